@@ -11,9 +11,15 @@
 // so parity with it is to tolerance only).  K is walked in chunks of 16: a lane loads four consecutive k of its
 // row (16 bytes) and the chunk's four MFMAs take k = 4g + j (g = lane / 16) -- a fixed permutation of the chunk,
 // so the summation order of an element is a function of K alone: row m never sees M, tiles or the launch.
-// This is a correctness path (fp32 matmuls are rare in the models the reference serves): operands are read
-// straight from global memory, 64x64 tile per work-group, 4 waves of 32x32.
+//
+// Bound: the fp32 matrix rate (154 TFLOP/s in a large product on this card) from about 64 rows on, the weight stream below.
+// A tile's operands go global -> LDS directly in slices of 32 k (128-byte rows, whole cache lines) through a ring of NS
+// slots; fragments are read one chunk ahead of the MFMAs and the one barrier of a slice sits between its two chunks, so
+// neither a memory round trip nor an LDS read is on the MFMA chain.  A wave's four MFMAs of an output tile and chunk are
+// 128 cycles of matrix work per two 16-byte reads: neither the LDS nor the L2 is near its limit with any tile.  What is
+// left is the barrier of a slice (a fifth of the time of a 64x64 tile); the tile is chosen for the grid (f32_pick).
 #include "common.h"
+#include "lds_direct.h"
 
 namespace tbik {
 
@@ -24,61 +30,106 @@ struct GemmF32Args {
   const float* bias;
   int64_t ldx, ldw, ldc;
   int M, N, K;
-  int T, flb, lb;  // leaves of 128, leaves per level-0 group, binary levels (TREE)
+  int flb, lb;     // leaves of 128 per level-0 group, binary levels (TREE)
+  int vec_store;
 };
 
 constexpr int F32_LBMAX = 8;
+constexpr int F32_SLICE = 32;   // k per ring slot: 128 bytes per row
 
-template <bool TREE>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmF32Args p) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int tiles_n = (p.N + 63) / 64;
-  const int m0 = (blockIdx.x / tiles_n) * 64 + wm * 32;
-  const int n0 = (blockIdx.x % tiles_n) * 64 + wn * 32;
+// WM x WN waves of TM x TN MFMA tiles (16x16) each; NS ring slots.
+template <int WM, int WN, int TM, int TN, int NS>
+struct F32Shape {
+  static constexpr int NWAVE = WM * WN, RX = WM * TM * 16, RW = WN * TN * 16;
+  static constexpr int NI = (RX + RW) / 8;      // direct loads (8 rows of 128 bytes each) per slice
+  static constexpr int PI = NI / NWAVE;         // ... of which each wave issues
+  static constexpr int STAGE = (RX + RW) * 128;
+  static_assert(NI % NWAVE == 0 && NS >= 4 && PI * (NS - 2) < 64 && NS * STAGE <= 160 * 1024, "ring");
+};
+
+template <int WM, int WN, int TM, int TN, int NS, bool TREE>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(const GemmF32Args p) {
+  typedef F32Shape<WM, WN, TM, TN, NS> S;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int tiles_m = (p.M + S::RX - 1) / S::RX;
+  const int tiles_n = (p.N + S::RW - 1) / S::RW;
+  // every XCD walks a contiguous range of tiles, eight rows of tiles at a time: neighbours share operand rows in its L2
+  const int lid = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  constexpr int GROUP = 8;
+  const int first_m = (lid / (GROUP * tiles_n)) * GROUP;
+  const int gsz = min(tiles_m - first_m, GROUP);
+  const int in_group = lid % (GROUP * tiles_n);
+  const int m0 = (first_m + in_group % gsz) * S::RX;
+  const int n0 = (in_group / gsz) * S::RW;
   const int r16 = lane & 15, g = lane >> 4;
 
-  const float* xp[2];
-  const float* wp[2];
+  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(p.X + (int64_t)m0 * p.ldx);
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.W + (int64_t)n0 * p.ldw);
+  // lane l of a load brings the 16-byte chunk that belongs at its linear place: row l / 8 of the eight, position l & 7,
+  // where row r keeps chunk c at position c ^ (r & 7) (sixteen lanes of a fragment read then cover all banks)
+  const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
+  uint32_t voff[S::PI];
 #pragma unroll
-  for (int a = 0; a < 2; a++) xp[a] = p.X + (int64_t)min(m0 + a * 16 + r16, p.M - 1) * p.ldx + 4 * g;
+  for (int i = 0; i < S::PI; i++) {
+    const int row = (wave * S::PI + i) * 8 + lrow;
+    if (row < S::RX) voff[i] = (uint32_t)((int64_t)(min(m0 + row, p.M - 1) - m0) * p.ldx * 4) + lchunk * 16;
+    else voff[i] = (uint32_t)((int64_t)(min(n0 + row - S::RX, p.N - 1) - n0) * p.ldw * 4) + lchunk * 16;
+  }
+  const int nchunks = p.K / 16;                // chunks of 16 k
+  const int nslices = (nchunks + 1) / 2;
+  // K may end in the middle of a slice: the lanes whose chunk lies behind it bring the first half again (never used)
+  const uint32_t tail_back = (nchunks & 1) && lchunk >= 4 ? 64u : 0u;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+  auto load_slice = [&](int s, int slot) __attribute__((always_inline)) {
+    const int sc = min(s, nslices - 1);        // slices past the end load the last one again: the count in flight stays
+    const uint32_t back = sc == nslices - 1 ? tail_back : 0u;
 #pragma unroll
-  for (int b = 0; b < 2; b++) wp[b] = p.W + (int64_t)min(n0 + b * 16 + r16, p.N - 1) * p.ldw + 4 * g;
+    for (int i = 0; i < S::PI; i++) {
+      const int q = wave * S::PI + i;
+      const uint8_t* b = (q < S::RX / 8 ? xbase : wbase) + (int64_t)sc * (F32_SLICE * 4);
+      dma16(lds0 + slot * S::STAGE + q * 1024, voff[i] - back, b);
+    }
+  };
+  const uint32_t frag = r16 * 128 + ((g ^ (r16 & 7)) << 4);
+  const uint32_t xfrag = frag + wm * TM * 2048, wfrag = frag + S::RX * 128 + wn * TN * 2048;
+  f32x4 fx[2][TM], fw[2][TN];
+  auto read_frags = [&](int buf, int slot, int c) __attribute__((always_inline)) {
+    const uint8_t* st = smem + slot * S::STAGE;
+#pragma unroll
+    for (int a = 0; a < TM; a++) fx[buf][a] = *reinterpret_cast<const f32x4*>(st + (xfrag ^ (c * 64)) + a * 2048);
+#pragma unroll
+    for (int b = 0; b < TN; b++) fw[buf][b] = *reinterpret_cast<const f32x4*>(st + (wfrag ^ (c * 64)) + b * 2048);
+  };
 
-  f32x4 acc[2][2];
-  f32x4 s0[2][2], sb[F32_LBMAX][2][2];
-  int c0 = 0, grp = 0;
+  f32x4 acc[TM][TN];
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int a = 0; a < TM; a++)
 #pragma unroll
-    for (int b = 0; b < 2; b++) acc[a][b] = zero;
+    for (int b = 0; b < TN; b++) acc[a][b] = zero;
+  auto multiply = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+      for (int a = 0; a < TM; a++)
+#pragma unroll
+        for (int b = 0; b < TN; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[buf][b][e], fx[buf][a][e], acc[a][b], 0, 0, 0);
+  };
 
-  const int nchunks = p.K / 16;
-  const int per_leaf = TREE ? 8 : nchunks;
-  const int nleaves = TREE ? p.T : 1;
-  int chunk = 0;
-  for (int j = 0; j < nleaves; j++) {
-    for (int i = 0; i < per_leaf; i++, chunk++) {
-      f32x4 fx[2], fw[2];
-#pragma unroll
-      for (int a = 0; a < 2; a++) fx[a] = *reinterpret_cast<const f32x4*>(xp[a] + (int64_t)chunk * 16);
-#pragma unroll
-      for (int b = 0; b < 2; b++) fw[b] = *reinterpret_cast<const f32x4*>(wp[b] + (int64_t)chunk * 16);
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-          for (int b = 0; b < 2; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[b][e], fx[a][e], acc[a][b], 0, 0, 0);
-    }
-    if (!TREE) break;
+  // merge state (TREE): running level-0 sum and the binary counter's levels, all in registers
+  constexpr int TA = TREE ? TM : 1, TB = TREE ? TN : 1;
+  f32x4 s0[TA][TB], sb[TREE ? F32_LBMAX : 1][TA][TB];
+  int c0 = 0, grp = 0;
+  auto merge_leaf = [&](bool last) __attribute__((always_inline)) {
     // leaf done: binary-counter merge in fp32 (all conditions are uniform over the block)
-    f32x4 t[2][2];
+    f32x4 t[TA][TB];
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < TA; a++)
 #pragma unroll
-      for (int b = 0; b < 2; b++) {
+      for (int b = 0; b < TB; b++) {
         t[a][b] = c0 != 0 ? s0[a][b] + acc[a][b] : acc[a][b];
         acc[a][b] = zero;
       }
@@ -91,45 +142,133 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmF32Args p) {
         if (!parked && l < p.lb) {
           if ((grp >> l) & 1) {
 #pragma unroll
-            for (int a = 0; a < 2; a++)
+            for (int a = 0; a < TA; a++)
 #pragma unroll
-              for (int b = 0; b < 2; b++) t[a][b] = sb[l][a][b] + t[a][b];
+              for (int b = 0; b < TB; b++) t[a][b] = sb[l][a][b] + t[a][b];
           } else {
 #pragma unroll
-            for (int a = 0; a < 2; a++)
+            for (int a = 0; a < TA; a++)
 #pragma unroll
-              for (int b = 0; b < 2; b++) sb[l][a][b] = t[a][b];
+              for (int b = 0; b < TB; b++) sb[l][a][b] = t[a][b];
             parked = true;
           }
         }
       }
       grp++;
-      if (j == nleaves - 1) {
+      if (last) {
 #pragma unroll
-        for (int a = 0; a < 2; a++)
+        for (int a = 0; a < TA; a++)
 #pragma unroll
-          for (int b = 0; b < 2; b++) acc[a][b] = t[a][b];  // the root
+          for (int b = 0; b < TB; b++) acc[a][b] = t[a][b];  // the root
       }
     } else {
 #pragma unroll
-      for (int a = 0; a < 2; a++)
+      for (int a = 0; a < TA; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++) s0[a][b] = t[a][b];
+        for (int b = 0; b < TB; b++) s0[a][b] = t[a][b];
     }
+  };
+
+  // prologue: NS - 1 slices in flight, slice 0 visible, its first fragments in registers
+#pragma unroll
+  for (int s = 0; s < NS - 1; s++) load_slice(s, s);
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(S::PI * (NS - 2)) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read_frags(0, 0, 0);
+  int slot = 0;
+  for (int s = 0; s < nslices; s++) {
+    const int next = slot + 1 == NS ? 0 : slot + 1;
+    const int prev = slot == 0 ? NS - 1 : slot - 1;
+    read_frags(1, slot, 1);
+    multiply(0);
+    // slice s + 1 has landed (this wave's share) and every fragment read of slice s is done; behind the barrier the slot
+    // of slice s - 1, which no wave reads any more, takes slice s + NS - 1
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(S::PI * (NS - 3)) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    load_slice(s + NS - 1, prev);
+    read_frags(0, next, 0);
+    if (2 * s + 1 < nchunks) multiply(1);
+    if (TREE && (s & 3) == 3) merge_leaf(s == nslices - 1);   // a leaf of 128 is four slices
+    slot = next;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // loads past the end of K have an address in this work-group's LDS
 
 #pragma unroll
-  for (int a = 0; a < 2; a++) {
-    const int m = m0 + a * 16 + r16;
+  for (int a = 0; a < TM; a++) {
+    const int m = m0 + (wm * TM + a) * 16 + r16;
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < TN; b++) {
+      const int n = n0 + (wn * TN + b) * 16 + 4 * g;
+      if (m >= p.M || n >= p.N) continue;
+      float* dst = p.C + (int64_t)m * p.ldc + n;
+      f32x4 v = acc[a][b];
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int n = n0 + b * 16 + 4 * g + e;
-        if (m < p.M && n < p.N) p.C[(int64_t)m * p.ldc + n] = acc[a][b][e] + (p.bias ? p.bias[n] : 0.f);
+      for (int e = 0; e < 4; e++) v[e] += p.bias && n + e < p.N ? p.bias[n + e] : 0.f;
+      if (p.vec_store && n + 3 < p.N) {
+        *reinterpret_cast<f32x4*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (n + e < p.N) dst[e] = v[e];
       }
     }
   }
+}
+
+template <int WM, int WN, int TM, int TN, int NS, bool TREE>
+static int f32_launch(const GemmF32Args& a, hipStream_t stream) {
+  typedef F32Shape<WM, WN, TM, TN, NS> S;
+  const int64_t tiles = (int64_t)((a.M + S::RX - 1) / S::RX) * ((a.N + S::RW - 1) / S::RW);
+  if (tiles > 0x7fffffff) return TBIK_ERR_INVALID;
+  const int64_t reach = 0xffffff00ll - 128;   // byte offsets inside a tile's operand rows are 32 bits
+  if (a.ldx * 4 * (S::RX - 1) > reach || a.ldw * 4 * (S::RW - 1) > reach) return TBIK_ERR_UNSUPPORTED;
+  static std::atomic<uint64_t> done{0};
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_f32_kernel<WM, WN, TM, TN, NS, TREE>), NS * S::STAGE, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL((gemm_f32_kernel<WM, WN, TM, TN, NS, TREE>), dim3((unsigned)tiles), dim3(64 * S::NWAVE), NS * S::STAGE, stream, a);
+  return hip_code(hipGetLastError());
+}
+
+// Which tile serves a call.  K cannot be cut (one accumulator, or one tree per element), so a call takes as many passes
+// over K as the fullest CU has tiles, and the tile whose passes add up to the least time wins.  Microseconds of a pass at
+// K = 4096 on MI355X, the first (launch and first loads included, 256 tiles) and each further one:
+//   mm    32x32, 4 waves 32 / 23.5   64x32, 4 waves 46.5 / 36.5   64x64, 16 waves 83 / 66.5   128x128, 8 waves 247 / 249
+//   tree  32x32, 4 waves 40 / 26     64x64, 16 waves 84 / 81
+// (matrix work alone: 13.7, 27.3, 54.6 and 218 us).  Several small waves per SIMD beat few large ones: 64x64 with four
+// waves of 32x32 takes 78 us for mm and 111 for the tree, whose merges then stand in the MFMAs' way.  Whole calls, before
+// (operands read straight from global memory, nothing prefetched) -> after: mm [256,4096]x[4096,4096] 136 -> 78 us,
+// [2048,4096]x[4096,6144] 1519 -> 745 (138 TFLOP/s), [16,4096]x[4096,4096] 114 -> 30; tree 139 -> 84, 1390 -> 969, 118 -> 38.
+struct F32Tile {
+  int rows, cols;
+  double first, next;
+};
+static int f32_pick(int M, int N, int K, bool tree) {
+  static const F32Tile mm[4] = {{32, 32, 32., 23.5}, {64, 32, 46.5, 36.5}, {64, 64, 83., 66.5}, {128, 128, 247., 249.}};
+  static const F32Tile tr[4] = {{32, 32, 40., 26.}, {64, 32, 1e9, 1e9}, {64, 64, 84., 81.}, {128, 128, 1e9, 1e9}};
+  int best = 0;
+  double best_t = 0.;
+  for (int c = 0; c < 4; c++) {
+    const F32Tile& t = tree ? tr[c] : mm[c];
+    const int64_t tiles = (((int64_t)M + t.rows - 1) / t.rows) * (((int64_t)N + t.cols - 1) / t.cols);
+    const double k = K / 4096.0;
+    const double us = 5.0 + (t.first - 5.0) * k + t.next * k * (double)((tiles + 255) / 256 - 1);
+    if (c == 0 || us < best_t) {
+      best_t = us;
+      best = c;
+    }
+  }
+  return best;
+}
+
+template <bool TREE>
+static int f32_run(const GemmF32Args& a, int cfg, hipStream_t stream) {
+  if (cfg == 0) return f32_launch<2, 2, 1, 1, 8, TREE>(a, stream);
+  if (cfg == 2 || TREE) return f32_launch<4, 4, 1, 1, 4, TREE>(a, stream);
+  if (cfg == 1) return f32_launch<2, 2, 2, 1, 6, false>(a, stream);
+  return f32_launch<2, 4, 4, 2, 4, false>(a, stream);
 }
 
 int gemm_f32_dispatch(bool tree, const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n, void* C,
@@ -143,22 +282,20 @@ int gemm_f32_dispatch(bool tree, const void* A, int64_t lda, const void* B, int6
   if (mis(A) || mis(B) || (lda & 3) || (ldb_n & 3) || (K & 15)) return TBIK_ERR_ALIGNMENT;
   if (reinterpret_cast<uintptr_t>(C) & 3) return TBIK_ERR_ALIGNMENT;
   GemmF32Args a{static_cast<const float*>(A), static_cast<const float*>(B), static_cast<float*>(C),
-                static_cast<const float*>(bias), lda, ldb_n, ldc, M, N, K, 0, 1, 0};
-  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-  if (tiles > 0x7fffffff) return TBIK_ERR_INVALID;
+                static_cast<const float*>(bias), lda, ldb_n, ldc, M, N, K, 1, 0, (ldc & 3) == 0 && !mis(C)};
   if (tree) {
     if (leaf_k != 128) return TBIK_ERR_UNSUPPORTED;
     int T, flb, level_k;
     if (tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return TBIK_ERR_INVALID;
     if (level_k - 1 > F32_LBMAX) return TBIK_ERR_UNSUPPORTED;
-    a.T = T;
     a.flb = flb;
     a.lb = level_k - 1;
-    hipLaunchKernelGGL(gemm_f32_kernel<true>, dim3((unsigned)tiles), dim3(256), 0, stream, a);
-  } else {
-    hipLaunchKernelGGL(gemm_f32_kernel<false>, dim3((unsigned)tiles), dim3(256), 0, stream, a);
   }
-  return hip_code(hipGetLastError());
+  // rows so far apart that a tile's rows do not fit 32-bit offsets go to the smallest tile, which reaches furthest
+  const int cfg = f32_pick(M, N, K, tree);
+  int rc = tree ? f32_run<true>(a, cfg, stream) : f32_run<false>(a, cfg, stream);
+  if (rc == TBIK_ERR_UNSUPPORTED && cfg != 0) rc = tree ? f32_run<true>(a, 0, stream) : f32_run<false>(a, 0, stream);
+  return rc;
 }
 
 }  // namespace tbik
