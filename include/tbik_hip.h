@@ -300,6 +300,19 @@ int bi_gemm_f32(const void* A, int64_t lda,
                 tbik_stream_t stream);
 
 /*
+ * Transposing copy of a row-major matrix of 2- or 4-byte elements: out[c, r] = x[r, c] for r < rows, zero for
+ * rows <= r < rows_out.  x [rows, cols] with row stride ldx, out [cols, rows_out] with row stride ldo (elements);
+ * out 16-byte aligned, ldo and rows_out multiples of 16 bytes, x aligned to its element.  It brings a matmul operand
+ * whose K runs across its rows (a row-major B, the left operand of a weight gradient) into the K-contiguous layout of
+ * the kernels above; K may be extended by zeros on the way (rows_out > rows), which does not change a sum over K.
+ * Replaces: the strided operand access of matmul_persistent, src/bio/batch_invariant_ops.py:175-196 (*a.stride(), *b.stride()).
+ */
+int bi_transpose(const void* x, int64_t ldx,
+                 void* out, int64_t ldo,
+                 int64_t rows, int64_t cols, int64_t rows_out, int elem_bytes,
+                 tbik_stream_t stream);
+
+/*
  * Gated activation in front of the row-split down projection:
  *   out[r, i] = bf16( bf16(silu(gate_up[r, i])) * gate_up[r, inter + i] ),  i < inter,  silu in fp32.
  * gate_up [rows, >= 2*inter] with row stride ld_in, out [rows, inter] with row stride ld_out (elements);

@@ -27,6 +27,8 @@ int qk_norm_rope_cache_dispatch(const void* qkv, int64_t ld, const void* q_weigh
                                 const float* inv_freq, const int64_t* positions, const int64_t* seq_of_token, void* q_out,
                                 void* k_cache, void* vt_cache, int64_t tokens, int q_heads, int kv_heads, int head_dim,
                                 int max_len, int batch, float eps, hipStream_t stream);
+int transpose_dispatch(const void* x, int64_t ldx, void* out, int64_t ldo, int64_t rows, int64_t cols, int64_t rows_out,
+                       int elem_bytes, hipStream_t stream);
 int silu_mul_dispatch(const void* gate_up, int64_t ld_in, void* out, int64_t ld_out, int64_t rows, int inter, bool f16,
                       hipStream_t stream);
 int rmsnorm_gemm_dispatch(const void* x, int64_t ldx, const void* res, int64_t ldr, const void* norm_w, float eps,
@@ -50,7 +52,7 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 extern "C" {
 
-int tbik_abi_version(void) { return 17; }
+int tbik_abi_version(void) { return 18; }
 
 const char* tbik_error_string(int code) {
   switch (code) {
@@ -208,6 +210,11 @@ int bi_gemm_f32(const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_
                 int N, int K, const void* bias_or_null, tbik_stream_t stream) {
   return tbik::gemm_f32_dispatch(false, A, lda, B, ldb_k, ldb_n, C, ldc, M, N, K, 0, bias_or_null,
                                  static_cast<hipStream_t>(stream));
+}
+
+int bi_transpose(const void* x, int64_t ldx, void* out, int64_t ldo, int64_t rows, int64_t cols, int64_t rows_out, int elem_bytes,
+                 tbik_stream_t stream) {
+  return tbik::transpose_dispatch(x, ldx, out, ldo, rows, cols, rows_out, elem_bytes, static_cast<hipStream_t>(stream));
 }
 
 int bi_silu_mul_bf16(const void* gate_up, int64_t ld_in, void* out, int64_t ld_out, int64_t rows, int inter,

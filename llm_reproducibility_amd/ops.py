@@ -49,11 +49,37 @@ def _is_f16(*tensors) -> bool:
     return dts == {torch.float16}
 
 
+def _k_across(t: torch.Tensor) -> bool:
+    """True for a matrix whose columns are contiguous and whose rows are not: the transposed view of a row-major one."""
+    return t.stride(0) == 1 and t.stride(1) != 1 and t.shape[0] > 1 and t.shape[1] > 1 and t.stride(1) >= t.shape[0]
+
+
+def _transposed(t: torch.Tensor, k: int):
+    """(copy of the `_k_across` matrix t with contiguous rows, its leading dimension): one pass of the transposing copy
+    kernel, the rows extended by zeros to k elements (a multiple of 16 bytes).  4.2 - 5.0 TB/s, where the library's
+    strided copy moves 1 TB/s in 16 bits and 2 in 32 ([12288,4096] bf16: 45 us against 196)."""
+    R, C = t.shape
+    out = torch.empty((R, k), device=t.device, dtype=t.dtype)
+    rc = _lib.lib().bi_transpose(t.data_ptr(), t.stride(1), out.data_ptr(), k, C, R, k, t.element_size(), _stream(t))
+    _lib.check(rc, "bi_transpose")
+    return out, k
+
+
+def _k_rows(t: torch.Tensor, k: int):
+    """(tensor, leading dimension) of t with contiguous rows, extended by zero columns to k."""
+    if _k_across(t):
+        return _transposed(t, k)
+    p = torch.nn.functional.pad(t, (0, k - t.shape[1]))
+    return p, p.stride(0)
+
+
 def _rows_f32(t: torch.Tensor):
     """fp32 operand with a contiguous last dim, 16-byte aligned rows (leading dimension a multiple of 4)."""
     ok = t.stride(1) == 1 and _aligned16(t) and (t.shape[0] == 1 or (t.stride(0) >= t.shape[1] and t.stride(0) % 4 == 0))
     if ok:
         return t, (t.shape[1] if t.shape[0] == 1 else t.stride(0))
+    if _k_across(t):
+        return _transposed(t, (t.shape[1] + 3) // 4 * 4)
     c = t.contiguous()
     if not _aligned16(c) or c.shape[1] % 4 != 0:
         c = torch.nn.functional.pad(c, (0, (-c.shape[1]) % 4))[:, : t.shape[1]] if c.shape[1] % 4 else c.clone()
@@ -64,12 +90,12 @@ def _gemm_f32(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor], le
     M, K = A.shape
     N = B.shape[1]
     if K % 16 != 0:  # only the single-accumulator form gets here: zero columns do not change a sequential sum
-        pad = (-K) % 16
-        A = torch.nn.functional.pad(A, (0, pad))
-        B = torch.nn.functional.pad(B, (0, 0, 0, pad))
-        K += pad
-    a, lda = _rows_f32(A)
-    w, ldw = _rows_f32(B.t())
+        K += (-K) % 16
+        a, lda = _k_rows(A, K)
+        w, ldw = _k_rows(B.t(), K)
+    else:
+        a, lda = _rows_f32(A)
+        w, ldw = _rows_f32(B.t())
     b = None if bias is None else bias.contiguous()
     C = torch.empty((M, N), device=A.device, dtype=torch.float32)
     L = _lib.lib()
@@ -90,36 +116,47 @@ def _rows16(t: torch.Tensor):
         return t, t.shape[1]
     if ok and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0:
         return t, t.stride(0)
+    if _k_across(t):
+        return _transposed(t, (t.shape[1] + 7) // 8 * 8)
     c = t.contiguous()
     if not _aligned16(c):
         c = c.clone()
     return c, c.shape[1]
 
 
-# Rows from which a row-major [K,N] operand is repacked into the native [N,K] layout instead of being consumed in
-# place.  In place it runs on the 64-row tiled kernels only (the pipelines with 128x256 tiles are built for [N,K]), so
-# the time grows with the rows; a repack costs one transposing copy of B (60 us for 4096 x 4096, 180 us for
-# 12288 x 4096 with the library's copy kernel) and then the fast kernels.  Measured on MI355X, bf16, B of 4096 x 4096 /
-# 12288 x 4096 / 4096 x 12288: the tree matmul in place wins up to 512 rows (74 / 199 / 197 us against 93 / 244 / 256)
-# and loses from 1024 on (133 / 382 / 393 against 110 / 305 / 303; at 4096 rows 523 / 1523 / 1567 against 205 / 594 /
-# 622); the single-accumulator mm, which cannot cut K, wins up to 1024 rows and loses from 2048 on (148 / 416 / 437
-# against 120 / 335 / 332).  Same bits either way.
-_REPACK_ROWS_TREE = 1024
-_REPACK_ROWS_MM = 2048
+# Where a row-major [K,N] operand is repacked into the native [N,K] layout instead of being consumed in place.  In place
+# it runs on the 64-row tiled kernels only (the other pipelines are built for [N,K]); a repack is one pass of the
+# transposing copy kernel (23 us for 4096 x 4096 in 16 bits, 45 us for 12288 x 4096) and then whatever kernel is best.
+# Measured on MI355X, bf16, us in place against repacked, same bits either way:
+#   tree matmul: in place cuts K and holds out until its 64-row tiles fill a second round of the chip, that is up to 128
+#     rows (12288 x 4096: 68 against 73; at 192 rows 99 against 79, at 1024 448 against 164), later for small matrices
+#     (2048 x 2048: 256 rows 17 against 24, 384 rows 28 against 22): a bound on rows * K * N.
+#   single-accumulator mm: in place cannot cut K, and every narrow matrix is a long chain on few work-groups (4096 x 4096:
+#     76 against 23 at one row, 69 against 30 at 64 rows).  Wide ones fill the chip and the copy costs more than it gives
+#     up to 128 rows (4096 x 24576: 70 against 112 at 64 rows, 78 against 134 at 128, 143 against 140 at 256).
+_REPACK_ROWS_TREE = 416      # for a matrix of 2048 x 1536, inversely to its size, but at least 129
+_REPACK_ROWS_MM = 1          # for matrices of fewer than _WIDE_N columns
+_REPACK_ROWS_MM_WIDE = 160
+_WIDE_N = 16384
+
+
+def _consumed_in_place(rows: int, K: int, N: int, tree: bool) -> bool:
+    if tree:
+        return rows <= 128 or rows * K * N < _REPACK_ROWS_TREE * (2048 * 1536)
+    return rows < (_REPACK_ROWS_MM_WIDE if N >= _WIDE_N else _REPACK_ROWS_MM)
 
 
 def _weight_operand(B: torch.Tensor, rows: int = 0, tree: bool = True):
     """How a [K,N] operand is handed to the kernels: (tensor whose data_ptr is passed, ldb_k, ldb_n).
 
     `weight.t()` of an nn.Linear weight ([N,K], K contiguous) is the native layout (ldb_k = 1), used without a copy; a
-    row-major [K,N] operand (N contiguous: a plain `x @ B`) is consumed in place too (ldb_n = 1) unless the product has
-    so many rows (`rows`) that a repack into the native layout pays.  Anything else -- neither dimension contiguous,
-    rows not 16-byte aligned -- is repacked as well."""
+    row-major [K,N] operand (N contiguous: a plain `x @ B`) is consumed in place too (ldb_n = 1) unless a repack into
+    the native layout pays for this many `rows`.  Anything else -- neither dimension contiguous, rows not 16-byte
+    aligned -- is repacked as well."""
     K, N = B.shape
     if B.stride(0) == 1 and _aligned16(B) and K % 8 == 0 and (N == 1 or (B.stride(1) >= K and B.stride(1) % 8 == 0)):
         return B, 1, (K if N == 1 else B.stride(1))
-    in_place = rows < (_REPACK_ROWS_TREE if tree else _REPACK_ROWS_MM)
-    if in_place and B.stride(1) == 1 and _aligned16(B) and B.stride(0) >= N and B.stride(0) % 8 == 0:
+    if (B.stride(1) == 1 and _aligned16(B) and B.stride(0) >= N and B.stride(0) % 8 == 0 and _consumed_in_place(rows, K, N, tree)):
         return B, B.stride(0), 1
     w, ldw = _rows16(B.t())
     return w, 1, ldw
@@ -206,18 +243,22 @@ def _bi_gemm_impl(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]
         return _gemm_f32(A, B, bias, 0, False)
     M, K = A.shape
     N = B.shape[1]
-    if K % 8 != 0:
-        # zero columns do not change a sequential fp32 accumulation
-        pad = (-K) % 8
-        A = torch.nn.functional.pad(A, (0, pad))
-        B = torch.nn.functional.pad(B, (0, 0, 0, pad))
-        K += pad
-    a, lda = _rows16(A)
-    w, ldb_k, ldb_n = _weight_operand(B, M, False)
+    f16 = _is_f16(A, B, bias)
+    if K % 8 != 0 or (K % 64 != 0 and _k_across(A) and _k_across(B.t())):
+        # zero columns do not change a sequential fp32 accumulation.  A K that no kernel takes is extended, and so is one
+        # that only the small-tile kernel takes when both operands are copied anyway (a weight gradient, whose K is
+        # the number of tokens): to whole slices of 64, which every kernel takes
+        K += (-K) % 64
+        a, lda = _k_rows(A, K)
+        w, ldb_n = _k_rows(B.t(), K)
+        ldb_k = 1
+    else:
+        a, lda = _rows16(A)
+        w, ldb_k, ldb_n = _weight_operand(B, M, False)
     b = None if bias is None else bias.contiguous()
     C = torch.empty((M, N), device=A.device, dtype=A.dtype)
     L = _lib.lib()
-    rc = (L.bi_gemm_f16 if _is_f16(A, B, bias) else L.bi_gemm_bf16)(a.data_ptr(), lda, w.data_ptr(), ldb_k, ldb_n, C.data_ptr(), C.stride(0),
+    rc = (L.bi_gemm_f16 if f16 else L.bi_gemm_bf16)(a.data_ptr(), lda, w.data_ptr(), ldb_k, ldb_n, C.data_ptr(), C.stride(0),
                                  M, N, K, None if b is None else b.data_ptr(), _stream(A))
     _lib.check(rc, "bi_gemm")
     return C
