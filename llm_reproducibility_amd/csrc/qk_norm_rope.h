@@ -10,8 +10,17 @@
 
 namespace tbik {
 
-__device__ __forceinline__ uint32_t qk_norm_rope_head(uint16_t r1, uint16_t r2, const uint16_t* w, int64_t pos,
-                                                      const float* inv_freq, float eps, int lane) {
+// The rotation of the pair (l, l + 64) at position `pos`: one per token, whatever the head.
+struct RopeFactors {
+  float c, s;
+  __device__ __forceinline__ RopeFactors(int64_t pos, const float* inv_freq, int lane) {
+#pragma clang fp contract(off)
+    const float ang = (float)pos * inv_freq[lane];
+    c = cosf(ang), s = sinf(ang);
+  }
+};
+
+__device__ __forceinline__ uint32_t qk_norm_rope_head(uint16_t r1, uint16_t r2, float w1, float w2, const RopeFactors& rope, float eps) {
   // every product and sum is rounded on its own, except where a fused multiply-add is written out: left to the
   // compiler, a multiplication could be fused with the next addition in one kernel and not in the other
 #pragma clang fp contract(off)
@@ -19,11 +28,15 @@ __device__ __forceinline__ uint32_t qk_norm_rope_head(uint16_t r1, uint16_t r2, 
   const float ss = wave_sum(__builtin_fmaf(x1, x1, x2 * x2));
   const float rs = 1.0f / sqrtf(ss * (1.0f / 128.0f) + eps);
   const uint32_t nrm = pack_bf16x2(x1 * rs, x2 * rs);
-  const uint32_t wv = pack_bf16x2(bf16_lo(nrm) * bf16_bits_to_f32(w[lane]), bf16_hi(nrm) * bf16_bits_to_f32(w[lane + 64]));
+  const uint32_t wv = pack_bf16x2(bf16_lo(nrm) * w1, bf16_hi(nrm) * w2);
   const float y1 = bf16_lo(wv), y2 = bf16_hi(wv);
-  const float ang = (float)pos * inv_freq[lane];
-  const float c = cosf(ang), s = sinf(ang);
-  return pack_bf16x2(y1 * c - y2 * s, y2 * c + y1 * s);
+  return pack_bf16x2(y1 * rope.c - y2 * rope.s, y2 * rope.c + y1 * rope.s);
+}
+
+__device__ __forceinline__ uint32_t qk_norm_rope_head(uint16_t r1, uint16_t r2, const uint16_t* w, int64_t pos,
+                                                      const float* inv_freq, float eps, int lane) {
+  const float w1 = bf16_bits_to_f32(w[lane]), w2 = bf16_bits_to_f32(w[lane + 64]);
+  return qk_norm_rope_head(r1, r2, w1, w2, RopeFactors(pos, inv_freq, lane), eps);
 }
 
 }  // namespace tbik
