@@ -231,6 +231,22 @@ int bi_attention_bf16(const void* q, const void* k_cache, const void* vt_cache, 
                       float scale, tbik_stream_t stream);
 
 /*
+ * bi_attention_bf16 with scratch memory, for calls with a few new queries per sequence against long caches: the chunks of
+ * 512 keys of a (sequence, KV head) are then shared by several work-groups and a second launch merges them in the order
+ * in which a single work-group would -- the same bits.  bi_attention_workspace_bytes(...) says how much scratch such a call
+ * uses (0: the call gains nothing, pass NULL); with less than that, or NULL, the call runs as bi_attention_bf16.
+ * The scratch (16-byte aligned) need not be initialised and must not be shared by calls that overlap.
+ * max_q_len = 1 gives the size for bi_attention_decode_qkv_ws_bf16.
+ * Replaces: as bi_attention_bf16 (the reference's alignment mode forces the kernel without such a split, because its merge
+ *           order would depend on the split: src/patch/patch_training_inference_align.py:548-561; here the chunks are fixed).
+ */
+size_t bi_attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len);
+int bi_attention_ws_bf16(const void* q, const void* k_cache, const void* vt_cache, void* out,
+                         const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
+                         int batch, int max_q_len, int q_heads, int kv_heads, int head_dim, int max_len,
+                         float scale, void* workspace_or_null, size_t workspace_bytes, tbik_stream_t stream);
+
+/*
  * fp16 counterparts of tbik_gemm_bf16 / tbik_gemm_workspace_bytes / tbik_tree_combine_bf16 / bi_gemm_bf16: same
  * arguments and contract, elements are IEEE half, leaves are chains of v_mfma_f32_16x16x32_f16 rounded once to
  * fp16, every tree node is one fp16 addition (round to nearest even).
@@ -362,6 +378,14 @@ int bi_attention_decode_qkv_bf16(const void* qkv, int64_t ld,
                                  const int32_t* ctx_len,
                                  int batch, int q_heads, int kv_heads, int head_dim, int max_len,
                                  float scale, float eps, tbik_stream_t stream);
+/* the same with scratch memory: see bi_attention_ws_bf16 */
+int bi_attention_decode_qkv_ws_bf16(const void* qkv, int64_t ld,
+                                    const void* q_weight, const void* k_weight, const float* inv_freq,
+                                    void* k_cache, void* vt_cache, void* out,
+                                    const int32_t* ctx_len,
+                                    int batch, int q_heads, int kv_heads, int head_dim, int max_len,
+                                    float scale, float eps, void* workspace_or_null, size_t workspace_bytes,
+                                    tbik_stream_t stream);
 
 /*
  * Greedy sampling: out[r] (int64) = index of the largest element of row r of x [rows, cols] (bf16, row stride ld

@@ -28,7 +28,7 @@ EXPORTS = (
     "tbik_gemm_bf16_static", "bi_log_softmax", "tbik_gemm_workspace_bytes_rowmajor_b", "tbik_gemm_plan_info",
     "bi_rmsnorm_gemm_bf16", "tbik_gemm_silu_mul_bf16", "bi_argmax_advance_bf16",
     "tbik_gemm_rmsnorm_bf16", "tbik_tree_combine_rmsnorm_bf16", "bi_attention_decode_qkv_bf16", "bi_gemm_silu_mul_bf16",
-    "bi_transpose",
+    "bi_transpose", "bi_attention_workspace_bytes", "bi_attention_ws_bf16", "bi_attention_decode_qkv_ws_bf16",
 )
 
 _lib = None
@@ -125,6 +125,12 @@ def lib() -> ctypes.CDLL:
     L.tbik_gemm_silu_mul_bf16.restype = i32
     L.bi_attention_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, f32, vp]
     L.bi_attention_bf16.restype = i32
+    L.bi_attention_workspace_bytes.argtypes = [i32, i32, i32, i32, i32]
+    L.bi_attention_workspace_bytes.restype = sz
+    L.bi_attention_ws_bf16.argtypes = L.bi_attention_bf16.argtypes[:-1] + [vp, sz, vp]
+    L.bi_attention_ws_bf16.restype = i32
+    L.bi_attention_decode_qkv_ws_bf16.argtypes = L.bi_attention_decode_qkv_bf16.argtypes[:-1] + [vp, sz, vp]
+    L.bi_attention_decode_qkv_ws_bf16.restype = i32
     if L.tbik_abi_version() != ABI_VERSION:
         raise RuntimeError(f"{LIB_PATH}: ABI version {L.tbik_abi_version()} does not match this package ({ABI_VERSION})")
     _lib = L

@@ -12,11 +12,14 @@
 // keys in tiles of 32, online softmax, no split over the key axis, the same kernel for prefill and decode).
 //
 // Invariance argument: a query row is owned by the four lanes {j, j+16, j+32, j+48}; its scores, its
-// running maximum / denominator and its output accumulators never mix with another row's.  Keys are
-// visited in ascending tiles of 32 whatever the batch or the block looks like; a tile that lies entirely
-// behind a row's causal horizon contributes exp(-inf) = 0 and a rescale by exactly 1.0, so the number of
-// tiles the BLOCK walks does not change the row.  Prefill (16 rows per block) and decode (1 valid row)
-// therefore produce the same bits for the same token, and heads can be sharded freely.
+// running maximum / denominator and its output accumulators never mix with another row's.  The keys are cut into
+// chunks of 512 at fixed positions.  Inside a chunk they are visited in ascending tiles of 32, starting from an empty
+// state (reference point, denominator, accumulators), whatever the batch or the block looks like; a tile that lies
+// entirely behind a row's causal horizon contributes exp(-inf) = 0 and a rescale by exactly 1.0, so the number of
+// tiles the BLOCK walks does not change the row.  The chunks' states are merged in ascending order (merge_chunk),
+// those behind a row's horizon left out.  Prefill (16 rows per block) and decode (1 valid row)
+// therefore produce the same bits for the same token, and heads can be sharded freely; and because no chunk waits for
+// another, a few sequences with long contexts spread their chunks over the chip.
 //
 // Layouts: q/out [tokens, q_heads, 128]; K cache [batch, kv_heads, max_len, 128]; V cache TRANSPOSED
 // [batch, kv_heads, 128, max_len] so that the P*V MFMA operand (8 consecutive keys of one channel) is a
@@ -40,6 +43,17 @@ struct AttnArgs {
 };
 
 constexpr int HD = 128;
+constexpr int CHUNK_TILES = 16;           // key tiles per chunk: 512 keys
+constexpr float kNoKey = -3e38f;          // reference point of an empty state: below every score, finite (see softmax_tile)
+
+// Where the chunks of a row go when different work-groups compute them (SPLIT): slot (sequence * max_q_len + query) *
+// q_heads + head of [nchunks] states.
+struct SplitArgs {
+  float* o;      // [slot][nchunks][128] accumulators
+  float* ml;     // [slot][nchunks][2] reference point, denominator
+  int nchunks;   // chunks of the cache length
+  int max_q_len;
+};
 
 // The decode kernel that forms its own queries and the new key/value (FUSED): sequence b's one new token is row b of the
 // fused qkv projection output, at position ctx_len[b] - 1.
@@ -89,7 +103,8 @@ __device__ __forceinline__ void softmax_tile(const f32x4 (&s)[2], int k0, int g,
   // probability, and out = o / l is the same quotient).  After the first tiles of a row it practically never moves, so
   // the rescale of the output accumulators is skipped for whole rows of tiles.  The rule looks at a row's own scores
   // in its fixed tile order only, so it is the same for prefill, chunked prefill and decode.
-  // Key 0 is visible to every query: the reference point is finite from tile 0 on.
+  // A row's first key of a chunk moves it from kNoKey to a score; in a tile that lies entirely behind the horizon it stays
+  // where it is (kNoKey is finite, so kNoKey - kNoKey is 0 and not NaN) and every probability is 2^-inf = 0.
   constexpr float kLazy = 8.0f;
   const float cand = tmax * scale_log2;
   const float m_new = cand > m + kLazy ? cand : m;
@@ -107,6 +122,21 @@ __device__ __forceinline__ void softmax_tile(const f32x4 (&s)[2], int k0, int g,
   // P as the MFMA "B" operand: k slots 0..3 = keys k0+4g.., slots 4..7 = keys k0+16+4g..
   p = __builtin_bit_cast(bf16x8, u32x4{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3]), pack_bf16x2(pv[4], pv[5]),
                                        pack_bf16x2(pv[6], pv[7])});
+}
+
+// The merge of a row's next chunk (m, l, and below each accumulator) into its state so far (M, L): both are brought to the
+// larger reference point, rounded as written in every kernel (no contraction).
+__device__ __forceinline__ void merge_chunk(float& M, float& L, float m, float l, float& fa, float& fb) {
+#pragma clang fp contract(off)
+  const float top = LaneMaxNaN::f(M, m);
+  fa = __builtin_amdgcn_exp2f(M - top);
+  fb = __builtin_amdgcn_exp2f(m - top);
+  M = top;
+  L = __builtin_fmaf(L, fa, l * fb);
+}
+__device__ __forceinline__ float merge_acc(float O, float fa, float o, float fb) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(O, fa, o * fb);
 }
 
 __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
@@ -137,12 +167,33 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
   f32x4 o[8];  // output accumulators, transposed: lane (j, g) holds out[j][16t + 4g .. +3] for the channel tiles t
 #pragma unroll
   for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY;  // reference point of the exponentials (base-2 domain; a lazily updated running maximum), identical in the four lanes of a row
+  float m = kNoKey;     // reference point of the exponentials (base-2 domain; a lazily updated running maximum), identical in the four lanes of a row
   float l = 0.f;        // running denominator
+  f32x4 ot[8];          // the merged chunks so far
+  float mt = 0.f, lt = 0.f;
+  // chunk `c` is complete: merged into the rows that see it, and an empty state for the next
+  auto end_chunk = [&](int c) {
+    if (c == 0) {
+      mt = m, lt = l;
+#pragma unroll
+      for (int t = 0; t < 8; t++) ot[t] = o[t];
+    } else if (qpos >= c * CHUNK_TILES * 32) {
+      float fa, fb;
+      merge_chunk(mt, lt, m, l, fa, fb);
+#pragma unroll
+      for (int t = 0; t < 8; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) ot[t][i] = merge_acc(ot[t][i], fa, o[t][i], fb);
+    }
+    m = kNoKey, l = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
 
   const int ntiles = last_pos / 32 + 1;
   for (int tile = 0; tile < ntiles; tile++) {
     const int k0 = tile * 32;
+    if (tile != 0 && tile % CHUNK_TILES == 0) end_chunk(tile / CHUNK_TILES - 1);
     // ---- scores: two 16-key sub-tiles; lane (j, g) receives keys k0 + 16u + 4g + i of query j
     f32x4 s[2];
 #pragma unroll
@@ -173,13 +224,14 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
       o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, scaled, 0, 0, 0);
     }
   }
+  end_chunk((ntiles - 1) / CHUNK_TILES);
   if (!qvalid) return;
-  const float inv = 1.0f / l;
+  const float inv = 1.0f / lt;
   uint16_t* op = a.out + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
 #pragma unroll
   for (int t = 0; t < 8; t++) {
-    const uint32_t lo = pack_bf16x2(o[t][0] * inv, o[t][1] * inv);
-    const uint32_t hi = pack_bf16x2(o[t][2] * inv, o[t][3] * inv);
+    const uint32_t lo = pack_bf16x2(ot[t][0] * inv, ot[t][1] * inv);
+    const uint32_t hi = pack_bf16x2(ot[t][2] * inv, ot[t][3] * inv);
     *reinterpret_cast<uint2*>(op + 16 * t + 4 * g) = make_uint2(lo, hi);
   }
 }
@@ -195,9 +247,15 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
 // NLD > 0: that many more wavefronts in the work-group do all the staging (loads, LDS writes) at the same barriers and
 // the G computing waves none of it: for launches that leave the chip short of work-groups, where a work-group's time is
 // its own chain of tiles rather than its share of a CU.
+// SPLIT: a work-group takes one chunk of the keys (blockIdx.z) and leaves its state in the workspace for
+// attention_merge_kernel: a few new tokens against a long cache are a handful of work-groups otherwise
+// (55 tokens at 8192 keys 133 -> 24 us, 16 tokens of two sequences at 16384 keys 227 -> 30).
 // ------------------------------------------------------------------------------------------------
-template <int G, bool DEEP, int NLD = 0>
-__global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const AttnArgs a) {
+// chunks: the cache has a single one / a work-group walks them all / a work-group takes one (SPLIT)
+enum { ONE_CHUNK, ALL_CHUNKS, SPLIT_CHUNKS };
+template <int G, bool DEEP, int NLD, int CHUNKS>
+__global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
+  constexpr bool SPLIT = CHUNKS == SPLIT_CHUNKS;
   __shared__ __attribute__((aligned(16))) uint8_t lds[2][16384];  // per buffer: K tile [32][128] (8 KiB), V^T tile [128][32] (8 KiB)
   const int b = blockIdx.y;
   // Work-groups are dealt to the eight XCDs round robin, each with an L2 of its own: with the KV head as the fastest
@@ -286,15 +344,18 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
     }
   };
 
-  const int ntiles = last_pos / 32 + 1;
+  // the tiles of this work-group: all of them, or (SPLIT) those of chunk blockIdx.z
+  const int tile0 = SPLIT ? (int)blockIdx.z * CHUNK_TILES : 0;
+  const int ntiles = SPLIT ? min(last_pos / 32 + 1, tile0 + CHUNK_TILES) : last_pos / 32 + 1;
+  if (SPLIT && tile0 >= ntiles) return;  // uniform over the work-group
   constexpr int UNROLL = DEPTH < 2 ? 2 : DEPTH;
   if (NLD && stid >= 0) {
     // ---- loader waves: the staging half of the loop below, at the same barriers
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_tile(d, d);
+    for (int d = 0; d < DEPTH; d++) load_tile(tile0 + d, d);
     store_tile(0, 0);
     __syncthreads();
-    for (int t0 = 0; t0 < ntiles; t0 += UNROLL) {
+    for (int t0 = tile0; t0 < ntiles; t0 += UNROLL) {
 #pragma unroll
       for (int d = 0; d < UNROLL; d++) {
         const int tile = t0 + d;
@@ -314,8 +375,39 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
   f32x4 o[8];
 #pragma unroll
   for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY;
+  float m = kNoKey;
   float l = 0.f;
+  // The merged chunks so far.  (They cost the full chip a wavefront per SIMD, three instead of four, and 7 % at 4096 keys;
+  // parked in scratch memory instead they cost 25 %: 557 MB of it for a prompt of 4096.)
+  f32x4 ot[8];
+  float mt = 0.f, lt = 0.f;
+  // chunk `c` is complete: merged into the rows that see it; after the last one the result stays in m, l and o,
+  // otherwise an empty state follows
+  auto end_chunk = [&](int c, bool last) __attribute__((always_inline)) {
+    if (c != 0) {
+      if (qpos >= c * CHUNK_TILES * 32) {
+        float fa, fb;
+        merge_chunk(mt, lt, m, l, fa, fb);
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) ot[t][i] = merge_acc(ot[t][i], fa, o[t][i], fb);
+      }
+    } else {
+      mt = m, lt = l;
+#pragma unroll
+      for (int t = 0; t < 8; t++) ot[t] = o[t];
+    }
+    if (last) {
+      l = lt;
+#pragma unroll
+      for (int t = 0; t < 8; t++) o[t] = ot[t];
+    } else {
+      m = kNoKey, l = 0.f;
+#pragma unroll
+      for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
 
   // LDS offsets of this lane's fragments inside a tile buffer, formed once: key row 16u + j of the K tile (256 bytes a
   // row, 16-byte chunk c*4 + g swizzled by the row; u adds 4096), channel row 16t + j of the V^T tile (64 bytes a row,
@@ -329,17 +421,20 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
   // number of loads in flight static, so the waits below can leave the newer tiles in flight
   if (!NLD) {
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_tile(d, d);
+    for (int d = 0; d < DEPTH; d++) load_tile(tile0 + d, d);
     store_tile(0, 0);
   }
   __syncthreads();
   // the loop body covers UNROLL (an even number of) tiles, so that the LDS buffer of each is a compile-time constant and
   // every LDS address is a per-thread offset plus an immediate
-  for (int t0 = 0; t0 < ntiles; t0 += UNROLL) {
+  static_assert(CHUNK_TILES % UNROLL == 0, "a chunk is a whole number of loop bodies");
+  for (int c0 = tile0; c0 < ntiles; c0 += CHUNK_TILES) {
+  const int ce = min(c0 + CHUNK_TILES, ntiles);
+  for (int t0 = c0; t0 < ce; t0 += UNROLL) {
 #pragma unroll
    for (int d = 0; d < UNROLL; d++) {
     const int tile = t0 + d;
-    if (tile >= ntiles) break;
+    if (tile >= ce) break;
     const int cur = d & 1;
     if (!NLD) load_tile(tile + DEPTH, d % DEPTH);  // that set held this tile and went to LDS a tile ago
     const int k0 = tile * 32;
@@ -378,7 +473,17 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
     __syncthreads();
    }
   }
+  if (CHUNKS == ALL_CHUNKS && ntiles > CHUNK_TILES) end_chunk(c0 / CHUNK_TILES, ce == ntiles);
+  }
   if (!qvalid) return;
+  if (SPLIT && qpos >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete here)
+    const int64_t at = ((int64_t)(b * sp.max_q_len + qrow) * a.q_heads + h) * sp.nchunks + blockIdx.z;
+#pragma unroll
+    for (int t = 0; t < 8; t++) *reinterpret_cast<f32x4*>(sp.o + at * HD + 16 * t + 4 * g) = o[t];
+    if (g == 0) *reinterpret_cast<f32x2*>(sp.ml + at * 2) = f32x2{m, l};
+    return;
+  }
+  if (SPLIT && blockIdx.z != 0) return;
   const float inv = 1.0f / l;
   uint16_t* op = a.out + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
 #pragma unroll
@@ -413,10 +518,14 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
 // and all eight waves meet at the barrier.  Tiles behind the last one are clamped to the last tile of the cache and
 // never used, so the number of loads in flight is static; nothing is in flight when a wave ends.
 // A row's arithmetic -- the lanes that own it, the MFMA chains over channels and key slots, the order of the softmax
-// updates -- is that of the kernels above: the same bits.
+// updates and of the chunks -- is that of the kernels above: the same bits.
+// SPLIT: gridDim.z work-groups per (KV head, sequence); work-group z takes the chunks z, z + gridDim.z, ... as one stream of
+// tiles and leaves each chunk's state in the workspace for attention_merge_kernel.  One work-group per (KV head,
+// sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8200 keys 113 us, with
+// the chunks spread over the chip 67 us (62 and the merge; the keys and values take 36 at the rate of a one-pass read).
 // ------------------------------------------------------------------------------------------------
-template <int G, bool FUSED>
-__global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a, const QkvArgs f) {
+template <int G, bool FUSED, bool SPLIT>
+__global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a, const QkvArgs f, const SplitArgs sp) {
   constexpr int NS = 4;               // ring slots per operand (2 x 4 x 8 KiB of LDS)
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_dyn[];
   uint8_t (*lds_k)[8192] = reinterpret_cast<uint8_t (*)[8192]>(lds_dyn);
@@ -427,6 +536,17 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   constexpr int PI = 8 / NL;          // load instructions per tile, operand and loader wave
   const int b = blockIdx.y;
   const int kvh = blockIdx.x;
+  const int z = SPLIT ? blockIdx.z : 0, nz = SPLIT ? gridDim.z : 1;
+  // tile i of this work-group's stream, and how many there are of ntiles in all
+  auto tile_of = [&](int i) __attribute__((always_inline)) {
+    return SPLIT ? (i / CHUNK_TILES * nz + z) * CHUNK_TILES + i % CHUNK_TILES : i;
+  };
+  auto tiles_here = [&](int ntiles) __attribute__((always_inline)) {
+    if (!SPLIT) return ntiles;
+    const int nch = (ntiles + CHUNK_TILES - 1) / CHUNK_TILES;
+    if (z >= nch) return 0;
+    return (nch - z + nz - 1) / nz * CHUNK_TILES - ((nch - 1) % nz == z ? nch * CHUNK_TILES - ntiles : 0);
+  };
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -460,11 +580,11 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
 #pragma unroll
       for (int i = 0; i < PI; i++) dma16(lv + slot * 8192 + i * 1024, vvoff[i], src);
     };
-    load_k(0, 0);
+    load_k(tile_of(0), 0);
 #pragma unroll
     for (int i = 0; i < NS - 1; i++) {
-      load_k(i + 1, i + 1);
-      load_v(i, i);
+      load_k(tile_of(i + 1), i + 1);
+      load_v(tile_of(i), i);
     }
     const int ctx = a.ctx_len[b];
     const int qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
@@ -473,12 +593,17 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       return;
     }
     const int last_pos = ctx - qlen + min(QMAX - 1, qlen - 1);
-    const int ntiles = last_pos / 32 + 1;
+    const int ntiles = tiles_here(last_pos / 32 + 1);
+    if (SPLIT && ntiles == 0) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      return;
+    }
     if (FUSED) {
       // loaders 0 and 1 form the new key and file the new value while the first tiles are on their way (the computing
       // waves form the query heads meanwhile); everything they have in flight is drained before the barrier, so the waits
       // below still count the tile loads alone
-      if (li < 2) {
+      // (SPLIT: the work-group that has the position's chunk)
+      if (li < 2 && (!SPLIT || ((ctx - 1) / (32 * CHUNK_TILES)) % nz == z)) {
         uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + 2 * NS * 8192);
         const int pos = ctx - 1;
         const uint16_t* src = f.qkv + (int64_t)b * f.ld + (int64_t)(a.q_heads + (li == 0 ? 0 : a.kv_heads) + kvh) * HD;
@@ -511,8 +636,8 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       for (int d = 0; d < NS; d++) {
         const int tile = t0 + d;
         if (tile >= ntiles) break;
-        load_k(tile + NS, d);                          // slot t % NS, read during iteration t - 1
-        load_v(tile + NS - 1, (d + NS - 1) % NS);      // slot (t - 1) % NS, likewise
+        load_k(tile_of(tile + NS), d);                       // slot t % NS, read during iteration t - 1
+        load_v(tile_of(tile + NS - 1), (d + NS - 1) % NS);   // slot (t - 1) % NS, likewise
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PI * (NS - 2)) : "memory");  // K tile t + 2, V^T tile t + 1
         __syncthreads();
       }
@@ -530,7 +655,8 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   const int qrow = min(qi, qlen - 1);
   const int qpos = ctx - qlen + qrow;
   const int last_pos = ctx - qlen + min(QMAX - 1, qlen - 1);
-  const int ntiles = last_pos / 32 + 1;
+  const int ntiles = tiles_here(last_pos / 32 + 1);
+  if (SPLIT && ntiles == 0) return;
   const int nfull = (ctx - qlen + 1) / 32;
   bf16x8 qf[4];
   // FUSED: the G query heads of this (sequence, KV head) are formed here, one head per wave at a time, the key and the
@@ -588,83 +714,226 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       s[u] = acc;
     }
   };
-  f32x4 o[CT];
+  f32x4 o[CT], ot[CT];
 #pragma unroll
   for (int i = 0; i < CT; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY;
-  float l = 0.f;
+  float m = kNoKey, mt = 0.f;
+  float l = 0.f, lsum = 0.f;
   __syncthreads();
-  if (FUSED && lt == 0) patch_k(0);
+  if (FUSED && tile_of(0) == lt) patch_k(0);
   f32x4 s_cur[2];
   scores(0, s_cur);
   __syncthreads();
-  for (int t0 = 0; t0 < ntiles; t0 += NS) {
+  for (int c0 = 0; c0 < ntiles; c0 += CHUNK_TILES) {
+    const int ce = min(c0 + CHUNK_TILES, ntiles);
+    for (int t0 = c0; t0 < ce; t0 += NS) {
 #pragma unroll
-    for (int d = 0; d < NS; d++) {
-      const int tile = t0 + d;
-      if (tile >= ntiles) break;
-      if (FUSED && tile == lt) patch_v(d);
-      if (FUSED && tile + 1 == lt) patch_k((d + 1) % NS);
-      bf16x8 vf[CT];
+      for (int d = 0; d < NS; d++) {
+        if (t0 + d >= ce) break;
+        const int tile = tile_of(t0 + d);
+        if (FUSED && tile == lt) patch_v(d);
+        if (FUSED && tile_of(t0 + d + 1) == lt) patch_k((d + 1) % NS);
+        bf16x8 vf[CT];
 #pragma unroll
-      for (int i = 0; i < CT; i++) {
-        const uint2 va = *reinterpret_cast<const uint2*>(&lds_v[d][vofs0 + i * 1024]);
-        const uint2 vb = *reinterpret_cast<const uint2*>(&lds_v[d][vofs1 + i * 1024]);
-        vf[i] = __builtin_bit_cast(bf16x8, u32x4{va.x, va.y, vb.x, vb.y});
+        for (int i = 0; i < CT; i++) {
+          const uint2 va = *reinterpret_cast<const uint2*>(&lds_v[d][vofs0 + i * 1024]);
+          const uint2 vb = *reinterpret_cast<const uint2*>(&lds_v[d][vofs1 + i * 1024]);
+          vf[i] = __builtin_bit_cast(bf16x8, u32x4{va.x, va.y, vb.x, vb.y});
+        }
+        f32x4 s_next[2];
+        scores((d + 1) % NS, s_next);
+        float alpha;
+        bf16x8 pf;
+        if (tile < nfull) softmax_tile<false>(s_cur, tile * 32, g, qpos, a.scale_log2, m, l, alpha, pf);
+        else softmax_tile<true>(s_cur, tile * 32, g, qpos, a.scale_log2, m, l, alpha, pf);
+#pragma unroll
+        for (int i = 0; i < CT; i++) o[i] = f32x4{o[i][0] * alpha, o[i][1] * alpha, o[i][2] * alpha, o[i][3] * alpha};
+#pragma unroll
+        for (int i = 0; i < CT; i++) o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i], pf, o[i], 0, 0, 0);
+        __syncthreads();
+        s_cur[0] = s_next[0];
+        s_cur[1] = s_next[1];
       }
-      f32x4 s_next[2];
-      scores((d + 1) % NS, s_next);
-      float alpha;
-      bf16x8 pf;
-      if (tile < nfull) softmax_tile<false>(s_cur, tile * 32, g, qpos, a.scale_log2, m, l, alpha, pf);
-      else softmax_tile<true>(s_cur, tile * 32, g, qpos, a.scale_log2, m, l, alpha, pf);
-#pragma unroll
-      for (int i = 0; i < CT; i++) o[i] = f32x4{o[i][0] * alpha, o[i][1] * alpha, o[i][2] * alpha, o[i][3] * alpha};
-#pragma unroll
-      for (int i = 0; i < CT; i++) o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i], pf, o[i], 0, 0, 0);
-      __syncthreads();
-      s_cur[0] = s_next[0];
-      s_cur[1] = s_next[1];
     }
+    // the chunk is complete
+    const int chunk = tile_of(c0) / CHUNK_TILES;
+    if (SPLIT && qpos >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete with it)
+      if (qvalid) {
+        const int64_t at = ((int64_t)(b * sp.max_q_len + qi) * a.q_heads + h) * sp.nchunks + chunk;
+#pragma unroll
+        for (int i = 0; i < CT; i++) *reinterpret_cast<f32x4*>(sp.o + at * HD + 16 * (CT * wv + i) + 4 * g) = o[i];
+        if (wv == 0 && g == 0) *reinterpret_cast<f32x2*>(sp.ml + at * 2) = f32x2{m, l};
+      }
+    } else if (chunk == 0) {
+      mt = m, lsum = l;
+#pragma unroll
+      for (int i = 0; i < CT; i++) ot[i] = o[i];
+    } else if (qpos >= chunk * CHUNK_TILES * 32) {
+      float fa, fb;
+      merge_chunk(mt, lsum, m, l, fa, fb);
+#pragma unroll
+      for (int i = 0; i < CT; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) ot[i][e] = merge_acc(ot[i][e], fa, o[i][e], fb);
+    }
+    m = kNoKey, l = 0.f;
+#pragma unroll
+    for (int i = 0; i < CT; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  if (!qvalid) return;
-  const float inv = 1.0f / l;
+  if (!qvalid || (SPLIT && (qpos >= 32 * CHUNK_TILES || z != 0))) return;
+  const float inv = 1.0f / lsum;
   uint16_t* op = a.out + ((int64_t)(FUSED ? b : a.q_start[b] + qi) * a.q_heads + h) * HD + 16 * CT * wv;
 #pragma unroll
   for (int i = 0; i < CT; i++) {
-    const uint32_t lo = pack_bf16x2(o[i][0] * inv, o[i][1] * inv);
-    const uint32_t hi = pack_bf16x2(o[i][2] * inv, o[i][3] * inv);
+    const uint32_t lo = pack_bf16x2(ot[i][0] * inv, ot[i][1] * inv);
+    const uint32_t hi = pack_bf16x2(ot[i][2] * inv, ot[i][3] * inv);
     *reinterpret_cast<uint2*>(op + 16 * i + 4 * g) = make_uint2(lo, hi);
   }
 }
 
+// The rows of several chunks, which different work-groups computed: one wavefront per (query, head), two channels per lane, the chunks
+// merged in ascending order exactly as the kernels above merge them.  Sixteen chunks' loads are in flight at a time.
+template <bool FUSED>
+__global__ __launch_bounds__(256) void attention_merge_kernel(const AttnArgs a, const SplitArgs sp) {
+  const int b = blockIdx.z, qi = blockIdx.y;
+  const int h = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (h >= a.q_heads) return;
+  int nch = 0, qlen = 0;
+  auto read_lengths = [&]() __attribute__((always_inline)) {
+    const int ctx = a.ctx_len[b];
+    qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
+    nch = qi < qlen ? (ctx - qlen + qi) / (32 * CHUNK_TILES) + 1 : 0;
+  };
+  // a chunk of a prompt has many rows, and possibly all of one chunk: they are not loaded before that is known.  A decode
+  // step has few: their states (behind the horizon, too) are loaded while the length is on its way, and possibly not used.
+  if (!FUSED) {
+    read_lengths();
+    if (nch <= 1) return;
+  }
+  const int64_t at = ((int64_t)(b * sp.max_q_len + qi) * a.q_heads + h) * sp.nchunks;
+  const f32x2* po = reinterpret_cast<const f32x2*>(sp.o + at * HD) + lane;
+  const f32x2* pm = reinterpret_cast<const f32x2*>(sp.ml + at * 2);
+  constexpr int NB = 16;
+  f32x2 O = {0.f, 0.f};
+  float M = 0.f, L = 0.f;
+  for (int c0 = 0; c0 < sp.nchunks; c0 += NB) {
+    f32x2 o[NB], ml[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      const int c = min(c0 + i, sp.nchunks - 1);
+      o[i] = po[(int64_t)c * (HD / 2)];
+      ml[i] = pm[c];
+    }
+    if (c0 == 0) {
+      if (FUSED) read_lengths();
+      M = ml[0][0], L = ml[0][1], O = o[0];
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      if (c0 + i == 0) continue;
+      if (c0 + i >= nch) break;
+      float fa, fb;
+      merge_chunk(M, L, ml[i][0], ml[i][1], fa, fb);
+      O = f32x2{merge_acc(O[0], fa, o[i][0], fb), merge_acc(O[1], fa, o[i][1], fb)};
+    }
+    if (c0 + NB >= nch) break;
+  }
+  if (nch <= 1) return;
+  const float inv = 1.0f / L;
+  uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)(FUSED ? b : a.q_start[b] + qi) * a.q_heads + h) * HD);
+  op[lane] = pack_bf16x2(O[0] * inv, O[1] * inv);
+}
+
+static int chunks_of(int max_len) { return (max_len + 32 * CHUNK_TILES - 1) / (32 * CHUNK_TILES); }
+
+// How many work-groups share the chunks of a (KV head, sequence) in the decode kernel: 1 = a single one walks them all.
+// Enough for 512 work-groups in all, two per CU; from 129 pairs on a chain per pair already draws the keys at the rate of
+// the memory and the second launch is lost (us, one chain against split: 16 sequences of 2300 keys on 8 KV heads 37.2 / 35.0,
+// of 8200 keys 130 / 116; 32 of 2300 55 / 62, of 8200 194 / 204), and with two chunks there is nothing to gain
+// (1 sequence of 600 keys 10.8 / 12.0; of 1200 17.4 / 12, of 4096 49.3 / 13.1, of 16384 186 / 22).
+static int decode_split(int64_t pairs, int max_len) {
+  const int nch = chunks_of(max_len);
+  if (nch < 3 || pairs > 128) return 1;
+  const int64_t want = 512 / pairs;
+  return (int)(want > nch ? nch : want);
+}
+// The same for the grouped kernel, whose work-groups then take a chunk each: worth it while they are few; the bound on
+// the product keeps the states (33 KiB per work-group and chunk) to 64 MiB.
+static bool group_split(int64_t groups, int max_len) {
+  const int nch = chunks_of(max_len);
+  return nch >= 3 && groups <= 128 && groups * nch <= 2048;
+}
+static bool grouped_cache(int G, int kv_heads, int max_len) {
+  return (max_len & 31) == 0 && (G == 1 || G == 2 || G == 4 || G == 8) && kv_heads <= 65535 && max_len <= (1 << 22);
+}
+size_t attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len) {
+  if (batch <= 0 || max_q_len <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || max_len < 32) return 0;
+  const int G = q_heads / kv_heads;
+  if (!grouped_cache(G, kv_heads, max_len)) return 0;
+  const bool split = (int64_t)max_q_len * G <= 16 ? decode_split((int64_t)batch * kv_heads, max_len) > 1
+                                                  : group_split((int64_t)((max_q_len + 15) / 16) * kv_heads * batch, max_len);
+  return split ? (size_t)batch * max_q_len * q_heads * chunks_of(max_len) * (HD + 2) * sizeof(float) : 0;
+}
+static SplitArgs split_args(void* ws, int batch, int max_q_len, int q_heads, int max_len) {
+  SplitArgs sp;
+  sp.nchunks = chunks_of(max_len);
+  sp.max_q_len = max_q_len;
+  sp.o = static_cast<float*>(ws);
+  sp.ml = sp.o + (int64_t)batch * max_q_len * q_heads * sp.nchunks * HD;
+  return sp;
+}
+
+template <bool FUSED>
+static void merge_launch(const AttnArgs& a, const SplitArgs& sp, int max_q_len, int batch, hipStream_t stream) {
+  const dim3 grid((unsigned)((a.q_heads + 3) / 4), (unsigned)max_q_len, (unsigned)batch);
+  hipLaunchKernelGGL(attention_merge_kernel<FUSED>, grid, dim3(256), 0, stream, a, sp);
+}
+
+template <int G, bool FUSED>
+static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max_q_len, void* ws, size_t ws_bytes, hipStream_t stream) {
+  const int lds = 2 * 4 * 8192 + (FUSED ? (G + 2) * HD * 2 : 0);
+  const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, a.q_heads, a.kv_heads, a.max_len) : 0;
+  if (need == 0 || ws_bytes < need) {
+    static std::atomic<uint64_t> done{0};
+    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, false>), lds, done);
+    if (e != hipSuccess) return hip_code(e);
+    hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, false>), dim3((unsigned)a.kv_heads, (unsigned)batch), dim3(512), lds, stream, a, f, SplitArgs{});
+    return hip_code(hipGetLastError());
+  }
+  const SplitArgs sp = split_args(ws, batch, max_q_len, a.q_heads, a.max_len);
+  static std::atomic<uint64_t> done{0};
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, true>), lds, done);
+  if (e != hipSuccess) return hip_code(e);
+  const int nz = decode_split((int64_t)batch * a.kv_heads, a.max_len);
+  hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, true>), dim3((unsigned)a.kv_heads, (unsigned)batch, (unsigned)nz), dim3(512), lds, stream, a, f, sp);
+  merge_launch<FUSED>(a, sp, max_q_len, batch, stream);
+  return hip_code(hipGetLastError());
+}
+
 int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache, void* out, const int* q_start,
                        const int* q_len, const int* ctx_len, int batch, int max_q_len, int q_heads, int kv_heads,
-                       int head_dim, int max_len, float scale, hipStream_t stream) {
+                       int head_dim, int max_len, float scale, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (!q || !k_cache || !vt_cache || !out || !q_start || !q_len || !ctx_len) return TBIK_ERR_INVALID;
   if (batch <= 0 || max_q_len <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0) return TBIK_ERR_INVALID;
   if (head_dim != HD) return TBIK_ERR_UNSUPPORTED;
   if (max_len < 32 || (max_len & 3)) return TBIK_ERR_ALIGNMENT;
   auto mis = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; };
-  if (mis(q) || mis(k_cache) || mis(vt_cache) || mis(out)) return TBIK_ERR_ALIGNMENT;
+  if (mis(q) || mis(k_cache) || mis(vt_cache) || mis(out) || mis(ws)) return TBIK_ERR_ALIGNMENT;
   if (batch > 65535 || q_heads > 65535) return TBIK_ERR_INVALID;
   AttnArgs a{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k_cache), static_cast<const uint16_t*>(vt_cache),
              static_cast<uint16_t*>(out), q_start, q_len, ctx_len, q_heads, kv_heads, max_len, scale * 1.4426950408889634f};
   // the grouped kernel needs whole 32-key tiles in the caches, at most 8 query heads per KV head and a (sequence, head)
   // slice of a cache below 2 GiB (32-bit byte offsets)
   const int G = q_heads / kv_heads;
-  const bool grouped = (max_len & 31) == 0 && (G == 1 || G == 2 || G == 4 || G == 8) && kv_heads <= 65535 && max_len <= (1 << 22);
+  const bool grouped = grouped_cache(G, kv_heads, max_len);
   if (grouped) {
     const bool deep = max_q_len <= 16;  // decode: one block of queries per sequence
     if ((int64_t)max_q_len * G <= 16) {  // all queries of a sequence and all heads of a group in one MFMA tile
-      const dim3 grid((unsigned)kv_heads, (unsigned)batch, 1u);
-      constexpr size_t lds = 2 * 4 * 8192;
       const QkvArgs none{};
-      if (G == 1) hipLaunchKernelGGL((attention_decode_kernel<1, false>), grid, dim3(512), lds, stream, a, none);
-      else if (G == 2) hipLaunchKernelGGL((attention_decode_kernel<2, false>), grid, dim3(512), lds, stream, a, none);
-      else if (G == 4) hipLaunchKernelGGL((attention_decode_kernel<4, false>), grid, dim3(512), lds, stream, a, none);
-      else hipLaunchKernelGGL((attention_decode_kernel<8, false>), grid, dim3(512), lds, stream, a, none);
-      return hip_code(hipGetLastError());
+      if (G == 1) return decode_launch<1, false>(a, none, batch, max_q_len, ws, ws_bytes, stream);
+      if (G == 2) return decode_launch<2, false>(a, none, batch, max_q_len, ws, ws_bytes, stream);
+      if (G == 4) return decode_launch<4, false>(a, none, batch, max_q_len, ws, ws_bytes, stream);
+      return decode_launch<8, false>(a, none, batch, max_q_len, ws, ws_bytes, stream);
     }
     const int64_t gx = (int64_t)((max_q_len + 15) / 16) * kv_heads;
     if (gx > 0x7fffffff) return TBIK_ERR_INVALID;
@@ -674,18 +943,33 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
     // sequences: up to two work-groups per CU: 3 - 18 % faster) and costs once the chip is full, where the extra waves
     // take the place of a whole work-group (from three per CU on: 35 % slower).  Same bits either way.
     const bool few = gx * batch <= 512;
-#define TBIK_ATTN_GROUP(GG)                                                                                              \
-  do {                                                                                                                   \
-    if (few && deep) hipLaunchKernelGGL((attention_group_kernel<GG, true, 2>), grid, dim3(64 * (GG + 2)), 0, stream, a);   \
-    else if (few) hipLaunchKernelGGL((attention_group_kernel<GG, false, 2>), grid, dim3(64 * (GG + 2)), 0, stream, a);    \
-    else if (deep) hipLaunchKernelGGL((attention_group_kernel<GG, true, 0>), grid, dim3(64 * GG), 0, stream, a);          \
-    else hipLaunchKernelGGL((attention_group_kernel<GG, false, 0>), grid, dim3(64 * GG), 0, stream, a);                   \
+    const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len) : 0;
+    const bool split = need != 0 && ws_bytes >= need;
+    const bool one = chunks_of(max_len) == 1;
+    const SplitArgs sp = split ? split_args(ws, batch, max_q_len, q_heads, max_len) : SplitArgs{};
+    const dim3 cgrid((unsigned)gx, (unsigned)batch, (unsigned)chunks_of(max_len));
+#define TBIK_ATTN_GROUP_RUN(GG, DEEP, NLD, CH, GRID)                                                                              \
+  hipLaunchKernelGGL((attention_group_kernel<GG, DEEP, NLD, CH>), GRID, dim3(64 * (GG + NLD)), 0, stream, a, sp)
+#define TBIK_ATTN_GROUP(GG)                                                                  \
+  do {                                                                                       \
+    if (split && deep) TBIK_ATTN_GROUP_RUN(GG, true, 2, SPLIT_CHUNKS, cgrid);                \
+    else if (split) TBIK_ATTN_GROUP_RUN(GG, false, 2, SPLIT_CHUNKS, cgrid);                  \
+    else if (one && few && deep) TBIK_ATTN_GROUP_RUN(GG, true, 2, ONE_CHUNK, grid);          \
+    else if (one && few) TBIK_ATTN_GROUP_RUN(GG, false, 2, ONE_CHUNK, grid);                 \
+    else if (one && deep) TBIK_ATTN_GROUP_RUN(GG, true, 0, ONE_CHUNK, grid);                 \
+    else if (one) TBIK_ATTN_GROUP_RUN(GG, false, 0, ONE_CHUNK, grid);                        \
+    else if (few && deep) TBIK_ATTN_GROUP_RUN(GG, true, 2, ALL_CHUNKS, grid);                \
+    else if (few) TBIK_ATTN_GROUP_RUN(GG, false, 2, ALL_CHUNKS, grid);                       \
+    else if (deep) TBIK_ATTN_GROUP_RUN(GG, true, 0, ALL_CHUNKS, grid);                       \
+    else TBIK_ATTN_GROUP_RUN(GG, false, 0, ALL_CHUNKS, grid);                                \
   } while (0)
     if (G == 1) TBIK_ATTN_GROUP(1);
     else if (G == 2) TBIK_ATTN_GROUP(2);
     else if (G == 4) TBIK_ATTN_GROUP(4);
     else TBIK_ATTN_GROUP(8);
 #undef TBIK_ATTN_GROUP
+#undef TBIK_ATTN_GROUP_RUN
+    if (split) merge_launch<false>(a, sp, max_q_len, batch, stream);
   } else {
     const dim3 grid((unsigned)((max_q_len + 15) / 16), (unsigned)q_heads, (unsigned)batch);
     hipLaunchKernelGGL(attention_kernel, grid, dim3(64), 0, stream, a);
@@ -700,14 +984,15 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
 // the caller makes the two calls.
 int attention_decode_qkv_dispatch(const void* qkv, int64_t ld, const void* q_weight, const void* k_weight, const float* inv_freq,
                                   void* k_cache, void* vt_cache, void* out, const int* ctx_len, int batch, int q_heads,
-                                  int kv_heads, int head_dim, int max_len, float scale, float eps, hipStream_t stream) {
+                                  int kv_heads, int head_dim, int max_len, float scale, float eps, void* ws, size_t ws_bytes,
+                                  hipStream_t stream) {
   if (!qkv || !q_weight || !k_weight || !inv_freq || !k_cache || !vt_cache || !out || !ctx_len) return TBIK_ERR_INVALID;
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0) return TBIK_ERR_INVALID;
   if (head_dim != HD) return TBIK_ERR_UNSUPPORTED;
   if (ld < (int64_t)(q_heads + 2 * kv_heads) * HD) return TBIK_ERR_INVALID;
   if (max_len < 32 || (max_len & 3)) return TBIK_ERR_ALIGNMENT;
   auto mis = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & m) != 0; };
-  if (mis(k_cache, 15) || mis(vt_cache, 15) || mis(out, 15) || mis(qkv, 1) || mis(q_weight, 1) || mis(k_weight, 1) || mis(inv_freq, 3))
+  if (mis(k_cache, 15) || mis(vt_cache, 15) || mis(out, 15) || mis(ws, 15) || mis(qkv, 1) || mis(q_weight, 1) || mis(k_weight, 1) || mis(inv_freq, 3))
     return TBIK_ERR_ALIGNMENT;
   if (batch > 65535 || kv_heads > 65535) return TBIK_ERR_INVALID;
   const int G = q_heads / kv_heads;
@@ -716,13 +1001,10 @@ int attention_decode_qkv_dispatch(const void* qkv, int64_t ld, const void* q_wei
              nullptr, nullptr, ctx_len, q_heads, kv_heads, max_len, scale * 1.4426950408889634f};
   const QkvArgs f{static_cast<const uint16_t*>(qkv), ld, static_cast<const uint16_t*>(q_weight), static_cast<const uint16_t*>(k_weight),
                   inv_freq, static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(vt_cache), eps};
-  const dim3 grid((unsigned)kv_heads, (unsigned)batch, 1u);
-  const size_t lds = 2 * 4 * 8192 + (size_t)(G + 2) * HD * 2;
-  if (G == 1) hipLaunchKernelGGL((attention_decode_kernel<1, true>), grid, dim3(512), lds, stream, a, f);
-  else if (G == 2) hipLaunchKernelGGL((attention_decode_kernel<2, true>), grid, dim3(512), lds, stream, a, f);
-  else if (G == 4) hipLaunchKernelGGL((attention_decode_kernel<4, true>), grid, dim3(512), lds, stream, a, f);
-  else hipLaunchKernelGGL((attention_decode_kernel<8, true>), grid, dim3(512), lds, stream, a, f);
-  return hip_code(hipGetLastError());
+  if (G == 1) return decode_launch<1, true>(a, f, batch, 1, ws, ws_bytes, stream);
+  if (G == 2) return decode_launch<2, true>(a, f, batch, 1, ws, ws_bytes, stream);
+  if (G == 4) return decode_launch<4, true>(a, f, batch, 1, ws, ws_bytes, stream);
+  return decode_launch<8, true>(a, f, batch, 1, ws, ws_bytes, stream);
 }
 
 }  // namespace tbik

@@ -17,7 +17,8 @@ int log_softmax_dispatch(const void* x, int64_t ldx, int in_dtype, void* out, in
                          int64_t cols, void* ws, size_t ws_bytes, int write_softmax, hipStream_t stream);
 int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache, void* out, const int* q_start,
                        const int* q_len, const int* ctx_len, int batch, int max_q_len, int q_heads, int kv_heads,
-                       int head_dim, int max_len, float scale, hipStream_t stream);
+                       int head_dim, int max_len, float scale, void* ws, size_t ws_bytes, hipStream_t stream);
+size_t attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len);
 int argmax_dispatch(const void* x, int64_t ld, void* out, int64_t rows, int cols, void* history, int64_t history_ld,
                     void* count, void* positions, void* ctx_len, hipStream_t stream);
 int mean_dispatch(const void* x, void* out, int64_t outer, int64_t n, int64_t inner, int dtype_code, hipStream_t stream);
@@ -36,7 +37,8 @@ int rmsnorm_gemm_dispatch(const void* x, int64_t ldx, const void* res, int64_t l
                           int M, int N, int K, const void* bias, hipStream_t stream);
 int attention_decode_qkv_dispatch(const void* qkv, int64_t ld, const void* q_weight, const void* k_weight, const float* inv_freq,
                                   void* k_cache, void* vt_cache, void* out, const int* ctx_len, int batch, int q_heads,
-                                  int kv_heads, int head_dim, int max_len, float scale, float eps, hipStream_t stream);
+                                  int kv_heads, int head_dim, int max_len, float scale, float eps, void* ws, size_t ws_bytes,
+                                  hipStream_t stream);
 int gemm_silu_mul_dispatch(const void* x, int64_t ldx, const void* W, int64_t ldw, void* out, int64_t ldo, int M, int inter, int K,
                            hipStream_t stream);
 int gemm_tree_rmsnorm_dispatch(bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n, int M, int N,
@@ -197,7 +199,18 @@ int bi_attention_bf16(const void* q, const void* k_cache, const void* vt_cache, 
                       const int32_t* q_len, const int32_t* ctx_len, int batch, int max_q_len, int q_heads, int kv_heads,
                       int head_dim, int max_len, float scale, tbik_stream_t stream) {
   return tbik::attention_dispatch(q, k_cache, vt_cache, out, q_start, q_len, ctx_len, batch, max_q_len, q_heads, kv_heads,
-                                  head_dim, max_len, scale, static_cast<hipStream_t>(stream));
+                                  head_dim, max_len, scale, nullptr, 0, static_cast<hipStream_t>(stream));
+}
+
+size_t bi_attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len) {
+  return tbik::attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len);
+}
+
+int bi_attention_ws_bf16(const void* q, const void* k_cache, const void* vt_cache, void* out, const int32_t* q_start,
+                         const int32_t* q_len, const int32_t* ctx_len, int batch, int max_q_len, int q_heads, int kv_heads,
+                         int head_dim, int max_len, float scale, void* workspace, size_t workspace_bytes, tbik_stream_t stream) {
+  return tbik::attention_dispatch(q, k_cache, vt_cache, out, q_start, q_len, ctx_len, batch, max_q_len, q_heads, kv_heads,
+                                  head_dim, max_len, scale, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 int tbik_gemm_f32(const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n, void* C, int64_t ldc, int M,
@@ -240,7 +253,16 @@ int bi_attention_decode_qkv_bf16(const void* qkv, int64_t ld, const void* q_weig
                                  void* k_cache, void* vt_cache, void* out, const int32_t* ctx_len, int batch, int q_heads,
                                  int kv_heads, int head_dim, int max_len, float scale, float eps, tbik_stream_t stream) {
   return tbik::attention_decode_qkv_dispatch(qkv, ld, q_weight, k_weight, inv_freq, k_cache, vt_cache, out, ctx_len, batch,
-                                             q_heads, kv_heads, head_dim, max_len, scale, eps, static_cast<hipStream_t>(stream));
+                                             q_heads, kv_heads, head_dim, max_len, scale, eps, nullptr, 0, static_cast<hipStream_t>(stream));
+}
+
+int bi_attention_decode_qkv_ws_bf16(const void* qkv, int64_t ld, const void* q_weight, const void* k_weight, const float* inv_freq,
+                                    void* k_cache, void* vt_cache, void* out, const int32_t* ctx_len, int batch, int q_heads,
+                                    int kv_heads, int head_dim, int max_len, float scale, float eps, void* workspace,
+                                    size_t workspace_bytes, tbik_stream_t stream) {
+  return tbik::attention_decode_qkv_dispatch(qkv, ld, q_weight, k_weight, inv_freq, k_cache, vt_cache, out, ctx_len, batch, q_heads,
+                                             kv_heads, head_dim, max_len, scale, eps, workspace, workspace_bytes,
+                                             static_cast<hipStream_t>(stream));
 }
 
 int bi_argmax_bf16(const void* x, int64_t ld, void* out, int64_t rows, int cols, tbik_stream_t stream) {

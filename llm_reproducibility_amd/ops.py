@@ -420,6 +420,12 @@ def _(x, dim, keepdim):
 # --------------------------------------------------------------------------------------------
 # fixed-order attention
 # --------------------------------------------------------------------------------------------
+def _attention_workspace(batch: int, max_q_len: int, q_heads: int, kv_heads: int, max_len: int, device):
+    """(scratch for the chunks of long caches that several work-groups share, its bytes); (None, 0) where none is used."""
+    n = _lib.lib().bi_attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len)
+    return (torch.empty(n, device=device, dtype=torch.uint8), n) if n else (None, 0)
+
+
 def _bi_attention_bf16_impl(q: torch.Tensor, k_cache: torch.Tensor, vt_cache: torch.Tensor, q_start: torch.Tensor,
                             q_len: torch.Tensor, ctx_len: torch.Tensor, max_q_len: int, scale: float) -> torch.Tensor:
     _require_gpu(q, k_cache, vt_cache, q_start, q_len, ctx_len)
@@ -431,10 +437,12 @@ def _bi_attention_bf16_impl(q: torch.Tensor, k_cache: torch.Tensor, vt_cache: to
     q = q.contiguous()
     assert k_cache.is_contiguous() and vt_cache.is_contiguous()
     out = torch.empty_like(q)
-    rc = _lib.lib().bi_attention_bf16(q.data_ptr(), k_cache.data_ptr(), vt_cache.data_ptr(), out.data_ptr(),
-                                      q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), batch, max_q_len,
-                                      q_heads, kv_heads, head_dim, max_len, scale, _stream(q))
-    _lib.check(rc, "bi_attention_bf16")
+    ws, ws_bytes = _attention_workspace(batch, max_q_len, q_heads, kv_heads, max_len, q.device)
+    rc = _lib.lib().bi_attention_ws_bf16(q.data_ptr(), k_cache.data_ptr(), vt_cache.data_ptr(), out.data_ptr(),
+                                         q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), batch, max_q_len,
+                                         q_heads, kv_heads, head_dim, max_len, scale,
+                                         None if ws is None else ws.data_ptr(), ws_bytes, _stream(q))
+    _lib.check(rc, "bi_attention_ws_bf16")
     return out
 
 
@@ -701,7 +709,7 @@ def bi_attention_decode_qkv(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight:
                             scale: float, eps: float) -> torch.Tensor:
     """A decode step of an attention block for sequences with one new token each (row b of qkv = sequence b's token at
     position ctx_len[b] - 1): per-head q/k norm, rotary embedding, cache write (in place) and attention in one launch
-    (`bi_attention_decode_qkv_bf16`), the two calls where that kernel does not apply.  Same bits either way."""
+    (`bi_attention_decode_qkv_ws_bf16`), the two calls where that kernel does not apply.  Same bits either way."""
     _require_gpu(qkv, q_weight, k_weight, inv_freq, k_cache, vt_cache, ctx_len)
     B = qkv.shape[0]
     assert qkv.dtype == torch.bfloat16 and qkv.stride(1) == 1 and qkv.shape[1] == (q_heads + 2 * kv_heads) * 128
@@ -710,14 +718,16 @@ def bi_attention_decode_qkv(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight:
     max_len = k_cache.shape[2]
     if ("attn_qkv", q_heads, kv_heads, max_len % 32) not in _declined:
         out = torch.empty((B, q_heads, 128), device=qkv.device, dtype=qkv.dtype)
-        rc = _lib.lib().bi_attention_decode_qkv_bf16(
+        ws, ws_bytes = _attention_workspace(B, 1, q_heads, kv_heads, max_len, qkv.device)
+        rc = _lib.lib().bi_attention_decode_qkv_ws_bf16(
             qkv.data_ptr(), qkv.stride(0) if B > 1 else max(qkv.stride(0), qkv.shape[1]), q_weight.contiguous().data_ptr(),
             k_weight.contiguous().data_ptr(), inv_freq.contiguous().data_ptr(), k_cache.data_ptr(), vt_cache.data_ptr(),
-            out.data_ptr(), ctx_len.data_ptr(), B, q_heads, kv_heads, 128, max_len, scale, eps, _stream(qkv))
+            out.data_ptr(), ctx_len.data_ptr(), B, q_heads, kv_heads, 128, max_len, scale, eps,
+            None if ws is None else ws.data_ptr(), ws_bytes, _stream(qkv))
         if rc == _lib.TBIK_OK:
             return out
         if rc != _lib.TBIK_ERR_UNSUPPORTED:
-            _lib.check(rc, "bi_attention_decode_qkv_bf16")
+            _lib.check(rc, "bi_attention_decode_qkv_ws_bf16")
         _declined.add(("attn_qkv", q_heads, kv_heads, max_len % 32))
     pos = (ctx_len - 1).to(torch.int64)
     seq = torch.arange(B, device=qkv.device, dtype=torch.int64)

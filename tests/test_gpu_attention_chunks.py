@@ -1,0 +1,85 @@
+"""Attention around the edges of its 512-key chunks: the kernels that walk all chunks, the ones that share them between
+work-groups and the one-wave kernel give the same bits, and the values are those of the float64 oracle."""
+import math
+
+import pytest
+import torch
+
+from llm_reproducibility_amd import _lib, ops
+from oracle import tbik_oracle as O
+
+pytestmark = pytest.mark.gpu
+D, SCALE = 128, 1.0 / math.sqrt(128)
+
+
+def _caches(ks, vs, L, dev):
+    kc = torch.zeros((len(ks), ks[0].shape[1], L, D), dtype=torch.bfloat16, device=dev)
+    vt = torch.zeros((len(ks), ks[0].shape[1], D, L), dtype=torch.bfloat16, device=dev)
+    for b, (k, v) in enumerate(zip(ks, vs)):
+        kc[b, :, : k.shape[0]] = k.transpose(0, 1)
+        vt[b, :, :, : v.shape[0]] = v.permute(1, 2, 0)
+    return kc, vt
+
+
+def _no_workspace(monkeypatch):
+    monkeypatch.setattr(ops, "_attention_workspace", lambda *a: (None, 0))
+
+
+# heads per KV head 4, 8, 1 (decode rows) and more new queries than a decode tile takes (the grouped kernel); contexts one key
+# around one, two and three chunks, and one whose queries straddle an edge
+@pytest.mark.parametrize("hq,hkv,new,ctxs", [
+    (8, 2, 1, [1, 511, 512, 513, 1023, 1024, 1025, 1537]),
+    (16, 2, 2, [513, 514, 1025, 2, 1600]),
+    (3, 3, 5, [515, 1027, 1540]),
+    (8, 2, 40, [40, 520, 530, 1056, 1560]),
+    (2, 2, 20, [1030, 1545]),
+])
+def test_chunk_edges(dev, monkeypatch, hq, hkv, new, ctxs):
+    torch.manual_seed(hq + new)
+    print("case chunks", hq, hkv, new, ctxs, flush=True)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    rnd = lambda *s: torch.randn(s, device=dev).to(torch.bfloat16)  # noqa: E731
+    ks, vs = [rnd(c, hkv, D) for c in ctxs], [rnd(c, hkv, D) for c in ctxs]
+    qlens = [min(new, c) - (b % 2 if min(new, c) > 1 else 0) for b, c in enumerate(ctxs)]      # ragged
+    qs = [rnd(n, hq, D) for n in qlens]
+    starts = [sum(qlens[:i]) for i in range(len(qlens))]
+    args = (i32(starts), i32(qlens), i32(ctxs), new, SCALE)
+    L = (max(ctxs) + 31) // 32 * 32
+    q = torch.cat(qs)
+    assert _lib.lib().bi_attention_workspace_bytes(len(ctxs), new, hq, hkv, L) > 0
+    kc, vt = _caches(ks, vs, L, dev)
+    shared = ops.bi_attention_bf16(q, kc, vt, *args)
+    for b, c in enumerate(ctxs):
+        want = O.causal_attention(qs[b].cpu(), ks[b].cpu(), vs[b].cpu(), SCALE).to(torch.bfloat16)
+        assert not O.outside_tolerance(shared[starts[b]: starts[b] + qlens[b]].cpu(), want).any(), c
+    kc2, vt2 = _caches(ks, vs, L + 4, dev)                      # no whole number of tiles: the one-wave kernel
+    assert torch.equal(ops.bi_attention_bf16(q, kc2, vt2, *args), shared)
+    kc3, vt3 = _caches(ks, vs, L + 4096, dev)                   # a longer cache: another number of chunks and work-groups
+    assert torch.equal(ops.bi_attention_bf16(q, kc3, vt3, *args), shared)
+    for b in (0, len(ctxs) - 1):                                # a sequence alone
+        kb, vb = _caches([ks[b]], [vs[b]], (ctxs[b] + 31) // 32 * 32, dev)
+        alone = ops.bi_attention_bf16(qs[b], kb, vb, i32([0]), i32([qlens[b]]), i32([ctxs[b]]), qlens[b], SCALE)
+        assert torch.equal(alone, shared[starts[b]: starts[b] + qlens[b]])
+    _no_workspace(monkeypatch)
+    assert torch.equal(ops.bi_attention_bf16(q, kc, vt, *args), shared)
+
+
+@pytest.mark.parametrize("ctxs", [[1537], [512, 513, 1024, 1025, 0, 1700], [600] * 20])
+def test_one_launch_decode_step_over_chunks(dev, monkeypatch, ctxs):
+    """The decode step that forms its own query, key and value: outputs and caches with and without the workspace."""
+    torch.manual_seed(len(ctxs))
+    print("case decode step", ctxs, flush=True)
+    hq, hkv, L, B = 8, 2, 1728, len(ctxs)
+    w = (1 + 0.1 * torch.randn(D, device=dev)).to(torch.bfloat16)
+    inv = O.rope_inv_freq(D, 1e6).to(dev)
+    qkv = torch.randn((B, (hq + 2 * hkv) * D), device=dev).to(torch.bfloat16)
+    kc = torch.randn((B, hkv, L, D), device=dev).to(torch.bfloat16)
+    vt = torch.randn((B, hkv, D, L), device=dev).to(torch.bfloat16)
+    ctx = torch.tensor(ctxs, dtype=torch.int32, device=dev)
+    assert _lib.lib().bi_attention_workspace_bytes(B, 1, hq, hkv, L) > 0
+    k1, v1, k2, v2 = kc.clone(), vt.clone(), kc.clone(), vt.clone()
+    live = ctx > 0
+    a = ops.bi_attention_decode_qkv(qkv, w, w, inv, k1, v1, ctx, hq, hkv, SCALE, 1e-6)
+    _no_workspace(monkeypatch)
+    b = ops.bi_attention_decode_qkv(qkv, w, w, inv, k2, v2, ctx, hq, hkv, SCALE, 1e-6)
+    assert torch.equal(a[live], b[live]) and torch.equal(k1, k2) and torch.equal(v1, v2)
