@@ -415,6 +415,202 @@ __global__ __launch_bounds__(512) void lsm_resident_kernel(const LsmArgs a) {
   }
 }
 
+// The resident schedule for 16-bit logits: the row stays packed, so half the chip's storage holds it and TWO rows are
+// resident on a CU, one being read or written while the other is being reduced (one row per CU leaves the memory idle for
+// the reduction).  One work-group of 256 threads per row; 28 segments in registers (8 of them per segment and thread, 224
+// of 256), the rest in 78 KiB of LDS.  Bound: memory, 4 bytes per element; bf16 [1000,151936] 191 -> 154 us, [4096,151936]
+// 752 -> 512 (4.9 TB/s, 95 % of a copy), to fp32 933 -> 726.  Up to 256 rows, one per CU, the kernel above is ahead (twice
+// the threads for the reduction: 46 against 51 us at 256 rows, 81 against 63 at 300).  Forming the sums while loads are still
+// arriving (a barrier per four segments) changed nothing.  Every reduction is the one of the two-launch schedule.
+constexpr int kPackedRegSegs = kResidentRegSegs;
+constexpr int kPackedLdsElems = kResidentLdsFloats;                       // the same row lengths as above
+constexpr int kPackedLdsBytes = kPackedLdsElems * 2 + 2048;               // ... and the statistics
+static_assert(kPackedLdsBytes <= 80 * 1024, "two work-groups per CU");
+
+template <int IN>
+__device__ __forceinline__ void unpack4(const uint2& q, float (&v)[4]) {
+  if (IN == LSM_BF16) {
+    v[0] = bf16_lo(q.x); v[1] = bf16_hi(q.x); v[2] = bf16_lo(q.y); v[3] = bf16_hi(q.y);
+  } else {
+    const f16x2 a = __builtin_bit_cast(f16x2, q.x), b = __builtin_bit_cast(f16x2, q.y);
+    v[0] = (float)a[0]; v[1] = (float)a[1]; v[2] = (float)b[0]; v[3] = (float)b[1];
+  }
+}
+template <int IN>
+__device__ __forceinline__ void unpack_seg(const uint2 (&q)[4], float (&v)[4][4]) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) unpack4<IN>(q[i], v[i]);
+}
+
+// Keeps the compiler from carrying a segment's unpacked values from one phase to the next (they would not fit), and one
+// segment's work from mixing with the next one's.
+__device__ __forceinline__ void opaque(uint2 (&q)[4]) {
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 4; i++) asm volatile("" : "+v"(q[i].x), "+v"(q[i].y));
+}
+
+template <int IN, int OUT, bool SOFTMAX>
+__global__ __launch_bounds__(256, 2) void lsm_resident_packed_kernel(const LsmArgs a) {
+  constexpr int RS = kPackedRegSegs;
+  constexpr int MAXSEG = (int)((kResidentMaxCols + kSeg - 1) / kSeg);
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
+  uint16_t* lds_row = reinterpret_cast<uint16_t*>(lds_bytes);
+  float* red = reinterpret_cast<float*>(lds_bytes + kPackedLdsElems * 2);   // [MAXSEG][4] wave partials of a segment
+  float* stat = red + MAXSEG * 4;                                           // [MAXSEG][2] (max, sum), then 2 row values
+  static_assert((MAXSEG * 6 + 2) * 4 <= 2048, "statistics");
+  typedef typename LsmElem<OUT>::type out_t;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t row = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  const uint16_t* xr = static_cast<const uint16_t*>(a.x) + row * a.ldx;
+  out_t* orow = static_cast<out_t*>(a.out) + row * a.ldo;
+  const int cols = (int)a.cols, segs = a.segs;
+  const int nfull = cols >> 12;               // full segments
+  const int nreg = nfull < RS ? nfull : RS;   // ... of which in registers
+  const int lds0 = nreg * kSeg;               // first row element that lives in LDS
+  const int t4 = 4 * t;                       // thread's chunk i of segment k starts at row element k*4096 + t4 + 1024*i
+  constexpr uint32_t ninf = IN == LSM_BF16 ? 0xff80ff80u : 0xfc00fc00u;
+
+  // the ragged segment: what lies behind the row reads as -inf
+  auto load_ragged = [&](int sg, uint2 (&q)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = sg * kSeg + t4 + 1024 * i;
+      if (e + 3 < cols) {
+        q[i] = *reinterpret_cast<const uint2*>(xr + e);
+      } else {
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = e + j < cols ? (uint32_t)xr[e + j] : (ninf & 0xffffu);
+        q[i] = make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+      }
+    }
+  };
+  auto from_lds = [&](int sg, uint2 (&q)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = sg * kSeg + t4 + 1024 * i;
+      q[i] = e < cols ? *reinterpret_cast<const uint2*>(lds_row + (e - lds0)) : make_uint2(ninf, ninf);
+    }
+  };
+  auto finish = [&](int sg, const uint2 (&q)[4], bool ragged) __attribute__((always_inline)) {
+    const float gm = stat[2 * MAXSEG], lg = stat[2 * MAXSEG + 1];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float u[4];
+      unpack4<IN>(q[i], u);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const float y = (u[j] - gm) - lg;
+        u[j] = SOFTMAX ? fast_exp(y) : y;
+      }
+      const int e = sg * kSeg + t4 + 1024 * i;
+      if (!ragged) LsmElem<OUT>::store4(orow + e, u);
+      else store_chunk<OUT>(orow, e, cols, 1, u);
+    }
+  };
+
+  // ---- read the row once: first the part that lives in LDS, four segments per round trip through registers that the
+  // register part does not occupy yet
+  constexpr int LB = 4;
+  for (int sg0 = nreg; sg0 < segs; sg0 += LB) {
+    uint2 u[LB][4];
+#pragma unroll
+    for (int b = 0; b < LB; b++) {
+      const int sg = sg0 + b;
+      if (sg < nfull) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) u[b][i] = *reinterpret_cast<const uint2*>(xr + sg * kSeg + t4 + 1024 * i);
+      } else if (sg < segs) {
+        load_ragged(sg, u[b]);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < LB; b++) {
+      const int sg = sg0 + b;
+      if (sg < segs) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int e = sg * kSeg + t4 + 1024 * i;
+          if (e < cols) *reinterpret_cast<uint2*>(lds_row + (e - lds0)) = u[b][i];
+        }
+      }
+    }
+  }
+  uint2 v[RS][4];
+#pragma unroll
+  for (int k = 0; k < RS; k++)
+    if (k < nreg) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[k][i] = *reinterpret_cast<const uint2*>(xr + k * kSeg + t4 + 1024 * i);
+    }
+
+  // ---- segment maxima: per thread, butterfly, then the four wavefronts in order
+  auto seg_max = [&](int sg, const uint2 (&q)[4]) __attribute__((always_inline)) {
+    float u[4][4];
+    unpack_seg<IN>(q, u);
+    const float m = wave_max(seg_thread_max(u));
+    if (lane == 0) red[sg * 4 + wave] = m;
+  };
+  auto seg_sum = [&](int sg, const uint2 (&q)[4]) __attribute__((always_inline)) {
+    float u[4][4];
+    unpack_seg<IN>(q, u);
+    const float sm = wave_sum(seg_thread_expsum(u, stat[2 * sg]));
+    if (lane == 0) red[sg * 4 + wave] = sm;
+  };
+#pragma unroll
+  for (int k = 0; k < RS; k++)
+    if (k < nreg) {
+      opaque(v[k]);
+      seg_max(k, v[k]);
+    }
+  for (int sg = nreg; sg < segs; sg++) {
+    uint2 q[4];
+    from_lds(sg, q);
+    seg_max(sg, q);
+  }
+  __syncthreads();
+  if (t < segs) stat[2 * t] = fmaxf(fmaxf(red[4 * t], red[4 * t + 1]), fmaxf(red[4 * t + 2], red[4 * t + 3]));
+  __syncthreads();
+  // ---- segment sums of exp(x - segment max)
+#pragma unroll
+  for (int k = 0; k < RS; k++)
+    if (k < nreg) {
+      opaque(v[k]);
+      seg_sum(k, v[k]);
+    }
+  for (int sg = nreg; sg < segs; sg++) {
+    uint2 q[4];
+    from_lds(sg, q);
+    seg_sum(sg, q);
+  }
+  __syncthreads();
+  if (t < segs) stat[2 * t + 1] = ((red[4 * t] + red[4 * t + 1]) + red[4 * t + 2]) + red[4 * t + 3];
+  __syncthreads();
+  if (t < 64) {
+    float gmax, lg;
+    merge_segments(stat, segs, t, gmax, lg);
+    if (t == 0) {
+      stat[2 * MAXSEG] = gmax;
+      stat[2 * MAXSEG + 1] = lg;
+    }
+  }
+  __syncthreads();
+  // ---- write the row once
+#pragma unroll
+  for (int k = 0; k < RS; k++)
+    if (k < nreg) {
+      opaque(v[k]);
+      finish(k, v[k], false);
+    }
+  for (int sg = nreg; sg < segs; sg++) {
+    uint2 q[4];
+    from_lds(sg, q);
+    if (sg < nfull) finish(sg, q, false);
+    else finish(sg, q, true);
+  }
+}
+
 // One launch with the row resident on chip once there are enough rows to occupy the CUs with one work-group each (same
 // bits either way); that schedule does not touch the workspace.
 static bool lsm_resident(int64_t rows, int64_t cols) { return cols <= kResidentMaxCols && rows >= 192; }
@@ -425,26 +621,31 @@ size_t lsm_workspace_bytes(int64_t rows, int64_t cols) {
   return (size_t)rows * (size_t)segs * 2 * sizeof(float);
 }
 
+template <int IN, int OUT, bool SOFTMAX>
+static int lsm_resident_launch(const LsmArgs& a, hipStream_t stream) {
+  if constexpr (IN != LSM_F32) {
+    if (a.rows > 256) {
+      static std::atomic<uint64_t> done{0};
+      const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(lsm_resident_packed_kernel<IN, OUT, SOFTMAX>), kPackedLdsBytes, done);
+      if (e != hipSuccess) return hip_code(e);
+      hipLaunchKernelGGL((lsm_resident_packed_kernel<IN, OUT, SOFTMAX>), dim3((unsigned)a.rows), dim3(256), kPackedLdsBytes, stream, a);
+      return hip_code(hipGetLastError());
+    }
+  }
+  constexpr int lds = 160 * 1024;
+  static std::atomic<uint64_t> done{0};
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(lsm_resident_kernel<IN, OUT, SOFTMAX>), lds, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL((lsm_resident_kernel<IN, OUT, SOFTMAX>), dim3((unsigned)a.rows), dim3(512), lds, stream, a);
+  return hip_code(hipGetLastError());
+}
+
 template <int IN, int OUT>
 static int lsm_launch(const LsmArgs& a, bool resident, hipStream_t stream) {
-  if (resident) {
-    constexpr int lds = 160 * 1024;
-    if (a.write_softmax) {
-      static std::atomic<uint64_t> done{0};
-      hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(lsm_resident_kernel<IN, OUT, true>), lds, done);
-      if (e != hipSuccess) return hip_code(e);
-      hipLaunchKernelGGL((lsm_resident_kernel<IN, OUT, true>), dim3((unsigned)a.rows), dim3(512), lds, stream, a);
-    } else {
-      static std::atomic<uint64_t> done{0};
-      hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(lsm_resident_kernel<IN, OUT, false>), lds, done);
-      if (e != hipSuccess) return hip_code(e);
-      hipLaunchKernelGGL((lsm_resident_kernel<IN, OUT, false>), dim3((unsigned)a.rows), dim3(512), lds, stream, a);
-    }
-  } else {
-    const dim3 grid((unsigned)(a.rows * a.segs)), block(256);
-    hipLaunchKernelGGL((lsm_partial_kernel<IN>), grid, block, 0, stream, a);
-    hipLaunchKernelGGL((lsm_write_kernel<IN, OUT>), grid, block, 0, stream, a);
-  }
+  if (resident) return a.write_softmax ? lsm_resident_launch<IN, OUT, true>(a, stream) : lsm_resident_launch<IN, OUT, false>(a, stream);
+  const dim3 grid((unsigned)(a.rows * a.segs)), block(256);
+  hipLaunchKernelGGL((lsm_partial_kernel<IN>), grid, block, 0, stream, a);
+  hipLaunchKernelGGL((lsm_write_kernel<IN, OUT>), grid, block, 0, stream, a);
   return hip_code(hipGetLastError());
 }
 
