@@ -412,6 +412,7 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // the bits do not change.  The wide kernel takes over once its 128x256 tiles (times the split) occupy the chip.
 struct Plan {
   bool wide;
+  int few_waves;   // up to 64 rows: waves of the ring kernel (gemm_tree_few.hip), 0: the tiled kernel
   int split;       // power of two, divides 2^lb
   int T, flb, lb;  // tree of ONE shard
   size_t partial_bytes, parked_bytes;
@@ -478,6 +479,30 @@ static int column_regions(int M, int N, int K, int leaf_k, bool f16) {
   return best_na;
 }
 
+// Up to 64 rows on the ring kernel: waves per work-group (32 columns each) and K split, from an estimate of the pass:
+// rounds of 256 work-groups (the ring takes a CU's whole LDS), each 2.5 us plus its bytes at the 24 GB/s that a CU gets
+// when all of them stream (X rows come from the L2 and count a third), plus the shard combine.
+static int few_waves(int M, int N, int K, int lb, int* best_split) {
+  const int max_split = lb >= 3 ? 8 : (1 << lb);
+  const int rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  double best = 0;
+  int waves = 0;
+  for (int sp = 1, ls = 0; sp <= max_split; sp *= 2, ls++) {
+    if (lb - ls > TREE_FEW_LEVELS) continue;
+    for (int nw = 2; nw <= 6; nw++) {
+      const int64_t tiles = ((int64_t)N + nw * 32 - 1) / (nw * 32);
+      double t = (double)((tiles * sp + 255) / 256) * (2.5 + (double)K / sp * 2 * (nw * 32 + rows * 0.33) / 24.0e3);
+      if (sp > 1) t += 4.0 + (double)(sp + 1) * M * N * 2.0 / 5.0e6;
+      if (!waves || t < best) {
+        best = t;
+        waves = nw;
+        *best_split = sp;
+      }
+    }
+  }
+  return waves;
+}
+
 static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool rowmajor_b = false) {
   int T, flb, level_k;
   if (M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
@@ -493,7 +518,8 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
     // [64,16384] x [16384,8192] 75 on 256 against 97
     wide = wide_tiles * split >= (M == 64 ? 160 : 64);
   }
-  if (!wide) {
+  pl->few_waves = !wide && !rowmajor_b && M <= 64 ? few_waves(M, N, K, lb, &split) : 0;
+  if (!wide && !pl->few_waves) {
     const int bm = M <= 16 ? 16 : ((M <= 64 || rowmajor_b) ? 64 : 128), bn = M <= 16 ? 64 : 128;
     const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     split = 1;
@@ -882,6 +908,9 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
                a.T, a.flb, a.lb, a.vec_store, a.k_shard, a.c_shard};
     rc = wide_uses_deep_kernel(leaf_k, f16, a.flb, a.lb) ? gemm_tree_deep_launch(w, pl.split, stream)
                                                          : gemm_tree_wide_launch(w, leaf_k, f16, pl.split, stream);
+  } else if (pl.few_waves && lda < (1 << 22) && ldb_n < (1 << 22)) {
+    const WideArgs w{a.X, a.W, a.C, a.bias, nullptr, a.ldx, a.ldw, a.ldc, M, N, a.K, a.T, a.flb, a.lb, a.vec_store, a.k_shard, a.c_shard};
+    rc = gemm_tree_few_launch(w, leaf_k, f16, pl.few_waves, pl.split, stream);
   } else {
     if (f16) rc = leaf_k == 256 ? launch_tree<4, true>(a, pl.split, stream) : launch_tree<2, true>(a, pl.split, stream);
     else rc = leaf_k == 256 ? launch_tree<4, false>(a, pl.split, stream) : launch_tree<2, false>(a, pl.split, stream);
