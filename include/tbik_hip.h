@@ -496,9 +496,11 @@ int tbik_tree_combine_rmsnorm_bf16(const void* const* parts, int nparts,
  *   the wave that owns 16 columns of `gate` also owns the same 16 columns of `up`, runs the fixed-order pass over K once per
  *   matrix and stores silu(gate) * up -- the consumer inside the producer again.  Both products are rounded to bf16 before
  *   the activation, so the result is bit-identical to the two calls.  inter a multiple of 16, K a multiple of 32, no bias.
- *   Returns TBIK_ERR_UNSUPPORTED (3), with nothing launched, outside 5 .. 64 rows (fewer rows: the tree matmul of down_proj
- *   forms the activation itself, tbik_gemm_silu_mul_bf16; more: the tile kernels, which have no such epilogue): the caller
- *   then makes the two calls.
+ *   With many rows (those for which the product of 2*inter columns takes the tiles of 256 / 192 rows, from 384 rows on for
+ *   inter = 12288; K a multiple of 64) the two products of a tile meet in the work-group's LDS instead.
+ *   Returns TBIK_ERR_UNSUPPORTED (3), with nothing launched, for up to 4 rows (the tree matmul of down_proj forms the
+ *   activation itself, tbik_gemm_silu_mul_bf16) and between 64 rows and those many (tile kernels without such an
+ *   epilogue): the caller then makes the two calls.
  *   Replaces: the merged column-parallel projection through aten::mm (src/bio/batch_invariant_ops.py:442-447) followed by
  *             SiluAndMul, in front of the patched down_proj (src/patch/patch_tp_invariant.py:10-48).
  */

@@ -56,10 +56,14 @@ struct QuadArgs {
   int M, N, K;
   int vec_store;
   int row_step = 0;    // rows a tile of gemm_single_acc_quad_kernel owns (0 = all 128; 64, 32 or 16: see the kernel)
+  const uint16_t* W2 = nullptr;  // gated form of gemm_single_acc_256.hip only: the up half [N,K], row stride ldw (no bias)
 };
 int gemm_single_acc_quad_launch(const QuadArgs& a, hipStream_t stream);
 int gemm_single_acc_slab_launch(const QuadArgs& a, hipStream_t stream);  // at most 128 rows; TBIK_ERR_UNSUPPORTED: use another kernel
 int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream);  // any row count: tile width from a cost model
+// C[M,N] = silu(X W^T) * (X W2^T), both products rounded to bf16 first, where the product of 2 N columns runs on the tiles
+// of gemm_single_acc_256.hip; TBIK_ERR_UNSUPPORTED (nothing launched) elsewhere
+int gemm_single_acc_gated_launch(const QuadArgs& a, hipStream_t stream);
 // gemm_single_acc_256.hip: the same GEMM on tiles of 256 or 192 rows by 256 or 192 columns, for grids of more than one
 // round; K % 64 == 0
 int gemm_single_acc_256_launch(const QuadArgs& a, int tile_rows, int tile_cols, hipStream_t stream);

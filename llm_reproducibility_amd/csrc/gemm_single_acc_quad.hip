@@ -271,8 +271,11 @@ int gemm_single_acc_slab_launch(const QuadArgs& a, hipStream_t stream) {
 // schedule beats one pass over the weights at 3.5 TB/s.  Every width issues the same MFMA chain per element, so the
 // choice never changes a bit.  Examples (us, before -> after, vendor library GEMM in brackets): qkv [M,4096]x[4096,6144]
 // at M=256 39 -> 24 (37), M=512 54 -> 31 (34); gate_up (N=24576) M=384 101 -> 85 (70); 8192x8192 at M=256 83 -> 42 (68).
-int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream) {
-  if (a.M <= 0 || a.N <= 0 || a.K < quad::BK || (a.K % quad::BK) != 0) return TBIK_ERR_UNSUPPORTED;
+struct BalancedTile {
+  int rows256, cols256;  // tile of gemm_single_acc_256.hip; 0: the quad kernel on `tn` times 32 columns
+  int tn;
+};
+static BalancedTile balanced_tile(const QuadArgs& a) {
   const double nsl = (double)(a.K / quad::BK);
   const int64_t tm = ((int64_t)a.M + quad::BM - 1) / quad::BM;
   const double floor_us = (double)a.N * a.K * 2.0 / 3.5e6;
@@ -340,8 +343,26 @@ int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream) {
       }
     }
     const double t128 = rounds8 >= 6.0 ? rounds8 * (3.0 + nsl * 0.83) : best_sustained;
-    if (tiles8 > 256 && t_sq < t128) return gemm_single_acc_256_launch(a, shape[pick][0], shape[pick][1], stream);
+    if (tiles8 > 256 && t_sq < t128) return {shape[pick][0], shape[pick][1], best};
   }
+  return {0, 0, best};
+}
+
+int gemm_single_acc_gated_launch(const QuadArgs& a, hipStream_t stream) {
+  if (a.M <= 128 || a.N <= 0 || a.N > (1 << 30) || a.K < quad::BK || (a.K % quad::BK) != 0 || !a.W2) return TBIK_ERR_UNSUPPORTED;
+  QuadArgs both = a;
+  both.N = 2 * a.N;
+  const BalancedTile t = balanced_tile(both);
+  if (!t.rows256) return TBIK_ERR_UNSUPPORTED;
+  return gemm_single_acc_256_launch(a, t.rows256, t.cols256, stream);
+}
+
+int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream) {
+  if (a.M <= 0 || a.N <= 0 || a.K < quad::BK || (a.K % quad::BK) != 0) return TBIK_ERR_UNSUPPORTED;
+  const BalancedTile tile = balanced_tile(a);
+  if (tile.rows256) return gemm_single_acc_256_launch(a, tile.rows256, tile.cols256, stream);
+  const int best = tile.tn;
+  const int64_t tm = ((int64_t)a.M + quad::BM - 1) / quad::BM;
   // at most one narrow tile per CU: the deep ring (see the kernel); qkv at M=160 31 -> 25 us, [M,12288]x[12288,4096]
   // at M=192 73 -> 51
   const bool deep = tm * (((int64_t)a.N + 32 * best - 1) / (32 * best)) <= 256;

@@ -976,7 +976,8 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 // The merged gate/up projection with the activation behind it in the same launch: out[M, inter] = silu(x Wg^T) * (x Wu^T),
 // W = [2*inter, K] (rows 0 .. inter-1 gate, the rest up; the nn.Linear layout), both products rounded to bf16 first.
-// TBIK_ERR_UNSUPPORTED (nothing launched) outside the row counts of the windowed streaming kernel.
+// Up to 64 rows on the windowed streaming kernel; with more, where the product of 2 * inter columns runs on the tiles of
+// gemm_single_acc_256.hip, on the gated form of those.  TBIK_ERR_UNSUPPORTED (nothing launched) elsewhere.
 int gemm_silu_mul_dispatch(const void* x, int64_t ldx, const void* W, int64_t ldw, void* out, int64_t ldo, int M, int inter, int K,
                            hipStream_t stream) {
   if (M < 0 || inter <= 0 || K <= 0) return TBIK_ERR_INVALID;
@@ -985,6 +986,13 @@ int gemm_silu_mul_dispatch(const void* x, int64_t ldx, const void* W, int64_t ld
   if (ldx < K || ldw < K || ldo < inter) return TBIK_ERR_INVALID;
   if (!aligned16(x) || !aligned16(W) || (ldx & 7) || (ldw & 7) || (K & 7)) return TBIK_ERR_ALIGNMENT;
   if (reinterpret_cast<uintptr_t>(out) & 1) return TBIK_ERR_ALIGNMENT;
+  if (M > 64) {
+    if ((K & 63) || ldx >= (1 << 22) || ldw >= (1 << 22)) return TBIK_ERR_UNSUPPORTED;
+    QuadArgs qa{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(W), static_cast<uint16_t*>(out), nullptr, ldx, ldw, ldo,
+                M, inter, K, 0};
+    qa.W2 = static_cast<const uint16_t*>(W) + (int64_t)inter * ldw;
+    return gemm_single_acc_gated_launch(qa, stream);
+  }
   StreamArgs sa{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(W), static_cast<uint16_t*>(out), nullptr, ldx, ldw, ldo,
                 M, inter, K, ((reinterpret_cast<uintptr_t>(out) & 7) == 0 && (ldo & 3) == 0) ? 1 : 0,
                 static_cast<const uint16_t*>(W) + (int64_t)inter * ldw};

@@ -575,11 +575,12 @@ def gemm_tree_silu_mul(gate: torch.Tensor, up: torch.Tensor, B: torch.Tensor, bi
 
 def gemm_silu_mul(x: torch.Tensor, W: torch.Tensor) -> torch.Tensor:
     """bi_silu_mul(bi_gemm(x, W.t())) for the merged gate/up weight W [2*inter, K] (nn.Linear layout): one launch
-    (`bi_gemm_silu_mul_bf16`) for 5 .. 64 bf16 rows, the two calls otherwise.  Same bits either way."""
+    (`bi_gemm_silu_mul_bf16`) for 5 .. 64 bf16 rows and for the many that run on its 256-row tiles, the two calls
+    otherwise.  Same bits either way."""
     _require_gpu(x, W)
     M, K = x.shape
     inter = W.shape[0] // 2
-    fusable = (x.dtype == torch.bfloat16 and W.dtype == torch.bfloat16 and 4 < M <= 64 and W.shape[0] == 2 * inter and inter % 16 == 0
+    fusable = (x.dtype == torch.bfloat16 and W.dtype == torch.bfloat16 and M > 4 and W.shape[0] == 2 * inter and inter % 16 == 0
                and K % 32 == 0 and W.stride(1) == 1 and W.stride(0) % 8 == 0 and _aligned16(W) and not torch.compiler.is_compiling()
                and ("mm_silu", M, inter, K) not in _declined)
     if fusable:
