@@ -481,14 +481,16 @@ static int column_regions(int M, int N, int K, int leaf_k, bool f16) {
 
 // Up to 64 rows on the ring kernel: waves per work-group (32 columns each) and K split, from an estimate of the pass:
 // rounds of 256 work-groups (the ring takes a CU's whole LDS), each 2.5 us plus its bytes at the 24 GB/s that a CU gets
-// when all of them stream (X rows come from the L2 and count a third), plus the shard combine.
+// when all of them stream (X rows come from the L2 and count a third), plus the shard combine.  No cut whose partial
+// results outgrow the static scratch: tbik_gemm_bf16_static takes every decode batch ([32,8192]x[8192,151936] would be
+// cut into four for the last round's sake, 37 MiB of partials).
 static int few_waves(int M, int N, int K, int lb, int* best_split) {
   const int max_split = lb >= 3 ? 8 : (1 << lb);
   const int rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
   double best = 0;
   int waves = 0;
   for (int sp = 1, ls = 0; sp <= max_split; sp *= 2, ls++) {
-    if (lb - ls > TREE_FEW_LEVELS) continue;
+    if (lb - ls > TREE_FEW_LEVELS || (sp > 1 && (int64_t)sp * M * N * 2 > TBIK_STATIC_SCRATCH_BYTES)) continue;
     for (int nw = 2; nw <= 6; nw++) {
       const int64_t tiles = ((int64_t)N + nw * 32 - 1) / (nw * 32);
       double t = (double)((tiles * sp + 255) / 256) * (2.5 + (double)K / sp * 2 * (nw * 32 + rows * 0.33) / 24.0e3);

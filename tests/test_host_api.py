@@ -106,6 +106,13 @@ def test_workspace_query_and_plan_come_from_one_decision():
     assert L.tbik_gemm_plan_info(8, 8, 256, 256, 0, 0, None) == _lib.TBIK_ERR_INVALID
 
 
+@pytest.mark.parametrize("M,N,K,leaf", [(29, 151936, 8192, 256), (63, 262144, 8192, 256), (47, 200000, 25600, 128), (63, 40000, 12288, 256)])
+def test_decode_batches_fit_the_static_scratch(M, N, K, leaf):
+    """However wide the matrix, a batch of fewer than 64 rows (64 may run on 128-row tiles) is not cut into more partial results than the array of
+    tbik_gemm_bf16_static holds."""
+    assert _lib.lib().tbik_gemm_workspace_bytes(M, N, K, leaf) <= 32 * 1024 * 1024
+
+
 def test_host_argument_checks_fire_before_any_launch():
     L = _lib.lib()
     # null pointers / bad sizes are rejected on the host, so these are safe without a GPU
