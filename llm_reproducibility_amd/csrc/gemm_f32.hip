@@ -224,7 +224,8 @@ static int f32_launch(const GemmF32Args& a, hipStream_t stream) {
   const int64_t tiles = (int64_t)((a.M + S::RX - 1) / S::RX) * ((a.N + S::RW - 1) / S::RW);
   if (tiles > 0x7fffffff) return TBIK_ERR_INVALID;
   const int64_t reach = 0xffffff00ll - 128;   // byte offsets inside a tile's operand rows are 32 bits
-  if (a.ldx * 4 * (S::RX - 1) > reach || a.ldw * 4 * (S::RW - 1) > reach) return TBIK_ERR_UNSUPPORTED;
+  const int rx = a.M < S::RX ? a.M : S::RX, rw = a.N < S::RW ? a.N : S::RW;
+  if ((rx > 1 && a.ldx > reach / 4 / (rx - 1)) || (rw > 1 && a.ldw > reach / 4 / (rw - 1))) return TBIK_ERR_UNSUPPORTED;
   static std::atomic<uint64_t> done{0};
   hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_f32_kernel<WM, WN, TM, TN, NS, TREE>), NS * S::STAGE, done);
   if (e != hipSuccess) return hip_code(e);
@@ -271,6 +272,31 @@ static int f32_run(const GemmF32Args& a, int cfg, hipStream_t stream) {
   return f32_launch<2, 4, 4, 2, 4, false>(a, stream);
 }
 
+// Rows so far apart that a tile's rows do not fit 32-bit offsets (138 MB for 32 rows) go to the smallest tile, which reaches
+// furthest, and beyond that to halves of the product: a single row has no distance to the next.
+template <bool TREE>
+static int f32_run_reaching(const GemmF32Args& a, int cfg, hipStream_t stream) {
+  int rc = f32_run<TREE>(a, cfg, stream);
+  if (rc == TBIK_ERR_UNSUPPORTED && cfg != 0) rc = f32_run<TREE>(a, 0, stream);
+  if (rc != TBIK_ERR_UNSUPPORTED || (a.M == 1 && a.N == 1)) return rc;
+  GemmF32Args lo = a, hi = a;
+  if (a.N == 1 || (a.M > 1 && a.ldx >= a.ldw)) {
+    lo.M = a.M / 2;
+    hi.M = a.M - lo.M;
+    hi.X += (int64_t)lo.M * a.ldx;
+    hi.C += (int64_t)lo.M * a.ldc;
+  } else {
+    lo.N = a.N / 2;
+    hi.N = a.N - lo.N;
+    hi.W += (int64_t)lo.N * a.ldw;
+    hi.C += lo.N;
+    if (a.bias) hi.bias += lo.N;
+    hi.vec_store = a.vec_store && (lo.N & 3) == 0;
+  }
+  rc = f32_run_reaching<TREE>(lo, 0, stream);
+  return rc == TBIK_OK ? f32_run_reaching<TREE>(hi, 0, stream) : rc;
+}
+
 int gemm_f32_dispatch(bool tree, const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n, void* C,
                       int64_t ldc, int M, int N, int K, int leaf_k, const void* bias, hipStream_t stream) {
   if (M < 0 || N < 0 || K <= 0) return TBIK_ERR_INVALID;
@@ -291,11 +317,8 @@ int gemm_f32_dispatch(bool tree, const void* A, int64_t lda, const void* B, int6
     a.flb = flb;
     a.lb = level_k - 1;
   }
-  // rows so far apart that a tile's rows do not fit 32-bit offsets go to the smallest tile, which reaches furthest
   const int cfg = f32_pick(M, N, K, tree);
-  int rc = tree ? f32_run<true>(a, cfg, stream) : f32_run<false>(a, cfg, stream);
-  if (rc == TBIK_ERR_UNSUPPORTED && cfg != 0) rc = tree ? f32_run<true>(a, 0, stream) : f32_run<false>(a, 0, stream);
-  return rc;
+  return tree ? f32_run_reaching<true>(a, cfg, stream) : f32_run_reaching<false>(a, cfg, stream);
 }
 
 }  // namespace tbik

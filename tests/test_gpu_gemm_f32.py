@@ -44,3 +44,14 @@ def test_fp32_tree_tile_edges(dev, M, N, K):
     xr, wr = xd + 0.37 * xd.sin(), wd * 0.13
     full = matmul_tp_persistent(xr, wr.t())
     assert torch.equal(matmul_tp_persistent(xr[-1:], wr.t()), full[-1:])
+
+
+def test_fp32_rows_far_apart(dev):
+    """Operand rows so far apart that a tile of 32 does not reach them all with 32-bit byte offsets."""
+    M, N, K, ld = 40, 33, 128, 36_000_000
+    x, w, xd, wd = _operands(M, N, K, dev)
+    far = torch.empty((M - 1) * ld + K, device=dev).as_strided((M, K), (ld, 1))
+    far.copy_(xd)
+    assert torch.equal(bio.matmul_persistent(far, wd.t()).cpu(), x @ w.t())
+    assert torch.equal(matmul_tp_persistent(wd, far.t()).cpu(), w @ x.t())
+    assert torch.equal(bio.matmul_persistent(far[:3], wd.t()).cpu(), (x @ w.t())[:3])
