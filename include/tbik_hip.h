@@ -89,8 +89,8 @@ size_t tbik_gemm_workspace_bytes_rowmajor_b(int M, int N, int K, int leaf_k, int
 /*
  * How tbik_gemm_bf16 (f16 != 0: tbik_gemm_f16) would run this problem: the decision the workspace size above comes
  * from, for callers and tests that want to see it (host only, launches nothing, no effect on any result).
- *   out5[0] path: 0 one launch with K cut over the waves of a work-group (a few rows), 1 128x128 tiles,
- *                 2 two column regions with a K split each, 3 one grid with one K split
+ *   out5[0] path: 0 one launch with K cut over the waves of a work-group (a few rows), 1 128x128 tiles (up to 512 rows),
+ *                 2 two column regions with a K split each, 3 one grid of any other kind with one K split
  *   out5[1] K split (of the first region for path 2, 0 if that region runs on 128x128 tiles; waves per strip for path 0)
  *   out5[2] columns of the first region (path 2), else 0
  *   out5[3] K split of the second region (path 2), else 0

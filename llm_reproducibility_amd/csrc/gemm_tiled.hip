@@ -540,15 +540,18 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
   return true;
 }
 
-// 64 .. 512 rows, leaves of 256: one to four rows of 128x256 tiles need a deep cut of K to occupy the chip, and the pass
-// over that many partial results then weighs as much as a quarter of the GEMM.  Tiles of 128 columns
-// (gemm_tree_quad.hip) occupy it with half the cut.  That kernel is slower per slice than the 128x256-tile kernels, so it
-// is taken only where a shard is short and the grid close to one work-group per CU, the region where sweeps over
-// N = 1024 .. 8192 and K = 2048 .. 16384 on MI355X measured it ahead:
-//   * 64 .. 128 rows (one row of tiles): shards of 512 .. 1024 of K on 160 .. 256 work-groups, or up to 1536 on
-//     224 .. 256 -- 8 % on average, up to 20 %; with fewer rows the 64-row tiles of the tiled kernel win;
-//   * 129 .. 512 rows (two to four rows of tiles): only shards of at most 1024 and a cut into at least four -- 6 % on
-//     average, ahead in every one of 59 shapes in three alternating repetitions each.
+// Short shards, leaves of 256: where K cannot be cut into long enough pieces, tiles of 128x256 leave half of the chip idle
+// or need a deep cut and a pass over that many partial results.  Tiles of 128x128 (gemm_tree_quad.hip) are twice as many.
+// That kernel is slower per slice than the 128x256-tile kernels, so it is taken only where a shard is short and the whole
+// grid one round of the chip.  Measured on MI355X against the 128x256-tile kernels with their own best split, M = 96 ..
+// 2048, N = 2048 .. 5120, K = 512 .. 6144, weights cold, bf16 and fp16 (240 shapes):
+//   * uncut (the K of a tensor-parallel rank), 96 .. 256 work-groups: 15 .. 60 % faster, [1024,1536]x[1536,4096] 24.9 ->
+//     19.6 us, [768,1024]x[1024,4096] 22.0 -> 13.7, [512,768]x[768,4096] 15.0 -> 11.6;
+//   * cut, shards of up to 768: 96 work-groups or more, 15 .. 27 %, [1024,1536]x[1536,2048] in fp16 19.6 -> 16.6; shards of
+//     up to 1024: from 192 work-groups on up to 26 %, 160 are level (up to 128 rows, whose other tiles are nearly empty, 160
+//     win as well); shards of up to 1536: from 224 on, 0 .. 8 % (192 and fewer lose up to 5 %).
+// Of several cuts the one of the least estimated time: 5.5 us + 8 ns per k and the shard combine.  A column region keeps
+// the narrower rule it was measured with (bf16, up to 512 rows): a region on these tiles is a launch of its own.
 // The shards are aligned subtrees like every other K split, so the bits do not change.
 struct NarrowPlan {
   int split;
@@ -556,25 +559,32 @@ struct NarrowPlan {
   size_t partial_bytes;
 };
 
-static bool narrow_plan(int M, int N, int K, int leaf_k, bool f16, NarrowPlan* np) {
+static bool narrow_plan(int M, int N, int K, int leaf_k, bool f16, bool whole_problem, NarrowPlan* np) {
   int T, flb, level_k;
-  if (f16 || leaf_k != 256 || M < 64 || M > 512 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
-  // exactly 64 rows: the 64-row tiles of the tiled kernel cut K at most eightfold, which fills the chip from 32 column
-  // tiles on and then beats 128-row tiles that are half empty ([64,8192] x [8192,4096] 25.6 -> 21.1 us, [64,4096] x
-  // [4096,4096] 14.7 -> 13.5); narrower matrices need the deeper cut of this plan (N = 2048: 15.5 against 16.8)
-  if (M == 64 && N >= 4096) return false;
+  if (leaf_k != 256 || M < 64 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
+  if (!whole_problem && (f16 || M > 512)) return false;
+  // exactly 64 rows: the kernels of up to 64 rows cut K at most eightfold, which fills the chip from 32 column tiles on and
+  // then beats 128-row tiles that are half empty ([64,8192] x [8192,4096] 25.6 -> 21.1 us, [64,4096] x [4096,4096] 14.7 ->
+  // 13.5); narrower matrices need the deeper cut of this plan (N = 2048: 15.5 against 16.8)
+  if (M == 64 && (f16 || N >= 4096)) return false;
   const int lb = level_k - 1;
-  const int64_t tiles = (((int64_t)N + 127) / 128) * ((M + 127) / 128);
+  const int64_t tiles = (((int64_t)N + 127) / 128) * (((int64_t)M + 127) / 128);
   int best = 0, best_ls = 0;
-  int64_t best_wgs = 0;
+  double best_t = 0;
   for (int ls = 0; ls <= lb && ls <= 5; ls++) {
     const int sp = 1 << ls;
     const int ks = K / sp;
     const int64_t wgs = tiles * sp;
-    if (lb - ls > 1 || ks < 512 || ks > 1536 || wgs > 256 || wgs < (ks > 1024 ? 224 : 160)) continue;
-    if (M > 128 && (sp < 4 || ks > 1024)) continue;
-    if (wgs > best_wgs) {
-      best_wgs = wgs;
+    if (lb - ls > 1 || ks < 512 || ks > 1536 || wgs > 256) continue;
+    if (whole_problem && M > 64) {
+      const int least = sp == 1 || ks <= 768 ? 96 : ks <= 1024 ? (M <= 128 ? 160 : 192) : 224;
+      if (wgs < least) continue;
+    } else {
+      if (wgs < (ks > 1024 ? 224 : 160) || (M > 128 && (sp < 4 || ks > 1024))) continue;
+    }
+    const double t = 5.5 + 0.008 * ks + (sp > 1 ? 3.0 + (double)(sp + 1) * M * N * 2.0 / 5.0e6 : 0.0);
+    if (!best || t < best_t) {
+      best_t = t;
       best = sp;
       best_ls = ls;
     }
@@ -603,7 +613,7 @@ struct RegionPlan {
 // it, so the bytes the caller is told to bring are the bytes the launch uses.
 enum TreePath {
   PATH_STRIP = 0,    // a few rows: one launch, K cut over the waves of a work-group, no workspace
-  PATH_NARROW = 1,   // 64 .. 512 rows, short shards: 128x128 tiles (narrow_plan)
+  PATH_NARROW = 1,   // short shards: 128x128 tiles (narrow_plan)
   PATH_REGIONS = 2,  // two column regions, each with a K split of its own (column_regions)
   PATH_SINGLE = 3,   // one grid of 128x256 tiles or of the small tiles, one K split (make_plan)
 };
@@ -657,7 +667,7 @@ static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b
       tp->path = PATH_STRIP;
       return true;
     }
-    if (narrow_plan(M, N, K, leaf_k, f16, &tp->narrow)) {
+    if (narrow_plan(M, N, K, leaf_k, f16, whole_problem, &tp->narrow)) {
       tp->path = PATH_NARROW;
       tp->bytes = tp->narrow.partial_bytes;
       return true;
@@ -680,14 +690,15 @@ size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowm
 }
 
 // What tree_plan() chose for a shape, for callers and tests that want to know (no effect on any result):
-// out[0] path (0 one-launch few-rows kernel, 1 128x128 tiles, 2 two column regions, 3 one grid), out[1] K split (of the
+// out[0] path (0 one-launch few-rows kernel, 1 128x128 tiles for up to 512 rows, 2 two column regions, 3 one grid of any
+// other kind, 128x128 tiles of more rows among them), out[1] K split (of the
 // first region for path 2; waves per strip for path 0), out[2] columns of the first region (path 2, else 0), out[3] K
 // split of the second region (path 2, else 0), out[4] 1 when the two regions go out as one launch.
 int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, int out[5]) {
   TreePlan tp;
   if (!out) return TBIK_ERR_INVALID;
   if (!tree_plan(M, N, K, leaf_k, f16, rowmajor_b, true, &tp)) return TBIK_ERR_INVALID;
-  out[0] = (int)tp.path;
+  out[0] = tp.path == PATH_NARROW && M > 512 ? (int)PATH_SINGLE : (int)tp.path;
   out[1] = tp.path == PATH_STRIP ? tp.strip_waves : tp.path == PATH_NARROW ? tp.narrow.split
            : tp.path == PATH_REGIONS ? (tp.regions.narrow_a ? 0 : tp.regions.a.split) : tp.single.split;
   out[2] = tp.path == PATH_REGIONS ? tp.regions.na : 0;
@@ -826,7 +837,21 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
       w.vec_store = (N & 3) == 0 ? 1 : 0;
       w.bias = nullptr;
     }
-    const int rc = gemm_tree_quad_launch(w, np.split, stream);
+    int rc;
+    if (lda < (1 << 22) && ldb_n < (1 << 22)) {
+      rc = gemm_tree_quad_launch(w, f16, np.split, stream);
+    } else {  // rows too far apart for that kernel's 32-bit offsets: the tiled kernel on the same shards
+      a.T = np.T;
+      a.flb = np.flb;
+      a.lb = np.lb;
+      a.k_shard = a.K = K / np.split;
+      a.C = w.C;
+      a.ldc = w.ldc;
+      a.c_shard = (int64_t)M * N;
+      a.vec_store = w.vec_store;
+      a.bias = w.bias;
+      rc = f16 ? launch_tree<4, true>(a, np.split, stream) : launch_tree<4, false>(a, np.split, stream);
+    }
     if (rc != TBIK_OK || np.split == 1) return rc;
     const void* parts[32];
     for (int i = 0; i < np.split; i++) parts[i] = static_cast<uint8_t*>(ws) + (size_t)i * M * N * sizeof(uint16_t);

@@ -1,11 +1,11 @@
-// Tree-ordered bf16 GEMM for gfx950, path of 64 .. 512 rows with short K shards: 128x128 tiles, 4 wavefronts (one per
+// Tree-ordered 16-bit GEMM for gfx950, path of short K shards (64 rows and more): 128x128 tiles, 4 wavefronts (one per
 // SIMD) of 64x64 each, K streamed through a 4-slot LDS ring in 64-element slices -- the pipeline of
 // gemm_single_acc_quad.hip with the merge tree of gemm_tree_wide.hip, and the whole tree of a shard in registers.
 // Replaces matmul_kernel_tp_persistent, src/tbik/tree_based_matmul.py:50-187, where one row of 128x256 tiles needs a
 // cut of K into sixteen shards (and a pass over sixteen partial results) to occupy the chip: with tiles half as wide
 // eight shards do.  Per element the arithmetic is that of every other tree kernel of this library (one chain of
 // 16x16x32 MFMAs per leaf over k ascending, one rounding per leaf, a left-to-right sum over the leaves of a group, an
-// adjacent-pair tree over the groups, every node rounded to bf16), so the bits are the same.
+// adjacent-pair tree over the groups, every node rounded), so the bits are the same.
 //
 // A wave's tile is 64x64: 32 packed registers per tree level, so the running sum, the pending leaf and one binary level
 // (shards of at most two groups of leaves) sit next to the accumulators without a workspace.  The finished leaf j is
@@ -23,6 +23,9 @@
 // 75 us against 70 us for the 128x256-tile kernels with their K split; [256,K]x[K,N] 10-20 % slower from K = 6144 on),
 // which is why the tile widths of 32, 64 and 96 columns, the deeper rings and the leaves of 128 that this pipeline
 // also allows were measured and are not built.
+// An uncut product of a short K (the shard of a tensor-parallel rank) gains most: no pass over partial results and twice
+// the work-groups ([1024,1536]x[1536,4096] 24.9 -> 19.6 us; the rule of the dispatch and its figures stand at narrow_plan in
+// gemm_tiled.hip).  fp16 merges a register with one packed addition.
 #include <type_traits>
 
 #include "common.h"
@@ -47,9 +50,10 @@ enum Kind { K_FIRST = 0, K_ADD = 1, K_CARRY = 2 };  // the pending leaf opens a 
 
 // TN: 16-column MFMA tiles per wave (4: the 128-column tile).  LS: slices per leaf (4: leaves of 256).  NSLOT: slices of
 // the ring.
-template <int TN, int NSLOT, int LS>
+template <int TN, int NSLOT, int LS, bool F16>
 __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p) {
   using namespace tq;
+  using Num = Num16<F16>;
   static_assert(NSLOT >= 3 && TN >= 1 && TN <= 4, "tile shape");
   constexpr int BN = Shape<TN>::BN, STAGE_BYTES = Shape<TN>::STAGE_BYTES, NDMA = Shape<TN>::NDMA;
   constexpr int NREG = TM * TN * 2;  // packed bf16 pairs per lane per tree level
@@ -169,6 +173,12 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
               const int u = r - r0;
               if (KIND == K_FIRST) {
                 if (pc == 0) s0[r] = t[r];
+              } else if (F16) {
+                if (pc == 0) v[u] = Num::add(s0[r], t[r]);  // one packed instruction
+                if (pc == 2) {
+                  if (KIND == K_ADD) s0[r] = v[u];
+                  if (KIND == K_CARRY) lv[0][r] = v[u];
+                }
               } else {
                 if (pc == 0) {
                   xl[u] = bf16_lo(t[r]);
@@ -207,15 +217,15 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
               if (i == LS - 1 && kk == 1 && q >= 1) prow = q - 1;
               if (i == 0 && kk == 0 && q == 0) prow = TM - 1;  // of the leaf before (zeros in front of the first leaf)
               if (prow >= 0) {
-                t[(prow * TN + jj) * 2] = pack_bf16x2(acc[prow][jj][0], acc[prow][jj][1]);
-                t[(prow * TN + jj) * 2 + 1] = pack_bf16x2(acc[prow][jj][2], acc[prow][jj][3]);
+                t[(prow * TN + jj) * 2] = Num::pack(acc[prow][jj][0], acc[prow][jj][1]);
+                t[(prow * TN + jj) * 2 + 1] = Num::pack(acc[prow][jj][2], acc[prow][jj][3]);
               }
             }
             __builtin_amdgcn_sched_barrier(0);
           };
 #pragma unroll
           for (int jj = 0; jj < TN; jj++) {
-            acc[q][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[kk][jj], fx[kk][q], (i == 0 && kk == 0) ? zero : acc[q][jj], 0, 0, 0);
+            acc[q][jj] = Num::mfma(fw[kk][jj], fx[kk][q], (i == 0 && kk == 0) ? zero : acc[q][jj]);
             behind(jj);
           }
 #pragma unroll
@@ -259,18 +269,18 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
   // the last leaf: its last row, then every level carries and t ends as the root
 #pragma unroll
   for (int b = 0; b < TN; b++) {
-    t[((TM - 1) * TN + b) * 2] = pack_bf16x2(acc[TM - 1][b][0], acc[TM - 1][b][1]);
-    t[((TM - 1) * TN + b) * 2 + 1] = pack_bf16x2(acc[TM - 1][b][2], acc[TM - 1][b][3]);
+    t[((TM - 1) * TN + b) * 2] = Num::pack(acc[TM - 1][b][0], acc[TM - 1][b][1]);
+    t[((TM - 1) * TN + b) * 2 + 1] = Num::pack(acc[TM - 1][b][2], acc[TM - 1][b][3]);
   }
   if (c0 != 0) {
 #pragma unroll
-    for (int r = 0; r < NREG; r++) t[r] = add_bf16x2(s0[r], t[r]);
+    for (int r = 0; r < NREG; r++) t[r] = Num::add(s0[r], t[r]);
   }
 #pragma unroll
   for (int l = 0; l < MAXL; l++) {
     if (l < p.lb) {
 #pragma unroll
-      for (int r = 0; r < NREG; r++) t[r] = add_bf16x2(lv[l][r], t[r]);
+      for (int r = 0; r < NREG; r++) t[r] = Num::add(lv[l][r], t[r]);
     }
   }
 
@@ -286,9 +296,9 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (n + e < p.N) bv[e] = bf16_bits_to_f32(p.bias[n + e]);
-        lo = add_bf16x2(lo, pack_bf16x2(bv[0], bv[1]));
-        hi = add_bf16x2(hi, pack_bf16x2(bv[2], bv[3]));
+          if (n + e < p.N) bv[e] = Num::to_f32(p.bias[n + e]);
+        lo = Num::add(lo, Num::pack(bv[0], bv[1]));
+        hi = Num::add(hi, Num::pack(bv[2], bv[3]));
       }
       uint16_t* dst = p.C + shard * p.c_shard + (int64_t)m * p.ldc + n;
       if (p.vec_store && n + 3 < p.N) {
@@ -303,7 +313,7 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
   }
 }
 
-template <int TN, int NSLOT, int LS>
+template <int TN, int NSLOT, int LS, bool F16>
 static int tq_launch(const WideArgs& a, int split, hipStream_t stream) {
   using namespace tq;
   constexpr int BN = Shape<TN>::BN;
@@ -314,14 +324,16 @@ static int tq_launch(const WideArgs& a, int split, hipStream_t stream) {
   if (a.T <= 0 || a.K != a.T * LS * BK || a.lb < 0 || a.lb > MAXL || a.flb < 1) return TBIK_ERR_UNSUPPORTED;
   if (a.ldx >= (1 << 22) || a.ldw >= (1 << 22)) return TBIK_ERR_UNSUPPORTED;  // 32-bit in-tile byte offsets
   static std::atomic<uint64_t> done{0};
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tree_quad_kernel<TN, NSLOT, LS>), (int)smem, done);
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tree_quad_kernel<TN, NSLOT, LS, F16>), (int)smem, done);
   if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((gemm_tree_quad_kernel<TN, NSLOT, LS>), dim3((unsigned)tiles, (unsigned)split), dim3(NT), smem, stream, a);
+  hipLaunchKernelGGL((gemm_tree_quad_kernel<TN, NSLOT, LS, F16>), dim3((unsigned)tiles, (unsigned)split), dim3(NT), smem, stream, a);
   return hip_code(hipGetLastError());
 }
 
 // a ring of four slices (128 KiB): 2-5 % ahead of three on half of the shapes measured, level with it on the rest; five
 // are no better than three
-int gemm_tree_quad_launch(const WideArgs& a, int split, hipStream_t stream) { return tq_launch<4, 4, 4>(a, split, stream); }
+int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream) {
+  return f16 ? tq_launch<4, 4, 4, true>(a, split, stream) : tq_launch<4, 4, 4, false>(a, split, stream);
+}
 
 }  // namespace tbik
