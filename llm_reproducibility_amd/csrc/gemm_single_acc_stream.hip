@@ -11,9 +11,12 @@
 // (double-buffered, one barrier per window), which keeps the vector-memory queue of every wave for the weights.
 // With a handful of rows all of X is staged up front and the waves never meet again; work-groups shrink to one
 // or two strips when N is small, so that every CU gets some.  Same MFMA chain per element as the tiled and the
-// quad kernels, hence the same bits.
+// quad kernels, hence the same bits.  Narrow matrices, lm_head and most gated calls take the ring kernel below.
+#include <algorithm>
+
 #include "common.h"
 #include "gemm_args.h"
+#include "lds_direct.h"
 #include "rmsnorm_row.h"
 #include "silu_mul.h"
 
@@ -311,6 +314,176 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_single_acc_stream_kernel(con
   }
 }
 
+// The ring kernel: weights and activations of a work-group go global -> LDS directly, slices of 128 k (rows of 256 bytes) up to
+// eleven slices ahead.  What bounds a decode-sized mm is bytes in flight: a wave of the windowed kernel holds one or two windows of
+// its strip in registers, and a matrix of few columns is a chain on few waves (K cannot be cut: one accumulator per element);
+// here the loads need no registers.  X travels with the weights through the ring, so its rows cost no wait of their own: the
+// time hardly grows with the rows (figures at ring_waves).
+// A wave multiplies one strip of 16 columns (GATED: of both halves) by all rows; it loads the weight rows that it alone
+// multiplies and its share of the X rows, and one barrier per slice hands the X rows around.
+namespace ring {
+constexpr int BK = 128, ROWB = BK * 2;
+template <int MB, int NW, bool GATED>
+struct Shape {
+  static constexpr int TN = GATED ? 2 : 1;
+  static constexpr int STAGE = (MB + NW * TN) * 16 * ROWB;
+  static constexpr int XDMA = (MB * 4 + NW - 1) / NW;  // direct loads of 4 X rows per wave and slice
+  static constexpr int NDMA = XDMA + TN * 4;           // ... and of 4 weight rows
+  static constexpr int FIT = 160 * 1024 / STAGE, CNT = 63 / NDMA + 1;
+  static constexpr int CAP = FIT < CNT ? FIT : CNT;
+  static constexpr int NSLOT = CAP < 12 ? CAP : 12;
+};
+}  // namespace ring
+
+template <int MB, int NW, bool F16, bool GATED>
+__global__ __launch_bounds__(NW * 64) void gemm_single_acc_ring_kernel(const StreamArgs p) {
+  using namespace ring;
+  using Num = Num16<F16>;
+  using S = Shape<MB, NW, GATED>;
+  constexpr int TN = S::TN, NDMA = S::NDMA, XDMA = S::XDMA, NSLOT = S::NSLOT;
+  static_assert(NSLOT >= 3 && (NSLOT - 1) * NDMA < 64 && NSLOT * S::STAGE <= 160 * 1024, "ring");
+  extern __shared__ __attribute__((aligned(16))) uint8_t xs[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = (xcd_contiguous_tile(blockIdx.x, gridDim.x) * NW + wave) * 16;  // the wave's strip
+  const int wrow = min(n0, p.N - 1);
+  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(p.X);
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.W + (int64_t)wrow * p.ldw);
+  const uint8_t* w2base = GATED ? reinterpret_cast<const uint8_t*>(p.W2 + (int64_t)wrow * p.ldw) : wbase;
+  // byte offsets of this lane's loads and the LDS place of each: row r of a group of 16 keeps chunk c at position c ^ r.
+  // Rows past the edge are clamped (their results are not stored); where NW does not divide the X rows the last waves load
+  // the last group once more: same bytes, same place.
+  uint32_t voff[NDMA], dst[NDMA];
+  {
+    const int r = lane >> 4, pos = lane & 15;
+#pragma unroll
+    for (int i = 0; i < XDMA; i++) {
+      const int grp = min(i * NW + wave, MB * 4 - 1), row = grp * 4 + r;
+      voff[i] = (uint32_t)(((int64_t)min(row, p.M - 1) * p.ldx + (pos ^ (row & 15)) * 8) * 2);
+      dst[i] = grp * 1024;
+    }
+#pragma unroll
+    for (int i = 0; i < TN * 4; i++) {
+      const int row = (i & 3) * 4 + r;
+      voff[XDMA + i] = (uint32_t)(((int64_t)(min(n0 + row, p.N - 1) - wrow) * p.ldw + (pos ^ row) * 8) * 2);
+      dst[XDMA + i] = (MB * 16 + wave * TN * 16) * ROWB + i * 1024;
+    }
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)xs;
+  auto issue = [&](int s, int slot) __attribute__((always_inline)) {
+    const uint32_t base = lds0 + slot * S::STAGE;
+#pragma unroll
+    for (int i = 0; i < NDMA; i++)
+      dma16(base + dst[i], voff[i], (i < XDMA ? xbase : i < XDMA + 4 ? wbase : w2base) + (int64_t)s * ROWB);
+  };
+  const int r = lane & 15, g = lane >> 4;
+  const uint32_t xfrag = r * ROWB, wfrag = (MB * 16 + wave * TN * 16 + r) * ROWB;
+
+  f32x4 acc[TN][MB];
+#pragma unroll
+  for (int t = 0; t < TN; t++)
+#pragma unroll
+    for (int b = 0; b < MB; b++) acc[t][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nst = p.K / BK;
+#pragma unroll
+  for (int s = 0; s < NSLOT - 1; s++)
+    if (s < nst) issue(s, s);
+  int slot = 0;
+  for (int s = 0; s < nst; s++) {
+    wait_slices<NDMA, NSLOT - 2>(nst - 1 - s);          // slice s has landed, this wave's share of it
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave has read slice s - 1
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + NSLOT - 1 < nst) issue(s + NSLOT - 1, slot == 0 ? NSLOT - 1 : slot - 1);  // over slice s - 1
+    const uint8_t* base = xs + slot * S::STAGE;
+    bf16x8 fx[4][MB], fw[4][TN];
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
+      const uint32_t c = ((kk * 4 + g) ^ r) * 16;
+#pragma unroll
+      for (int t = 0; t < TN; t++) fw[kk][t] = *reinterpret_cast<const bf16x8*>(base + wfrag + c + t * 16 * ROWB);
+#pragma unroll
+      for (int b = 0; b < MB; b++) fx[kk][b] = *reinterpret_cast<const bf16x8*>(base + xfrag + c + b * 16 * ROWB);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+      for (int t = 0; t < TN; t++)
+#pragma unroll
+        for (int b = 0; b < MB; b++) acc[t][b] = Num::mfma(fw[kk][t], fx[kk][b], acc[t][b]);
+    slot = slot + 1 == NSLOT ? 0 : slot + 1;
+  }
+  if (n0 >= p.N) return;
+  if constexpr (GATED) stream_store_gated<MB, F16>(p, acc[0], acc[TN - 1], n0, r, g);
+  else stream_store<MB, F16>(p, acc[0], n0, r, g);
+}
+
+template <int MB, int NW, bool F16, bool GATED>
+static int ring_launch_nw(const StreamArgs& a, hipStream_t stream) {
+  using S = ring::Shape<MB, NW, GATED>;
+  constexpr int smem = S::NSLOT * S::STAGE;
+  const int64_t groups = ((int64_t)a.N + 16 * NW - 1) / (16 * NW);
+  if (groups > 0x7fffffff) return TBIK_ERR_INVALID;
+  static std::atomic<uint64_t> done{0};
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_single_acc_ring_kernel<MB, NW, F16, GATED>), smem, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL((gemm_single_acc_ring_kernel<MB, NW, F16, GATED>), dim3((unsigned)groups), dim3(NW * 64), smem, stream, a);
+  return hip_code(hipGetLastError());
+}
+
+// Waves per work-group of the ring kernel for a call, 0: the windowed kernel.  Measured on MI355X, weights cold, against that
+// kernel (us, windowed -> ring; hidden 4096 unless stated):
+//   mm, up to 8192 columns: one strip per work-group for one block of rows (two work-groups share a CU), two strips for more.
+//     [8,4096]x[4096,4096] 12.5 -> 11.0, [32,4096]x[4096,6144] 17.5 -> 14.6, [32,4096]x[4096,1024] 16.2 -> 13.1,
+//     [8,12288]x[12288,4096] 33.3 -> 27.5; fp16 at 64 rows 33.1 -> 20.4.
+//   mm, up to 10240 columns: three strips, a round of the chip, [32,5120]x[5120,10240] 28.4 -> 26.0 and [8,4096]x[4096,9216] 18.7
+//     -> 18.2, but not for longer K ([8,8192]x[8192,10240] 36.3 -> 38.2).  Wider ones fill the chip with the windowed kernel
+//     just as well ([8,4096]x[4096,12288] 22.6 -> 23.7, x[4096,24576] level) as long as there are one or two blocks of rows
+//     (fp16 at 64 rows: 34.9 -> 26.6 and 57.2 -> 46.2).
+//   mm, more than 65536 columns (lm_head): four strips, [32,4096]x[4096,151936] 238 -> 229, [8,...] 223 -> 215.
+//   gated: 64 rows of 2 x 12288 columns 65.7 -> 43.7, 32 rows 43.9 -> 42.5, [8,5120] of 2 x 25600 115 -> 101, of 2 x 1536 columns
+//     20.9 -> 13.5; one block of rows where the windowed kernel's groups fill their rounds stays there (2 x 8192: 28.8
+//     against 30.8, 2 x 12288: 40.3 against 41.1).
+// The strips of a work-group otherwise follow from the rounds of 256 work-groups, each as long as its weight rows, its
+// X rows at a third of their price (they come from the L2) and a fixed part.
+static int ring_waves(int mb, int64_t strips, int K, bool gated, double windowed_fill) {
+  if (K % ring::BK != 0) return 0;
+  if (!gated) {
+    if (strips <= 512) return mb == 1 ? 1 : 2;
+    if (mb <= 2) return strips <= 640 && K <= 5120 ? 3 : strips > 4096 ? 4 : 0;
+    if (strips > 4096) return 0;
+  } else if (mb == 1 && windowed_fill > 0.9) {
+    return 0;
+  }
+  static const int cand[5] = {1, 2, 3, 4, 6};
+  int best = 0;
+  double best_t = 0;
+  for (int i = gated ? 0 : 1; i < (gated ? 4 : 5); i++) {
+    const int64_t groups = (strips + cand[i] - 1) / cand[i];
+    const double t = (double)((groups + 255) / 256) * (8.0 + 16.0 * cand[i] * (gated ? 2 : 1) + 0.33 * 16 * mb);
+    if (!best || t < best_t) {
+      best_t = t;
+      best = cand[i];
+    }
+  }
+  return best;
+}
+
+template <int MB, bool F16, bool GATED>
+static int ring_launch(const StreamArgs& a, int waves, hipStream_t stream) {
+  switch (waves) {
+    case 1: return ring_launch_nw<MB, 1, F16, GATED>(a, stream);
+    case 2: return ring_launch_nw<MB, 2, F16, GATED>(a, stream);
+    case 3: return ring_launch_nw<MB, 3, F16, GATED>(a, stream);
+    case 4: return ring_launch_nw<MB, 4, F16, GATED>(a, stream);
+    default: break;
+  }
+  if constexpr (!GATED && MB >= 3) {
+    if (waves == 6) return ring_launch_nw<MB, 6, F16, GATED>(a, stream);
+  }
+  return TBIK_ERR_INVALID;
+}
+
 template <int MB, int WS, int NWAVES, bool F16, bool GATED = false>
 static int stream_launch_nw(const StreamArgs& a, hipStream_t stream) {
   const int64_t groups = ((int64_t)a.N + 16 * NWAVES - 1) / (16 * NWAVES);
@@ -336,6 +509,16 @@ static int stream_launch(const StreamArgs& a, hipStream_t stream) {
   // four (two on every second CU), 41.2 us as 256 groups of six; [32,4096]x[4096,18432] 48.6 -> 35.4; lm_head (9496
   // strips, ten rounds of groups of four) is within 2 % for three, four and six.
   const int64_t strips = ((int64_t)a.N + 15) / 16;
+  const bool near_rows = a.ldx < (1 << 22) && a.ldw < (1 << 22);  // the ring kernel's 32-bit byte offsets
+  if (near_rows) {
+    double fill = 0.0;
+    for (int nw : {6, 4, 3, 2}) {
+      const int64_t groups = (strips + nw - 1) / nw;
+      fill = std::max(fill, (double)groups / (double)(((groups + 255) / 256) * 256));
+    }
+    const int waves = ring_waves(MB, strips, a.K, GATED, fill);
+    if (waves) return ring_launch<MB, F16, GATED>(a, waves, stream);
+  }
   // grids of many rounds do not run in rounds: the last one matters little there, the restaging of X more
   if (strips > 4 * 1024) return MB >= 3 ? stream_launch_nw<MB, WS, 8, F16, GATED>(a, stream) : stream_launch_nw<MB, WS, 4, F16, GATED>(a, stream);
   static const int cand[5] = {8, 6, 4, 3, 2};

@@ -41,15 +41,6 @@ struct Shape {
   static constexpr int CNT = 63 / NDMA + 1;
   static constexpr int NSLOT = FIT < CNT ? (FIT < 8 ? FIT : 8) : (CNT < 8 ? CNT : 8);
 };
-// wait until at most `left` slices of this wave's loads are in flight (left <= MAXL, wave-uniform)
-template <int NDMA, int MAXL>
-__device__ __forceinline__ void wait_slices(int left) {
-  if (left >= MAXL) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA * MAXL) : "memory");
-  } else if constexpr (MAXL > 0) {
-    wait_slices<NDMA, MAXL - 1>(left);
-  }
-}
 }  // namespace few
 
 // MT: 16-row tiles; NW: waves, 32 columns each; LS: slices per leaf

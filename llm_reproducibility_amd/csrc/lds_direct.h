@@ -38,4 +38,14 @@ __device__ __forceinline__ void store16_sbase(void* base, uint32_t voff, u32x4 v
   asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2\n\ts_nop 1" : : "v"(voff), "v"(v), "s"(base) : "memory");
 }
 
+// Wait until at most `left` slices of this wave's direct loads (NDMA each) are in flight; left <= MAXL, wave-uniform.
+template <int NDMA, int MAXL>
+__device__ __forceinline__ void wait_slices(int left) {
+  if (left >= MAXL) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA * MAXL) : "memory");
+  } else if constexpr (MAXL > 0) {
+    wait_slices<NDMA, MAXL - 1>(left);
+  }
+}
+
 }  // namespace tbik
