@@ -220,7 +220,8 @@ int bi_mean_dim(const void* x, void* out,
  *   k_cache     [batch, kv_heads, max_len, 128]
  *   vt_cache    [batch, kv_heads, 128, max_len]   (V stored transposed; entries behind ctx_len must be finite)
  *   q_start/q_len/ctx_len  device int32 [batch]: first token row, number of new tokens, cache length
- *                          including the new tokens (query r of sequence b sits at position ctx_len-q_len+r)
+ *                          including the new tokens (query r of sequence b sits at position ctx_len-q_len+r).  A
+ *                          sequence whose ctx_len exceeds max_len has no meaningful output; the others are not affected
  * Replaces: the fixed-tile attention of the train/inference alignment patch,
  *           _kernel_unified_attention_2d, src/patch/patch_training_inference_align.py:171-487 (its KV-order
  *           rule, not vLLM's paged-cache plumbing).

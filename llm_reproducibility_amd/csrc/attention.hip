@@ -543,6 +543,9 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   };
   auto tiles_here = [&](int ntiles) __attribute__((always_inline)) {
     if (!SPLIT) return ntiles;
+    // lengths are device data: a sequence that ran off its cache has no chunk behind the last one of its slot in the
+    // workspace, where the states of the next row begin (the merge is bounded likewise)
+    ntiles = min(ntiles, a.max_len >> 5);
     const int nch = (ntiles + CHUNK_TILES - 1) / CHUNK_TILES;
     if (z >= nch) return 0;
     return (nch - z + nz - 1) / nz * CHUNK_TILES - ((nch - 1) % nz == z ? nch * CHUNK_TILES - ntiles : 0);
@@ -802,7 +805,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const AttnArgs a, 
   auto read_lengths = [&]() __attribute__((always_inline)) {
     const int ctx = a.ctx_len[b];
     qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
-    nch = qi < qlen ? (ctx - qlen + qi) / (32 * CHUNK_TILES) + 1 : 0;
+    nch = qi < qlen ? min((ctx - qlen + qi) / (32 * CHUNK_TILES) + 1, sp.nchunks) : 0;
   };
   // a chunk of a prompt has many rows, and possibly all of one chunk: they are not loaded before that is known.  A decode
   // step has few: their states (behind the horizon, too) are loaded while the length is on its way, and possibly not used.

@@ -83,3 +83,46 @@ def test_one_launch_decode_step_over_chunks(dev, monkeypatch, ctxs):
     _no_workspace(monkeypatch)
     b = ops.bi_attention_decode_qkv(qkv, w, w, inv, k2, v2, ctx, hq, hkv, SCALE, 1e-6)
     assert torch.equal(a[live], b[live]) and torch.equal(k1, k2) and torch.equal(v1, v2)
+
+
+def _guarded(nbytes, dev):
+    """Scratch of nbytes with a pattern behind it that no kernel may touch."""
+    return torch.full((nbytes + 4096,), 0xA5, dtype=torch.uint8, device=dev)
+
+
+def _untouched(ws, nbytes):
+    return bool((ws[nbytes:] == 0xA5).all())
+
+
+@pytest.mark.parametrize("over", [1, 31, 513, 5000])
+@pytest.mark.parametrize("which", [1, 3])
+def test_a_sequence_past_its_cache_spoils_no_other(dev, which, over):
+    """ctx_len is device data and may run off the cache (a finished sequence in a replayed graph): the chunk states of the
+    other rows and the memory behind the workspace stay what they are.  `which`: in the middle of the batch, and the last."""
+    print("case past the cache", which, over, flush=True)
+    hq, hkv, L, B = 8, 2, 2048, 4
+    gen = torch.Generator(device=dev).manual_seed(over)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    qkv, kc, vt = rnd(B, (hq + 2 * hkv) * D), rnd(B, hkv, L, D), rnd(B, hkv, D, L)
+    w, inv = (1 + 0.1 * torch.randn(D, generator=gen, device=dev)).to(torch.bfloat16), O.rope_inv_freq(D, 1e6).to(dev)
+    lib, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    nbytes = lib.bi_attention_workspace_bytes(B, 1, hq, hkv, L)
+    others = [b for b in range(B) if b != which]
+    one, starts = torch.ones(B, dtype=torch.int32, device=dev), torch.arange(B, dtype=torch.int32, device=dev)
+    q = qkv[:, : hq * D].contiguous()
+    got = []
+    for last in (L, L + over):
+        ctxs = [700, 2048, 1500, 600]
+        ctxs[which] = last
+        ctx = torch.tensor(ctxs, dtype=torch.int32, device=dev)
+        k1, v1, ws = kc.clone(), vt.clone(), _guarded(nbytes, dev)
+        fused, plain = torch.zeros((B, hq, D), dtype=torch.bfloat16, device=dev), torch.zeros((B, hq, D), dtype=torch.bfloat16, device=dev)
+        assert lib.bi_attention_decode_qkv_ws_bf16(qkv.data_ptr(), qkv.stride(0), w.data_ptr(), w.data_ptr(), inv.data_ptr(), k1.data_ptr(),
+                                                   v1.data_ptr(), fused.data_ptr(), ctx.data_ptr(), B, hq, hkv, D, L, SCALE, 1e-6,
+                                                   ws.data_ptr(), nbytes, s) == _lib.TBIK_OK
+        assert _untouched(ws, nbytes)
+        assert lib.bi_attention_ws_bf16(q.data_ptr(), kc.data_ptr(), vt.data_ptr(), plain.data_ptr(), starts.data_ptr(), one.data_ptr(),
+                                        ctx.data_ptr(), B, 1, hq, hkv, D, L, SCALE, ws.data_ptr(), nbytes, s) == _lib.TBIK_OK
+        assert _untouched(ws, nbytes)
+        got.append((fused[others], plain[others], k1[others], v1[others]))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
