@@ -46,13 +46,14 @@ constexpr int HD = 128;
 constexpr int CHUNK_TILES = 16;           // key tiles per chunk: 512 keys
 constexpr float kNoKey = -3e38f;          // reference point of an empty state: below every score, finite (see softmax_tile)
 
-// Where the chunks of a row go when different work-groups compute them (SPLIT): slot (sequence * max_q_len + query) *
-// q_heads + head of [nchunks] states.
+// Where the chunks of a row go when different work-groups compute them (SPLIT): slot (sequence * q_rows + query) *
+// q_heads + head of [nchunks] states.  q_rows are the queries per sequence that the kernels' tiles have room for and not
+// the caller's max_q_len: they compute every row that the device's q_len says there is, up to those.
 struct SplitArgs {
   float* o;      // [slot][nchunks][128] accumulators
   float* ml;     // [slot][nchunks][2] reference point, denominator
   int nchunks;   // chunks of the cache length
-  int max_q_len;
+  int q_rows;
 };
 
 // The decode kernel that forms its own queries and the new key/value (FUSED): sequence b's one new token is row b of the
@@ -477,7 +478,7 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
   }
   if (!qvalid) return;
   if (SPLIT && qpos >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete here)
-    const int64_t at = ((int64_t)(b * sp.max_q_len + qrow) * a.q_heads + h) * sp.nchunks + blockIdx.z;
+    const int64_t at = ((int64_t)(b * sp.q_rows + qrow) * a.q_heads + h) * sp.nchunks + blockIdx.z;
 #pragma unroll
     for (int t = 0; t < 8; t++) *reinterpret_cast<f32x4*>(sp.o + at * HD + 16 * t + 4 * g) = o[t];
     if (g == 0) *reinterpret_cast<f32x2*>(sp.ml + at * 2) = f32x2{m, l};
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
     const int chunk = tile_of(c0) / CHUNK_TILES;
     if (SPLIT && qpos >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete with it)
       if (qvalid) {
-        const int64_t at = ((int64_t)(b * sp.max_q_len + qi) * a.q_heads + h) * sp.nchunks + chunk;
+        const int64_t at = ((int64_t)(b * sp.q_rows + qi) * a.q_heads + h) * sp.nchunks + chunk;
 #pragma unroll
         for (int i = 0; i < CT; i++) *reinterpret_cast<f32x4*>(sp.o + at * HD + 16 * (CT * wv + i) + 4 * g) = o[i];
         if (wv == 0 && g == 0) *reinterpret_cast<f32x2*>(sp.ml + at * 2) = f32x2{m, l};
@@ -813,7 +814,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const AttnArgs a, 
     read_lengths();
     if (nch <= 1) return;
   }
-  const int64_t at = ((int64_t)(b * sp.max_q_len + qi) * a.q_heads + h) * sp.nchunks;
+  const int64_t at = ((int64_t)(b * sp.q_rows + qi) * a.q_heads + h) * sp.nchunks;
   const f32x2* po = reinterpret_cast<const f32x2*>(sp.o + at * HD) + lane;
   const f32x2* pm = reinterpret_cast<const f32x2*>(sp.ml + at * 2);
   constexpr int NB = 16;
@@ -869,26 +870,28 @@ static bool group_split(int64_t groups, int max_len) {
 static bool grouped_cache(int G, int kv_heads, int max_len) {
   return (max_len & 31) == 0 && (G == 1 || G == 2 || G == 4 || G == 8) && kv_heads <= 65535 && max_len <= (1 << 22);
 }
+// Queries per sequence that a call's tiles hold: all of a decode tile, or whole blocks of 16.
+static int query_rows(int max_q_len, int G) { return (int64_t)max_q_len * G <= 16 ? 16 / G : (max_q_len + 15) / 16 * 16; }
 size_t attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len) {
   if (batch <= 0 || max_q_len <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || max_len < 32) return 0;
   const int G = q_heads / kv_heads;
   if (!grouped_cache(G, kv_heads, max_len)) return 0;
   const bool split = (int64_t)max_q_len * G <= 16 ? decode_split((int64_t)batch * kv_heads, max_len) > 1
                                                   : group_split((int64_t)((max_q_len + 15) / 16) * kv_heads * batch, max_len);
-  return split ? (size_t)batch * max_q_len * q_heads * chunks_of(max_len) * (HD + 2) * sizeof(float) : 0;
+  return split ? (size_t)batch * query_rows(max_q_len, G) * q_heads * chunks_of(max_len) * (HD + 2) * sizeof(float) : 0;
 }
-static SplitArgs split_args(void* ws, int batch, int max_q_len, int q_heads, int max_len) {
+static SplitArgs split_args(void* ws, int batch, int max_q_len, int q_heads, int kv_heads, int max_len) {
   SplitArgs sp;
   sp.nchunks = chunks_of(max_len);
-  sp.max_q_len = max_q_len;
+  sp.q_rows = query_rows(max_q_len, q_heads / kv_heads);
   sp.o = static_cast<float*>(ws);
-  sp.ml = sp.o + (int64_t)batch * max_q_len * q_heads * sp.nchunks * HD;
+  sp.ml = sp.o + (int64_t)batch * sp.q_rows * q_heads * sp.nchunks * HD;
   return sp;
 }
 
 template <bool FUSED>
-static void merge_launch(const AttnArgs& a, const SplitArgs& sp, int max_q_len, int batch, hipStream_t stream) {
-  const dim3 grid((unsigned)((a.q_heads + 3) / 4), (unsigned)max_q_len, (unsigned)batch);
+static void merge_launch(const AttnArgs& a, const SplitArgs& sp, int batch, hipStream_t stream) {
+  const dim3 grid((unsigned)((a.q_heads + 3) / 4), FUSED ? 1u : (unsigned)sp.q_rows, (unsigned)batch);
   hipLaunchKernelGGL(attention_merge_kernel<FUSED>, grid, dim3(256), 0, stream, a, sp);
 }
 
@@ -903,13 +906,13 @@ static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max
     hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, false>), dim3((unsigned)a.kv_heads, (unsigned)batch), dim3(512), lds, stream, a, f, SplitArgs{});
     return hip_code(hipGetLastError());
   }
-  const SplitArgs sp = split_args(ws, batch, max_q_len, a.q_heads, a.max_len);
+  const SplitArgs sp = split_args(ws, batch, max_q_len, a.q_heads, a.kv_heads, a.max_len);
   static std::atomic<uint64_t> done{0};
   const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, true>), lds, done);
   if (e != hipSuccess) return hip_code(e);
   const int nz = decode_split((int64_t)batch * a.kv_heads, a.max_len);
   hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, true>), dim3((unsigned)a.kv_heads, (unsigned)batch, (unsigned)nz), dim3(512), lds, stream, a, f, sp);
-  merge_launch<FUSED>(a, sp, max_q_len, batch, stream);
+  merge_launch<FUSED>(a, sp, batch, stream);
   return hip_code(hipGetLastError());
 }
 
@@ -949,7 +952,7 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
     const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len) : 0;
     const bool split = need != 0 && ws_bytes >= need;
     const bool one = chunks_of(max_len) == 1;
-    const SplitArgs sp = split ? split_args(ws, batch, max_q_len, q_heads, max_len) : SplitArgs{};
+    const SplitArgs sp = split ? split_args(ws, batch, max_q_len, q_heads, kv_heads, max_len) : SplitArgs{};
     const dim3 cgrid((unsigned)gx, (unsigned)batch, (unsigned)chunks_of(max_len));
 #define TBIK_ATTN_GROUP_RUN(GG, DEEP, NLD, CH, GRID)                                                                              \
   hipLaunchKernelGGL((attention_group_kernel<GG, DEEP, NLD, CH>), GRID, dim3(64 * (GG + NLD)), 0, stream, a, sp)
@@ -972,7 +975,7 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
     else TBIK_ATTN_GROUP(8);
 #undef TBIK_ATTN_GROUP
 #undef TBIK_ATTN_GROUP_RUN
-    if (split) merge_launch<false>(a, sp, max_q_len, batch, stream);
+    if (split) merge_launch<false>(a, sp, batch, stream);
   } else {
     const dim3 grid((unsigned)((max_q_len + 15) / 16), (unsigned)q_heads, (unsigned)batch);
     hipLaunchKernelGGL(attention_kernel, grid, dim3(64), 0, stream, a);

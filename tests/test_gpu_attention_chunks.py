@@ -126,3 +126,28 @@ def test_a_sequence_past_its_cache_spoils_no_other(dev, which, over):
         assert _untouched(ws, nbytes)
         got.append((fused[others], plain[others], k1[others], v1[others]))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("hq,hkv,qlens,max_q_len", [
+    (8, 2, [1, 4, 1, 3], 1),          # decode tiles: room for 16 / 4 queries
+    (4, 4, [2, 16, 1, 9], 2),         # ... for 16
+    (8, 2, [20, 32, 17, 30], 20),     # two blocks of 16
+])
+def test_more_queries_than_the_call_says(dev, hq, hkv, qlens, max_q_len):
+    """q_len is device data: rows beyond the caller's max_q_len that still fit the tiles come out as without the workspace,
+    and nothing is written outside it."""
+    print("case more queries", hq, hkv, qlens, max_q_len, flush=True)
+    gen = torch.Generator(device=dev).manual_seed(max_q_len)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    L, B = 2048, len(qlens)
+    q, kc, vt = rnd(sum(qlens), hq, D), rnd(B, hkv, L, D), rnd(B, hkv, D, L)
+    starts, n, ctx = i32([sum(qlens[:i]) for i in range(B)]), i32(qlens), i32([2048, 1700, 600, 1025])
+    lib, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    nbytes = lib.bi_attention_workspace_bytes(B, max_q_len, hq, hkv, L)
+    assert nbytes > 0
+    ws, out, want = _guarded(nbytes, dev), torch.zeros_like(q), torch.zeros_like(q)
+    for o, w, wb in ((want, None, 0), (out, ws.data_ptr(), nbytes)):
+        assert lib.bi_attention_ws_bf16(q.data_ptr(), kc.data_ptr(), vt.data_ptr(), o.data_ptr(), starts.data_ptr(), n.data_ptr(),
+                                        ctx.data_ptr(), B, max_q_len, hq, hkv, D, L, SCALE, w, wb, s) == _lib.TBIK_OK
+    assert _untouched(ws, nbytes) and torch.equal(out, want)
