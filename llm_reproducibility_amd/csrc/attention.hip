@@ -44,7 +44,7 @@ struct AttnArgs {
 
 constexpr int HD = 128;
 constexpr int CHUNK_TILES = 16;           // key tiles per chunk: 512 keys
-constexpr float kNoKey = -3e38f;          // reference point of an empty state: below every score, finite (see softmax_tile)
+constexpr float kNoKey = -__FLT_MAX__;    // reference point of an empty state: no finite score lies below it (see softmax_tile)
 
 // Where the chunks of a row go when different work-groups compute them (SPLIT): slot (sequence * q_rows + query) *
 // q_heads + head of [nchunks] states.  q_rows are the queries per sequence that the kernels' tiles have room for and not

@@ -151,3 +151,38 @@ def test_more_queries_than_the_call_says(dev, hq, hkv, qlens, max_q_len):
         assert lib.bi_attention_ws_bf16(q.data_ptr(), kc.data_ptr(), vt.data_ptr(), o.data_ptr(), starts.data_ptr(), n.data_ptr(),
                                         ctx.data_ptr(), B, max_q_len, hq, hkv, D, L, SCALE, w, wb, s) == _lib.TBIK_OK
     assert _untouched(ws, nbytes) and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("ctx", [40, 520, 1100])
+def test_scores_at_the_ends_of_fp32(dev, monkeypatch, ctx):
+    """Rows whose scores all lie near the lowest finite fp32 (the mean of the values, exactly 1), rows with some keys at
+    -inf (without weight, a whole chunk of them too), and a row with a NaN: every kernel, with and without the workspace."""
+    print("case extreme scores", ctx, flush=True)
+    hq, hkv, L = 8, 2, 2048
+    q = torch.zeros((1, hq, D), dtype=torch.bfloat16, device=dev)
+    q[:, :, 0] = 1
+    one, start, n = (torch.tensor([v], dtype=torch.int32, device=dev) for v in (1, 0, ctx))
+    scale = 1.3862943649291992                              # times log2(e) in fp32: exactly 2, so that large scores scale exactly
+    low = torch.tensor(-1.6e38).to(torch.bfloat16).item()   # -3.2e38 after it
+    cases = {"low": low, "some": 0.0, "nan": 0.0}
+    for name, fill in cases.items():
+        k = torch.zeros((L, D))
+        k[:, 0] = fill
+        v = torch.ones((L, D))
+        if name == "some":
+            k[: min(ctx - 8, 1024), 0] = -math.inf          # the whole of the first chunks, or all but a few keys
+            v[: min(ctx - 8, 1024)] = 7.0
+        if name == "nan":
+            k[ctx // 2, 0] = math.nan
+        for length in (L, L + 4):
+            kc = torch.zeros((1, hkv, length, D), dtype=torch.bfloat16, device=dev)
+            vt = torch.zeros((1, hkv, D, length), dtype=torch.bfloat16, device=dev)
+            kc[0, :, :L], vt[0, :, :, :L] = k.to(torch.bfloat16).to(dev), v.t().to(torch.bfloat16).to(dev)
+            for shared in (True, False):
+                with monkeypatch.context() as m:
+                    if not shared:
+                        _no_workspace(m)
+                    got = ops.bi_attention_bf16(q, kc, vt, start, one, n, 1, scale)
+                    wide = ops.bi_attention_bf16(q.expand(20, hq, D).contiguous(), kc, vt, start, one * 20, n, 20, scale)[-1:]
+                for o in (got, wide):
+                    assert torch.isnan(o).all() if name == "nan" else torch.equal(o, torch.ones_like(o)), (name, length, shared)
