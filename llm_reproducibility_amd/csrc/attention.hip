@@ -861,8 +861,7 @@ static int decode_split(int64_t pairs, int max_len) {
   const int64_t want = 512 / pairs;
   return (int)(want > nch ? nch : want);
 }
-// The same for the grouped kernel, whose work-groups then take a chunk each: worth it while they are few; the bound on
-// the product keeps the states (33 KiB per work-group and chunk) to 64 MiB.
+// The same for the grouped kernel, whose work-groups then take a chunk each: worth it while they are few.
 static bool group_split(int64_t groups, int max_len) {
   const int nch = chunks_of(max_len);
   return nch >= 3 && groups <= 128 && groups * nch <= 2048;
@@ -878,7 +877,11 @@ size_t attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_h
   if (!grouped_cache(G, kv_heads, max_len)) return 0;
   const bool split = (int64_t)max_q_len * G <= 16 ? decode_split((int64_t)batch * kv_heads, max_len) > 1
                                                   : group_split((int64_t)((max_q_len + 15) / 16) * kv_heads * batch, max_len);
-  return split ? (size_t)batch * query_rows(max_q_len, G) * q_heads * chunks_of(max_len) * (HD + 2) * sizeof(float) : 0;
+  // A state is a row of 128 accumulators and two numbers.  The grouped kernel's bound above keeps them to 2^18 (130 MiB, at
+  // 8 query heads per KV head); the decode kernel's is reached by 128 pairs with 65,536 keys each, which one work-group
+  // per pair reads at the rate of the memory.
+  const int64_t states = (int64_t)batch * query_rows(max_q_len, G) * q_heads * chunks_of(max_len);
+  return split && states <= (1 << 18) ? (size_t)states * (HD + 2) * sizeof(float) : 0;
 }
 static SplitArgs split_args(void* ws, int batch, int max_q_len, int q_heads, int kv_heads, int max_len) {
   SplitArgs sp;

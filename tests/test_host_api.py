@@ -113,6 +113,16 @@ def test_decode_batches_fit_the_static_scratch(M, N, K, leaf):
     assert _lib.lib().tbik_gemm_workspace_bytes(M, N, K, leaf) <= 32 * 1024 * 1024
 
 
+@pytest.mark.parametrize("kv_heads", [1, 2, 8])
+@pytest.mark.parametrize("heads_per_kv", [1, 2, 4, 8])
+def test_attention_scratch_is_bounded(heads_per_kv, kv_heads):
+    """Whatever the cache length (up to the 2^22 of the grouped kernels), a call asks for at most 2^18 chunk states of 130 floats."""
+    f = _lib.lib().bi_attention_workspace_bytes
+    most = max(f(batch, new, heads_per_kv * kv_heads, kv_heads, max_len) for batch in (1, 5, 16, 64, 128)
+               for new in (1, 2, 16, 17, 256, 2048) for max_len in (1024, 8192, 65536, 1 << 20, 1 << 22))
+    assert 0 < most <= (1 << 18) * 130 * 4
+
+
 def test_host_argument_checks_fire_before_any_launch():
     L = _lib.lib()
     # null pointers / bad sizes are rejected on the host, so these are safe without a GPU
