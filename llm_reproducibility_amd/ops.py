@@ -55,9 +55,10 @@ def _is_f16(*tensors) -> bool:
 
 
 def _k_across(t: torch.Tensor) -> bool:
-    """True for a matrix whose columns are contiguous and whose rows are not: the transposed view of a row-major one."""
+    """True for a matrix whose columns are contiguous and whose rows are not, the transposed view of a row-major one, in an
+    element size that the transposing copy takes (other types are refused further on, as what they are)."""
     (rows, cols), (s0, s1) = t.shape, t.stride()
-    return s0 == 1 and s1 != 1 and rows > 1 and cols > 1 and s1 >= rows
+    return s0 == 1 and s1 != 1 and rows > 1 and cols > 1 and s1 >= rows and t.element_size() in (2, 4)
 
 
 def _transposed(t: torch.Tensor, k: int):

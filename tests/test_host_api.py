@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import llm_reproducibility_amd as pkg
-from llm_reproducibility_amd import _lib, utils
+from llm_reproducibility_amd import _lib, ops, utils
 from llm_reproducibility_amd.tbik import choose_leaf_k, matmul_tp_persistent, tree_combine
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -121,6 +121,17 @@ def test_attention_scratch_is_bounded(heads_per_kv, kv_heads):
     most = max(f(batch, new, heads_per_kv * kv_heads, kv_heads, max_len) for batch in (1, 5, 16, 64, 128)
                for new in (1, 2, 16, 17, 256, 2048) for max_len in (1024, 8192, 65536, 1 << 20, 1 << 22))
     assert 0 < most <= (1 << 18) * 130 * 4
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.complex64, torch.int8])
+def test_transposed_operands_of_other_types_are_refused_as_such(monkeypatch, dtype):
+    """A transposed view of an element size that no copy kernel takes is refused by its type, like any other layout."""
+    monkeypatch.setattr(ops, "_require_gpu", lambda *t: None)
+    A, B = torch.zeros((256, 32), dtype=dtype).t(), torch.zeros((256, 16), dtype=dtype)
+    for call in (lambda: ops._gemm_tree_impl(A, B, None, 256), lambda: ops._bi_gemm_impl(A, B, None),
+                 lambda: ops._bi_rmsnorm_impl(A, None, 1e-6), lambda: ops._bi_add_rmsnorm_impl(A, A, None, 1e-6)):
+        with pytest.raises(NotImplementedError):
+            call()
 
 
 def test_host_argument_checks_fire_before_any_launch():
