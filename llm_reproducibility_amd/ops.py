@@ -520,9 +520,11 @@ def _(gate_up):
 # --------------------------------------------------------------------------------------------
 # one-launch compositions for decode-sized batches (bit-identical to the two-launch forms they fall back to)
 # --------------------------------------------------------------------------------------------
-# Shapes for which a one-launch entry point answered 'unsupported': whether it applies depends on the shape alone, so the
-# next call of the same shape goes to the separate calls at once (no output allocated for a call that will not run).
+# Shapes for which a one-launch entry point answered 'unsupported': whether it applies depends on the shape alone (what
+# depends on strides is asked before the call), so the next call of the same shape goes to the separate calls at once (no
+# output allocated for a call that will not run).
 _declined: set = set()
+_FAR_ROWS = 1 << 22   # row stride from which the 256-row tiles' 32-bit byte offsets do not reach
 
 
 def rmsnorm_gemm(x: torch.Tensor, norm_weight: Optional[torch.Tensor], eps: float, residual: Optional[torch.Tensor],
@@ -602,13 +604,15 @@ def gemm_silu_mul(x: torch.Tensor, W: torch.Tensor) -> torch.Tensor:
     _require_gpu(x, W)
     M, K = x.shape
     inter = W.shape[0] // 2
+    ldw = W.stride(0)
     fusable = (x.dtype == torch.bfloat16 and W.dtype == torch.bfloat16 and M > 4 and W.shape[0] == 2 * inter and inter % 16 == 0
-               and K % 32 == 0 and W.stride(1) == 1 and W.stride(0) % 8 == 0 and _aligned16(W) and not torch.compiler.is_compiling()
-               and ("mm_silu", M, inter, K) not in _declined)
+               and K % 32 == 0 and W.stride(1) == 1 and ldw >= K and ldw % 8 == 0 and _aligned16(W)
+               and (M <= 64 or (ldw < _FAR_ROWS and x.stride(0) < _FAR_ROWS))
+               and not torch.compiler.is_compiling() and ("mm_silu", M, inter, K) not in _declined)
     if fusable:
         x2, ldx = _rows16(x)
         out = torch.empty((M, inter), device=x.device, dtype=x.dtype)
-        rc = _lib.lib().bi_gemm_silu_mul_bf16(x2.data_ptr(), ldx, W.data_ptr(), W.stride(0), out.data_ptr(), out.stride(0), M, inter, K,
+        rc = _lib.lib().bi_gemm_silu_mul_bf16(x2.data_ptr(), ldx, W.data_ptr(), ldw, out.data_ptr(), out.stride(0), M, inter, K,
                                               _stream(x))
         if rc == _lib.TBIK_OK:
             return out

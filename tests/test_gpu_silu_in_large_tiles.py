@@ -29,3 +29,21 @@ def test_equals_the_two_calls(dev, M, K, inter):
         assert torch.equal(out[:, :inter], want) and not out[:, inter:].any()
     assert torch.equal(ops.gemm_silu_mul(x, W), want)
     assert torch.equal(ops.gemm_silu_mul(x[M - 70:], W), want[M - 70:])   # the two calls
+
+
+def test_strides_decide_for_their_own_call_only(dev):
+    """Rows too far apart for the tiles' 32-bit offsets and a weight of one repeated row go to the two calls; neither is
+    remembered against the shape."""
+    M, K, inter = 1025, 256, 4096
+    gen = torch.Generator(device=dev).manual_seed(7)
+    x = torch.randn((M, K), generator=gen, device=dev).bfloat16()
+    W = (torch.randn((2 * inter, K), generator=gen, device=dev) * 0.05).bfloat16()
+    far = torch.empty((M - 1) * (1 << 22) + K, device=dev, dtype=torch.bfloat16).as_strided((M, K), (1 << 22, 1))
+    far.copy_(x)
+    want = ops.bi_silu_mul(bio.matmul_persistent(x, W.t()))
+    assert torch.equal(ops.gemm_silu_mul(far, W), want)
+    del far
+    same = W[:1].expand(2 * inter, K)
+    assert torch.equal(ops.gemm_silu_mul(x, same), ops.bi_silu_mul(bio.matmul_persistent(x, same.contiguous().t())))
+    assert ("mm_silu", M, inter, K) not in ops._declined
+    assert torch.equal(ops.gemm_silu_mul(x, W), want) and ("mm_silu", M, inter, K) not in ops._declined
