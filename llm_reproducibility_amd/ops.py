@@ -522,9 +522,16 @@ def _(gate_up):
 # --------------------------------------------------------------------------------------------
 # Shapes for which a one-launch entry point answered 'unsupported': whether it applies depends on the shape alone (what
 # depends on strides is asked before the call), so the next call of the same shape goes to the separate calls at once (no
-# output allocated for a call that will not run).
+# output allocated for a call that will not run).  Row counts of a serving program are many: the set starts anew when full.
 _declined: set = set()
+_DECLINED_MAX = 4096
 _FAR_ROWS = 1 << 22   # row stride from which the 256-row tiles' 32-bit byte offsets do not reach
+
+
+def _decline(key) -> None:
+    if len(_declined) >= _DECLINED_MAX:
+        _declined.clear()
+    _declined.add(key)
 
 
 def rmsnorm_gemm(x: torch.Tensor, norm_weight: Optional[torch.Tensor], eps: float, residual: Optional[torch.Tensor],
@@ -554,7 +561,7 @@ def rmsnorm_gemm(x: torch.Tensor, norm_weight: Optional[torch.Tensor], eps: floa
             return C, rout
         if rc != _lib.TBIK_ERR_UNSUPPORTED:
             _lib.check(rc, "bi_rmsnorm_gemm_bf16")
-        _declined.add(("norm_mm", M, N, K))
+        _decline(("norm_mm", M, N, K))
     if residual is None:
         h, rout = bi_rmsnorm(x, norm_weight, eps), None
     else:
@@ -586,7 +593,7 @@ def gemm_tree_silu_mul(gate: torch.Tensor, up: torch.Tensor, B: torch.Tensor, bi
             return C
         if rc != _lib.TBIK_ERR_UNSUPPORTED:
             _lib.check(rc, "tbik_gemm_silu_mul_bf16")
-        _declined.add(("silu_tree", M, N, K, leaf_k))
+        _decline(("silu_tree", M, N, K, leaf_k))
     if (gate.dim() == 2 and up.shape == gate.shape and gate.stride(1) == 1 and up.stride(1) == 1 and gate.stride(0) == up.stride(0)
             and gate.dtype == up.dtype and up.data_ptr() == gate.data_ptr() + K * gate.element_size()
             and (M == 1 or gate.stride(0) >= 2 * K)):
@@ -618,7 +625,7 @@ def gemm_silu_mul(x: torch.Tensor, W: torch.Tensor) -> torch.Tensor:
             return out
         if rc != _lib.TBIK_ERR_UNSUPPORTED:
             _lib.check(rc, "bi_gemm_silu_mul_bf16")
-        _declined.add(("mm_silu", M, inter, K))
+        _decline(("mm_silu", M, inter, K))
     return bi_silu_mul(bi_gemm(x, W.t(), None))
 
 
@@ -668,7 +675,7 @@ def gemm_tree_add_rmsnorm(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch
                 return out, rout
             if rc != _lib.TBIK_ERR_UNSUPPORTED:
                 _lib.check(rc, "tbik_gemm_rmsnorm_bf16")
-            _declined.add(("tree_norm", M, N, K, leaf_k))
+            _decline(("tree_norm", M, N, K, leaf_k))
     return _norm_after(gemm_tree(A, B, bias, leaf_k), residual, norm_weight, eps)
 
 
@@ -755,7 +762,7 @@ def bi_attention_decode_qkv(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight:
             return out
         if rc != _lib.TBIK_ERR_UNSUPPORTED:
             _lib.check(rc, "bi_attention_decode_qkv_ws_bf16")
-        _declined.add(("attn_qkv", q_heads, kv_heads, max_len % 32))
+        _decline(("attn_qkv", q_heads, kv_heads, max_len % 32))
     pos = (ctx_len - 1).to(torch.int64)
     seq = torch.arange(B, device=qkv.device, dtype=torch.int64)
     q = bi_qk_norm_rope_cache_bf16(qkv, q_weight, k_weight, inv_freq, pos, seq, k_cache, vt_cache, q_heads, kv_heads, eps)

@@ -134,6 +134,13 @@ def test_transposed_operands_of_other_types_are_refused_as_such(monkeypatch, dty
             call()
 
 
+def test_declined_shapes_are_a_bounded_memory(monkeypatch):
+    monkeypatch.setattr(ops, "_declined", set())
+    for rows in range(3 * ops._DECLINED_MAX):
+        ops._decline(("mm_silu", rows, 64, 64))
+        assert ("mm_silu", rows, 64, 64) in ops._declined and len(ops._declined) <= ops._DECLINED_MAX
+
+
 def test_host_argument_checks_fire_before_any_launch():
     L = _lib.lib()
     # null pointers / bad sizes are rejected on the host, so these are safe without a GPU
