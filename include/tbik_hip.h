@@ -89,12 +89,13 @@ size_t tbik_gemm_workspace_bytes_rowmajor_b(int M, int N, int K, int leaf_k, int
 /*
  * How tbik_gemm_bf16 (f16 != 0: tbik_gemm_f16) would run this problem: the decision the workspace size above comes
  * from, for callers and tests that want to see it (host only, launches nothing, no effect on any result).
- *   out5[0] path: 0 one launch with K cut over the waves of a work-group (a few rows), 1 128x128 tiles (up to 512 rows),
+ *   out5[0] path: 0 one launch with K cut over the waves of a work-group (a few rows), 1 128x128 tiles (short K shards),
  *                 2 two column regions with a K split each, 3 one grid of any other kind with one K split
  *   out5[1] K split (of the first region for path 2, 0 if that region runs on 128x128 tiles; waves per strip for path 0)
  *   out5[2] columns of the first region (path 2), else 0
  *   out5[3] K split of the second region (path 2), else 0
- *   out5[4] 1 when both regions go out as one launch
+ *   out5[4] path 2: 1 when both regions go out as one launch; path 3: waves per work-group of the ring kernel that serves
+ *           up to 64 rows (32 columns each), 0 where another kernel does; else 0
  * Every choice yields the same bits (shard tree o leaf tree = full tree).
  * Replaces: the fixed launch configuration of the reference, src/tbik/tree_based_matmul.py:206-238 (no counterpart
  * for the K split: the reference cuts K only across GPUs).

@@ -690,20 +690,19 @@ size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowm
 }
 
 // What tree_plan() chose for a shape, for callers and tests that want to know (no effect on any result):
-// out[0] path (0 one-launch few-rows kernel, 1 128x128 tiles for up to 512 rows, 2 two column regions, 3 one grid of any
-// other kind, 128x128 tiles of more rows among them), out[1] K split (of the
-// first region for path 2; waves per strip for path 0), out[2] columns of the first region (path 2, else 0), out[3] K
-// split of the second region (path 2, else 0), out[4] 1 when the two regions go out as one launch.
+// out[0] path (TreePath), out[1] K split (of the first region for path 2; waves per strip for path 0), out[2] columns of
+// the first region (path 2, else 0), out[3] K split of the second region (path 2, else 0), out[4] for path 2: 1 when the
+// two regions go out as one launch; for path 3: waves of the ring kernel for decode batches, 0 on the other kernels.
 int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, int out[5]) {
   TreePlan tp;
   if (!out) return TBIK_ERR_INVALID;
   if (!tree_plan(M, N, K, leaf_k, f16, rowmajor_b, true, &tp)) return TBIK_ERR_INVALID;
-  out[0] = tp.path == PATH_NARROW && M > 512 ? (int)PATH_SINGLE : (int)tp.path;
+  out[0] = (int)tp.path;
   out[1] = tp.path == PATH_STRIP ? tp.strip_waves : tp.path == PATH_NARROW ? tp.narrow.split
            : tp.path == PATH_REGIONS ? (tp.regions.narrow_a ? 0 : tp.regions.a.split) : tp.single.split;
   out[2] = tp.path == PATH_REGIONS ? tp.regions.na : 0;
   out[3] = tp.path == PATH_REGIONS ? (tp.regions.narrow_b ? 0 : tp.regions.b.split) : 0;
-  out[4] = tp.path == PATH_REGIONS && tp.regions.pair ? 1 : 0;
+  out[4] = tp.path == PATH_REGIONS ? (tp.regions.pair ? 1 : 0) : tp.path == PATH_SINGLE ? tp.single.few_waves : 0;
   return TBIK_OK;
 }
 

@@ -82,13 +82,14 @@ def test_workspace_query_and_plan_come_from_one_decision():
                 if path == 0:
                     assert ws == 0 and M <= 16 and split in (2, 4, 8)
                 elif path == 1:
-                    assert 64 <= M <= 512 and leaf == 256 and ws == (0 if split == 1 else (split * M * N * 2 + 255) // 256 * 256)
+                    assert M >= 64 and leaf == 256 and ws == (0 if split == 1 else (split * M * N * 2 + 255) // 256 * 256)
                 elif path == 2:
                     assert 0 < na < N and na % 256 == 0 and M >= 64
                     parts = [(sp, n) for sp, n in ((split, na), (split_b, N - na)) if sp > 1]
                     need = [sp * M * n * 2 for sp, n in parts]
                     assert ws >= (sum(need) if pair else max(need, default=0))
                 else:
+                    assert pair == 0 or (M <= 64 and 2 <= pair <= 6)      # waves of the decode-batch ring kernel
                     assert split >= 1 and (split & (split - 1)) == 0 and ws >= (split * M * N * 2 if split > 1 else 0)
                 assert ws % 16 == 0
                 # a row-major B runs on the tiled kernels only: one grid, partial results only
@@ -100,6 +101,8 @@ def test_workspace_query_and_plan_come_from_one_decision():
     assert plan(1, 4096, 12288, 256)[0] == 0                                # decode: one launch
     assert plan(128, 4096, 12288, 256)[:2] == [1, 8]                        # down_proj 8B at 128 rows: 128x128 tiles, K in 8
     assert plan(2048, 4096, 12288, 256) == [3, 1, 0, 0, 0]                  # the benchmark shape: one round of 256 tiles, no cut
+    assert plan(1024, 2048, 1536, 256)[:2] == [1, 2]                        # a tensor-parallel rank's short K: 128x128 tiles
+    assert plan(49, 5120, 25600, 128) == [3, 8, 0, 0, 5]                    # a decode batch on the 32B down_proj: 5 waves, K in 8
     p = plan(4096, 5120, 8192, 256)                                         # o_proj 32B: two regions in one launch
     assert p[0] == 2 and p[2] == 1024 and p[4] == 1
     assert L.tbik_gemm_plan_info(8, 8, 100, 256, 0, 0, out) == _lib.TBIK_ERR_INVALID   # K is not a whole number of leaves
