@@ -60,8 +60,8 @@ int tbik_tree_params(int K, int leaf_k, int* T, int* flb, int* level_k);
  *      consumed in place by the tiled kernels, which transpose 8x8 blocks in registers on the way to LDS -- same
  *      MFMA chain, same bits, no copy (the large-M pipelines are built for [N,K] only: measured on MI355X,
  *      [M,12288] x [12288,4096] row-major takes 60 / 762 us at M = 128 / 2048 against 32 / 200 us for the [N,K]
- *      form, so a caller with many rows should hand over [N,K]; the Python wrappers repack from 1024
- *      rows on).  The contiguous dimension's partner stride must be a multiple of 8 elements;
+ *      form, so a caller with many rows should hand over [N,K]; the Python wrappers repack, with bi_transpose,
+ *      where that is the faster way).  The contiguous dimension's partner stride must be a multiple of 8 elements;
  *      neither stride equal to 1 returns TBIK_ERR_UNSUPPORTED.
  *      For ldb_n == 1 the workspace size is tbik_gemm_workspace_bytes_rowmajor_b(M,N,K,leaf_k,f16).
  *   C: element (m,n) at C[m*ldc + n]

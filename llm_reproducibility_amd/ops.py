@@ -146,23 +146,34 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
 # Where a row-major [K,N] operand is repacked into the native [N,K] layout instead of being consumed in place.  In place
 # it runs on the 64-row tiled kernels only (the other pipelines are built for [N,K]); a repack is one pass of the
 # transposing copy kernel (23 us for 4096 x 4096 in 16 bits, 45 us for 12288 x 4096) and then whatever kernel is best.
-# Measured on MI355X, bf16, us in place against repacked, same bits either way:
+# Same bits either way.  Measured on MI355X, us in place against repacked:
 #   tree matmul: in place cuts K and holds out until its 64-row tiles fill a second round of the chip, that is up to 128
 #     rows (12288 x 4096: 68 against 73; at 192 rows 99 against 79, at 1024 448 against 164), later for small matrices
-#     (2048 x 2048: 256 rows 17 against 24, 384 rows 28 against 22): a bound on rows * K * N.
-#   single-accumulator mm: in place cannot cut K, and every narrow matrix is a long chain on few work-groups (4096 x 4096:
-#     76 against 23 at one row, 69 against 30 at 64 rows).  Wide ones fill the chip and the copy costs more than it gives
-#     up to 128 rows (4096 x 24576: 70 against 112 at 64 rows, 78 against 134 at 128, 143 against 140 at 256).
-_REPACK_ROWS_TREE = 416      # for a matrix of 2048 x 1536, inversely to its size, but at least 129
-_REPACK_ROWS_MM = 1          # for matrices of fewer than _WIDE_N columns
-_REPACK_ROWS_MM_WIDE = 160
-_WIDE_N = 16384
+#     (2048 x 1536: 256 rows 16 against 20, 384 rows 27 against 21; 1024 x 1024: 1024 rows 16.3 against 17.4, 1536 rows 26.5
+#     against 18.1; 512 x 1536: 1536 rows, 288 tiles, 22.8 against 14.4): bounds on rows * K * N and on the tiles.
+#   single-accumulator mm: in place cannot cut K, so a call takes as long as one chain per round of 512 work-groups (two on
+#     a CU), whatever it fills them with; narrow matrices are repacked (4096 x 4096: 88 against 27 at one row, 77 against 34 at
+#     64), wide ones not while they are one round (12288 x 16384: 220 against 273 at 64 rows, 248 against 318 at 256; 4096 x
+#     24576: 93 against 123 at 128 rows, 158 against 138 at 160).  K, the type (fp16 has slower tiles above 64 rows:
+#     12288 x 10240 at 256 rows 182 against 244, bf16 201 against 201) and the rounds move the line, so both times are estimated.
+#     Over 4,862 points of 1 .. 3072 rows, K = 512 .. 25600, N = 512 .. 151936 in both types the choice is 0.25 % from the
+#     better of the two on average and 23 % at worst.
+_TREE_IN_PLACE_MACS = 416 * 2048 * 1536
 
 
-def _consumed_in_place(rows: int, K: int, N: int, tree: bool) -> bool:
+def _consumed_in_place(rows: int, K: int, N: int, tree: bool, f16: bool = False) -> bool:
+    tiles = -(-rows // 64) * -(-N // 128)
     if tree:
-        return rows <= 128 or rows * K * N < _REPACK_ROWS_TREE * (2048 * 1536)
-    return rows < (_REPACK_ROWS_MM_WIDE if N >= _WIDE_N else _REPACK_ROWS_MM)
+        return rows <= 128 or (rows * K * N < _TREE_IN_PLACE_MACS and tiles <= 256)
+    groups = -(-N // 64) if rows <= 16 else tiles
+    in_place = (7.0 + 0.0222 * K) * max(1, -(-groups // 512))
+    copied = 4.0 * K * N    # bytes; up to 256 MB the cache behind the L2s holds them
+    product = max(K * N / 3.5e6, 0.0048 * K if rows > 64 else 0.0)
+    if f16 and rows > 64:
+        product = max(product, 0.0098 * K * -(-(-(-rows // 128) * -(-N // 128)) // 256))
+    else:
+        product = max(product, rows * K * N / 0.72e9)
+    return in_place < 11.8 + copied / (4.1e6 if copied <= 256e6 else 3.3e6) + product
 
 
 def _weight_operand(B: torch.Tensor, rows: int = 0, tree: bool = True):
@@ -175,7 +186,7 @@ def _weight_operand(B: torch.Tensor, rows: int = 0, tree: bool = True):
     (K, N), (s0, s1) = B.shape, B.stride()
     if s0 == 1 and _aligned16(B) and K % 8 == 0 and (N == 1 or (s1 >= K and s1 % 8 == 0)):
         return B, 1, (K if N == 1 else s1)
-    if s1 == 1 and _aligned16(B) and s0 >= N and s0 % 8 == 0 and _consumed_in_place(rows, K, N, tree):
+    if s1 == 1 and _aligned16(B) and s0 >= N and s0 % 8 == 0 and _consumed_in_place(rows, K, N, tree, B.dtype is torch.float16):
         return B, s0, 1
     w, ldw = _rows16(B.t())
     return w, 1, ldw

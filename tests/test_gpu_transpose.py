@@ -46,7 +46,7 @@ def test_linear_backward_operands(dev, dtype, tokens):
 def test_repacked_and_in_place_agree_around_the_rule(dev, K, N):
     B = O.gaussian_bf16((K, N), 0.02, 3).to(dev)
     Wt = B.t().contiguous().t()
-    last = max(128, (ops._REPACK_ROWS_TREE * 2048 * 1536 - 1) // (K * N))
+    last = max(128, (ops._TREE_IN_PLACE_MACS - 1) // (K * N))
     for M, tree, in_place in ((last, True, True), (last + 1, True, False), (1, False, False)):
         print("case rule", K, N, M, tree, flush=True)
         A = O.gaussian_bf16((M, K), 1.0, M).to(dev)

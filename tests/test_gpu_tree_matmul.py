@@ -309,25 +309,37 @@ def test_row_major_b_simulated_tp_as_the_reference_script_runs_it(dev):
     assert_close_to_oracle(full, O.matmul_tree(A.cpu(), B.cpu()), "row-major B, Gaussian")
 
 
-def test_row_major_b_repacked_from_many_rows_on_gives_the_same_bits(dev):
-    """From 1024 rows on (2048 for the single-accumulator mm) the wrappers repack a row-major [K,N] operand into the
-    native layout, because the in-place path runs on the small tiles only; on either side of the switch the bits are
-    those of the [N,K] form."""
+# (K, N, tree, rows consumed in place, rows repacked): both sides of the line, next to each other where the rows decide
+ROWMAJOR_LINE = [
+    (2048, 1536, True, 415, 416), (4096, 4096, True, 128, 129), (512, 1536, True, 1344, 1345),     # K * N, a second round, tiles
+    (256, 16384, False, 256, 257), (256, 16381, False, 256, 257), (1024, 32768, False, 128, 512),  # mm: a second round
+    (256, 20480, False, 1, 193), (4096, 16384, False, 128, 300),
+    (2048, 4096, False, None, 1), (2048, 14336, False, None, 8), (8192, 8192, False, None, 64),    # mm: narrow matrices
+]
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("K,N,tree,in_place,repacked", ROWMAJOR_LINE)
+def test_row_major_b_in_place_and_repacked_gives_the_same_bits(dev, K, N, tree, in_place, repacked, f16):
+    """A row-major [K,N] operand is consumed in place or repacked into the native layout, by an estimate of both; on either
+    side of the line the layout handed over is the expected one and the bits are those of the [N,K] form."""
     from llm_reproducibility_amd import ops
     from llm_reproducibility_amd.bio import batch_invariant_ops as bio
-    K, N = 2048, 1536
-    B = O.gaussian_bf16((K, N), 0.02, 3).to(dev)                 # row-major [K,N]
-    Wt = B.t().contiguous().t()                                  # the same matrix as an [N,K] weight, transposed view
+    dt = torch.float16 if f16 else torch.bfloat16
+    B = O.gaussian_bf16((K, N + (-N) % 8), 0.02, 3).to(dev).to(dt)[:, :N]      # row-major [K,N]
+    Wt = B.t().contiguous().t()                                               # the same matrix as an [N,K] weight, transposed view
     assert B.stride(1) == 1 and Wt.stride(0) == 1
-    for M in (ops._REPACK_ROWS_TREE - 1, ops._REPACK_ROWS_TREE, ops._REPACK_ROWS_MM - 1, ops._REPACK_ROWS_MM):
-        print("case row-major B rows", M, flush=True)
-        A = O.gaussian_bf16((M, K), 1.0, M).to(dev)
-        assert_bitwise(matmul_tp_persistent(A, B), matmul_tp_persistent(A, Wt), f"tree matmul, {M} rows")
-        assert torch.equal(bio.matmul_persistent(A, B), bio.matmul_persistent(A, Wt)), M
-    assert ops._weight_operand(B, ops._REPACK_ROWS_TREE - 1, True)[1] != 1      # in place
-    assert ops._weight_operand(B, ops._REPACK_ROWS_TREE, True)[1:] == (1, K)    # repacked: [N,K], K contiguous
-    assert ops._weight_operand(B, ops._REPACK_ROWS_MM - 1, False)[1] != 1
-    assert ops._weight_operand(B, ops._REPACK_ROWS_MM, False)[1:] == (1, K)
+    for M, stays in ((in_place, True), (repacked, False)):
+        if M is None:
+            continue
+        print("case row-major B", M, K, N, tree, f16, flush=True)
+        A = O.gaussian_bf16((M, K), 1.0, M).to(dev).to(dt)
+        if tree:
+            assert_bitwise(matmul_tp_persistent(A, B), matmul_tp_persistent(A, Wt), f"tree matmul, {M} rows")
+        else:
+            assert torch.equal(bio.matmul_persistent(A, B), bio.matmul_persistent(A, Wt)), M
+        layout = ops._weight_operand(B, M, tree)[1:]
+        assert layout == ((B.stride(0), 1) if stays else (1, K)), (M, layout)
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (128, 512, 12288), (16, 256, 12288), (1, 128, 8192)])
