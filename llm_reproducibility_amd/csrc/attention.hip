@@ -522,8 +522,8 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
 // updates and of the chunks -- is that of the kernels above: the same bits.
 // SPLIT: gridDim.z work-groups per (KV head, sequence); work-group z takes the chunks z, z + gridDim.z, ... as one stream of
 // tiles and leaves each chunk's state in the workspace for attention_merge_kernel.  One work-group per (KV head,
-// sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8200 keys 113 us, with
-// the chunks spread over the chip 67 us (62 and the merge; the keys and values take 36 at the rate of a one-pass read).
+// sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8000 keys 102 us, with
+// the chunks spread over the chip 57 us, the merge included (the keys and values take 42 at the rate of a one-pass read).
 // ------------------------------------------------------------------------------------------------
 template <int G, bool FUSED, bool SPLIT>
 __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a, const QkvArgs f, const SplitArgs sp) {
@@ -584,12 +584,18 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
 #pragma unroll
       for (int i = 0; i < PI; i++) dma16(lv + slot * 8192 + i * 1024, vvoff[i], src);
     };
-    load_k(tile_of(0), 0);
+    auto first_tiles = [&]() __attribute__((always_inline)) {
+      load_k(tile_of(0), 0);
 #pragma unroll
-    for (int i = 0; i < NS - 1; i++) {
-      load_k(tile_of(i + 1), i + 1);
-      load_v(tile_of(i), i);
-    }
+      for (int i = 0; i < NS - 1; i++) {
+        load_k(tile_of(i + 1), i + 1);
+        load_v(tile_of(i), i);
+      }
+    };
+    // on their way before the lengths are known, except where there may be no such chunk: in a cache that is mostly empty
+    // most of these work-groups have nothing to do (8 sequences of 300 keys in a cache of 8192: 12.1 -> 9.0 us; the wait
+    // costs full caches at most 1 us of 57)
+    if (z == 0) first_tiles();
     const int ctx = a.ctx_len[b];
     const int qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
     if (qlen <= 0) {
@@ -602,6 +608,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       return;
     }
+    if (z != 0) first_tiles();
     if (FUSED) {
       // loaders 0 and 1 form the new key and file the new value while the first tiles are on their way (the computing
       // waves form the query heads meanwhile); everything they have in flight is drained before the barrier, so the waits
@@ -802,36 +809,29 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const AttnArgs a, 
   const int b = blockIdx.z, qi = blockIdx.y;
   const int h = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (h >= a.q_heads) return;
-  int nch = 0, qlen = 0;
-  auto read_lengths = [&]() __attribute__((always_inline)) {
-    const int ctx = a.ctx_len[b];
-    qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
-    nch = qi < qlen ? min((ctx - qlen + qi) / (32 * CHUNK_TILES) + 1, sp.nchunks) : 0;
-  };
-  // a chunk of a prompt has many rows, and possibly all of one chunk: they are not loaded before that is known.  A decode
-  // step has few: their states (behind the horizon, too) are loaded while the length is on its way, and possibly not used.
-  if (!FUSED) {
-    read_lengths();
-    if (nch <= 1) return;
-  }
+  // the lengths first: a row of one chunk is complete already, and of a cache that is mostly empty only the chunks in use
+  // are read (states loaded while the lengths were on their way, all that the cache has room for, gained long contexts
+  // nothing and cost short ones 1 .. 3 us)
+  const int ctx = a.ctx_len[b];
+  const int qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
+  if (qi >= qlen) return;
+  const int nch = min((ctx - qlen + qi) / (32 * CHUNK_TILES) + 1, sp.nchunks);
+  if (nch <= 1) return;
   const int64_t at = ((int64_t)(b * sp.q_rows + qi) * a.q_heads + h) * sp.nchunks;
   const f32x2* po = reinterpret_cast<const f32x2*>(sp.o + at * HD) + lane;
   const f32x2* pm = reinterpret_cast<const f32x2*>(sp.ml + at * 2);
   constexpr int NB = 16;
   f32x2 O = {0.f, 0.f};
   float M = 0.f, L = 0.f;
-  for (int c0 = 0; c0 < sp.nchunks; c0 += NB) {
+  for (int c0 = 0; c0 < nch; c0 += NB) {
     f32x2 o[NB], ml[NB];
 #pragma unroll
     for (int i = 0; i < NB; i++) {
-      const int c = min(c0 + i, sp.nchunks - 1);
+      const int c = min(c0 + i, nch - 1);
       o[i] = po[(int64_t)c * (HD / 2)];
       ml[i] = pm[c];
     }
-    if (c0 == 0) {
-      if (FUSED) read_lengths();
-      M = ml[0][0], L = ml[0][1], O = o[0];
-    }
+    if (c0 == 0) M = ml[0][0], L = ml[0][1], O = o[0];
 #pragma unroll
     for (int i = 0; i < NB; i++) {
       if (c0 + i == 0) continue;
@@ -840,9 +840,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const AttnArgs a, 
       merge_chunk(M, L, ml[i][0], ml[i][1], fa, fb);
       O = f32x2{merge_acc(O[0], fa, o[i][0], fb), merge_acc(O[1], fa, o[i][1], fb)};
     }
-    if (c0 + NB >= nch) break;
   }
-  if (nch <= 1) return;
   const float inv = 1.0f / L;
   uint32_t* op = reinterpret_cast<uint32_t*>(a.out + ((int64_t)(FUSED ? b : a.q_start[b] + qi) * a.q_heads + h) * HD);
   op[lane] = pack_bf16x2(O[0] * inv, O[1] * inv);
@@ -851,17 +849,22 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const AttnArgs a, 
 static int chunks_of(int max_len) { return (max_len + 32 * CHUNK_TILES - 1) / (32 * CHUNK_TILES); }
 
 // How many work-groups share the chunks of a (KV head, sequence) in the decode kernel: 1 = a single one walks them all.
-// Enough for 512 work-groups in all, two per CU; from 129 pairs on a chain per pair already draws the keys at the rate of
-// the memory and the second launch is lost (us, one chain against split: 16 sequences of 2300 keys on 8 KV heads 37.2 / 35.0,
-// of 8200 keys 130 / 116; 32 of 2300 55 / 62, of 8200 194 / 204), and with two chunks there is nothing to gain
-// (1 sequence of 600 keys 10.8 / 12.0; of 1200 17.4 / 12, of 4096 49.3 / 13.1, of 16384 186 / 22).
+// Enough for 512 work-groups in all, two per CU.  From 97 pairs on a chain per pair draws the keys nearly at the rate of
+// the memory and the second launch is lost; with two chunks there is nothing to gain.  The lengths are the device's, so the
+// rule has only the cache to go by: with few keys in a large cache the second launch is 2 us too many, from 1000 keys (64
+// pairs) or 1500 (96) on the split wins (us, 8 KV heads, cache of 8192, one chain against split at 300, 600, 1000, 2000 and
+// 8000 keys: 1 sequence 6.4 / 8.5, 9.9 / 12.1, 14.4 / 12.2, 25 / 12.3, 93 / 15; 8 sequences 6.6 / 9.0, 10.2 / 12.4,
+// 16.0 / 13.0, 28 / 17, 102 / 57; 12 sequences 7.0 / 9.2, 10.8 / 14.3, 16.6 / 15.9, 29 / 27, 108 / 85; 16 sequences
+// 7.3 / 12.5, 10.8 / 16.7, 15.5 / 20.0, 32 / 33, 122 / 120).
 static int decode_split(int64_t pairs, int max_len) {
   const int nch = chunks_of(max_len);
-  if (nch < 3 || pairs > 128) return 1;
+  if (nch < 3 || pairs > 96) return 1;
   const int64_t want = 512 / pairs;
   return (int)(want > nch ? nch : want);
 }
-// The same for the grouped kernel, whose work-groups then take a chunk each: worth it while they are few.
+// The same for the grouped kernel, whose work-groups then take a chunk each: worth it while they are few (64 new tokens in
+// a cache of 8192, one chain against split at 300, 600, 1000, 2000 and 8000 keys: 1 sequence 8.4 / 10.1, 13.1 / 15.9, 20 / 16,
+// 36 / 17, 187 / 27; 4 sequences, 128 work-groups, 8.6 / 10.9, 13.8 / 22.4, 20 / 23, 44 / 30, 195 / 91).
 static bool group_split(int64_t groups, int max_len) {
   const int nch = chunks_of(max_len);
   return nch >= 3 && groups <= 128 && groups * nch <= 2048;
