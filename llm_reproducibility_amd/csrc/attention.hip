@@ -238,8 +238,8 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Grouped variant: one work-group per (16 consecutive queries, KV head, sequence); its G wavefronts are the G query
-// heads that share the KV head.  Each 32-key tile of K and of V^T is fetched from global memory ONCE per group with
+// Grouped variant: one work-group per (16 * QB consecutive queries, KV head, sequence); its G * QB wavefronts are the G
+// query heads that share the KV head, for each of the QB blocks of 16 queries.  Each 32-key tile of K and of V^T is fetched from global memory ONCE per group with
 // coalesced 16-byte loads, staged in LDS (double buffered; K rows XOR-swizzled against bank conflicts, V^T rows stored in
 // fragment order) and read from there
 // by every wave.  A row's arithmetic -- the lanes that own it, the MFMA chain, the order of the softmax updates --
@@ -254,9 +254,15 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
 // ------------------------------------------------------------------------------------------------
 // chunks: the cache has a single one / a work-group walks them all / a work-group takes one (SPLIT)
 enum { ONE_CHUNK, ALL_CHUNKS, SPLIT_CHUNKS };
-template <int G, bool DEEP, int NLD, int CHUNKS>
-__global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
+template <int G, int QB, bool DEEP, int NLD, int CHUNKS>
+__global__ __launch_bounds__(64 * (G * QB + NLD)) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
   constexpr bool SPLIT = CHUNKS == SPLIT_CHUNKS;
+  constexpr int NW = G * QB;   // computing wavefronts
+  // The merged chunks (32 registers a lane, touched once in sixteen tiles) would cost work-groups of eight wavefronts the
+  // second one of a CU: half of them lie in LDS there, which two such work-groups have to spare (64 of 80 KiB), and four
+  // wavefronts fit a SIMD again (144 -> 124 registers).
+  constexpr int PARK = CHUNKS == ALL_CHUNKS && NW == 8 && NLD == 0 ? 4 : 0;
+  __shared__ f32x4 parked[PARK ? PARK : 1][PARK ? 64 * NW : 1];
   __shared__ __attribute__((aligned(16))) uint8_t lds[2][16384];  // per buffer: K tile [32][128] (8 KiB), V^T tile [128][32] (8 KiB)
   const int b = blockIdx.y;
   // Work-groups are dealt to the eight XCDs round robin, each with an L2 of its own: with the KV head as the fastest
@@ -267,30 +273,32 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
   const int kvh = blockIdx.x % a.kv_heads;
   const int qb = gridDim.x / a.kv_heads - 1 - blockIdx.x / a.kv_heads;
   const int qlen = a.q_len[b];
-  if (qb * 16 >= qlen) return;  // uniform over the work-group
+  if (qb * (16 * QB) >= qlen) return;  // uniform over the work-group
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int h = kvh * G + (tid >> 6);
+  const int wave = tid >> 6;
+  const int h = kvh * G + (QB == 1 ? wave : wave % G);
   const int j = lane & 15;
   const int g = lane >> 4;
   const int ctx = a.ctx_len[b];
-  const int qrow = qb * 16 + j;
+  const int qrow = qb * (16 * QB) + (QB == 1 ? 0 : wave / G * 16) + j;
   const bool qvalid = qrow < qlen;
   const int qpos = ctx - qlen + min(qrow, qlen - 1);
-  const int last_pos = ctx - qlen + min(qb * 16 + 15, qlen - 1);
+  const int last_pos = ctx - qlen + min(qb * (16 * QB) + (16 * QB - 1), qlen - 1);
 
   const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.k_cache + ((int64_t)b * a.kv_heads + kvh) * a.max_len * HD);
   const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vt_cache + ((int64_t)b * a.kv_heads + kvh) * (int64_t)HD * a.max_len);
 
   // cooperative staging: 512 16-byte chunks per tile and operand, NCH per thread
   // (NLD loader waves, where the kernel has them, do all of it; the computing waves then neither load nor store tiles)
-  constexpr int NT = NLD ? 64 * NLD : 64 * G;
-  const int stid = NLD ? tid - 64 * G : tid;   // staging thread
+  constexpr int NT = NLD ? 64 * NLD : 64 * NW;
+  const int stid = NLD ? tid - 64 * NW : tid;   // staging thread
   constexpr int NCH = (512 + NT - 1) / NT;
   // Key tiles are fetched DEPTH tiles ahead into DEPTH register sets (set = tile % DEPTH).  DEEP is for decode: a
   // single block of queries per sequence makes the kernel a chain of memory round trips, and one tile of arithmetic
-  // hides none of them.  Prefill has arithmetic to overlap and prefers the registers (more waves per SIMD).
-  constexpr int DEPTH = !DEEP ? 1 : (NCH <= 2 ? 4 : (NCH <= 4 ? 2 : 1));
+  // hides none of them.  Prefill has arithmetic to overlap and prefers the registers (more waves per SIMD), and so does
+  // decode where they decide about the second work-group of a CU (8 heads, 128 sequences of 1000 keys 151 -> 116 us).
+  constexpr int DEPTH = !DEEP ? 1 : PARK ? 2 : (NCH <= 2 ? 4 : (NCH <= 4 ? 2 : 1));
   u32x4 kregs[DEPTH][NCH], vregs[DEPTH][NCH];
   // A K tile is 8 KiB of consecutive bytes (32 rows of 256), chunk ch at byte 16 ch; a V^T tile is 128 rows of 64 bytes,
   // max_len elements apart.  Per-thread byte offsets inside a tile (global and LDS side) are formed once; per tile only
@@ -378,9 +386,13 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
   for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = kNoKey;
   float l = 0.f;
-  // The merged chunks so far.  (They cost the full chip a wavefront per SIMD, three instead of four, and 7 % at 4096 keys;
-  // parked in scratch memory instead they cost 25 %: 557 MB of it for a prompt of 4096.)
-  f32x4 ot[8];
+  // The merged chunks so far.  (All of them parked in scratch memory cost 25 %: 557 MB of it for a prompt of 4096.)
+  f32x4 ot[8 - PARK];
+  auto merged = [&](int t) __attribute__((always_inline)) { return t < 8 - PARK ? ot[t] : parked[t - (8 - PARK)][tid]; };
+  auto set_merged = [&](int t, f32x4 v) __attribute__((always_inline)) {
+    if (t < 8 - PARK) ot[t] = v;
+    else parked[t - (8 - PARK)][tid] = v;
+  };
   float mt = 0.f, lt = 0.f;
   // chunk `c` is complete: merged into the rows that see it; after the last one the result stays in m, l and o,
   // otherwise an empty state follows
@@ -390,19 +402,22 @@ __global__ __launch_bounds__(64 * (G + NLD)) void attention_group_kernel(const A
         float fa, fb;
         merge_chunk(mt, lt, m, l, fa, fb);
 #pragma unroll
-        for (int t = 0; t < 8; t++)
+        for (int t = 0; t < 8; t++) {
+          f32x4 u = merged(t);
 #pragma unroll
-          for (int i = 0; i < 4; i++) ot[t][i] = merge_acc(ot[t][i], fa, o[t][i], fb);
+          for (int i = 0; i < 4; i++) u[i] = merge_acc(u[i], fa, o[t][i], fb);
+          set_merged(t, u);
+        }
       }
     } else {
       mt = m, lt = l;
 #pragma unroll
-      for (int t = 0; t < 8; t++) ot[t] = o[t];
+      for (int t = 0; t < 8; t++) set_merged(t, o[t]);
     }
     if (last) {
       l = lt;
 #pragma unroll
-      for (int t = 0; t < 8; t++) o[t] = ot[t];
+      for (int t = 0; t < 8; t++) o[t] = merged(t);
     } else {
       m = kNoKey, l = 0.f;
 #pragma unroll
@@ -922,6 +937,58 @@ static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max
   return hip_code(hipGetLastError());
 }
 
+template <int G, int QB, bool DEEP, int NLD, int CHUNKS>
+static void group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_q_len, hipStream_t stream) {
+  const int64_t blocks = ((int64_t)max_q_len + 16 * QB - 1) / (16 * QB);
+  const dim3 grid((unsigned)(blocks * a.kv_heads), (unsigned)batch, CHUNKS == SPLIT_CHUNKS ? (unsigned)sp.nchunks : 1u);
+  hipLaunchKernelGGL((attention_group_kernel<G, QB, DEEP, NLD, CHUNKS>), grid, dim3(64 * (G * QB + NLD)), 0, stream, a, sp);
+}
+
+// The form of the grouped kernel, same bits in all.  Lengths are the device's, so what is known is the number of
+// work-groups of one block of 16 queries and the cache length.
+// Two more waves per work-group that only stage the tiles (NLD = 2) take the loads and LDS writes out of the computing
+// waves' instruction streams.  That pays while the launch leaves CUs short of work-groups (a chunk of a prompt, a few
+// sequences: up to two work-groups per CU: 3 - 18 % faster) and costs once the chip is full, where the extra waves
+// take the place of a whole work-group (from three per CU on: 35 % slower).
+// In a cache of several chunks the accumulators of the merged chunks take a wavefront per SIMD from the others, and a
+// block of 16 queries at a time is 7 - 40 % slower than a walk without chunks is.  There two blocks share a work-group
+// (one of eight heads has eight wavefronts by itself) once a launch of that form fills the chip; before that, four
+// heads have a range in which one block without loader waves is ahead, and one or two heads keep the loader waves for as
+// long as all their work-groups are resident at once.  Measured on MI355X, us, a walk without chunks / one block / the form
+// chosen here:
+//   4 heads: 3 prompts of 4096, 3136 and 2176 tokens 327 / 347 / 308, 1 of 8192 655 / 705 / 615, 32 chunks of 64 tokens at
+//     4000 keys 206 / 273 / 182, 16 prompts of 400 in a cache of 8192 47.1 / 48.2 / 50.0; 1040 tokens (520 blocks) 24.6 /
+//     26.6 / 26.6, against 30.1 with two blocks and 24.7 with loader waves (which take 123 against 103 where 4000 keys are
+//     cached already); at 1024 blocks 2 prompts of 1020 35.6 / 35.3 / 40.2 but 8 chunks of 250 at 800 keys 39 / 45.5 / 37.7;
+//   8 heads: prompt of 4096 298 / 420 / 310, 16 of 400 87 / 111 / 87;   2 heads: 125 / 130 / 102, 1040 tokens 22.6 / 26.3 / 20.8;
+//   1 head: 217 / 225 / 126, 1040 tokens 27.0 / 28.2 / 20.8.
+// What is left of the cost of the chunks is their merge, where a launch is a chain (520 tokens 12.6 -> 13.7) or its rounds
+// are few.
+template <int G>
+static void group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
+  const bool deep = max_q_len <= 16;  // decode: one block of queries per sequence
+  const int64_t groups = ((int64_t)max_q_len + 15) / 16 * a.kv_heads * batch;
+#define TBIK_ATTN_GROUP(...) group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
+  if (split) {
+    if (deep) TBIK_ATTN_GROUP(1, true, 2, SPLIT_CHUNKS);
+    else TBIK_ATTN_GROUP(1, false, 2, SPLIT_CHUNKS);
+  } else if (chunks_of(a.max_len) == 1) {
+    if (groups <= 512 && deep) TBIK_ATTN_GROUP(1, true, 2, ONE_CHUNK);
+    else if (groups <= 512) TBIK_ATTN_GROUP(1, false, 2, ONE_CHUNK);
+    else if (deep) TBIK_ATTN_GROUP(1, true, 0, ONE_CHUNK);
+    else TBIK_ATTN_GROUP(1, false, 0, ONE_CHUNK);
+  } else if (deep) {
+    if (groups <= 512) TBIK_ATTN_GROUP(1, true, 2, ALL_CHUNKS);
+    else TBIK_ATTN_GROUP(1, true, 0, ALL_CHUNKS);
+  } else {
+    constexpr int LOADERS = G == 1 ? 1280 : G == 2 ? 1024 : 512, SINGLE = G == 4 ? 768 : 0, QB = G == 8 ? 1 : 2;
+    if (groups <= LOADERS) TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS);
+    else if (groups <= SINGLE) TBIK_ATTN_GROUP(1, false, 0, ALL_CHUNKS);
+    else TBIK_ATTN_GROUP(QB, false, 0, ALL_CHUNKS);
+  }
+#undef TBIK_ATTN_GROUP
+}
+
 int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache, void* out, const int* q_start,
                        const int* q_len, const int* ctx_len, int batch, int max_q_len, int q_heads, int kv_heads,
                        int head_dim, int max_len, float scale, void* ws, size_t ws_bytes, hipStream_t stream) {
@@ -939,7 +1006,6 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
   const int G = q_heads / kv_heads;
   const bool grouped = grouped_cache(G, kv_heads, max_len);
   if (grouped) {
-    const bool deep = max_q_len <= 16;  // decode: one block of queries per sequence
     if ((int64_t)max_q_len * G <= 16) {  // all queries of a sequence and all heads of a group in one MFMA tile
       const QkvArgs none{};
       if (G == 1) return decode_launch<1, false>(a, none, batch, max_q_len, ws, ws_bytes, stream);
@@ -949,38 +1015,13 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
     }
     const int64_t gx = (int64_t)((max_q_len + 15) / 16) * kv_heads;
     if (gx > 0x7fffffff) return TBIK_ERR_INVALID;
-    const dim3 grid((unsigned)gx, (unsigned)batch, 1u);
-    // Two more waves per work-group that only stage the tiles (NLD = 2) take the loads and LDS writes out of the computing
-    // waves' instruction streams.  That pays while the launch leaves CUs short of work-groups (a chunk of a prompt, a few
-    // sequences: up to two work-groups per CU: 3 - 18 % faster) and costs once the chip is full, where the extra waves
-    // take the place of a whole work-group (from three per CU on: 35 % slower).  Same bits either way.
-    const bool few = gx * batch <= 512;
     const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len) : 0;
     const bool split = need != 0 && ws_bytes >= need;
-    const bool one = chunks_of(max_len) == 1;
     const SplitArgs sp = split ? split_args(ws, batch, max_q_len, q_heads, kv_heads, max_len) : SplitArgs{};
-    const dim3 cgrid((unsigned)gx, (unsigned)batch, (unsigned)chunks_of(max_len));
-#define TBIK_ATTN_GROUP_RUN(GG, DEEP, NLD, CH, GRID)                                                                              \
-  hipLaunchKernelGGL((attention_group_kernel<GG, DEEP, NLD, CH>), GRID, dim3(64 * (GG + NLD)), 0, stream, a, sp)
-#define TBIK_ATTN_GROUP(GG)                                                                  \
-  do {                                                                                       \
-    if (split && deep) TBIK_ATTN_GROUP_RUN(GG, true, 2, SPLIT_CHUNKS, cgrid);                \
-    else if (split) TBIK_ATTN_GROUP_RUN(GG, false, 2, SPLIT_CHUNKS, cgrid);                  \
-    else if (one && few && deep) TBIK_ATTN_GROUP_RUN(GG, true, 2, ONE_CHUNK, grid);          \
-    else if (one && few) TBIK_ATTN_GROUP_RUN(GG, false, 2, ONE_CHUNK, grid);                 \
-    else if (one && deep) TBIK_ATTN_GROUP_RUN(GG, true, 0, ONE_CHUNK, grid);                 \
-    else if (one) TBIK_ATTN_GROUP_RUN(GG, false, 0, ONE_CHUNK, grid);                        \
-    else if (few && deep) TBIK_ATTN_GROUP_RUN(GG, true, 2, ALL_CHUNKS, grid);                \
-    else if (few) TBIK_ATTN_GROUP_RUN(GG, false, 2, ALL_CHUNKS, grid);                       \
-    else if (deep) TBIK_ATTN_GROUP_RUN(GG, true, 0, ALL_CHUNKS, grid);                       \
-    else TBIK_ATTN_GROUP_RUN(GG, false, 0, ALL_CHUNKS, grid);                                \
-  } while (0)
-    if (G == 1) TBIK_ATTN_GROUP(1);
-    else if (G == 2) TBIK_ATTN_GROUP(2);
-    else if (G == 4) TBIK_ATTN_GROUP(4);
-    else TBIK_ATTN_GROUP(8);
-#undef TBIK_ATTN_GROUP
-#undef TBIK_ATTN_GROUP_RUN
+    if (G == 1) group_launch<1>(a, sp, split, batch, max_q_len, stream);
+    else if (G == 2) group_launch<2>(a, sp, split, batch, max_q_len, stream);
+    else if (G == 4) group_launch<4>(a, sp, split, batch, max_q_len, stream);
+    else group_launch<8>(a, sp, split, batch, max_q_len, stream);
     if (split) merge_launch<false>(a, sp, batch, stream);
   } else {
     const dim3 grid((unsigned)((max_q_len + 15) / 16), (unsigned)q_heads, (unsigned)batch);

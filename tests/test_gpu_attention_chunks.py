@@ -64,6 +64,33 @@ def test_chunk_edges(dev, monkeypatch, hq, hkv, new, ctxs):
     assert torch.equal(ops.bi_attention_bf16(q, kc, vt, *args), shared)
 
 
+# one launch of each form that the grouped kernel takes once the chip is full (query heads, KV heads, sequences, longest
+# number of new tokens): two blocks of queries per work-group, eight heads, one block, and eight heads of a few queries
+@pytest.mark.parametrize("hq,hkv,B,new", [(32, 8, 20, 80), (16, 8, 26, 80), (16, 16, 17, 80), (64, 8, 13, 80), (32, 8, 16, 80), (64, 8, 65, 8)])
+def test_forms_for_a_full_chip(dev, hq, hkv, B, new):
+    """Ragged prompts and chunks around the edges of blocks of 16 and 32 queries, of tiles and of chunks: the bits of the
+    one-wave kernel, and of a sequence alone in a short cache."""
+    print("case full chip", hq, hkv, B, new, flush=True)
+    gen = torch.Generator(device=dev).manual_seed(hq + B)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    qlens = [min(new, (80, 1, 17, 32, 33, 79, 16, 49)[b % 8]) for b in range(B)]
+    ctxs = [max(n, (1100, 512, 513, 80, 1024, 1025, 530, 545, 1056)[b % 9]) for b, n in enumerate(qlens)]
+    L = 1120
+    assert ((new + 15) // 16) * hkv * B > 512                   # beyond the forms with loader waves
+    starts = [sum(qlens[:i]) for i in range(B)]
+    q, kc, vt = rnd(sum(qlens), hq, D), rnd(B, hkv, L, D), rnd(B, hkv, D, L)
+    args = (i32(starts), i32(qlens), i32(ctxs), new, SCALE)
+    got = ops.bi_attention_bf16(q, kc, vt, *args)
+    pad = torch.nn.functional.pad
+    assert torch.equal(ops.bi_attention_bf16(q, pad(kc, (0, 0, 0, 4)), pad(vt, (0, 4)), *args), got)   # the one-wave kernel
+    for b in (0, 5, B - 1):
+        n, short = qlens[b], (ctxs[b] + 31) // 32 * 32
+        alone = ops.bi_attention_bf16(q[starts[b]: starts[b] + n], kc[b: b + 1, :, :short].contiguous(), vt[b: b + 1, :, :, :short].contiguous(),
+                                      i32([0]), i32([n]), i32([ctxs[b]]), n, SCALE)
+        assert torch.equal(alone, got[starts[b]: starts[b] + n])
+
+
 @pytest.mark.parametrize("ctxs", [[1537], [512, 513, 1024, 1025, 0, 1700], [600] * 20])
 def test_one_launch_decode_step_over_chunks(dev, monkeypatch, ctxs):
     """The decode step that forms its own query, key and value: outputs and caches with and without the workspace."""
