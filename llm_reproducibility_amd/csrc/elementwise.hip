@@ -72,9 +72,10 @@ namespace tbik {
 // Bound: memory (12 KiB in and out per token at 32/8 heads) once two things are out of its way.  Sine and cosine belong
 // to the token, not to the head: a wavefront takes HPW heads of one token and forms them once (formed per head they kept
 // the vector units busy three times as long as the memory).  And the transposed values: stored by the wavefront of a
-// token they are 2-byte pieces max_len apart, so work-groups of 64 tokens x one value head pass them through LDS and
-// store, per channel, what consecutive tokens leave at consecutive positions.  9,096 tokens of three prompts: 132 -> 47 us
-// (a copy of the bytes takes 44), 1000 tokens 17.3 -> 9.1, a few tokens 5 as before.
+// token they are 2-byte pieces max_len apart, so work-groups of 64 tokens x 128 / VS channels of a value head pass them
+// through LDS and store, per channel, what consecutive tokens leave at consecutive positions.  9,096 tokens of three
+// prompts: 132 -> 47 us (a copy of the bytes takes 44).  A call of fewer tokens is a chain of latencies and of stores that
+// may all be scattered (one new token for each of many sequences), and takes smaller pieces; see the dispatch.
 // ------------------------------------------------------------------------------------------------
 struct QkRopeArgs {
   const uint16_t* qkv;
@@ -94,30 +95,33 @@ struct QkRopeArgs {
 
 constexpr int VT_TOKENS = 64;   // tokens per work-group of the value part
 
-// Work-groups [0, value_groups): 64 tokens of one value head each; the others: four wavefronts of HPW query or key heads.
-constexpr int HPW = 8;   // heads per wavefront (1, 2, 4: 103, 69, 54 us at 9,096 tokens; no difference below 200)
-
+// Work-groups [0, value_groups): 64 tokens of 128 / VS channels of one value head each; the others: four wavefronts of HPW
+// query or key heads.
+template <int VS, int HPW>
 __global__ __launch_bounds__(256) void qk_norm_rope_cache_kernel(const QkRopeArgs a, int value_groups, int q_units, int units) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if ((int)blockIdx.x < value_groups) {
-    __shared__ uint16_t tile[VT_TOKENS][130];   // rows an odd number of words apart: a column is free of bank conflicts
-    const int h = blockIdx.x % a.kv_heads;
-    const int64_t t0 = (int64_t)(blockIdx.x / a.kv_heads) * VT_TOKENS;
-    const uint16_t* src = a.qkv + t0 * a.ld + (int64_t)(a.q_heads + a.kv_heads + h) * 128;
+    constexpr int NC = 128 / VS, PAIRS = NC / 2;   // channels of the work-group
+    __shared__ uint16_t tile[VT_TOKENS][NC + 2];   // rows an odd number of words apart: a column is free of bank conflicts
+    const int unit = blockIdx.x / VS, c0 = blockIdx.x % VS * NC;
+    const int h = unit % a.kv_heads;
+    const int64_t t0 = (int64_t)(unit / a.kv_heads) * VT_TOKENS;
+    const uint16_t* src = a.qkv + t0 * a.ld + (int64_t)(a.q_heads + a.kv_heads + h) * 128 + c0;
     const int nt = (int)(a.tokens - t0 < VT_TOKENS ? a.tokens - t0 : VT_TOKENS);
 #pragma unroll
-    for (int i = 0; i < VT_TOKENS / 4; i++) {   // wavefront w: tokens w, w + 4, ..., two channels per lane
-      const int t = min(i * 4 + wave, nt - 1);
-      uint16_t lo = src[t * a.ld + 2 * lane], hi = src[t * a.ld + 2 * lane + 1];
-      *reinterpret_cast<uint32_t*>(&tile[i * 4 + wave][2 * lane]) = (uint32_t)lo | ((uint32_t)hi << 16);
+    for (int i = 0; i < VT_TOKENS * PAIRS / 256; i++) {   // two channels of a token per thread
+      const int e = i * 256 + threadIdx.x, row = e / PAIRS, c = 2 * (e % PAIRS);
+      const int t = min(row, nt - 1);
+      uint16_t lo = src[t * a.ld + c], hi = src[t * a.ld + c + 1];
+      *reinterpret_cast<uint32_t*>(&tile[row][c]) = (uint32_t)lo | ((uint32_t)hi << 16);
     }
     __syncthreads();
     if (lane >= nt) return;
     const int64_t pos = a.pos[t0 + lane], sq = a.seq[t0 + lane];
     if (sq < 0 || sq >= a.batch || pos < 0 || pos >= a.max_len) return;
-    uint16_t* dst = a.vt_cache + ((sq * a.kv_heads + h) * 128 + wave * 32) * (int64_t)a.max_len + pos;
+    uint16_t* dst = a.vt_cache + ((sq * a.kv_heads + h) * 128 + c0 + wave * (NC / 4)) * (int64_t)a.max_len + pos;
 #pragma unroll 8
-    for (int c = 0; c < 32; c++) dst[(int64_t)c * a.max_len] = tile[lane][wave * 32 + c];
+    for (int c = 0; c < NC / 4; c++) dst[(int64_t)c * a.max_len] = tile[lane][wave * (NC / 4) + c];
     return;
   }
   const int64_t unit = (int64_t)(blockIdx.x - value_groups) * 4 + wave;
@@ -159,6 +163,26 @@ __global__ __launch_bounds__(256) void qk_norm_rope_cache_kernel(const QkRopeArg
   }
 }
 
+template <int VS, int HPW>
+static int qk_rope_launch(const QkRopeArgs& a, hipStream_t stream) {
+  const int q_units = (a.q_heads + HPW - 1) / HPW, units = q_units + (a.kv_heads + HPW - 1) / HPW;
+  const int64_t vg = (a.tokens + VT_TOKENS - 1) / VT_TOKENS * a.kv_heads * VS, blocks = vg + (a.tokens * units + 3) / 4;
+  if (blocks > 0x7fffffff) return TBIK_ERR_INVALID;
+  hipLaunchKernelGGL((qk_norm_rope_cache_kernel<VS, HPW>), dim3((unsigned)blocks), dim3(256), 0, stream, a, (int)vg, q_units, units);
+  return hip_code(hipGetLastError());
+}
+// Heads per wavefront: by the (token, head) pairs there are, so that they still occupy the chip.  us of one launch in a graph
+// at 32/8 heads, 1, 2, 4, 8 heads (a wavefront and value per token and head before): 1 token 2.4, 2.5, 2.9, 3.7 (2.2);
+// 64 tokens of one prompt 2.9, 2.8, 3.2, 4.0 (2.9); 256 5.1, 4.2, 4.1, 4.7 (6.2); 1000 13.5, 10.1, 8.7, 8.6 (16.1).
+template <int VS>
+static int qk_rope_by_heads(const QkRopeArgs& a, hipStream_t stream) {
+  const int64_t pairs = a.tokens * (a.q_heads + a.kv_heads);
+  if (pairs <= 2048) return qk_rope_launch<VS, 1>(a, stream);
+  if (pairs <= 8192) return qk_rope_launch<VS, 2>(a, stream);
+  if (pairs <= 32768) return qk_rope_launch<VS, 4>(a, stream);
+  return qk_rope_launch<VS, 8>(a, stream);
+}
+
 int qk_norm_rope_cache_dispatch(const void* qkv, int64_t ld, const void* q_weight, const void* k_weight,
                                 const float* inv_freq, const int64_t* positions, const int64_t* seq_of_token, void* q_out,
                                 void* k_cache, void* vt_cache, int64_t tokens, int q_heads, int kv_heads, int head_dim,
@@ -172,11 +196,13 @@ int qk_norm_rope_cache_dispatch(const void* qkv, int64_t ld, const void* q_weigh
   QkRopeArgs a{static_cast<const uint16_t*>(qkv), ld, static_cast<const uint16_t*>(q_weight),
                static_cast<const uint16_t*>(k_weight), inv_freq, positions, seq_of_token, static_cast<uint16_t*>(q_out),
                static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(vt_cache), tokens, q_heads, kv_heads, max_len, batch, eps};
-  const int q_units = (q_heads + HPW - 1) / HPW, units = q_units + (kv_heads + HPW - 1) / HPW;
-  const int64_t vg = (tokens + VT_TOKENS - 1) / VT_TOKENS * kv_heads, blocks = vg + (tokens * units + 3) / 4;
-  if (blocks > 0x7fffffff) return TBIK_ERR_INVALID;
-  hipLaunchKernelGGL(qk_norm_rope_cache_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a, (int)vg, q_units, units);
-  return hip_code(hipGetLastError());
+  // Channels per work-group of the values, for stores that are scattered: sequences with one token each at 8 KV heads,
+  // VS = 1, 4, 16 (before): 64 of them 11.7, 4.9, 3.5 us (3.9), 200 10.7, 6.7, 6.3 (6.0), 400 12.1, 9.6, 10.3 (9.8); 200 at 16
+  // KV heads 13.0, 8.3, 9.3 (7.6).  A prompt of 2000 tokens 14.1, 15.4, 19.9 (30.9).
+  const int64_t tiles = (tokens + VT_TOKENS - 1) / VT_TOKENS * kv_heads;
+  if (tiles <= 32) return qk_rope_by_heads<16>(a, stream);
+  if (tiles < 256) return qk_rope_by_heads<4>(a, stream);
+  return qk_rope_by_heads<1>(a, stream);
 }
 
 }  // namespace tbik

@@ -1,5 +1,5 @@
-"""q/k norm, rotary embedding and cache write at the edges of the kernel's units: 64 tokens per value tile, eight heads
-per wavefront."""
+"""q/k norm, rotary embedding and cache write at the edges of the kernel's units: 64 tokens and 128, 32 or 8 channels per
+value tile, one to eight heads per wavefront, tokens side by side and one for each of many sequences."""
 import pytest
 import torch
 
@@ -9,7 +9,8 @@ from oracle import tbik_oracle as O
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("hq,hkv,lens,prefix", [(8, 1, [1], 0), (5, 3, [63, 2], 7), (32, 8, [64], 0), (9, 9, [65, 30, 40], 3), (16, 2, [300], 33)])
+@pytest.mark.parametrize("hq,hkv,lens,prefix", [(8, 1, [1], 0), (5, 3, [63, 2], 7), (32, 8, [64], 0), (9, 9, [65, 30, 40], 3), (16, 2, [300], 33),
+                                                (4, 1, [1] * 70, 5), (8, 8, [1] * 257, 2), (8, 16, [1000], 0), (64, 8, [513], 1)])
 def test_units_and_remainders(dev, hq, hkv, lens, prefix):
     print("case qk_norm_rope", hq, hkv, lens, flush=True)
     T, B, L = sum(lens), len(lens), (max(lens) + prefix + 31) // 32 * 32
