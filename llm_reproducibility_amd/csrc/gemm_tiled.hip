@@ -481,27 +481,32 @@ static int column_regions(int M, int N, int K, int leaf_k, bool f16) {
 
 // Up to 64 rows on the ring kernel: waves per work-group (32 columns each) and K split, from an estimate of the pass:
 // rounds of 256 work-groups (the ring takes a CU's whole LDS), each 2.5 us plus its bytes at the 24 GB/s that a CU gets
-// when all of them stream (X rows come from the L2 and count a third), plus the shard combine.  No cut whose partial
-// results outgrow the static scratch: tbik_gemm_bf16_static takes every decode batch ([32,8192]x[8192,151936] would be
-// cut into four for the last round's sake, 37 MiB of partials).
+// when all of them stream (X rows come from the L2 and count a third), plus the shard combine.  That is 4 us, but only 2
+// for two parts, which are priced so against an uncut product alone: against four parts they lose ([33,1024]x[1024,768] with
+// leaves of 128 in four, in two 6.9, 9.0 us; in two instead of uncut with leaves of 256 9.6 -> 8.0, [33,4608]x[4608,16384]
+// 42.0 -> 31.6; over 307 such shapes -6 % on average).  No cut whose partial results outgrow the static scratch:
+// tbik_gemm_bf16_static takes every decode batch ([32,8192]x[8192,151936] would be cut into four for the last round's sake,
+// 37 MiB of partials).
 static int few_waves(int M, int N, int K, int lb, int* best_split) {
   const int max_split = lb >= 3 ? 8 : (1 << lb);
   const int rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
   double best = 0;
   int waves = 0;
-  for (int sp = 1, ls = 0; sp <= max_split; sp *= 2, ls++) {
-    if (lb - ls > TREE_FEW_LEVELS || (sp > 1 && (int64_t)sp * M * N * 2 > TBIK_STATIC_SCRATCH_BYTES)) continue;
+  auto price = [&](int sp, int ls, double combine_us) {
+    if (lb - ls > TREE_FEW_LEVELS || (sp > 1 && (int64_t)sp * M * N * 2 > TBIK_STATIC_SCRATCH_BYTES)) return;
     for (int nw = 2; nw <= 6; nw++) {
       const int64_t tiles = ((int64_t)N + nw * 32 - 1) / (nw * 32);
       double t = (double)((tiles * sp + 255) / 256) * (2.5 + (double)K / sp * 2 * (nw * 32 + rows * 0.33) / 24.0e3);
-      if (sp > 1) t += 4.0 + (double)(sp + 1) * M * N * 2.0 / 5.0e6;
+      if (sp > 1) t += combine_us + (double)(sp + 1) * M * N * 2.0 / 5.0e6;
       if (!waves || t < best) {
         best = t;
         waves = nw;
         *best_split = sp;
       }
     }
-  }
+  };
+  for (int sp = 1, ls = 0; sp <= max_split; sp *= 2, ls++) price(sp, ls, 4.0);
+  if (waves && *best_split == 1 && max_split > 1) price(2, 1, 2.0);
   return waves;
 }
 

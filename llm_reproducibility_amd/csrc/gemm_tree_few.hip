@@ -13,7 +13,9 @@
 //
 // Measured with cold weights, shard combine included, tiled kernel -> this: [49,25600]x[25600,5120] 67.1 -> 56.9 us,
 // [32,25600]x[25600,5120] 63.3 -> 53.0 (5.0 TB/s), [32,8192]x[8192,5120] 25.0 -> 20.2, [32,12288]x[12288,4096] 25.9 -> 24.3,
-// [16,12288]x[12288,4096] 24.2 -> 23.2; never behind by more than 2 % over 5 .. 64 rows of nine layer shapes.
+// [16,12288]x[12288,4096] 24.2 -> 23.2; never behind by more than 2 % over 5 .. 64 rows of nine layer shapes.  Over 1479 points
+// of N = 64 .. 51200 and K = 256 .. 32768 8 % faster on average, 8 % of them more than 4 % slower: a few rows on tiny
+// matrices (0.4 .. 1 us) and N = 16384 and more on a K cut in two ([32,12288]x[12288,16384] 80 -> 97).
 //
 // The arithmetic per element is that of gemm_tiled.hip: one chain of 16x16x32 MFMAs over ascending k per leaf, one
 // rounding per leaf, left to right over the leaves of a group, adjacent pairs above, every node rounded; the whole tree

@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
     (49, 24570, 512, 256),   # no cut of K, a level of the tree inside the shard
     (48, 300, 3200, 128),    # groups of 25 leaves, fewer slices in the ring than in the shard
     (20, 1000, 256, 256),    # one leaf: fewer slices than the ring holds
+    (33, 300, 1024, 256),    # K in two rather than uncut
 ])
 def test_oracle_and_larger_batch(dev, M, N, K, leaf, f16):
     print("case few", M, N, K, leaf, f16, flush=True)

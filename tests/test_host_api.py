@@ -103,6 +103,7 @@ def test_workspace_query_and_plan_come_from_one_decision():
     assert plan(2048, 4096, 12288, 256) == [3, 1, 0, 0, 0]                  # the benchmark shape: one round of 256 tiles, no cut
     assert plan(1024, 2048, 1536, 256)[:2] == [1, 2]                        # a tensor-parallel rank's short K: 128x128 tiles
     assert plan(49, 5120, 25600, 128) == [3, 8, 0, 0, 5]                    # a decode batch on the 32B down_proj: 5 waves, K in 8
+    assert plan(33, 2048, 1024, 256) == [3, 2, 0, 0, 2]                     # a short K: two parts and their combine beat the uncut chain
     p = plan(4096, 5120, 8192, 256)                                         # o_proj 32B: two regions in one launch
     assert p[0] == 2 and p[2] == 1024 and p[4] == 1
     assert L.tbik_gemm_plan_info(8, 8, 100, 256, 0, 0, out) == _lib.TBIK_ERR_INVALID   # K is not a whole number of leaves
