@@ -214,9 +214,9 @@ int bi_mean_dim(const void* x, void* out,
                 tbik_stream_t stream);
 
 /*
- * Causal grouped-query attention with a fixed key order (tiles of 32 keys, ascending, online softmax, one
- * pass, no split over keys), bf16, head_dim 128; prefill, chunked prefill and decode run the same arithmetic
- * per row (whichever kernel takes the call), and a token's output does not depend on the batch it is computed in.
+ * Causal grouped-query attention with a fixed key order (tiles of 32 keys, ascending, online softmax, in chunks of 512
+ * keys at fixed positions whose states are merged in ascending order), bf16, head_dim 128; prefill, chunked prefill and
+ * decode run the same arithmetic per row (whichever kernel takes the call), and a token's output does not depend on the batch it is computed in.
  *   q, out      [tokens, q_heads, 128]
  *   k_cache     [batch, kv_heads, max_len, 128]
  *   vt_cache    [batch, kv_heads, 128, max_len]   (V stored transposed; entries behind ctx_len must be finite)
@@ -236,7 +236,9 @@ int bi_attention_bf16(const void* q, const void* k_cache, const void* vt_cache, 
  * bi_attention_bf16 with scratch memory, for calls with a few new queries per sequence against long caches: the chunks of
  * 512 keys of a (sequence, KV head) are then shared by several work-groups and a second launch merges them in the order
  * in which a single work-group would -- the same bits.  bi_attention_workspace_bytes(...) says how much scratch such a call
- * uses (0: the call gains nothing, pass NULL); with less than that, or NULL, the call runs as bi_attention_bf16.
+ * uses (0: the call gains nothing, pass NULL); with less than that, or NULL, the call runs as bi_attention_bf16.  It goes by
+ * max_len, the only length the host knows: a caller that knows its contexts to be short in a long cache (below some 700
+ * keys, where the second launch costs 2 us and gains nothing) passes NULL as well.
  * The scratch (16-byte aligned) need not be initialised and must not be shared by calls that overlap.
  * max_q_len = 1 gives the size for bi_attention_decode_qkv_ws_bf16.
  * Replaces: as bi_attention_bf16 (the reference's alignment mode forces the kernel without such a split, because its merge
@@ -350,7 +352,7 @@ int bi_silu_mul_bf16(const void* gate_up, int64_t ld_in,
  *   q_out    [tokens, q_heads, 128]
  *   k_cache  [batch, kv_heads, max_len, 128]   row (seq_of_token[t], h, positions[t]) is written
  *   vt_cache [batch, kv_heads, 128, max_len]   column positions[t] is written
- * positions / seq_of_token: device int64 [tokens].  One wavefront per (token, head): batch invariant.
+ * positions / seq_of_token: device int64 [tokens].  Every head of a token is formed on its own: batch invariant.
  * Replaces: the rotary-embedding patch of the alignment mode and the engine code around it,
  *           src/patch/patch_training_inference_align.py:35-44; model wiring simple_rl.py:320-338 (qk_norm, head_dim 128).
  */

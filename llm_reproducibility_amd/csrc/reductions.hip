@@ -419,7 +419,7 @@ __global__ __launch_bounds__(512) void lsm_resident_kernel(const LsmArgs a) {
 // resident on a CU, one being read or written while the other is being reduced (one row per CU leaves the memory idle for
 // the reduction).  One work-group of 256 threads per row; 28 segments in registers (8 of them per segment and thread, 224
 // of 256), the rest in 78 KiB of LDS.  Bound: memory, 4 bytes per element; bf16 [1000,151936] 191 -> 154 us, [4096,151936]
-// 752 -> 512 (4.9 TB/s, 95 % of a copy), to fp32 933 -> 726.  Up to 256 rows, one per CU, the kernel above is ahead (twice
+// 752 -> 512 (4.9 TB/s), to fp32 933 -> 726.  Up to 256 rows, one per CU, the kernel above is ahead (twice
 // the threads for the reduction: 46 against 51 us at 256 rows, 81 against 63 at 300).  Forming the sums while loads are still
 // arriving (a barrier per four segments) changed nothing.  Every reduction is the one of the two-launch schedule.
 constexpr int kPackedRegSegs = kResidentRegSegs;
