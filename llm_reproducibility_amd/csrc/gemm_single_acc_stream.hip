@@ -319,6 +319,7 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_single_acc_stream_kernel(con
 // its strip in registers, and a matrix of few columns is a chain on few waves (K cannot be cut: one accumulator per element);
 // here the loads need no registers.  X travels with the weights through the ring, so its rows cost no wait of their own: the
 // time hardly grows with the rows (figures at ring_waves).
+// The weights are loaded with the non-temporal hint (dma16_once): gate/up at 32 rows 45.6 -> 40.7 us, lm_head at 8 rows 217 -> 196.
 // A wave multiplies one strip of 16 columns (GATED: of both halves) by all rows; it loads the weight rows that it alone
 // multiplies and its share of the X rows, and one barrier per slice hands the X rows around.
 namespace ring {
@@ -373,8 +374,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_single_acc_ring_kernel(const Str
   auto issue = [&](int s, int slot) __attribute__((always_inline)) {
     const uint32_t base = lds0 + slot * S::STAGE;
 #pragma unroll
-    for (int i = 0; i < NDMA; i++)
-      dma16(base + dst[i], voff[i], (i < XDMA ? xbase : i < XDMA + 4 ? wbase : w2base) + (int64_t)s * ROWB);
+    for (int i = 0; i < XDMA; i++) dma16(base + dst[i], voff[i], xbase + (int64_t)s * ROWB);
+#pragma unroll
+    for (int i = XDMA; i < NDMA; i++) dma16_once(base + dst[i], voff[i], (i < XDMA + 4 ? wbase : w2base) + (int64_t)s * ROWB);
   };
   const int r = lane & 15, g = lane >> 4;
   const uint32_t xfrag = r * ROWB, wfrag = (MB * 16 + wave * TN * 16 + r) * ROWB;

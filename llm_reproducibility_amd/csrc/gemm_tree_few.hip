@@ -17,6 +17,9 @@
 // of N = 64 .. 51200 and K = 256 .. 32768 8 % faster on average, 8 % of them more than 4 % slower: a few rows on tiny
 // matrices (0.4 .. 1 us) and N = 16384 and more on a K cut in two ([32,12288]x[12288,16384] 80 -> 97).
 //
+// The weights are loaded with the non-temporal hint (dma16_once): [16,25600]x[25600,5120] 54.5 -> 48.4 us (5.4 TB/s),
+// [32,12288]x[12288,4096] 24.9 -> 22.7, [8,4096]x[4096,4096] 11.8 -> 10.9; at 64 rows level.
+//
 // The arithmetic per element is that of gemm_tiled.hip: one chain of 16x16x32 MFMAs over ascending k per leaf, one
 // rounding per leaf, left to right over the leaves of a group, adjacent pairs above, every node rounded; the whole tree
 // of a shard lives in registers.  Hence the same bits.
@@ -83,7 +86,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_tree_few_kernel(const WideArgs p
   auto issue = [&](int s, int slot) __attribute__((always_inline)) {
     const uint32_t base = lds0 + slot * S::STAGE_BYTES;
 #pragma unroll
-    for (int i = 0; i < NDMA; i++) dma16(base + dst[i], voff[i], (i < XDMA ? xbase : wbase) + (int64_t)s * (BK * 2));
+    for (int i = 0; i < XDMA; i++) dma16(base + dst[i], voff[i], xbase + (int64_t)s * (BK * 2));
+#pragma unroll
+    for (int i = XDMA; i < NDMA; i++) dma16_once(base + dst[i], voff[i], wbase + (int64_t)s * (BK * 2));
   };
 
   const int frow = lane & 15, fchk = lane >> 4;

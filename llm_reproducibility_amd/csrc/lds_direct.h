@@ -20,6 +20,18 @@ __device__ __forceinline__ void dma16(uint32_t lds_addr, uint32_t voff, const vo
                : "memory", "m0");
 }
 
+// The same load with the non-temporal hint, for bytes that one work-group reads once: the weights of a decode batch.  They
+// leave no line behind in the caches on their way, and the memory delivers 6.15 -> 6.80 TB/s (two billion bytes read by 2048
+// work-groups in pieces of 1 KiB: 355 -> 321 us).  Only where a wave asks for whole lines of 128 bytes: a line fetched in two halves
+// by two instructions is fetched twice (one strip of 16 rows x 64 bytes per instruction: 46 -> 51 us per 201 MB).
+__device__ __forceinline__ void dma16_once(uint32_t lds_addr, uint32_t voff, const void* base) {
+  const void* base_copy;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0 nt"
+               : "=&s"(base_copy)
+               : "s"(lds_addr), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+
 // The same load to lds_base + offset, the offset a compile-time constant: the sum is formed in m0 itself (one scalar
 // instruction instead of an add and a move; the scalar condition code is clobbered).
 __device__ __forceinline__ void dma16_at(uint32_t lds_base, int offset, uint32_t voff, const void* base) {
