@@ -11,7 +11,8 @@
 // (double-buffered, one barrier per window), which keeps the vector-memory queue of every wave for the weights.
 // With a handful of rows all of X is staged up front and the waves never meet again; work-groups shrink to one
 // or two strips when N is small, so that every CU gets some.  Same MFMA chain per element as the tiled and the
-// quad kernels, hence the same bits.  Narrow matrices, lm_head and most gated calls take the ring kernel below.
+// quad kernels, hence the same bits.  Most calls take the ring kernel below; these two keep the short K of wide matrices, a K
+// that is no multiple of 128, a single row or two of a small matrix, and the projections that normalise their input.
 #include <algorithm>
 
 #include "common.h"
@@ -438,25 +439,20 @@ static int ring_launch_nw(const StreamArgs& a, hipStream_t stream) {
 //   mm, up to 8192 columns: one strip per work-group for one block of rows (two work-groups share a CU), two strips for more.
 //     [8,4096]x[4096,4096] 12.5 -> 11.0, [32,4096]x[4096,6144] 17.5 -> 14.6, [32,4096]x[4096,1024] 16.2 -> 13.1,
 //     [8,12288]x[12288,4096] 33.3 -> 27.5; fp16 at 64 rows 33.1 -> 20.4.
-//   mm, up to 10240 columns: three strips, a round of the chip, [32,5120]x[5120,10240] 28.4 -> 26.0 and [8,4096]x[4096,9216] 18.7
-//     -> 18.2, but not for longer K ([8,8192]x[8192,10240] 36.3 -> 38.2).  Wider ones fill the chip with the windowed kernel
-//     just as well ([8,4096]x[4096,12288] 22.6 -> 23.7, x[4096,24576] level) as long as there are one or two blocks of rows
-//     (fp16 at 64 rows: 34.9 -> 26.6 and 57.2 -> 46.2).
-//   mm, more than 65536 columns (lm_head): four strips, [32,4096]x[4096,151936] 238 -> 229, [8,...] 223 -> 215.
-//   gated: 64 rows of 2 x 12288 columns 65.7 -> 43.7, 32 rows 43.9 -> 42.5, [8,5120] of 2 x 25600 115 -> 101, of 2 x 1536 columns
-//     20.9 -> 13.5; one block of rows where the windowed kernel's groups fill their rounds stays there (2 x 8192: 28.8
-//     against 30.8, 2 x 12288: 40.3 against 41.1).
+//   wider mm of up to 32 rows, K from 1024 on: three strips up to 12288 columns ([8,4096]x[4096,12288] 22.6 -> 20.9,
+//     [16,8192]x[8192,10240] 36.4 -> 34.0), four up to 16384, then six or, with K of 4096 and more, three ([16,2048]x[2048,24576] 24.9 ->
+//     21.2 with six and 22.7 with three, [16,4096]x[4096,24576] 42.6 -> 37.4 with three and 39.0 with six, [32,...] 43.8 -> 38.7),
+//     four beyond 24576 ([16,5120]x[5120,51200] 122.5 -> 99, [1,4096]x[4096,151936] 213 -> 192, [8,...] 217 -> 196).  Shorter K is a
+//     prologue: windowed ([16,512]x[512,51200] 13.1 against 13.7 and 15.1).
+//   more rows: fp16 at 64 rows 34.9 -> 26.6 and 57.2 -> 46.2 at 12288 and 24576 columns.
+//   gated: 64 rows of 2 x 12288 columns 65.7 -> 41.0, 32 rows 45.0 -> 39.6, 16 rows 41.3 -> 38.7, [16,5120] of 2 x 12288 48.5 -> 40.1,
+//     [8,5120] of 2 x 25600 115 -> 91, of 2 x 1536 columns 20.9 -> 13.5.
 // The strips of a work-group otherwise follow from the rounds of 256 work-groups, each as long as its weight rows, its
 // X rows at a third of their price (they come from the L2) and a fixed part.
-static int ring_waves(int mb, int64_t strips, int K, bool gated, double windowed_fill) {
+static int ring_waves(int mb, int64_t strips, int K, bool gated) {
   if (K % ring::BK != 0) return 0;
-  if (!gated) {
-    if (strips <= 512) return mb == 1 ? 1 : 2;
-    if (mb <= 2) return strips <= 640 && K <= 5120 ? 3 : strips > 4096 ? 4 : 0;
-    if (strips > 4096) return 0;
-  } else if (mb == 1 && windowed_fill > 0.9) {
-    return 0;
-  }
+  if (!gated && strips <= 512) return mb == 1 ? 1 : 2;
+  if (!gated && mb <= 2) return K < 1024 ? 0 : strips <= 768 ? 3 : strips <= 1024 || strips > 1536 ? 4 : K < 4096 ? 6 : 3;
   static const int cand[5] = {1, 2, 3, 4, 6};
   int best = 0;
   double best_t = 0;
@@ -480,7 +476,7 @@ static int ring_launch(const StreamArgs& a, int waves, hipStream_t stream) {
     case 4: return ring_launch_nw<MB, 4, F16, GATED>(a, stream);
     default: break;
   }
-  if constexpr (!GATED && MB >= 3) {
+  if constexpr (!GATED) {
     if (waves == 6) return ring_launch_nw<MB, 6, F16, GATED>(a, stream);
   }
   return TBIK_ERR_INVALID;
@@ -513,12 +509,7 @@ static int stream_launch(const StreamArgs& a, hipStream_t stream) {
   const int64_t strips = ((int64_t)a.N + 15) / 16;
   const bool near_rows = a.ldx < (1 << 22) && a.ldw < (1 << 22);  // the ring kernel's 32-bit byte offsets
   if (near_rows) {
-    double fill = 0.0;
-    for (int nw : {6, 4, 3, 2}) {
-      const int64_t groups = (strips + nw - 1) / nw;
-      fill = std::max(fill, (double)groups / (double)(((groups + 255) / 256) * 256));
-    }
-    const int waves = ring_waves(MB, strips, a.K, GATED, fill);
+    const int waves = ring_waves(MB, strips, a.K, GATED);
     if (waves) return ring_launch<MB, F16, GATED>(a, waves, stream);
   }
   // grids of many rounds do not run in rounds: the last one matters little there, the restaging of X more
@@ -607,7 +598,8 @@ static bool stream_rows_pays(const StreamArgs& a) {
 #endif
   const int64_t xe = (int64_t)a.M * a.K;
   if (a.K < 512) return true;   // shorter than one window: nothing to stage behind
-  return a.N >= 10240 || xe <= 2048 || (xe <= 4096 && a.N <= 4096) || (xe <= 8192 && a.N <= 3072);
+  if (a.N >= 10240 && a.K % ring::BK != 0) return true;   // (the ring kernel is ahead of both, but does not take it)
+  return xe <= 2048 || (xe <= 4096 && a.N <= 4096) || (xe <= 8192 && a.N <= 3072);
 }
 
 // Requires 0 < M <= 64 and K a multiple of 32 (checked by the dispatcher).
