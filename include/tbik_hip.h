@@ -125,6 +125,23 @@ int tbik_gemm_bf16_static(const void* A, int64_t lda,
                           tbik_stream_t stream);
 
 /*
+ * All `shards` ranks of a row-split layer on one GPU: the product of every rank from its K / shards columns of A and of the
+ * [N,K] weight (K contiguous, row stride ldb_n; f16 != 0: fp16, else bf16), rounded to the element type, and the adjacent-pair tree
+ * over the ranks' products, bias behind it.  The bits of `shards` calls of tbik_gemm_bf16 / _f16 on column slices followed by
+ * tbik_tree_combine_bf16 / _f16 (an aligned rank may be cut further), in one grid and one combine.  shards: a power of two up to
+ * 32, K a multiple of shards * leaf_k; everything else as for tbik_gemm_bf16.
+ * Replaces: the simulated tensor parallelism of the reference, simple_matmul.py:16-43 (one matmul per rank, then the tree).
+ */
+size_t tbik_gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, int f16);
+int tbik_gemm_sharded(const void* A, int64_t lda,
+                      const void* B, int64_t ldb_n,
+                      void* C, int64_t ldc,
+                      int M, int N, int K, int leaf_k, int shards, int f16,
+                      const void* bias_or_null,
+                      void* workspace, size_t workspace_bytes,
+                      tbik_stream_t stream);
+
+/*
  * out[i] = adjacent-pair binary tree over parts[0..nparts-1][i], bf16 adds (round to nearest even
  * at every node); nparts a power of two up to 32; all buffers contiguous, numel elements, 2-byte aligned
  * (16-byte aligned buffers take the vector path).  `out` may alias parts[0].

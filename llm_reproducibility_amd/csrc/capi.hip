@@ -7,6 +7,9 @@ int gemm_dispatch(bool tree, bool f16, const void* A, int64_t lda, const void* B
                   int64_t ldc, int M, int N, int K, int leaf_k, const void* bias, void* ws, size_t ws_bytes,
                   hipStream_t stream);
 size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b = false);
+size_t gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, bool f16);
+int gemm_sharded_dispatch(bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K,
+                          int leaf_k, int shards, const void* bias, void* ws, size_t ws_bytes, hipStream_t stream);
 int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, int out[5]);
 int tree_combine_dispatch(const void* const* parts, int nparts, void* out, int64_t numel, bool f16, hipStream_t stream);
 int tree_combine_f32_dispatch(const void* const* parts, int nparts, void* out, int64_t numel, hipStream_t stream);
@@ -54,7 +57,7 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 extern "C" {
 
-int tbik_abi_version(void) { return 18; }
+int tbik_abi_version(void) { return 19; }
 
 const char* tbik_error_string(int code) {
   switch (code) {
@@ -95,6 +98,16 @@ int tbik_gemm_bf16(const void* A, int64_t lda, const void* B, int64_t ldb_k, int
                    tbik_stream_t stream) {
   return tbik::gemm_dispatch(true, false, A, lda, B, ldb_k, ldb_n, C, ldc, M, N, K, leaf_k, bias_or_null, workspace,
                              workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+size_t tbik_gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, int f16) {
+  return tbik::gemm_sharded_workspace_bytes(M, N, K, leaf_k, shards, f16 != 0);
+}
+
+int tbik_gemm_sharded(const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K, int leaf_k,
+                      int shards, int f16, const void* bias_or_null, void* workspace, size_t workspace_bytes, tbik_stream_t stream) {
+  return tbik::gemm_sharded_dispatch(f16 != 0, A, lda, B, ldb_n, C, ldc, M, N, K, leaf_k, shards, bias_or_null, workspace, workspace_bytes,
+                                     static_cast<hipStream_t>(stream));
 }
 
 int tbik_tree_combine_bf16(const void* const* parts, int nparts, void* out, int64_t numel, tbik_stream_t stream) {

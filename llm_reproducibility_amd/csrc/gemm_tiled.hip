@@ -432,18 +432,22 @@ static bool wide_uses_deep_kernel(int leaf_k, bool f16, int flb, int lb) {
 // the rate of the kernel that shard would run on, plus the shard-combine pass over (split + 1) [M,N] arrays.  Constants
 // measured on MI355X: 5.5 us per round; 16.5 ns per k (15.0 on the kernel for deep trees); 5 TB/s and 4 us for the
 // combine.
-static double wide_cost_us(int M, int N, int K, int leaf_k, bool f16, int flb, int lb, int* best_split) {
-  const int max_split = lb >= 5 ? 32 : (1 << lb);
+//
+// shards (here and in the plans below): the ranks that K is cut into before any of that, 1 unless the caller wants the
+// ranks' products (gemm_dispatch_sharded); flb and lb are then those of a rank's tree, and a split is the ranks times the
+// parts each is cut into.
+static double wide_cost_us(int M, int N, int K, int leaf_k, bool f16, int flb, int lb, int* best_split, int shards = 1) {
+  const int max_split = lb >= 5 || (shards << lb) > 32 ? 32 : (shards << lb);
   const int64_t wide_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
   double best = 0;
-  int split = 1, ls = 0;
-  for (int sp = 1; sp <= max_split; sp *= 2, ls++) {
-    if (sp > 8 && wide_tiles * sp > 256) break;  // finer cuts only while the whole grid still runs as one round
+  int split = shards, ls = 0;
+  for (int sp = shards; sp <= max_split; sp *= 2, ls++) {
+    if (sp > 8 && sp > shards && wide_tiles * sp > 256) break;  // finer cuts only while the whole grid still runs as one round
     const double rounds = (double)((wide_tiles * sp + 255) / 256);
     const double ns_per_k = wide_uses_deep_kernel(leaf_k, f16, flb, lb - ls) ? 0.0150 : 0.0165;
     double t = rounds * (5.5 + ((double)K / sp) * ns_per_k);
     if (sp > 1) t += 4.0 + (double)(sp + 1) * M * N * 2.0 / 5.0e6;
-    if (sp == 1 || t < best) {
+    if (sp == shards || t < best) {
       best = t;
       split = sp;
     }
@@ -487,8 +491,8 @@ static int column_regions(int M, int N, int K, int leaf_k, bool f16) {
 // 42.0 -> 31.6; over 307 such shapes -6 % on average).  No cut whose partial results outgrow the static scratch:
 // tbik_gemm_bf16_static takes every decode batch ([32,8192]x[8192,151936] would be cut into four for the last round's sake,
 // 37 MiB of partials).
-static int few_waves(int M, int N, int K, int lb, int* best_split) {
-  const int max_split = lb >= 3 ? 8 : (1 << lb);
+static int few_waves(int M, int N, int K, int lb, int* best_split, int shards) {
+  const int max_split = std::max(shards, lb >= 3 ? 8 : std::min(8, shards << lb));
   const int rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
   double best = 0;
   int waves = 0;
@@ -505,38 +509,38 @@ static int few_waves(int M, int N, int K, int lb, int* best_split) {
       }
     }
   };
-  for (int sp = 1, ls = 0; sp <= max_split; sp *= 2, ls++) price(sp, ls, 4.0);
+  for (int sp = shards, ls = 0; sp <= max_split; sp *= 2, ls++) price(sp, ls, 4.0);
   if (waves && *best_split == 1 && max_split > 1) price(2, 1, 2.0);
   return waves;
 }
 
-static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool rowmajor_b = false) {
+static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool rowmajor_b = false, int shards = 1) {
   int T, flb, level_k;
-  if (M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
+  if (M <= 0 || N <= 0 || tbik_tree_params(K / shards, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
   const int lb = level_k - 1;
-  const int max_split = lb >= 5 ? 32 : (1 << lb);
+  const int max_split = lb >= 5 || (shards << lb) > 32 ? 32 : (shards << lb);
   const int64_t wide_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
-  int split = 1;
+  int split = shards;
   bool wide = false;
   if (M >= 64 && !rowmajor_b) {  // the wide kernels exist for [N,K] weights only
-    wide_cost_us(M, N, K, leaf_k, f16, flb, lb, &split);
+    wide_cost_us(M, N, K, leaf_k, f16, flb, lb, &split, shards);
     // exactly 64 rows fit one 64-row tile of the tiled kernel, which half-empty 128-row tiles only beat on a grid that
     // fills most of the chip: [64,25600] x [25600,4096] 66 us on 128 work-groups of the wide kernel, 51 on the tiled one;
     // [64,16384] x [16384,8192] 75 on 256 against 97
     wide = wide_tiles * split >= (M == 64 ? 160 : 64);
   }
-  pl->few_waves = !wide && !rowmajor_b && M <= 64 ? few_waves(M, N, K, lb, &split) : 0;
+  pl->few_waves = !wide && !rowmajor_b && M <= 64 ? few_waves(M, N, K, lb, &split, shards) : 0;
   if (!wide && !pl->few_waves) {
     const int bm = M <= 16 ? 16 : ((M <= 64 || rowmajor_b) ? 64 : 128), bn = M <= 16 ? 64 : 128;
     const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    split = 1;
+    split = shards;
     while (tiles * split < 512 && split < max_split && split < 8) split *= 2;
   }
   int ls = 0;
-  while ((1 << ls) < split) ls++;
+  while ((shards << ls) < split) ls++;
   pl->wide = wide;
   pl->split = split;
-  pl->T = T / split;
+  pl->T = T / (split / shards);
   pl->flb = flb;
   pl->lb = lb - ls;
   pl->partial_bytes = split > 1 ? (size_t)split * M * N * sizeof(uint16_t) : 0;
@@ -564,9 +568,9 @@ struct NarrowPlan {
   size_t partial_bytes;
 };
 
-static bool narrow_plan(int M, int N, int K, int leaf_k, bool f16, bool whole_problem, NarrowPlan* np) {
+static bool narrow_plan(int M, int N, int K, int leaf_k, bool f16, bool whole_problem, NarrowPlan* np, int shards = 1) {
   int T, flb, level_k;
-  if (leaf_k != 256 || M < 64 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
+  if (leaf_k != 256 || M < 64 || tbik_tree_params(K / shards, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
   if (!whole_problem && (f16 || M > 512)) return false;
   // exactly 64 rows: the kernels of up to 64 rows cut K at most eightfold, which fills the chip from 32 column tiles on and
   // then beats 128-row tiles that are half empty ([64,8192] x [8192,4096] 25.6 -> 21.1 us, [64,4096] x [4096,4096] 14.7 ->
@@ -576,8 +580,8 @@ static bool narrow_plan(int M, int N, int K, int leaf_k, bool f16, bool whole_pr
   const int64_t tiles = (((int64_t)N + 127) / 128) * (((int64_t)M + 127) / 128);
   int best = 0, best_ls = 0;
   double best_t = 0;
-  for (int ls = 0; ls <= lb && ls <= 5; ls++) {
-    const int sp = 1 << ls;
+  for (int ls = 0; ls <= lb && (shards << ls) <= 32; ls++) {
+    const int sp = shards << ls;
     const int ks = K / sp;
     const int64_t wgs = tiles * sp;
     if (lb - ls > 1 || ks < 512 || ks > 1536 || wgs > 256) continue;
@@ -596,7 +600,7 @@ static bool narrow_plan(int M, int N, int K, int leaf_k, bool f16, bool whole_pr
   }
   if (!best) return false;
   np->split = best;
-  np->T = T / best;
+  np->T = T >> best_ls;
   np->flb = flb;
   np->lb = lb - best_ls;
   np->partial_bytes = best > 1 ? (((size_t)best * M * N * sizeof(uint16_t) + 255) & ~(size_t)255) : 0;
@@ -631,7 +635,7 @@ struct TreePlan {
   size_t bytes;        // workspace of the chosen path
 };
 
-static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, bool whole_problem, TreePlan* tp);
+static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, bool whole_problem, TreePlan* tp, int shards = 1);
 
 static bool plan_regions(int M, int N, int K, int leaf_k, bool f16, RegionPlan* rp) {
   rp->na = column_regions(M, N, K, leaf_k, f16);
@@ -661,29 +665,30 @@ static bool plan_regions(int M, int N, int K, int leaf_k, bool f16, RegionPlan* 
 
 // whole_problem: the call may still be cut into column regions (false for a region itself).  Returns false for shapes
 // no tree exists for (K not a whole number of leaves).
-static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, bool whole_problem, TreePlan* tp) {
+static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, bool whole_problem, TreePlan* tp, int shards) {
   int T, flb, level_k;
   if (M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return false;
   tp->bytes = 0;
   tp->strip_waves = 0;
   if (!rowmajor_b) {
-    tp->strip_waves = gemm_tree_strip_waves(M, N, K, level_k - 1);
+    // (neither of the paths that keep a shard's value on chip or cut each region's K for itself gives the ranks' products)
+    tp->strip_waves = shards > 1 ? 0 : gemm_tree_strip_waves(M, N, K, level_k - 1);
     if (tp->strip_waves) {
       tp->path = PATH_STRIP;
       return true;
     }
-    if (narrow_plan(M, N, K, leaf_k, f16, whole_problem, &tp->narrow)) {
+    if (narrow_plan(M, N, K, leaf_k, f16, whole_problem, &tp->narrow, shards)) {
       tp->path = PATH_NARROW;
       tp->bytes = tp->narrow.partial_bytes;
       return true;
     }
-    if (whole_problem && plan_regions(M, N, K, leaf_k, f16, &tp->regions)) {
+    if (shards == 1 && whole_problem && plan_regions(M, N, K, leaf_k, f16, &tp->regions)) {
       tp->path = PATH_REGIONS;
       tp->bytes = tp->regions.bytes;
       return true;
     }
   }
-  if (!make_plan(M, N, K, leaf_k, f16, &tp->single, rowmajor_b)) return false;
+  if (!make_plan(M, N, K, leaf_k, f16, &tp->single, rowmajor_b, shards)) return false;
   tp->path = PATH_SINGLE;
   tp->bytes = tp->single.partial_bytes + tp->single.parked_bytes;
   return true;
@@ -692,6 +697,15 @@ static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b
 size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b) {
   TreePlan tp;
   return tree_plan(M, N, K, leaf_k, f16, rowmajor_b, true, &tp) ? tp.bytes : 0;
+}
+
+// `shards` ranks of a row-split layer: a power of two, each a whole number of leaves
+static bool ranks_ok(int K, int leaf_k, int shards) {
+  return shards >= 1 && shards <= 32 && (shards & (shards - 1)) == 0 && K > 0 && (leaf_k == 256 || leaf_k == 128) && K % (shards * leaf_k) == 0;
+}
+size_t gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, bool f16) {
+  TreePlan tp;
+  return ranks_ok(K, leaf_k, shards) && tree_plan(M, N, K, leaf_k, f16, false, true, &tp, shards) ? tp.bytes : 0;
 }
 
 // What tree_plan() chose for a shape, for callers and tests that want to know (no effect on any result):
@@ -713,12 +727,23 @@ int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, i
 
 static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n,
                               void* C, int64_t ldc, int M, int N, int K, int leaf_k, const void* bias, void* ws,
-                              size_t ws_bytes, hipStream_t stream, bool whole_problem, const NormEpilogue* ep = nullptr);
+                              size_t ws_bytes, hipStream_t stream, bool whole_problem, const NormEpilogue* ep = nullptr,
+                              int shards = 1);
 
 int gemm_dispatch(bool tree, bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n, void* C,
                   int64_t ldc, int M, int N, int K, int leaf_k, const void* bias, void* ws, size_t ws_bytes,
                   hipStream_t stream) {
   return gemm_dispatch_impl(tree, f16, A, lda, B, ldb_k, ldb_n, C, ldc, M, N, K, leaf_k, bias, ws, ws_bytes, stream, true);
+}
+
+// All ranks of a row-split layer on one GPU: every rank's product from its columns of A and of the [N,K] weight, rounded to
+// the element type, then the shard tree.  What `shards` calls of gemm_dispatch on column slices and a combine compute, but
+// the ranks share one grid: a rank alone leaves most of the chip idle ([232,3200]x[3200,5120], leaves of 128, is 40 tiles on 256
+// CUs; eight of them 505 us in eight launches, 120 in one).  Same bits; norm_w / res as for gemm_tree_rmsnorm_dispatch when `ep`.
+int gemm_sharded_dispatch(bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K,
+                          int leaf_k, int shards, const void* bias, void* ws, size_t ws_bytes, hipStream_t stream) {
+  if (!ranks_ok(K, leaf_k, shards)) return TBIK_ERR_INVALID;
+  return gemm_dispatch_impl(true, f16, A, lda, B, 1, ldb_n, C, ldc, M, N, K, leaf_k, bias, ws, ws_bytes, stream, true, nullptr, shards);
 }
 
 // The tree matmul with the (add-)RMSNorm of its result inside the launch of its shard combine: `out` receives the
@@ -738,7 +763,7 @@ int gemm_tree_rmsnorm_dispatch(bool f16, const void* A, int64_t lda, const void*
 
 static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_k, int64_t ldb_n,
                               void* C, int64_t ldc, int M, int N, int K, int leaf_k, const void* bias, void* ws,
-                              size_t ws_bytes, hipStream_t stream, bool whole_problem, const NormEpilogue* ep) {
+                              size_t ws_bytes, hipStream_t stream, bool whole_problem, const NormEpilogue* ep, int shards) {
   if (M < 0 || N < 0 || K <= 0) return TBIK_ERR_INVALID;
   if (M == 0 || N == 0) return TBIK_OK;  // nothing to do (empty tensors may come with null pointers)
   if (!A || !B || !C) return TBIK_ERR_INVALID;
@@ -809,7 +834,7 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
 
   if (leaf_k != 256 && leaf_k != 128) return TBIK_ERR_UNSUPPORTED;
   TreePlan tp;
-  if (!tree_plan(M, N, K, leaf_k, f16, rowmajor_b, whole_problem, &tp)) return TBIK_ERR_INVALID;
+  if (!tree_plan(M, N, K, leaf_k, f16, rowmajor_b, whole_problem, &tp, shards)) return TBIK_ERR_INVALID;
   if (ep) {
     // the norm rides on the shard combine of ONE K split over all columns: nothing else has a pass over whole rows
     const bool combines = (tp.path == PATH_NARROW && tp.narrow.split > 1) || (tp.path == PATH_SINGLE && tp.single.split > 1);

@@ -234,6 +234,39 @@ def _(A, B, bias, leaf_k):
     return A.new_empty((A.shape[0], B.shape[1]))
 
 
+def _gemm_tree_sharded_impl(A: torch.Tensor, W: torch.Tensor, leaf_k: int, shards: int) -> torch.Tensor:
+    _require_gpu(A, W)
+    M, K = A.shape
+    N = W.shape[0]
+    a, lda = _rows16(A)
+    w, ldw = _rows16(W)
+    f16 = _is_f16(A, W)
+    C = torch.empty((M, N), device=A.device, dtype=A.dtype)
+    L = _lib.lib()
+    ws_bytes = L.tbik_gemm_sharded_workspace_bytes(M, N, K, leaf_k, shards, int(f16))
+    ws = torch.empty(ws_bytes, device=A.device, dtype=torch.uint8) if ws_bytes else None
+    rc = L.tbik_gemm_sharded(a.data_ptr(), lda, w.data_ptr(), ldw, C.data_ptr(), C.stride(0), M, N, K, leaf_k, shards, int(f16), None,
+                             None if ws is None else ws.data_ptr(), ws_bytes, _stream(A))
+    _lib.check(rc, "tbik_gemm_sharded")
+    return C
+
+
+_gemm_tree_sharded_op = torch.library.custom_op("tbik::gemm_tree_sharded", _gemm_tree_sharded_impl, mutates_args=(), device_types="cuda")
+
+
+def gemm_tree_sharded(A: torch.Tensor, W: torch.Tensor, leaf_k: int, shards: int) -> torch.Tensor:
+    """The products of all `shards` ranks of a row-split layer (weight W [N,K], 16 bits) and the shard tree over them: one grid
+    and one combine, the bits of a `gemm_tree` per rank and `tree_combine`.  shards: a power of two up to 32."""
+    if torch.compiler.is_compiling():
+        return _gemm_tree_sharded_op(A, W, leaf_k, shards)
+    return _gemm_tree_sharded_impl(A, W, leaf_k, shards)
+
+
+@_gemm_tree_sharded_op.register_fake
+def _(A, W, leaf_k, shards):
+    return A.new_empty((A.shape[0], W.shape[0]))
+
+
 def _tree_combine_impl(parts: List[torch.Tensor]) -> torch.Tensor:
     _require_gpu(*parts)
     ps = [p.contiguous() for p in parts]
