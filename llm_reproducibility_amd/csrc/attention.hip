@@ -254,7 +254,7 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
 // ------------------------------------------------------------------------------------------------
 // chunks: the cache has a single one / a work-group walks them all / a work-group takes one (SPLIT)
 enum { ONE_CHUNK, ALL_CHUNKS, SPLIT_CHUNKS };
-template <int G, int QB, bool DEEP, int NLD, int CHUNKS>
+template <int G, int QB, bool DEEP, int NLD, int CHUNKS, int AHEAD>
 __global__ __launch_bounds__(64 * (G * QB + NLD)) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
   constexpr bool SPLIT = CHUNKS == SPLIT_CHUNKS;
   constexpr int NW = G * QB;   // computing wavefronts
@@ -298,7 +298,9 @@ __global__ __launch_bounds__(64 * (G * QB + NLD)) void attention_group_kernel(co
   // single block of queries per sequence makes the kernel a chain of memory round trips, and one tile of arithmetic
   // hides none of them.  Prefill has arithmetic to overlap and prefers the registers (more waves per SIMD), and so does
   // decode where they decide about the second work-group of a CU (8 heads, 128 sequences of 1000 keys 151 -> 116 us).
-  constexpr int DEPTH = !DEEP ? 1 : PARK ? 2 : (NCH <= 2 ? 4 : (NCH <= 4 ? 2 : 1));
+  // Loader waves without DEEP fetch AHEAD tiles ahead: with one, a tile is stored in the iteration that asked for it and the
+  // barrier waits for the memory (0.8 us per tile where several sequences share an L2 and read their own keys).
+  constexpr int DEPTH = !DEEP ? AHEAD : PARK ? 2 : (NCH <= 2 ? 4 : (NCH <= 4 ? 2 : 1));
   u32x4 kregs[DEPTH][NCH], vregs[DEPTH][NCH];
   // A K tile is 8 KiB of consecutive bytes (32 rows of 256), chunk ch at byte 16 ch; a V^T tile is 128 rows of 64 bytes,
   // max_len elements apart.  Per-thread byte offsets inside a tile (global and LDS side) are formed once; per tile only
@@ -937,11 +939,11 @@ static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max
   return hip_code(hipGetLastError());
 }
 
-template <int G, int QB, bool DEEP, int NLD, int CHUNKS>
+template <int G, int QB, bool DEEP, int NLD, int CHUNKS, int AHEAD = NLD ? 2 : 1>
 static void group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_q_len, hipStream_t stream) {
   const int64_t blocks = ((int64_t)max_q_len + 16 * QB - 1) / (16 * QB);
   const dim3 grid((unsigned)(blocks * a.kv_heads), (unsigned)batch, CHUNKS == SPLIT_CHUNKS ? (unsigned)sp.nchunks : 1u);
-  hipLaunchKernelGGL((attention_group_kernel<G, QB, DEEP, NLD, CHUNKS>), grid, dim3(64 * (G * QB + NLD)), 0, stream, a, sp);
+  hipLaunchKernelGGL((attention_group_kernel<G, QB, DEEP, NLD, CHUNKS, AHEAD>), grid, dim3(64 * (G * QB + NLD)), 0, stream, a, sp);
 }
 
 // The form of the grouped kernel, same bits in all.  Lengths are the device's, so what is known is the number of
@@ -962,6 +964,9 @@ static void group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max
 //     cached already); at 1024 blocks 2 prompts of 1020 35.6 / 35.3 / 40.2 but 8 chunks of 250 at 800 keys 39 / 45.5 / 37.7;
 //   8 heads: prompt of 4096 298 / 420 / 310, 16 of 400 87 / 111 / 87;   2 heads: 125 / 130 / 102, 1040 tokens 22.6 / 26.3 / 20.8;
 //   1 head: 217 / 225 / 126, 1040 tokens 27.0 / 28.2 / 20.8.
+// Up to 512 work-groups the loader waves fetch two tiles ahead: 4 sequences of 128 tokens at 8000 keys 194 -> 142 us, 2 of 196 at 4251
+// 105 -> 76, 2 heads 16 of 20 at 8000 207 -> 143, 1 head 4 of 64 at 1500 40 -> 27; one sequence alone, whose keys wait in the L2, 34.2 ->
+// 32.1 (405 tokens at 1633).  Beyond that the registers cost one or two heads work-groups of a CU (1 head 2 of 600 at 1870 58 -> 66).
 // What is left of the cost of the chunks is their merge, where a launch is a chain (520 tokens 12.6 -> 13.7) or its rounds
 // are few.
 template <int G>
@@ -982,7 +987,8 @@ static void group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int
     else TBIK_ATTN_GROUP(1, true, 0, ALL_CHUNKS);
   } else {
     constexpr int LOADERS = G == 1 ? 1280 : G == 2 ? 1024 : 512, SINGLE = G == 4 ? 768 : 0, QB = G == 8 ? 1 : 2;
-    if (groups <= LOADERS) TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS);
+    if (groups <= 512) TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS);
+    else if (groups <= LOADERS) TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS, 1);
     else if (groups <= SINGLE) TBIK_ATTN_GROUP(1, false, 0, ALL_CHUNKS);
     else TBIK_ATTN_GROUP(QB, false, 0, ALL_CHUNKS);
   }
