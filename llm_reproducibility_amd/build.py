@@ -1,5 +1,6 @@
-"""Builds libtbik_hip.so (the gfx950 kernels + their C ABI) in-tree with hipcc, and beside it measure/libtbik_measure.so
-(the benchmark's machine probes, which are not part of the product library).
+"""Builds libtbik_hip.so (the gfx950 kernels + their C ABI) in-tree with hipcc, beside it _fast.so (a Python extension with the
+common calls of the row-wise operators, host code only) and measure/libtbik_measure.so (the benchmark's machine probes,
+which are not part of the product library).
 
     python -m llm_reproducibility_amd.build            # compile every source, link
     python -m llm_reproducibility_amd.build --if-stale # only when a source is newer than the library
@@ -19,6 +20,8 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libtbik_hip.so")
+FAST_SRC = os.path.join(PKG_DIR, "csrc_host", "fast_ops.cpp")
+FAST_PATH = os.path.join(PKG_DIR, "_fast.so")
 MEASURE_DIR = os.path.join(PKG_DIR, "measure")
 MEASURE_LIB_PATH = os.path.join(MEASURE_DIR, "libtbik_measure.so")
 OBJ_DIR = os.path.join(PKG_DIR, "build")
@@ -54,14 +57,15 @@ def measure_sources():
 
 def _deps():
     deps = sources() + measure_sources() + [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".h")]
-    deps += [os.path.join(INCLUDE, "tbik_hip.h"), os.path.join(INCLUDE, "tbik_measure.h")]
+    deps += [os.path.join(INCLUDE, "tbik_hip.h"), os.path.join(INCLUDE, "tbik_measure.h"), FAST_SRC]
     return deps
 
 
 def is_stale() -> bool:
-    if not os.path.exists(LIB_PATH) or not os.path.exists(MEASURE_LIB_PATH):
+    built = (LIB_PATH, MEASURE_LIB_PATH, FAST_PATH)
+    if not all(os.path.exists(p) for p in built):
         return True
-    t = min(os.path.getmtime(LIB_PATH), os.path.getmtime(MEASURE_LIB_PATH))
+    t = min(os.path.getmtime(p) for p in built)
     return any(os.path.getmtime(d) > t for d in _deps())
 
 
@@ -90,13 +94,45 @@ def _link(objs, path: str) -> None:
     os.replace(tmp, path)
 
 
+def _compile_fast() -> str:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(OBJ_DIR, "fast_ops.o")
+    includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[a for p in includes for a in ("-isystem", p)],
+           "-c", FAST_SRC, "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on {FAST_SRC}:\n{r.stdout}\n{r.stderr}")
+    return obj
+
+
+def _link_fast(obj: str) -> None:
+    import torch
+
+    tmp = FAST_PATH + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, "-L", os.path.join(os.path.dirname(torch.__file__), "lib"), "-ltorch_cpu", "-ltorch_python",
+           "-lc10", "-lc10_hip", "-L", PKG_DIR, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, FAST_PATH)
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs, msrcs = sources(), measure_sources()
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + len(msrcs))) as ex:
+        fast = ex.submit(_compile_fast)
         objs = list(ex.map(_compile, srcs + msrcs))
+        fast_obj = fast.result()
     _link(objs[:len(srcs)], LIB_PATH)
     _link(objs[len(srcs):], MEASURE_LIB_PATH)
+    _link_fast(fast_obj)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources and {MEASURE_LIB_PATH} from {len(msrcs)}")
     return LIB_PATH

@@ -32,6 +32,24 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+_fast_module = None
+
+
+def _fast():
+    """The extension with the common calls of the row-wise operators (csrc_host/fast_ops.cpp): each gives the result, or None
+    for a call that is not the plain case, which then goes the way written out here."""
+    global _fast_module
+    if _fast_module is None:
+        _lib.lib()   # a missing library is reported as such
+        try:
+            from . import _fast as module
+        except ImportError as e:
+            raise RuntimeError("llm_reproducibility_amd/_fast.so is missing or does not load: run "
+                               "`python -m llm_reproducibility_amd.build`") from e
+        _fast_module = module
+    return _fast_module
+
+
 def _require_gpu(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if t is not None and not t.is_cuda:
@@ -362,7 +380,8 @@ _bi_rmsnorm_op = torch.library.custom_op("tbik::bi_rmsnorm", _bi_rmsnorm_impl, m
 def bi_rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float) -> torch.Tensor:
     if torch.compiler.is_compiling():
         return _bi_rmsnorm_op(x, weight, eps)
-    return _bi_rmsnorm_impl(x, weight, eps)
+    out = (_fast_module or _fast()).rms_norm(x, weight, eps)
+    return _bi_rmsnorm_impl(x, weight, eps) if out is None else out
 
 
 @_bi_rmsnorm_op.register_fake
@@ -395,7 +414,8 @@ def bi_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: Optional[tor
                         eps: float) -> List[torch.Tensor]:
     if torch.compiler.is_compiling():
         return _bi_add_rmsnorm_op(x, residual, weight, eps)
-    return _bi_add_rmsnorm_impl(x, residual, weight, eps)
+    out = (_fast_module or _fast()).add_rms_norm(x, residual, weight, eps)
+    return _bi_add_rmsnorm_impl(x, residual, weight, eps) if out is None else out
 
 
 @_bi_add_rmsnorm_op.register_fake
@@ -432,7 +452,8 @@ _bi_log_softmax_op = torch.library.custom_op("tbik::bi_log_softmax", _bi_log_sof
 def bi_log_softmax(x: torch.Tensor, write_softmax: bool, to_float: bool = False) -> torch.Tensor:
     if torch.compiler.is_compiling():
         return _bi_log_softmax_op(x, write_softmax, to_float)
-    return _bi_log_softmax_impl(x, write_softmax, to_float)
+    out = (_fast_module or _fast()).log_softmax(x, write_softmax, to_float)
+    return _bi_log_softmax_impl(x, write_softmax, to_float) if out is None else out
 
 
 @_bi_log_softmax_op.register_fake
@@ -472,7 +493,8 @@ _bi_mean_dim_op = torch.library.custom_op("tbik::bi_mean_dim", _bi_mean_dim_impl
 def bi_mean_dim(x: torch.Tensor, dim: int, keepdim: bool) -> torch.Tensor:
     if torch.compiler.is_compiling():
         return _bi_mean_dim_op(x, dim, keepdim)
-    return _bi_mean_dim_impl(x, dim, keepdim)
+    out = (_fast_module or _fast()).mean_last(x, keepdim) if dim == -1 or dim == x.ndim - 1 else None
+    return _bi_mean_dim_impl(x, dim, keepdim) if out is None else out
 
 
 @_bi_mean_dim_op.register_fake
@@ -560,7 +582,8 @@ def bi_silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """act = silu(gate_up[..., :I]) * gate_up[..., I:] (I = half the last dimension), fused, bf16."""
     if torch.compiler.is_compiling():
         return _bi_silu_mul_op(gate_up)
-    return _bi_silu_mul_impl(gate_up)
+    out = (_fast_module or _fast()).silu_mul(gate_up)
+    return _bi_silu_mul_impl(gate_up) if out is None else out
 
 
 @_bi_silu_mul_op.register_fake
