@@ -168,6 +168,21 @@ int bi_gemm_bf16(const void* A, int64_t lda,
                  tbik_stream_t stream);
 
 /*
+ * bi_gemm_bf16 with operands that lie K-major, read in place: B is [K,N] (row stride ldb), A is [M,K] or, with a_kmajor, [K,M]
+ * (row stride lda; the weight gradient grad_out^T x of a linear layer takes both this way).  The same MFMA chain per element, hence
+ * the bits of bi_gemm_bf16 on transposed copies.  16-byte aligned operands, strides multiples of 8.
+ * TBIK_ERR_UNSUPPORTED (3), nothing launched: N (with a_kmajor also M) is no multiple of 8, K is no multiple of 64 (without a_kmajor), or
+ * copies and the kernels for K-contiguous operands are faster.
+ * Replaces: as bi_gemm_bf16 (the backward products of the reference's aten::mm override).
+ */
+int bi_gemm_kmajor_bf16(const void* A, int64_t lda, int a_kmajor,
+                        const void* B, int64_t ldb,
+                        void* C, int64_t ldc,
+                        int M, int N, int K,
+                        const void* bias_or_null,
+                        tbik_stream_t stream);
+
+/*
  * RMSNorm over the last dimension, bf16 in/out, fp32 arithmetic, one wavefront per row in a fixed
  * lane->element order (row i's result does not depend on `rows`):
  *   x32 = x (+ residual);  residual_out = bf16(x32)          (only when residual != NULL)

@@ -59,6 +59,8 @@ struct QuadArgs {
   const uint16_t* W2 = nullptr;  // gated form of gemm_single_acc_256.hip only: the up half [N,K], row stride ldw (no bias)
 };
 int gemm_single_acc_quad_launch(const QuadArgs& a, hipStream_t stream);
+// the right operand [K,N], the left one [K,M] too with x_kmajor (ldw / ldx their row strides), read in place
+int gemm_single_acc_kmajor_launch(const QuadArgs& a, bool x_kmajor, hipStream_t stream);
 int gemm_single_acc_slab_launch(const QuadArgs& a, hipStream_t stream);  // at most 128 rows; TBIK_ERR_UNSUPPORTED: use another kernel
 int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream);  // any row count: tile width from a cost model
 // C[M,N] = silu(X W^T) * (X W2^T), both products rounded to bf16 first, where the product of 2 N columns runs on the tiles

@@ -14,6 +14,7 @@
 //     ahead of the MFMAs, also across the barrier; scheduling fences keep that order in the generated code.
 #include "common.h"
 #include "gemm_args.h"
+#include "kmajor.h"
 #include "lds_direct.h"
 
 namespace tbik {
@@ -39,7 +40,10 @@ struct Shape {
 // p.row_step < 128: a tile owns only its first row_step rows (it still stages and multiplies 128, the rest clamped to its
 // last row and never stored).  For a grid that would leave most CUs without a tile: a work-group's time is its chain of
 // slices whatever the rows in its tile, so the same rows spread over two to eight times the work-groups finish sooner.
-template <int TN, int NSLOT>
+// XT, WT: that operand lies K-major ([K,M], [K,N]; p.ldx / p.ldw its row stride) and is read in place (kmajor.h); M / N is then a
+// multiple of 8.  With both K-major (a weight gradient, whose K is the number of tokens) K may be any number: the rows of
+// the last slice behind it are zeroed in LDS by the wave that loaded them.
+template <int TN, int NSLOT, bool XT = false, bool WT = false>
 __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const QuadArgs p) {
   using namespace quad;
   static_assert(NSLOT >= 3, "the schedule needs a slice in use, one landing and one in flight");
@@ -67,35 +71,68 @@ __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const Qu
   const int m0 = pid_m * row_step, n0 = pid_n * BN;
   const int m_end = min(p.M, m0 + row_step);
 
-  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(p.X + (int64_t)m0 * p.ldx);
-  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.W + (int64_t)n0 * p.ldw);
+  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(p.X + (XT ? (int64_t)m0 : (int64_t)m0 * p.ldx));
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.W + (WT ? (int64_t)n0 : (int64_t)n0 * p.ldw));
+  const int64_t xstep = XT ? p.ldx * (BK * 2) : BK * 2, wstep = WT ? p.ldw * (BK * 2) : BK * 2;   // bytes from slice to slice
+  const int nstages = (p.K + BK - 1) / BK;
+  // rows of the last slice that there are (both K-major); its other rows are loaded from the last one and zeroed
+  const int tail = p.K - (nstages - 1) * BK;
   uint32_t voff[NDMA];
   {
     const int r = lane >> 3, c = (lane & 7) ^ r;
 #pragma unroll
     for (int i = 0; i < NDMA; i++) {
       const int row = (i * NWAVE + wave) * 8 + r;  // 0..383: X rows, then W rows; rows past the edge are clamped
-      if (i < XDMA) voff[i] = (uint32_t)(((min(m0 + row, m_end - 1) - m0) * p.ldx + c * 8) * 2);
+      if (XT && i < XDMA) voff[i] = kmajor::load_offset<BM>(i * NWAVE + wave, lane, p.ldx, p.M - m0);
+      else if (WT && i >= XDMA) voff[i] = kmajor::load_offset<WT ? BN : BM>((i - XDMA) * NWAVE + wave, lane, p.ldw, p.N - n0);
+      else if (i < XDMA) voff[i] = (uint32_t)(((min(m0 + row, m_end - 1) - m0) * p.ldx + c * 8) * 2);
       else voff[i] = (uint32_t)(((min(n0 + row - BM, p.N - 1) - n0) * p.ldw + c * 8) * 2);
     }
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
-  const int nstages = p.K / BK;
   auto dma_one = [&](int s, int slot, int i) __attribute__((always_inline)) {
-    const uint8_t* b = (i < XDMA ? xbase : wbase) + (int64_t)min(s, nstages - 1) * (BK * 2);
-    dma16(lds0 + slot * STAGE_BYTES + (i * NWAVE + wave) * 1024, voff[i], b);
+    const int sl = min(s, nstages - 1);
+    const uint8_t* b = (i < XDMA ? xbase : wbase) + sl * (i < XDMA ? xstep : wstep);
+    uint32_t off = voff[i];
+    if (XT && WT && sl == nstages - 1) {   // (uniform) rows behind K: the last one there is
+      const int k = i < XDMA ? kmajor::load_row<BM>(i * NWAVE + wave, lane) : kmajor::load_row<WT ? BN : BM>((i - XDMA) * NWAVE + wave, lane);
+      off -= (uint32_t)(max(k - (tail - 1), 0) * (i < XDMA ? p.ldx : p.ldw) * 2);
+    }
+    dma16(lds0 + slot * STAGE_BYTES + (i * NWAVE + wave) * 1024, off, b);
+  };
+  // this wave's rows of the last slice that lie behind K, once they have landed (0 x 0: whatever the rows loaded in their
+  // place hold)
+  auto zero_tail = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NDMA; i++) {
+      const int k = i < XDMA ? kmajor::load_row<BM>(i * NWAVE + wave, lane) : kmajor::load_row<WT ? BN : BM>((i - XDMA) * NWAVE + wave, lane);
+      if (k >= tail) *reinterpret_cast<u32x4*>(smem + slot * STAGE_BYTES + (i * NWAVE + wave) * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
   const int frow = lane & 15, fchk = lane >> 4;
   const uint32_t xfrag = ((wm * TM * 16 + frow) * BK + ((fchk ^ (frow & 7)) << 3)) * 2;
   const uint32_t wfrag = (BM * BK + (wn * TN * 16 + frow) * BK + ((fchk ^ (frow & 7)) << 3)) * 2;
 
+  uint32_t xt[XT ? TM : 1], wt[WT ? TN : 1];
+  if (XT) {
+#pragma unroll
+    for (int a = 0; a < TM; a++) xt[a] = kmajor::frag_offset<BM>(wm * TM + a, lane);
+  }
+  if (WT) {
+#pragma unroll
+    for (int b = 0; b < TN; b++) wt[b] = BM * BK * 2 + kmajor::frag_offset<WT ? BN : BM>(wn * TN + b, lane);
+  }
+
   f32x4 acc[TM][TN];
   bf16x8 fx[2][TM], fw[2][TN];
   auto read_x = [&](int buf, int slot, int kk, int a) __attribute__((always_inline)) {
-    fx[buf][a] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (xfrag ^ (kk * 64)) + a * 16 * BK * 2);
+    if (XT) fx[buf][a] = kmajor::read<BM>(smem + slot * STAGE_BYTES, xt[a], kk);
+    else fx[buf][a] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (xfrag ^ (kk * 64)) + a * 16 * BK * 2);
   };
   auto read_w = [&](int buf, int slot, int kk, int b) __attribute__((always_inline)) {
-    fw[buf][b] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (wfrag ^ (kk * 64)) + b * 16 * BK * 2);
+    if (WT) fw[buf][b] = kmajor::read<WT ? BN : BM>(smem + slot * STAGE_BYTES, wt[b], kk);
+    else fw[buf][b] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (wfrag ^ (kk * 64)) + b * 16 * BK * 2);
   };
 
   // prologue: three slices in flight, slice 0 visible, fragments of the first k step loaded
@@ -104,6 +141,7 @@ __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const Qu
 #pragma unroll
     for (int i = 0; i < NDMA; i++) dma_one(s, s, i);
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NSLOT - 1) * NDMA) : "memory");
+  if (XT && WT && nstages == 1 && tail < BK) zero_tail(0);
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
@@ -157,6 +195,7 @@ __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const Qu
       if (kk == 0) {
         // mid-slice: slice s+1 has landed (this wave's share) and every fragment read of slice s is done
         asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NSLOT - 2) * NDMA) : "memory");
+        if (XT && WT && s + 2 == nstages && tail < BK) zero_tail(nslot);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -274,37 +313,42 @@ int gemm_single_acc_slab_launch(const QuadArgs& a, hipStream_t stream) {
 struct BalancedTile {
   int rows256, cols256;  // tile of gemm_single_acc_256.hip; 0: the quad kernel on `tn` times 32 columns
   int tn;
+  double us;
 };
+struct QuadTime {
+  double us, sustained;  // the second without the overlap of later rounds (see below)
+};
+static QuadTime quad_time(int tn, int64_t tiles, double nsl) {
+  const double s0 = 0.185 + 0.0665 * tn;
+  if (tn <= 2) {  // up to two work-groups per CU
+    if (tiles <= 256) {
+      const double t = 3.0 + nsl * s0 * (1.0 + 0.16 * (double)tiles / 256.0);
+      return {t, t};
+    }
+    const double rounds = (double)((tiles + 511) / 512), round = 3.0 + nsl * s0 * 1.7;
+    return {round * (1.0 + 0.9 * (rounds - 1.0)), round * rounds};
+  }
+  QuadTime q{0.0, 0.0};
+  for (int r = 0; tiles > 0; r++, tiles -= 256) {
+    const double fill = (double)(tiles < 256 ? tiles : 256) / 256.0;
+    const double round = 3.0 + nsl * s0 * (1.0 + 0.16 * fill);
+    q.us += (r == 0 ? 1.0 : 0.9) * round;
+    q.sustained += round;
+  }
+  return q;
+}
 static BalancedTile balanced_tile(const QuadArgs& a) {
   const double nsl = (double)(a.K / quad::BK);
   const int64_t tm = ((int64_t)a.M + quad::BM - 1) / quad::BM;
   const double floor_us = (double)a.N * a.K * 2.0 / 3.5e6;
   static const int widths[6] = {8, 6, 4, 3, 2, 1};
   int best = 8;
-  double best_t = 0.0, best_sustained = 0.0;  // the second without the overlap of later rounds (see below)
+  double best_t = 0.0, best_sustained = 0.0;
   for (int i = 0; i < 6; i++) {
     const int tn = widths[i];
     const int64_t tiles = tm * (((int64_t)a.N + 32 * tn - 1) / (32 * tn));
-    const double s0 = 0.185 + 0.0665 * tn;
-    double t, ts;
-    if (tn <= 2) {  // up to two work-groups per CU
-      if (tiles <= 256) {
-        t = ts = 3.0 + nsl * s0 * (1.0 + 0.16 * (double)tiles / 256.0);
-      } else {
-        const double rounds = (double)((tiles + 511) / 512);
-        t = (3.0 + nsl * s0 * 1.7) * (1.0 + 0.9 * (rounds - 1.0));
-        ts = (3.0 + nsl * s0 * 1.7) * rounds;
-      }
-    } else {
-      t = ts = 0.0;
-      int64_t left = tiles;
-      for (int r = 0; left > 0; r++, left -= 256) {
-        const double fill = (double)(left < 256 ? left : 256) / 256.0;
-        const double round = 3.0 + nsl * s0 * (1.0 + 0.16 * fill);
-        t += (r == 0 ? 1.0 : 0.9) * round;
-        ts += round;
-      }
-    }
+    const QuadTime qt = quad_time(tn, tiles, nsl);
+    double t = qt.us, ts = qt.sustained;
     if (t < floor_us) t = floor_us + 1e-3 * t;  // memory-bound either way: keep the order of the compute estimates
     if (ts < floor_us) ts = floor_us + 1e-3 * ts;
     if (i == 0 || t < best_t) {
@@ -343,9 +387,9 @@ static BalancedTile balanced_tile(const QuadArgs& a) {
       }
     }
     const double t128 = rounds8 >= 6.0 ? rounds8 * (3.0 + nsl * 0.83) : best_sustained;
-    if (tiles8 > 256 && t_sq < t128) return {shape[pick][0], shape[pick][1], best};
+    if (tiles8 > 256 && t_sq < t128) return {shape[pick][0], shape[pick][1], best, t_sq};
   }
-  return {0, 0, best};
+  return {0, 0, best, best_t};
 }
 
 int gemm_single_acc_gated_launch(const QuadArgs& a, hipStream_t stream) {
@@ -384,6 +428,89 @@ int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream) {
     case 2: return deep ? quad_launch<2, 6>(a, stream) : quad_launch<2>(a, stream);
     default: return deep ? quad_launch<1, 6>(a, stream) : quad_launch<1>(a, stream);
   }
+}
+
+template <int TN, int NSLOT, bool XT>
+static int quad_kmajor_launch(const QuadArgs& a, hipStream_t stream) {
+  using namespace quad;
+  constexpr size_t smem = (size_t)NSLOT * Shape<TN>::STAGE_BYTES;
+  static_assert(smem <= 160 * 1024 && (NSLOT - 1) * Shape<TN>::NDMA < 64, "ring does not fit the LDS or the wait counter");
+  const int64_t tiles = (int64_t)((a.M + BM - 1) / BM) * ((a.N + Shape<TN>::BN - 1) / Shape<TN>::BN);
+  if (tiles <= 0 || tiles > 0x7fffffff) return TBIK_ERR_UNSUPPORTED;
+  static std::atomic<uint64_t> done{0};
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_single_acc_quad_kernel<TN, NSLOT, XT, true>), (int)smem, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL((gemm_single_acc_quad_kernel<TN, NSLOT, XT, true>), dim3((unsigned)tiles), dim3(NT), smem, stream, a);
+  return hip_code(hipGetLastError());
+}
+
+// Whether `in_place` us (of quad_time) beat a transposing copy per K-major operand (3 us and two passes at 4.1 TB/s) and the
+// kernel for K-contiguous ones.  quad_time misses the reads that transpose (10 % on one operand, 25 % on both); the kernels of
+// many rows run 10 % under the sum of balanced_tile's rounds.  A long K over few columns is a few long chains on an idle chip
+// (and a small copy: [1,25600]x[25600,1024] 71 us with it, 97 in place; [128,12288]x[12288,512] 47 and 53), elsewhere the
+// copy outlasts the product up to 128 rows.  Measured on MI355X over K = 2048 .. 25600, N = 1024 .. 51200, us with copies -> in place:
+//   one operand: [1,4096]x[4096,24576] 108 -> 37, [64,12288]x[12288,4096] 93 -> 71, [200,25600]x[25600,5120] 272 -> 181,
+//     [1024,4096]x[4096,4096] 52 -> 33, [2048,6144]x[6144,4096] 110 -> 92, [2048,12288]x[12288,4096] 196 -> 163; more rounds
+//     of 128x256 tiles lose to the tiles of gemm_single_acc_256.hip: [2048,4096]x[4096,24576] 343 against 368, [4096,25600]x
+//     [25600,5120] 900 against 988.
+//   both (M, K = tokens, N): 1024, 1000, 4096 24 -> 14; 2048, 2048, 2048 32 -> 23; 6144, 500, 4096 49 -> 43; but 6144, 2048, 4096
+//     98 against 104 and 24576, 2048, 4096 340 against 420.
+static bool kmajor_pays(const QuadArgs& a, bool x_kmajor, double in_place) {
+  if (a.K > 4096 && a.K > 8 * (int64_t)a.N) return false;
+  const double kn = (double)a.K * a.N, km = (double)a.K * a.M;
+  double copied = 3.0 + kn * 4.0 / 4.1e6;
+  if (x_kmajor) copied += 3.0 + km * 4.0 / 4.1e6;
+  QuadArgs native = a;
+  native.K = (a.K + quad::BK - 1) / quad::BK * quad::BK;
+  copied += a.M <= 128 && !x_kmajor ? 3.0 + kn / 3.5e6 : 0.9 * balanced_tile(native).us;
+  const double read = kn * 2.0 / 4.5e6;
+  return (in_place < read ? read : in_place) * (x_kmajor ? 1.25 : 1.10) < copied;
+}
+
+// Operands that lie K-major in place (the right one as [K,N], a.ldw its row stride; with x_kmajor the left one too, as [K,M], a.ldx its
+// row stride) on 128-row tiles of 256, 128, 64 or 32 columns.  TBIK_ERR_UNSUPPORTED (nothing launched) where the columns
+// are no whole chunks of 16 bytes, rows lie too far apart, K is no whole number of slices and only one operand is K-major,
+// or where the estimate says that transposing copies and the kernels for K-contiguous operands are faster.
+int gemm_single_acc_kmajor_launch(const QuadArgs& a, bool x_kmajor, hipStream_t stream) {
+  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || (a.N & 7) || (x_kmajor && (a.M & 7)) || (!x_kmajor && a.K % quad::BK != 0)) return TBIK_ERR_UNSUPPORTED;
+  if (a.ldx >= (1 << 22) || a.ldw >= (1 << 22)) return TBIK_ERR_UNSUPPORTED;  // 32-bit in-tile byte offsets
+  const double nsl = (double)((a.K + quad::BK - 1) / quad::BK);
+  const int64_t tm = ((int64_t)a.M + quad::BM - 1) / quad::BM;
+  static const int widths[4] = {8, 4, 2, 1};
+  int tn = 8;
+  double in_place = 0.0;
+  for (int i = 0; i < 4; i++) {
+    const double t = quad_time(widths[i], tm * (((int64_t)a.N + 32 * widths[i] - 1) / (32 * widths[i])), nsl).sustained;
+    if (i == 0 || t < in_place) {
+      in_place = t;
+      tn = widths[i];
+    }
+  }
+  if (!kmajor_pays(a, x_kmajor, in_place)) return TBIK_ERR_UNSUPPORTED;
+  switch (tn) {
+    case 8: return x_kmajor ? quad_kmajor_launch<8, 3, true>(a, stream) : quad_kmajor_launch<8, 3, false>(a, stream);
+    case 4: return x_kmajor ? quad_kmajor_launch<4, 5, true>(a, stream) : quad_kmajor_launch<4, 5, false>(a, stream);
+    case 2:
+      if (x_kmajor) return quad_kmajor_launch<2, 3, true>(a, stream);
+      return tm * (((int64_t)a.N + 63) / 64) <= 256 ? quad_kmajor_launch<2, 6, false>(a, stream) : quad_kmajor_launch<2, 3, false>(a, stream);
+    default:
+      if (x_kmajor) return quad_kmajor_launch<1, 3, true>(a, stream);
+      return tm * (((int64_t)a.N + 31) / 32) <= 256 ? quad_kmajor_launch<1, 6, false>(a, stream) : quad_kmajor_launch<1, 3, false>(a, stream);
+  }
+}
+
+int gemm_kmajor_dispatch(const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M, int N,
+                         int K, const void* bias, hipStream_t stream) {
+  if (M < 0 || N < 0 || K <= 0) return TBIK_ERR_INVALID;
+  if (M == 0 || N == 0) return TBIK_OK;
+  if (!A || !B || !C) return TBIK_ERR_INVALID;
+  if (lda < (a_kmajor ? M : K) || ldb < N || ldc < N) return TBIK_ERR_INVALID;
+  auto aligned16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+  if (!aligned16(A) || !aligned16(B) || (lda & 7) || (ldb & 7) || (reinterpret_cast<uintptr_t>(C) & 1)) return TBIK_ERR_ALIGNMENT;
+  const QuadArgs a{static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(B), static_cast<uint16_t*>(C),
+                   static_cast<const uint16_t*>(bias), lda, ldb, ldc, M, N, K,
+                   ((reinterpret_cast<uintptr_t>(C) & 7) == 0 && (ldc & 3) == 0) ? 1 : 0};
+  return gemm_single_acc_kmajor_launch(a, a_kmajor, stream);
 }
 
 }  // namespace tbik

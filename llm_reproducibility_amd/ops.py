@@ -319,6 +319,28 @@ def _(parts):
 # --------------------------------------------------------------------------------------------
 # batch-invariant ops
 # --------------------------------------------------------------------------------------------
+def _bi_gemm_kmajor(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """bf16 A @ B with a row-major B (and, in a weight gradient, an A whose columns are contiguous) read in place; None
+    where the library prefers copies or an operand lies otherwise.  Same bits either way."""
+    (M, K), N = A.shape, B.shape[1]
+    across = _k_across(A)
+    lda, ldb = A.stride(1 if across else 0), B.stride(0)
+    if M == 1 and not across:
+        lda = K
+    if not ((across and M % 8 == 0) or (A.stride(1) == 1 and K % 64 == 0 and lda >= K)):
+        return None
+    if K == 1 or ldb < N or ldb % 8 or lda % 8 or not _aligned16(A) or not _aligned16(B):
+        return None
+    b = None if bias is None else bias.contiguous()
+    C = torch.empty((M, N), device=A.device, dtype=A.dtype)
+    rc = _lib.lib().bi_gemm_kmajor_bf16(A.data_ptr(), lda, int(across), B.data_ptr(), ldb, C.data_ptr(), C.stride(0), M, N, K,
+                                        None if b is None else b.data_ptr(), _stream(A))
+    if rc == _lib.TBIK_ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc, "bi_gemm_kmajor")
+    return C
+
+
 def _bi_gemm_impl(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     _require_gpu(A, B, bias)
     if A.dtype == torch.float32 and B.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32):
@@ -326,6 +348,10 @@ def _bi_gemm_impl(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]
     M, K = A.shape
     N = B.shape[1]
     f16 = _is_f16(A, B, bias)
+    if not f16 and B.stride(1) == 1 and N % 8 == 0:
+        C = _bi_gemm_kmajor(A, B, bias)
+        if C is not None:
+            return C
     if K % 8 != 0 or (K % 64 != 0 and _k_across(A) and _k_across(B.t())):
         # zero columns do not change a sequential fp32 accumulation.  A K that no kernel takes is extended, and so is one
         # that only the small-tile kernel takes when both operands are copied anyway (a weight gradient, whose K is

@@ -1,0 +1,71 @@
+"""The single-accumulator matmul on K-major operands read in place (a row-major right operand, and with it the transposed left operand of a
+weight gradient): the bits of the same product on K-contiguous copies, at the edges of its tiles and slices."""
+import pytest
+import torch
+
+from llm_reproducibility_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+# widths of 32, 64, 128 and 256 columns are chosen by the grid; columns and rows end inside tiles, chunks and slices
+ONE = [(1, 64, 8), (1, 4096, 4096), (16, 4096, 24576), (40, 128, 1000), (127, 192, 264), (129, 256, 40), (300, 1024, 4104),
+       (512, 64, 2048), (1024, 4096, 4096), (1000, 320, 6152), (2048, 128, 8192)]
+BOTH = [(8, 1, 8), (8, 63, 264), (136, 64, 1000), (264, 65, 4096), (1024, 127, 1032), (2048, 200, 2048), (1000, 129, 40), (4096, 33, 8192)]
+
+
+def _operand(g, rows, cols, extra=0):
+    t = torch.randn(rows, cols + extra, device="cuda", generator=g).to(torch.bfloat16)
+    return t[:, :cols]
+
+
+def _check(A, B, bias, in_place):
+    """in_place: the size is one that the library takes so (None: either way)."""
+    direct = ops._bi_gemm_kmajor(A, B, bias)
+    if in_place is not None:
+        assert (direct is not None) == in_place
+    want = ops.bi_gemm(A.contiguous(), B.t().contiguous().t(), bias)
+    got = ops.bi_gemm(A, B, bias)
+    for out in (got, direct):
+        if out is not None:
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    return want
+
+
+@pytest.mark.parametrize("M,K,N", ONE)
+@pytest.mark.parametrize("extra", [0, 24])
+def test_row_major_right_operand(M, K, N, extra):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    A, B = _operand(g, M, K, extra), _operand(g, K, N, extra)
+    bias = _operand(g, 1, N)[0] if extra else None
+    want = _check(A, B, bias, True)
+    # one rounding to bf16 (2^-8) of a sum whose own error is at most K rounding steps of 2^-24 of the sum of magnitudes
+    ref = A.double() @ B.double() + (0 if bias is None else bias.double())
+    mag = A.double().abs() @ B.double().abs()
+    assert ((want.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * (K + 1) * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("M,K,N", BOTH)
+@pytest.mark.parametrize("extra", [0, 8])
+def test_both_operands_k_major(M, K, N, extra):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    At, B = _operand(g, K, M, extra), _operand(g, K, N, extra)
+    _check(At.t(), B, None, None if K == 1 else True)
+    At[-1, 0], B[-1, -1] = float("inf"), float("nan")    # the last row is what stands in for the rows behind K
+    _check(At.t(), B, None, None if K == 1 else True)
+
+
+def test_what_is_left_to_copies():
+    g = torch.Generator(device="cuda").manual_seed(5)
+    _check(_operand(g, 64, 72), _operand(g, 72, 64), None, False)          # K no whole number of slices
+    _check(_operand(g, 64, 64), _operand(g, 64, 60, 4), None, False)       # columns no whole chunks
+    _check(_operand(g, 64, 64), _operand(g, 64, 64, 3), None, False)       # rows not aligned
+    _check(_operand(g, 64, 65)[:, 1:], _operand(g, 64, 64), None, False)   # left operand not aligned
+    _check(_operand(g, 8, 8192), _operand(g, 8192, 128), None, False)      # a few long chains
+    _check(_operand(g, 72, 63).t(), _operand(g, 72, 64), None, False)      # M no whole chunks
+
+
+@pytest.mark.parametrize("M", [0, 3])
+def test_empty(M):
+    A = torch.empty(M, 64, device="cuda", dtype=torch.bfloat16)
+    for N in (0, 8):
+        assert ops.bi_gemm(A, torch.empty(64, N, device="cuda", dtype=torch.bfloat16), None).shape == (M, N)
