@@ -86,6 +86,10 @@ int tbik_gemm_bf16(const void* A, int64_t lda,
 size_t tbik_gemm_workspace_bytes(int M, int N, int K, int leaf_k);
 /* The same for a row-major B[K,N] (ldb_n == 1); f16 != 0: for tbik_gemm_f16. */
 size_t tbik_gemm_workspace_bytes_rowmajor_b(int M, int N, int K, int leaf_k, int f16);
+
+/* 1 where a row-major B is better passed in place (ldb_n == 1), 0 where a copy as [N,K] (bi_transpose) and that product are faster.  Either way
+ * gives the same bits. */
+int tbik_gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
 /*
  * How tbik_gemm_bf16 (f16 != 0: tbik_gemm_f16) would run this problem: the decision the workspace size above comes
  * from, for callers and tests that want to see it (host only, launches nothing, no effect on any result).

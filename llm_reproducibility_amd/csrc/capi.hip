@@ -8,6 +8,7 @@ int gemm_dispatch(bool tree, bool f16, const void* A, int64_t lda, const void* B
                   hipStream_t stream);
 size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b = false);
 size_t gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, bool f16);
+bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
 int gemm_kmajor_dispatch(const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M, int N,
                          int K, const void* bias, hipStream_t stream);
 int gemm_sharded_dispatch(bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K,
@@ -59,7 +60,7 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 extern "C" {
 
-int tbik_abi_version(void) { return 20; }
+int tbik_abi_version(void) { return 21; }
 
 const char* tbik_error_string(int code) {
   switch (code) {
@@ -91,6 +92,7 @@ size_t tbik_gemm_f16_workspace_bytes(int M, int N, int K, int leaf_k) { return t
 size_t tbik_gemm_workspace_bytes_rowmajor_b(int M, int N, int K, int leaf_k, int f16) {
   return tbik::gemm_workspace_bytes(M, N, K, leaf_k, f16 != 0, true);
 }
+int tbik_gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k) { return tbik::gemm_rowmajor_b_pays(M, N, K, leaf_k) ? 1 : 0; }
 int tbik_gemm_plan_info(int M, int N, int K, int leaf_k, int f16, int rowmajor_b, int* out5) {
   return tbik::gemm_plan_info(M, N, K, leaf_k, f16 != 0, rowmajor_b != 0, out5);
 }

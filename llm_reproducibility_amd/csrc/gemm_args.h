@@ -40,7 +40,7 @@ int gemm_tree_deep_pair_launch(const WidePair& a, hipStream_t stream);
 
 // gemm_tree_quad.hip: tree-ordered bf16 GEMM with leaves of 256 on 128x128 tiles (one wave per SIMD, the tree of a shard
 // in registers: a.lb <= 1, a.ws unused); grid.y = split as for the kernels above
-int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream);
+int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream, bool w_kmajor = false);
 // gemm_tree_few.hip: up to 64 rows, bf16 / fp16, tiles of `waves` (2 .. 6) times 32 columns, shards of at most
 // TREE_FEW_LEVELS binary levels; no parked levels (a.ws is not used)
 constexpr int TREE_FEW_LEVELS = 3;

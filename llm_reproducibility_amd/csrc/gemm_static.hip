@@ -47,12 +47,14 @@ extern "C" int tbik_gemm_bf16_static(const void* A, int64_t lda, const void* B, 
   if (M < 0 || N < 0 || K <= 0) return TBIK_ERR_INVALID;
   if (M == 0 || N == 0) return TBIK_OK;
   const size_t need = tbik::gemm_workspace_bytes(M, N, K, leaf_k, false, ldb_k != 1);
-  if (need > (size_t)TBIK_STATIC_SCRATCH_BYTES) return TBIK_ERR_SCRATCH_LIMIT;  // before anything is launched
+  // before anything is launched; a row-major B that does not fit runs on tiles that need less scratch, where those fit
+  if (need > (size_t)TBIK_STATIC_SCRATCH_BYTES && ldb_k == 1) return TBIK_ERR_SCRATCH_LIMIT;
   void* ws = nullptr;
   if (need > 0) {
     const int rc = scratch_for_current_device(&ws);
     if (rc != TBIK_OK) return rc;
   }
-  return tbik::gemm_dispatch(true, false, A, lda, B, ldb_k, ldb_n, C, ldc, M, N, K, leaf_k, bias_or_null, ws,
-                             need > 0 ? (size_t)TBIK_STATIC_SCRATCH_BYTES : 0, static_cast<hipStream_t>(stream));
+  const int rc = tbik::gemm_dispatch(true, false, A, lda, B, ldb_k, ldb_n, C, ldc, M, N, K, leaf_k, bias_or_null, ws,
+                                     need > 0 ? (size_t)TBIK_STATIC_SCRATCH_BYTES : 0, static_cast<hipStream_t>(stream));
+  return rc == TBIK_ERR_WORKSPACE ? TBIK_ERR_SCRATCH_LIMIT : rc;
 }

@@ -416,6 +416,7 @@ struct Plan {
   int split;       // power of two, divides 2^lb
   int T, flb, lb;  // tree of ONE shard
   size_t partial_bytes, parked_bytes;
+  bool kmajor;     // a row-major B on the 128x128 tiles of gemm_tree_quad.hip (kmajor_plan)
 };
 
 // Which of the two 128x256-tile kernels runs a shard whose tree has groups of `flb` leaves and `lb` binary levels.  The
@@ -522,6 +523,7 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
   const int64_t wide_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
   int split = shards;
   bool wide = false;
+  pl->kmajor = false;
   if (M >= 64 && !rowmajor_b) {  // the wide kernels exist for [N,K] weights only
     wide_cost_us(M, N, K, leaf_k, f16, flb, lb, &split, shards);
     // exactly 64 rows fit one 64-row tile of the tiled kernel, which half-empty 128-row tiles only beat on a grid that
@@ -547,6 +549,52 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
   pl->partial_bytes = (pl->partial_bytes + 255) & ~(size_t)255;
   pl->parked_bytes = wide ? wide_workspace_bytes(M, N, pl->lb, split, wide_uses_deep_kernel(leaf_k, f16, flb, pl->lb) ? 2 : 1) : 0;
   return true;
+}
+
+// A row-major B with leaves of 256 and columns in whole chunks of eight: in place on the 128x128 tiles of gemm_tree_quad.hip,
+// which take it K-major (kmajor.h).  K is cut until at most two groups of leaves are left to a shard (the tree that kernel
+// holds), once or not at all beyond that: the cheaper by 3 us, 0.3 us + 12.3 ns per k of a shard for every round of 256
+// work-groups, and the combine.  Returns that time in us, 0 where the kernel does not apply.  Measured on MI355X against the 64-row
+// tiles, the other kernels that read a row-major B, over M = 1 .. 2048, K = 512 .. 12288, N = 2048 .. 16384 in both types: faster
+// everywhere, [1,4096]x[4096,4096] 16.8 -> 13.4 us, [16,12288]x[12288,16384] 154 -> 85, [100,12288]x[12288,4096] 68 -> 30,
+// [1024,1536]x[1536,2048] 33.8 -> 16.7, [2048,2048]x[2048,4096] 137 -> 64.
+static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
+  int T, flb, level_k;
+  if (leaf_k != 256 || (N & 7) || M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return 0.0;
+  const int lb = level_k - 1;
+  const int64_t tiles = (((int64_t)N + 127) / 128) * (((int64_t)M + 127) / 128);
+  double best = 0.0;
+  for (int ls = lb > 1 ? lb - 1 : 0; ls <= lb && ls <= 5; ls++) {
+    const int sp = 1 << ls;
+    const double t = 3.0 + (double)((tiles * sp + 255) / 256) * (0.3 + 0.0123 * (K / sp)) +
+                     (sp > 1 ? 3.0 + (double)(sp + 1) * M * N * 2.0 / 5.0e6 : 0.0);
+    if (best > 0.0 && t >= best) continue;
+    best = t;
+    *pl = Plan{};
+    pl->kmajor = true;
+    pl->split = sp;
+    pl->T = T >> ls;
+    pl->flb = flb;
+    pl->lb = lb - ls;
+    pl->partial_bytes = sp > 1 ? (((size_t)sp * M * N * sizeof(uint16_t) + 255) & ~(size_t)255) : 0;
+  }
+  return best;
+}
+
+// Whether a row-major B is better read in place than through a transposing copy (23 us for 4096 x 4096, 45 us for 12288 x 4096)
+// and the kernels for [N,K] weights.  On the 128x128 tiles: by the estimate above against the copy's two passes at 4.1 TB/s and
+// the product at 1.1 PFLOP/s (700 rows: 4096 x 4096 51 us against 57, 8192 x 5120 128 against 107, 12288 x 4096 133 against 137;
+// 0.4 % from the better of the two on average over 99 shapes of the sweep above, 15 % at worst).  On the 64-row tiles (leaves of
+// 128, odd columns): they cut K and hold out until they fill a second round of the chip, that is up to 128 rows (12288 x 4096:
+// 68 against 73; at 192 rows 99 against 79, at 1024 448 against 164), later for small matrices (2048 x 1536: 256 rows 16 against
+// 20, 384 rows 27 against 21; 1024 x 1024: 1024 rows 16.3 against 17.4, 1536 rows 26.5 against 18.1; 512 x 1536: 1536 rows,
+// 288 tiles, 22.8 against 14.4): bounds on M * K * N and on the tiles.
+bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k) {
+  Plan pl;
+  const double mkn = (double)M * K * N;
+  const double in_place = kmajor_plan(M, N, K, leaf_k, &pl);
+  if (in_place > 0.0) return 0.9 * in_place < 9.0 + (double)K * N * 4.0 / 4.1e6 + std::max(mkn / 0.55e9, 3.0 + (double)K * N * 2.0 / 5.0e6);
+  return M <= 128 || (mkn < 416.0 * 2048 * 1536 && (((int64_t)M + 63) / 64) * (((int64_t)N + 127) / 128) <= 256);
 }
 
 // Short shards, leaves of 256: where K cannot be cut into long enough pieces, tiles of 128x256 leave half of the chip idle
@@ -687,6 +735,11 @@ static bool tree_plan(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b
       tp->bytes = tp->regions.bytes;
       return true;
     }
+  }
+  if (rowmajor_b && kmajor_plan(M, N, K, leaf_k, &tp->single) > 0.0) {
+    tp->path = PATH_SINGLE;
+    tp->bytes = tp->single.partial_bytes;
+    return true;
   }
   if (!make_plan(M, N, K, leaf_k, f16, &tp->single, rowmajor_b, shards)) return false;
   tp->path = PATH_SINGLE;
@@ -938,6 +991,11 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
     }
     return rc;
   }
+  if (tp.path == PATH_SINGLE && tp.single.kmajor && tp.bytes > ws_bytes) {
+    // less scratch than these tiles ask for (a fixed array, say): the 64-row tiles need less or none
+    if (!make_plan(M, N, K, leaf_k, f16, &tp.single, true)) return TBIK_ERR_INVALID;
+    tp.bytes = tp.single.partial_bytes;
+  }
   const Plan& pl = tp.single;
   if (tp.bytes > 0 && (!ws || ws_bytes < tp.bytes || !aligned16(ws))) return TBIK_ERR_WORKSPACE;
   uint8_t* wsb = static_cast<uint8_t*>(ws);
@@ -957,6 +1015,11 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
   int rc;
   if (rowmajor_b) {
     if (a.lb > 6) return TBIK_ERR_UNSUPPORTED;
+    if (pl.kmajor && lda < (1 << 22) && ldw < (1 << 22)) {  // else rows too far apart for 32-bit offsets: the 64-row tiles on the same shards
+      const WideArgs w{a.X, a.W, a.C, a.bias, nullptr, a.ldx, a.ldw, a.ldc, M, N, a.K, a.T, a.flb, a.lb, a.vec_store, a.k_shard,
+                       pl.split > 1 ? a.c_shard : 0};
+      rc = gemm_tree_quad_launch(w, f16, pl.split, stream, true);
+    } else
     if (f16) rc = leaf_k == 256 ? launch_rowmajor_b<4, 6, true, true>(a, pl.split, stream) : launch_rowmajor_b<2, 6, true, true>(a, pl.split, stream);
     else rc = leaf_k == 256 ? launch_rowmajor_b<4, 6, true, false>(a, pl.split, stream) : launch_rowmajor_b<2, 6, true, false>(a, pl.split, stream);
   } else if (pl.wide) {

@@ -30,6 +30,7 @@
 
 #include "common.h"
 #include "gemm_args.h"
+#include "kmajor.h"
 #include "lds_direct.h"
 
 namespace tbik {
@@ -49,8 +50,8 @@ enum Kind { K_FIRST = 0, K_ADD = 1, K_CARRY = 2 };  // the pending leaf opens a 
 }  // namespace tq
 
 // TN: 16-column MFMA tiles per wave (4: the 128-column tile).  LS: slices per leaf (4: leaves of 256).  NSLOT: slices of
-// the ring.
-template <int TN, int NSLOT, int LS, bool F16>
+// the ring.  WT: the right operand lies K-major ([K,N], p.ldw its row stride, N a multiple of 8) and is read in place (kmajor.h).
+template <int TN, int NSLOT, int LS, bool F16, bool WT = false>
 __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p) {
   using namespace tq;
   using Num = Num16<F16>;
@@ -81,7 +82,8 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
   const int m0 = pid_m * BM, n0 = pid_n * BN;
 
   const uint8_t* xbase = reinterpret_cast<const uint8_t*>(p.X + (int64_t)m0 * p.ldx + shard * p.k_shard);
-  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.W + (int64_t)n0 * p.ldw + shard * p.k_shard);
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(WT ? p.W + shard * p.k_shard * p.ldw + n0 : p.W + (int64_t)n0 * p.ldw + shard * p.k_shard);
+  const int64_t wstep = WT ? p.ldw * (BK * 2) : BK * 2;  // bytes from slice to slice
   uint32_t voff[NDMA];
   {
     const int r = lane >> 3, c = (lane & 7) ^ r;
@@ -89,17 +91,24 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
     for (int i = 0; i < NDMA; i++) {
       const int row = (i * NWAVE + wave) * 8 + r;  // X rows, then W rows; rows past the edge are clamped
       if (i < XDMA) voff[i] = (uint32_t)(((min(m0 + row, p.M - 1) - m0) * p.ldx + c * 8) * 2);
+      else if (WT) voff[i] = kmajor::load_offset<BN>((i - XDMA) * NWAVE + wave, lane, p.ldw, p.N - n0);
       else voff[i] = (uint32_t)(((min(n0 + row - BM, p.N - 1) - n0) * p.ldw + c * 8) * 2);
     }
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   const int nstages = p.T * LS;
   auto dma_one = [&](int s, int slot, int i) __attribute__((always_inline)) {
-    const uint8_t* b = (i < XDMA ? xbase : wbase) + (int64_t)min(s, nstages - 1) * (BK * 2);
+    const int64_t sl = min(s, nstages - 1);
+    const uint8_t* b = i < XDMA ? xbase + sl * (BK * 2) : wbase + sl * wstep;
     dma16(lds0 + slot * STAGE_BYTES + (i * NWAVE + wave) * 1024, voff[i], b);
   };
   const int frow = lane & 15, fchk = lane >> 4;
   const uint32_t xfrag = ((wm * TM * 16 + frow) * BK + ((fchk ^ (frow & 7)) << 3)) * 2;
+  uint32_t wt[WT ? TN : 1];
+  if (WT) {
+#pragma unroll
+    for (int b = 0; b < TN; b++) wt[b] = BM * BK * 2 + kmajor::frag_offset<BN>(wn * TN + b, lane);
+  }
   const uint32_t wfrag = (BM * BK + (wn * TN * 16 + frow) * BK + ((fchk ^ (frow & 7)) << 3)) * 2;
 
   f32x4 acc[TM][TN];
@@ -112,7 +121,8 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
     fx[buf][a] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (xfrag ^ (kk * 64)) + a * 16 * BK * 2);
   };
   auto read_w = [&](int buf, int slot, int kk, int b) __attribute__((always_inline)) {
-    fw[buf][b] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (wfrag ^ (kk * 64)) + b * 16 * BK * 2);
+    if (WT) fw[buf][b] = kmajor::read<BN>(smem + slot * STAGE_BYTES, wt[b], kk);
+    else fw[buf][b] = *reinterpret_cast<const bf16x8*>(smem + slot * STAGE_BYTES + (wfrag ^ (kk * 64)) + b * 16 * BK * 2);
   };
 
   // tree state, packed bf16 pairs: register (a * TN + b) * 2 + h holds elements 2h, 2h+1 of MFMA tile (a, b)
@@ -313,7 +323,7 @@ __global__ __launch_bounds__(tq::NT) void gemm_tree_quad_kernel(const WideArgs p
   }
 }
 
-template <int TN, int NSLOT, int LS, bool F16>
+template <int TN, int NSLOT, int LS, bool F16, bool WT = false>
 static int tq_launch(const WideArgs& a, int split, hipStream_t stream) {
   using namespace tq;
   constexpr int BN = Shape<TN>::BN;
@@ -323,16 +333,18 @@ static int tq_launch(const WideArgs& a, int split, hipStream_t stream) {
   if (tiles <= 0 || tiles > 0x7fffffff || split <= 0 || split > 65535) return TBIK_ERR_UNSUPPORTED;
   if (a.T <= 0 || a.K != a.T * LS * BK || a.lb < 0 || a.lb > MAXL || a.flb < 1) return TBIK_ERR_UNSUPPORTED;
   if (a.ldx >= (1 << 22) || a.ldw >= (1 << 22)) return TBIK_ERR_UNSUPPORTED;  // 32-bit in-tile byte offsets
+  if (WT && (a.N & 7)) return TBIK_ERR_UNSUPPORTED;
   static std::atomic<uint64_t> done{0};
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tree_quad_kernel<TN, NSLOT, LS, F16>), (int)smem, done);
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tree_quad_kernel<TN, NSLOT, LS, F16, WT>), (int)smem, done);
   if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((gemm_tree_quad_kernel<TN, NSLOT, LS, F16>), dim3((unsigned)tiles, (unsigned)split), dim3(NT), smem, stream, a);
+  hipLaunchKernelGGL((gemm_tree_quad_kernel<TN, NSLOT, LS, F16, WT>), dim3((unsigned)tiles, (unsigned)split), dim3(NT), smem, stream, a);
   return hip_code(hipGetLastError());
 }
 
 // a ring of four slices (128 KiB): 2-5 % ahead of three on half of the shapes measured, level with it on the rest; five
 // are no better than three
-int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream) {
+int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream, bool w_kmajor) {
+  if (w_kmajor) return f16 ? tq_launch<4, 4, 4, true, true>(a, split, stream) : tq_launch<4, 4, 4, false, true>(a, split, stream);
   return f16 ? tq_launch<4, 4, 4, true>(a, split, stream) : tq_launch<4, 4, 4, false>(a, split, stream);
 }
 

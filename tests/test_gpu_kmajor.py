@@ -1,9 +1,11 @@
-"""The single-accumulator matmul on K-major operands read in place (a row-major right operand, and with it the transposed left operand of a
-weight gradient): the bits of the same product on K-contiguous copies, at the edges of its tiles and slices."""
+"""Matmuls on K-major operands read in place (a row-major right operand, and with it the transposed left operand of a weight
+gradient): the bits of the same product on K-contiguous copies, at the edges of tiles and slices."""
 import pytest
 import torch
 
-from llm_reproducibility_amd import ops
+from llm_reproducibility_amd import _lib, ops
+from llm_reproducibility_amd.tbik import matmul_tp_persistent
+from oracle import tbik_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +71,39 @@ def test_empty(M):
     A = torch.empty(M, 64, device="cuda", dtype=torch.bfloat16)
     for N in (0, 8):
         assert ops.bi_gemm(A, torch.empty(64, N, device="cuda", dtype=torch.bfloat16), None).shape == (M, N)
+
+
+# shards of one and of two groups of leaves, groups of one and of several leaves, tiles that end in rows and columns
+TREE = [(1, 256, 8), (3, 4096, 4096), (16, 12288, 1000), (64, 768, 136), (65, 512, 264), (128, 6144, 2048), (129, 25600, 128),
+        (300, 2048, 1032), (1024, 1536, 2048), (1000, 8192, 520), (40, 32768, 64)]
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M,K,N", TREE)
+def test_tree_row_major(M, K, N, f16):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    dt = torch.float16 if f16 else torch.bfloat16
+    A = torch.randn(M, K + 8, device="cuda", generator=g).to(dt)[:, :K]
+    B = (torch.randn(K, N + 16, device="cuda", generator=g) * 0.05).to(dt)[:, :N]
+    bias = torch.randn(N, device="cuda", generator=g).to(dt)
+    native = B.t().contiguous().t()
+    want = matmul_tp_persistent(A, native, leaf_k=256)
+    assert torch.equal(matmul_tp_persistent(A, B, leaf_k=256), want)
+    assert torch.equal(ops.gemm_tree(A, B, bias, 256), ops.gemm_tree(A, native, bias, 256))
+    # in place whatever the rule prefers, and with no scratch at all (tiles that need none, or a refusal)
+    L, out = _lib.lib(), torch.empty(M, N, device="cuda", dtype=dt)
+    f = L.tbik_gemm_f16 if f16 else L.tbik_gemm_bf16
+    for nbytes in (L.tbik_gemm_workspace_bytes_rowmajor_b(M, N, K, 256, int(f16)), 0):
+        ws = torch.empty(max(nbytes, 16), device="cuda", dtype=torch.uint8)
+        out.zero_()
+        rc = f(A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), 1, out.data_ptr(), N, M, N, K, 256, None, ws.data_ptr(), nbytes,
+               torch.cuda.current_stream().cuda_stream)
+        assert rc == _lib.TBIK_OK or (nbytes == 0 and rc == _lib.TBIK_ERR_WORKSPACE)
+        if rc == _lib.TBIK_OK:
+            assert torch.equal(out, want)
+
+
+def test_tree_row_major_against_the_oracle():
+    x, w = O.integer_bf16((70, 3072), -9, 9, 0), O.integer_bf16((200, 3072), -7, 7, 1)
+    B = w.t().contiguous()
+    assert torch.equal(matmul_tp_persistent(x.cuda(), B.cuda(), leaf_k=256).cpu(), O.matmul_tree(x, B, leaf=256))
