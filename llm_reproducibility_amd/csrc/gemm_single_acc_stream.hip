@@ -321,6 +321,8 @@ __global__ __launch_bounds__(NWAVES * 64) void gemm_single_acc_stream_kernel(con
 // here the loads need no registers.  X travels with the weights through the ring, so its rows cost no wait of their own: the
 // time hardly grows with the rows (figures at ring_waves).
 // The weights are loaded with the non-temporal hint (dma16_once): gate/up at 32 rows 45.6 -> 40.7 us, lm_head at 8 rows 217 -> 196.
+// Not on the groups of one or two waves, which a narrow matrix gets: it may lie in the 256 MB cache behind the L2s from the last
+// pass, and the hint gives that up ([16,4096]x[4096,6144] from memory 12.7 -> 12.1 us, but the same 50 MB again and again 11.0 -> 11.7).
 // A wave multiplies one strip of 16 columns (GATED: of both halves) by all rows; it loads the weight rows that it alone
 // multiplies and its share of the X rows, and one barrier per slice hands the X rows around.
 namespace ring {
@@ -377,7 +379,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_single_acc_ring_kernel(const Str
 #pragma unroll
     for (int i = 0; i < XDMA; i++) dma16(base + dst[i], voff[i], xbase + (int64_t)s * ROWB);
 #pragma unroll
-    for (int i = XDMA; i < NDMA; i++) dma16_once(base + dst[i], voff[i], (i < XDMA + 4 ? wbase : w2base) + (int64_t)s * ROWB);
+    for (int i = XDMA; i < NDMA; i++) {
+      const uint8_t* from = (i < XDMA + 4 ? wbase : w2base) + (int64_t)s * ROWB;
+      if (GATED || NW > 2) dma16_once(base + dst[i], voff[i], from);
+      else dma16(base + dst[i], voff[i], from);
+    }
   };
   const int r = lane & 15, g = lane >> 4;
   const uint32_t xfrag = r * ROWB, wfrag = (MB * 16 + wave * TN * 16 + r) * ROWB;
@@ -628,7 +634,7 @@ int gemm_single_acc_stream_launch(const StreamArgs& a, bool f16, hipStream_t str
   }
 }
 
-// The gated form: only the windowed kernel has it (5 .. 64 rows: fewer rows take the whole-X kernel, whose consumer, the
+// The gated form: the ring and the windowed kernel have it (5 .. 64 rows: fewer rows take the whole-X kernel, whose consumer, the
 // tree matmul of down_proj, forms the activation itself).
 int gemm_single_acc_stream_gated_launch(const StreamArgs& a, hipStream_t stream) {
   if (a.M <= 0 || a.M > 64 || (a.K & 31) != 0 || a.K < 32 * 16 || !a.W2 || a.bias || (a.N & 15) != 0) return TBIK_ERR_UNSUPPORTED;

@@ -792,7 +792,7 @@ int gemm_dispatch(bool tree, bool f16, const void* A, int64_t lda, const void* B
 // All ranks of a row-split layer on one GPU: every rank's product from its columns of A and of the [N,K] weight, rounded to
 // the element type, then the shard tree.  What `shards` calls of gemm_dispatch on column slices and a combine compute, but
 // the ranks share one grid: a rank alone leaves most of the chip idle ([232,3200]x[3200,5120], leaves of 128, is 40 tiles on 256
-// CUs; eight of them 505 us in eight launches, 120 in one).  Same bits; norm_w / res as for gemm_tree_rmsnorm_dispatch when `ep`.
+// CUs; eight of them 512 us in eight launches, 127 in one).  Same bits.
 int gemm_sharded_dispatch(bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K,
                           int leaf_k, int shards, const void* bias, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (!ranks_ok(K, leaf_k, shards)) return TBIK_ERR_INVALID;
@@ -1095,7 +1095,7 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 // The merged gate/up projection with the activation behind it in the same launch: out[M, inter] = silu(x Wg^T) * (x Wu^T),
 // W = [2*inter, K] (rows 0 .. inter-1 gate, the rest up; the nn.Linear layout), both products rounded to bf16 first.
-// Up to 64 rows on the windowed streaming kernel; with more, where the product of 2 * inter columns runs on the tiles of
+// Up to 64 rows on the ring kernel (the windowed one where K is no whole number of its slices); with more, where the product of 2 * inter columns runs on the tiles of
 // gemm_single_acc_256.hip, on the gated form of those.  TBIK_ERR_UNSUPPORTED (nothing launched) elsewhere.
 int gemm_silu_mul_dispatch(const void* x, int64_t ldx, const void* W, int64_t ldw, void* out, int64_t ldo, int M, int inter, int K,
                            hipStream_t stream) {
