@@ -87,8 +87,8 @@ size_t tbik_gemm_workspace_bytes(int M, int N, int K, int leaf_k);
 /* The same for a row-major B[K,N] (ldb_n == 1); f16 != 0: for tbik_gemm_f16. */
 size_t tbik_gemm_workspace_bytes_rowmajor_b(int M, int N, int K, int leaf_k, int f16);
 
-/* 1 where a row-major B is better passed in place (ldb_n == 1), 0 where a copy as [N,K] (bi_transpose) and that product are faster.  Either way
- * gives the same bits. */
+/* 1 where the kernel that reads a row-major B K-major in place (ldb_n == 1; leaves of 256, N a multiple of 8) takes the problem and beats a
+ * copy as [N,K] (bi_transpose) and that product.  Either way gives the same bits. */
 int tbik_gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
 /*
  * How tbik_gemm_bf16 (f16 != 0: tbik_gemm_f16) would run this problem: the decision the workspace size above comes
@@ -172,14 +172,20 @@ int bi_gemm_bf16(const void* A, int64_t lda,
                  tbik_stream_t stream);
 
 /*
- * bi_gemm_bf16 with operands that lie K-major, read in place: B is [K,N] (row stride ldb), A is [M,K] or, with a_kmajor, [K,M]
+ * bi_gemm_bf16 / bi_gemm_f16 with operands that lie K-major, read in place: B is [K,N] (row stride ldb), A is [M,K] or, with a_kmajor, [K,M]
  * (row stride lda; the weight gradient grad_out^T x of a linear layer takes both this way).  The same MFMA chain per element, hence
- * the bits of bi_gemm_bf16 on transposed copies.  16-byte aligned operands, strides multiples of 8.
+ * the bits of those calls on transposed copies.  16-byte aligned operands, strides multiples of 8.
  * TBIK_ERR_UNSUPPORTED (3), nothing launched: N (with a_kmajor also M) is no multiple of 8, K is no multiple of 64 (without a_kmajor), or
  * copies and the kernels for K-contiguous operands are faster.
  * Replaces: as bi_gemm_bf16 (the backward products of the reference's aten::mm override).
  */
 int bi_gemm_kmajor_bf16(const void* A, int64_t lda, int a_kmajor,
+                        const void* B, int64_t ldb,
+                        void* C, int64_t ldc,
+                        int M, int N, int K,
+                        const void* bias_or_null,
+                        tbik_stream_t stream);
+int bi_gemm_kmajor_f16(const void* A, int64_t lda, int a_kmajor,
                         const void* B, int64_t ldb,
                         void* C, int64_t ldc,
                         int M, int N, int K,

@@ -9,8 +9,8 @@ int gemm_dispatch(bool tree, bool f16, const void* A, int64_t lda, const void* B
 size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b = false);
 size_t gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, bool f16);
 bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
-int gemm_kmajor_dispatch(const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M, int N,
-                         int K, const void* bias, hipStream_t stream);
+int gemm_kmajor_dispatch(bool f16, const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M,
+                         int N, int K, const void* bias, hipStream_t stream);
 int gemm_sharded_dispatch(bool f16, const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K,
                           int leaf_k, int shards, const void* bias, void* ws, size_t ws_bytes, hipStream_t stream);
 int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, int out[5]);
@@ -60,7 +60,7 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 extern "C" {
 
-int tbik_abi_version(void) { return 21; }
+int tbik_abi_version(void) { return 22; }
 
 const char* tbik_error_string(int code) {
   switch (code) {
@@ -147,7 +147,11 @@ int bi_gemm_bf16(const void* A, int64_t lda, const void* B, int64_t ldb_k, int64
 
 int bi_gemm_kmajor_bf16(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M, int N, int K,
                         const void* bias_or_null, tbik_stream_t stream) {
-  return tbik::gemm_kmajor_dispatch(A, lda, a_kmajor != 0, B, ldb, C, ldc, M, N, K, bias_or_null, static_cast<hipStream_t>(stream));
+  return tbik::gemm_kmajor_dispatch(false, A, lda, a_kmajor != 0, B, ldb, C, ldc, M, N, K, bias_or_null, static_cast<hipStream_t>(stream));
+}
+int bi_gemm_kmajor_f16(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M, int N, int K,
+                       const void* bias_or_null, tbik_stream_t stream) {
+  return tbik::gemm_kmajor_dispatch(true, A, lda, a_kmajor != 0, B, ldb, C, ldc, M, N, K, bias_or_null, static_cast<hipStream_t>(stream));
 }
 
 int bi_rmsnorm_gemm_bf16(const void* x, int64_t ldx, const void* residual_or_null, int64_t ldr, const void* norm_weight_or_null,

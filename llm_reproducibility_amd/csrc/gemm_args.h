@@ -46,7 +46,7 @@ int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t st
 constexpr int TREE_FEW_LEVELS = 3;
 int gemm_tree_few_launch(const WideArgs& a, int leaf_k, bool f16, int waves, int split, hipStream_t stream);
 
-// gemm_single_acc_quad.hip: single-accumulator bf16 GEMM, one wave per SIMD
+// gemm_single_acc_quad.hip: single-accumulator 16-bit GEMM, one wave per SIMD
 struct QuadArgs {
   const uint16_t* X;   // [M,K], row stride ldx
   const uint16_t* W;   // [N,K], row stride ldw
@@ -56,7 +56,8 @@ struct QuadArgs {
   int M, N, K;
   int vec_store;
   int row_step = 0;    // rows a tile of gemm_single_acc_quad_kernel owns (0 = all 128; 64, 32 or 16: see the kernel)
-  const uint16_t* W2 = nullptr;  // gated form of gemm_single_acc_256.hip only: the up half [N,K], row stride ldw (no bias)
+  const uint16_t* W2 = nullptr;  // gated form of gemm_single_acc_256.hip only: the up half [N,K], row stride ldw (no bias; bf16)
+  bool f16 = false;              // elements are fp16 (chooses the instantiation)
 };
 int gemm_single_acc_quad_launch(const QuadArgs& a, hipStream_t stream);
 // the right operand [K,N], the left one [K,M] too with x_kmajor (ldw / ldx their row strides), read in place

@@ -1,4 +1,4 @@
-// Batch-invariant bf16 GEMM (one fp32 accumulator per element, K strictly ascending) for gfx950, path of the shapes
+// Batch-invariant 16-bit GEMM (one fp32 accumulator per element, K strictly ascending) for gfx950, path of the shapes
 // with many rounds of tiles: 256x256 output tile per work-group, 4 wavefronts (one per SIMD) of 128x128 each, K
 // streamed in 64-element slices through a ring of ten 16 KiB blocks that fills the 160 KiB of LDS.  Replaces
 // matmul_kernel_persistent, src/bio/batch_invariant_ops.py:42-124, where the 128x256 tile of
@@ -45,11 +45,15 @@ constexpr __device__ __forceinline__ int wrap(int pos) { return pos >= NBLOCK ? 
 // such a statement: inside the loop an accumulator is touched by nothing but its own MFMA (the next one 64 MFMAs
 // later), the fragment registers are written by LDS reads that the compiler orders itself, and the epilogue waits
 // before anything else reads the results (mfma_results_ready).
+template <bool F16>
 __device__ __forceinline__ void mfma_in_agprs(f32x4& acc, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  if (F16) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
+template <bool F16>
 __device__ __forceinline__ void mfma_in_vgprs(f32x4& acc, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+  if (F16) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
 __device__ __forceinline__ void mfma_results_ready() {
   // an 8-pass MFMA needs up to 18 wait states before another kind of instruction may read its result; the scheduling
@@ -66,7 +70,7 @@ __device__ __forceinline__ void mfma_results_ready() {
 // up, so silu(gate) * up of a tile meets in its own LDS and the product of twice the columns never goes to memory (a
 // write and a read of it at 6 TB/s, and half of the burst of stores at a round's end).  Two calls -> this, hidden 4096,
 // 2 x 12288 columns: 512 rows 81 -> 75 us, 2048 rows 299 -> 276, 10944 rows 1673 -> 1541.
-template <int TM, int TN, bool GATED = false>
+template <int TM, int TN, bool GATED, bool F16>
 __global__ __launch_bounds__(sq::NT) void gemm_single_acc_256_kernel(const QuadArgs p) {
   using namespace sq;
   constexpr int BM = 2 * TM * 16, BN = (GATED ? 1 : 2) * TN * 16;  // BN: output columns
@@ -176,8 +180,8 @@ __global__ __launch_bounds__(sq::NT) void gemm_single_acc_256_kernel(const QuadA
       for (int q = 0; q < TM; q++) {
 #pragma unroll
         for (int b = 0; b < TN; b++) {
-          if (TN < 8 || b < TN - 1) mfma_in_agprs(acc[q][b], fw[kk][b], fx[kk][q]);
-          else mfma_in_vgprs(acc[q][b], fw[kk][b], fx[kk][q]);
+          if (TN < 8 || b < TN - 1) mfma_in_agprs<F16>(acc[q][b], fw[kk][b], fx[kk][q]);
+          else mfma_in_vgprs<F16>(acc[q][b], fw[kk][b], fx[kk][q]);
           if (b < 2 * RPR - 1 && (RPR == 3 || (b & 1) == 0)) {
             // fragments of the next k step: the second of this slice, or the first of the next slice (behind the
             // last slice that reads blocks whose loads have landed and are never used)
@@ -286,10 +290,10 @@ __global__ __launch_bounds__(sq::NT) void gemm_single_acc_256_kernel(const QuadA
         if (p.bias) {
           const int n = n0 + (wn * TN + b) * 16 + fchk * 4;
 #pragma unroll
-          for (int e = 0; e < 4; e++) bv[e] = bf16_bits_to_f32(p.bias[n + e]);
+          for (int e = 0; e < 4; e++) bv[e] = Num16<F16>::to_f32(p.bias[n + e]);
         }
-        const uint32_t lo = pack_bf16x2(acc[a][b][0] + bv[0], acc[a][b][1] + bv[1]);
-        const uint32_t hi = pack_bf16x2(acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]);
+        const uint32_t lo = Num16<F16>::pack(acc[a][b][0] + bv[0], acc[a][b][1] + bv[1]);
+        const uint32_t hi = Num16<F16>::pack(acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]);
         *reinterpret_cast<uint2*>(stage + (a * 16 + frow) * ROWB + (b * 16 + fchk * 4) * 2) = make_uint2(lo, hi);
       }
     }
@@ -318,10 +322,10 @@ __global__ __launch_bounds__(sq::NT) void gemm_single_acc_256_kernel(const QuadA
       if (p.bias) {
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (n + e < p.N) bv[e] = bf16_bits_to_f32(p.bias[n + e]);
+          if (n + e < p.N) bv[e] = Num16<F16>::to_f32(p.bias[n + e]);
       }
-      const uint32_t lo = pack_bf16x2(acc[a][b][0] + bv[0], acc[a][b][1] + bv[1]);
-      const uint32_t hi = pack_bf16x2(acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]);
+      const uint32_t lo = Num16<F16>::pack(acc[a][b][0] + bv[0], acc[a][b][1] + bv[1]);
+      const uint32_t hi = Num16<F16>::pack(acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]);
       uint16_t* dst = p.C + (int64_t)m * p.ldc + n;
       if (p.vec_store && n + 3 < p.N) {
         *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(sq::NT) void gemm_single_acc_256_kernel(const QuadA
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int TM, int TN, bool GATED>
+template <int TM, int TN, bool GATED, bool F16>
 static int sq_launch(const QuadArgs& a, hipStream_t stream) {
   using namespace sq;
   constexpr int BM = 2 * TM * 16, BN = (GATED ? 1 : 2) * TN * 16;
@@ -346,23 +350,24 @@ static int sq_launch(const QuadArgs& a, hipStream_t stream) {
   if (tiles <= 0 || tiles > 0x7fffffff || a.K < BK || (a.K % BK) != 0) return TBIK_ERR_UNSUPPORTED;
   if (a.ldx >= (1 << 22) || a.ldw >= (1 << 22)) return TBIK_ERR_UNSUPPORTED;  // 32-bit in-tile byte offsets
   static std::atomic<uint64_t> done{0};
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_single_acc_256_kernel<TM, TN, GATED>), (int)smem, done);
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_single_acc_256_kernel<TM, TN, GATED, F16>), (int)smem, done);
   if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((gemm_single_acc_256_kernel<TM, TN, GATED>), dim3((unsigned)tiles), dim3(NT), smem, stream, a);
+  hipLaunchKernelGGL((gemm_single_acc_256_kernel<TM, TN, GATED, F16>), dim3((unsigned)tiles), dim3(NT), smem, stream, a);
   return hip_code(hipGetLastError());
 }
 
-template <bool GATED>
+template <bool GATED, bool F16>
 static int sq_by_tile(const QuadArgs& a, int tile_rows, int tile_cols, hipStream_t stream) {
-  if (tile_rows == 256 && tile_cols == 256) return sq_launch<8, 8, GATED>(a, stream);
-  if (tile_rows == 256 && tile_cols == 192) return sq_launch<8, 6, GATED>(a, stream);
-  if (tile_rows == 192 && tile_cols == 256) return sq_launch<6, 8, GATED>(a, stream);
-  if (tile_rows == 192 && tile_cols == 192) return sq_launch<6, 6, GATED>(a, stream);
+  if (tile_rows == 256 && tile_cols == 256) return sq_launch<8, 8, GATED, F16>(a, stream);
+  if (tile_rows == 256 && tile_cols == 192) return sq_launch<8, 6, GATED, F16>(a, stream);
+  if (tile_rows == 192 && tile_cols == 256) return sq_launch<6, 8, GATED, F16>(a, stream);
+  if (tile_rows == 192 && tile_cols == 192) return sq_launch<6, 6, GATED, F16>(a, stream);
   return TBIK_ERR_UNSUPPORTED;
 }
 
 int gemm_single_acc_256_launch(const QuadArgs& a, int tile_rows, int tile_cols, hipStream_t stream) {
-  return a.W2 ? sq_by_tile<true>(a, tile_rows, tile_cols, stream) : sq_by_tile<false>(a, tile_rows, tile_cols, stream);
+  if (a.f16) return a.W2 ? TBIK_ERR_UNSUPPORTED : sq_by_tile<false, true>(a, tile_rows, tile_cols, stream);
+  return a.W2 ? sq_by_tile<true, false>(a, tile_rows, tile_cols, stream) : sq_by_tile<false, false>(a, tile_rows, tile_cols, stream);
 }
 
 }  // namespace tbik

@@ -1,4 +1,4 @@
-// Batch-invariant bf16 GEMM (one fp32 accumulator per element, K strictly ascending) for gfx950, large-M path:
+// Batch-invariant 16-bit GEMM (one fp32 accumulator per element, K strictly ascending) for gfx950, large-M path:
 // 128x256 output tile per work-group, 4 wavefronts (one per SIMD) of 64x128 each, K streamed through a 3-slot
 // LDS ring in 64-element slices.  Replaces matmul_kernel_persistent, src/bio/batch_invariant_ops.py:42-124, for
 // shapes that fill the chip; per element it issues the same MFMA chain as the small-tile kernel in gemm_tiled.hip,
@@ -43,7 +43,7 @@ struct Shape {
 // XT, WT: that operand lies K-major ([K,M], [K,N]; p.ldx / p.ldw its row stride) and is read in place (kmajor.h); M / N is then a
 // multiple of 8.  With both K-major (a weight gradient, whose K is the number of tokens) K may be any number: the rows of
 // the last slice behind it are zeroed in LDS by the wave that loaded them.
-template <int TN, int NSLOT, bool XT = false, bool WT = false>
+template <int TN, int NSLOT, bool F16, bool XT = false, bool WT = false>
 __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const QuadArgs p) {
   using namespace quad;
   static_assert(NSLOT >= 3, "the schedule needs a slice in use, one landing and one in flight");
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const Qu
 #pragma unroll
         for (int j = 0; j < GM; j++) {
           const int a = TN > 4 ? q >> 1 : q, b = TN > 4 ? (q & 1) * (TN / 2) + j : j;
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[kk][b], fx[kk][a], (s == 0 && kk == 0) ? zero : acc[a][b], 0, 0, 0);
+          acc[a][b] = Num16<F16>::mfma(fw[kk][b], fx[kk][a], (s == 0 && kk == 0) ? zero : acc[a][b]);
           if (j < 3) other(j);
         }
 #pragma unroll
@@ -215,10 +215,10 @@ __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const Qu
       if (p.bias) {
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (n + e < p.N) bv[e] = bf16_bits_to_f32(p.bias[n + e]);
+          if (n + e < p.N) bv[e] = Num16<F16>::to_f32(p.bias[n + e]);
       }
-      const uint32_t lo = pack_bf16x2(acc[a][b][0] + bv[0], acc[a][b][1] + bv[1]);
-      const uint32_t hi = pack_bf16x2(acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]);
+      const uint32_t lo = Num16<F16>::pack(acc[a][b][0] + bv[0], acc[a][b][1] + bv[1]);
+      const uint32_t hi = Num16<F16>::pack(acc[a][b][2] + bv[2], acc[a][b][3] + bv[3]);
       uint16_t* dst = p.C + (int64_t)m * p.ldc + n;
       if (p.vec_store && n + 3 < p.N) {
         *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
@@ -232,22 +232,28 @@ __global__ __launch_bounds__(quad::NT) void gemm_single_acc_quad_kernel(const Qu
   }
 }
 
+template <int TN, int NSLOT, bool F16, bool XT = false, bool WT = false>
+static int quad_launch_as(const QuadArgs& a, int64_t tiles, hipStream_t stream) {
+  constexpr size_t smem = (size_t)NSLOT * quad::Shape<TN>::STAGE_BYTES;  // 144 KiB for the 256-wide tile
+  static_assert(smem <= 160 * 1024 && (NSLOT - 1) * quad::Shape<TN>::NDMA < 64, "ring does not fit the LDS or the wait counter");
+  auto kern = gemm_single_acc_quad_kernel<TN, NSLOT, F16, XT, WT>;
+  static std::atomic<uint64_t> done{0};
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), (int)smem, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(quad::NT), smem, stream, a);
+  return hip_code(hipGetLastError());
+}
+
 template <int TN, int NSLOT = 3>
 static int quad_launch(const QuadArgs& a, hipStream_t stream) {
   using namespace quad;
   constexpr int BN = Shape<TN>::BN;
-  constexpr size_t smem = (size_t)NSLOT * Shape<TN>::STAGE_BYTES;  // 144 KiB for the 256-wide tile
-  static_assert(smem <= 160 * 1024 && (NSLOT - 1) * Shape<TN>::NDMA < 64, "ring does not fit the LDS or the wait counter");
   const int row_step = a.row_step > 0 ? a.row_step : BM;
   if (row_step > BM || (row_step & 15)) return TBIK_ERR_INVALID;
   const int64_t tiles = (int64_t)((a.M + row_step - 1) / row_step) * ((a.N + BN - 1) / BN);
   if (tiles <= 0 || tiles > 0x7fffffff || a.K < BK || (a.K % BK) != 0) return TBIK_ERR_UNSUPPORTED;
   if (a.ldx >= (1 << 22) || a.ldw >= (1 << 22)) return TBIK_ERR_UNSUPPORTED;  // 32-bit in-tile byte offsets
-  static std::atomic<uint64_t> done{0};
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_single_acc_quad_kernel<TN, NSLOT>), (int)smem, done);
-  if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((gemm_single_acc_quad_kernel<TN, NSLOT>), dim3((unsigned)tiles), dim3(NT), smem, stream, a);
-  return hip_code(hipGetLastError());
+  return a.f16 ? quad_launch_as<TN, NSLOT, true>(a, tiles, stream) : quad_launch_as<TN, NSLOT, false>(a, tiles, stream);
 }
 
 int gemm_single_acc_quad_launch(const QuadArgs& a, hipStream_t stream) { return quad_launch<8>(a, stream); }
@@ -433,15 +439,9 @@ int gemm_single_acc_balanced_launch(const QuadArgs& a, hipStream_t stream) {
 template <int TN, int NSLOT, bool XT>
 static int quad_kmajor_launch(const QuadArgs& a, hipStream_t stream) {
   using namespace quad;
-  constexpr size_t smem = (size_t)NSLOT * Shape<TN>::STAGE_BYTES;
-  static_assert(smem <= 160 * 1024 && (NSLOT - 1) * Shape<TN>::NDMA < 64, "ring does not fit the LDS or the wait counter");
   const int64_t tiles = (int64_t)((a.M + BM - 1) / BM) * ((a.N + Shape<TN>::BN - 1) / Shape<TN>::BN);
   if (tiles <= 0 || tiles > 0x7fffffff) return TBIK_ERR_UNSUPPORTED;
-  static std::atomic<uint64_t> done{0};
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_single_acc_quad_kernel<TN, NSLOT, XT, true>), (int)smem, done);
-  if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((gemm_single_acc_quad_kernel<TN, NSLOT, XT, true>), dim3((unsigned)tiles), dim3(NT), smem, stream, a);
-  return hip_code(hipGetLastError());
+  return a.f16 ? quad_launch_as<TN, NSLOT, true, XT, true>(a, tiles, stream) : quad_launch_as<TN, NSLOT, false, XT, true>(a, tiles, stream);
 }
 
 // Whether `in_place` us (of quad_time) beat a transposing copy per K-major operand (3 us and two passes at 4.1 TB/s) and the
@@ -499,17 +499,18 @@ int gemm_single_acc_kmajor_launch(const QuadArgs& a, bool x_kmajor, hipStream_t 
   }
 }
 
-int gemm_kmajor_dispatch(const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M, int N,
-                         int K, const void* bias, hipStream_t stream) {
+int gemm_kmajor_dispatch(bool f16, const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M,
+                         int N, int K, const void* bias, hipStream_t stream) {
   if (M < 0 || N < 0 || K <= 0) return TBIK_ERR_INVALID;
   if (M == 0 || N == 0) return TBIK_OK;
   if (!A || !B || !C) return TBIK_ERR_INVALID;
   if (lda < (a_kmajor ? M : K) || ldb < N || ldc < N) return TBIK_ERR_INVALID;
   auto aligned16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   if (!aligned16(A) || !aligned16(B) || (lda & 7) || (ldb & 7) || (reinterpret_cast<uintptr_t>(C) & 1)) return TBIK_ERR_ALIGNMENT;
-  const QuadArgs a{static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(B), static_cast<uint16_t*>(C),
-                   static_cast<const uint16_t*>(bias), lda, ldb, ldc, M, N, K,
-                   ((reinterpret_cast<uintptr_t>(C) & 7) == 0 && (ldc & 3) == 0) ? 1 : 0};
+  QuadArgs a{static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(B), static_cast<uint16_t*>(C),
+             static_cast<const uint16_t*>(bias), lda, ldb, ldc, M, N, K,
+             ((reinterpret_cast<uintptr_t>(C) & 7) == 0 && (ldc & 3) == 0) ? 1 : 0};
+  a.f16 = f16;
   return gemm_single_acc_kmajor_launch(a, a_kmajor, stream);
 }
 

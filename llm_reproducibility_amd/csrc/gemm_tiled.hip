@@ -581,20 +581,15 @@ static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
   return best;
 }
 
-// Whether a row-major B is better read in place than through a transposing copy (23 us for 4096 x 4096, 45 us for 12288 x 4096)
-// and the kernels for [N,K] weights.  On the 128x128 tiles: by the estimate above against the copy's two passes at 4.1 TB/s and
-// the product at 1.1 PFLOP/s (700 rows: 4096 x 4096 51 us against 57, 8192 x 5120 128 against 107, 12288 x 4096 133 against 137;
-// 0.4 % from the better of the two on average over 99 shapes of the sweep above, 15 % at worst).  On the 64-row tiles (leaves of
-// 128, odd columns): they cut K and hold out until they fill a second round of the chip, that is up to 128 rows (12288 x 4096:
-// 68 against 73; at 192 rows 99 against 79, at 1024 448 against 164), later for small matrices (2048 x 1536: 256 rows 16 against
-// 20, 384 rows 27 against 21; 1024 x 1024: 1024 rows 16.3 against 17.4, 1536 rows 26.5 against 18.1; 512 x 1536: 1536 rows,
-// 288 tiles, 22.8 against 14.4): bounds on M * K * N and on the tiles.
+// Whether a row-major B is better read by those tiles than through a transposing copy (23 us for 4096 x 4096, 45 us for 12288 x
+// 4096) and the kernels for [N,K] weights: the estimate above against the copy's two passes at 4.1 TB/s and the product at 1.1
+// PFLOP/s (700 rows: 4096 x 4096 51 us against 57, 8192 x 5120 128 against 107, 12288 x 4096 133 against 137; 0.4 % from the
+// better of the two on average over 99 shapes of the sweep above, 15 % at worst).
 bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k) {
   Plan pl;
   const double mkn = (double)M * K * N;
   const double in_place = kmajor_plan(M, N, K, leaf_k, &pl);
-  if (in_place > 0.0) return 0.9 * in_place < 9.0 + (double)K * N * 4.0 / 4.1e6 + std::max(mkn / 0.55e9, 3.0 + (double)K * N * 2.0 / 5.0e6);
-  return M <= 128 || (mkn < 416.0 * 2048 * 1536 && (((int64_t)M + 63) / 64) * (((int64_t)N + 127) / 128) <= 256);
+  return in_place > 0.0 && 0.9 * in_place < 9.0 + (double)K * N * 4.0 / 4.1e6 + std::max(mkn / 0.55e9, 3.0 + (double)K * N * 2.0 / 5.0e6);
 }
 
 // Short shards, leaves of 256: where K cannot be cut into long enough pieces, tiles of 128x256 leave half of the chip idle
@@ -855,8 +850,12 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
     // 33..128 rows: one row of 128-row tiles whose width balances the grid, when such a grid exists (same MFMA chain
     // per element again; measured faster than the streaming kernel from 33 rows on)
     const bool narrow_n = N < 4096;   // no one-row grid of at least 128 tiles, whatever their width
-    if (!f16 && M > 32 && M <= 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
+    // fp16 takes all of these since they were built for it: [128,12288]x[12288,4096] 117 -> 49 us, [512,4096]x[4096,6144] 61 -> 34,
+    // [2048,4096]x[4096,24576] 492 -> 296, [4096,12288]x[12288,4096] 463 -> 275 against the tiled kernel; up to 64 rows of a
+    // wide matrix the ring kernel stays ([33,4096]x[4096,24576] 39 against 42, [48,12288]x[12288,4096] 43.5 against 46)
+    if ((!f16 || M > 64 || narrow_n) && M > 32 && M <= 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
       QuadArgs qa{a.X, a.W, a.C, a.bias, a.ldx, a.ldw, a.ldc, M, N, K, a.vec_store};
+      qa.f16 = f16;
       if (!narrow_n) {
         const int rc = gemm_single_acc_slab_launch(qa, stream);
         if (rc != TBIK_ERR_UNSUPPORTED) return rc;
@@ -869,12 +868,14 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
       }
     }
     // more rows: the same pipeline with the tile width that spreads the grid over the chip (128x256 on large shapes)
-    if (!f16 && M > 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
+    if (M > 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
       QuadArgs qa{a.X, a.W, a.C, a.bias, a.ldx, a.ldw, a.ldc, M, N, K, a.vec_store};
+      qa.f16 = f16;
       return gemm_single_acc_balanced_launch(qa, stream);
     }
-    if (!f16 && M > 64 && wide_tiles >= 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
+    if (M > 64 && wide_tiles >= 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
       QuadArgs qa{a.X, a.W, a.C, a.bias, a.ldx, a.ldw, a.ldc, M, N, K, a.vec_store};
+      qa.f16 = f16;
       return gemm_single_acc_quad_launch(qa, stream);
     }
     // a handful of rows: one pass over the weights, every 16x16 tile its own wave (same chain per element again)

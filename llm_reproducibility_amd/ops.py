@@ -162,45 +162,61 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
     return out if len(shape) == 2 else out.reshape(shape)
 
 
-# Where a row-major [K,N] operand of the single-accumulator mm that bi_gemm_kmajor_bf16 does not take (fp16, K that is no multiple of
-# 64, odd columns) is repacked into the native [N,K] layout instead of being consumed in place.  In place it runs on the
-# 64-row tiled kernels only (the other pipelines are built for [N,K]); a repack is one pass of the transposing copy
-# kernel (23 us for 4096 x 4096 in 16 bits, 45 us for 12288 x 4096) and then whatever kernel is best.  Same bits either way.
-# In place cannot cut K, so a call takes as long as one chain per round of 512 work-groups (two on a CU), whatever it
-# fills them with; narrow matrices are repacked (4096 x 4096: 88 us against 27 at one row, 77 against 34 at 64), wide ones
-# not while they are one round (12288 x 16384: 220 against 273 at 64 rows, 248 against 318 at 256; 4096 x 24576: 93 against
-# 123 at 128 rows, 158 against 138 at 160).  K, the type (fp16 has slower tiles above 64 rows: 12288 x 10240 at 256 rows 182
-# against 244, bf16 201 against 201) and the rounds move the line, so both times are estimated.  Over 4,862 points of 1 ..
-# 3072 rows, K = 512 .. 25600, N = 512 .. 151936 in both types the choice is 0.25 % from the better of the two on average and
-# 23 % at worst.
-def _mm_in_place(rows: int, K: int, N: int, f16: bool) -> bool:
+# Where a row-major [K,N] operand that the K-major kernels do not take (`_bi_gemm_kmajor`, `_tree_operand`: odd columns, leaves of
+# 128, a K that is no multiple of 64) is repacked into the native [N,K] layout instead of being consumed in place.  In place
+# it runs on the 64-row tiled kernels; a repack is one pass of the transposing copy kernel (23 us for 4096 x 4096 in 16 bits,
+# 45 us for 12288 x 4096) and then whatever kernel is best.  Same bits either way.  Measured on MI355X, us in place against repacked:
+#   tree matmul: in place cuts K and holds out until its 64-row tiles fill a second round of the chip, that is up to 128
+#     rows (12288 x 4096: 68 against 73; at 192 rows 99 against 79, at 1024 448 against 164), later for small matrices
+#     (2048 x 1536: 256 rows 16 against 20, 384 rows 27 against 21; 1024 x 1024: 1024 rows 16.3 against 17.4, 1536 rows 26.5
+#     against 18.1; 512 x 1536: 1536 rows, 288 tiles, 22.8 against 14.4): bounds on rows * K * N and on the tiles.
+#   single-accumulator mm: in place cannot cut K, so a call takes as long as one chain per round of 512 work-groups (two on
+#     a CU), whatever it fills them with; narrow matrices are repacked (4096 x 4096: 88 against 27 at one row, 77 against 34 at
+#     64), wide ones not while they are one round (12288 x 16384: 220 against 273 at 64 rows, 248 against 318 at 256; 4096 x
+#     24576: 93 against 123 at 128 rows, 158 against 138 at 160).  K, the type (fp16 has slower tiles above 64 rows:
+#     12288 x 10240 at 256 rows 182 against 244, bf16 201 against 201) and the rounds move the line, so both times are estimated.
+#     Over 4,862 points of 1 .. 3072 rows, K = 512 .. 25600, N = 512 .. 151936 in both types the choice is 0.25 % from the
+#     better of the two on average and 23 % at worst.
+_TREE_IN_PLACE_MACS = 416 * 2048 * 1536
+
+
+def _consumed_in_place(rows: int, K: int, N: int, tree: bool, f16: bool = False) -> bool:
     tiles = -(-rows // 64) * -(-N // 128)
+    if tree:
+        return rows <= 128 or (rows * K * N < _TREE_IN_PLACE_MACS and tiles <= 256)
     groups = -(-N // 64) if rows <= 16 else tiles
     in_place = (7.0 + 0.0222 * K) * max(1, -(-groups // 512))
     copied = 4.0 * K * N    # bytes; up to 256 MB the cache behind the L2s holds them
     product = max(K * N / 3.5e6, 0.0048 * K if rows > 64 else 0.0)
-    if f16 and rows > 64:
+    if f16 and rows > 64 and K % 64:
         product = max(product, 0.0098 * K * -(-(-(-rows // 128) * -(-N // 128)) // 256))
     else:
         product = max(product, rows * K * N / 0.72e9)
     return in_place < 11.8 + copied / (4.1e6 if copied <= 256e6 else 3.3e6) + product
 
 
-def _weight_operand(B: torch.Tensor, rows: int = 0, leaf_k: Optional[int] = 256):
+def _weight_operand(B: torch.Tensor, rows: int = 0, tree: bool = True):
     """How a [K,N] operand is handed to the kernels: (tensor whose data_ptr is passed, ldb_k, ldb_n).
 
     `weight.t()` of an nn.Linear weight ([N,K], K contiguous) is the native layout (ldb_k = 1), used without a copy; a
     row-major [K,N] operand (N contiguous: a plain `x @ B`) is consumed in place too (ldb_n = 1) unless a repack into
-    the native layout pays for this many `rows` of a tree matmul (leaf_k; None: the single-accumulator mm).  Anything else
-    -- neither dimension contiguous, rows not 16-byte aligned -- is repacked as well."""
+    the native layout pays for this many `rows`.  Anything else -- neither dimension contiguous, rows not 16-byte
+    aligned -- is repacked as well."""
     (K, N), (s0, s1) = B.shape, B.stride()
     if s0 == 1 and _aligned16(B) and K % 8 == 0 and (N == 1 or (s1 >= K and s1 % 8 == 0)):
         return B, 1, (K if N == 1 else s1)
-    if s1 == 1 and _aligned16(B) and s0 >= N and s0 % 8 == 0:
-        if _lib.lib().tbik_gemm_rowmajor_b_pays(rows, N, K, leaf_k) if leaf_k else _mm_in_place(rows, K, N, B.dtype is torch.float16):
-            return B, s0, 1
+    if s1 == 1 and _aligned16(B) and s0 >= N and s0 % 8 == 0 and _consumed_in_place(rows, K, N, tree, B.dtype is torch.float16):
+        return B, s0, 1
     w, ldw = _rows16(B.t())
     return w, 1, ldw
+
+
+def _tree_operand(B: torch.Tensor, rows: int, leaf_k: int):
+    """`_weight_operand` of a tree matmul: a row-major operand also stays where the library reads it K-major at a gain."""
+    (K, N), (s0, s1) = B.shape, B.stride()
+    if s1 == 1 and _aligned16(B) and s0 >= N and s0 % 8 == 0 and _lib.lib().tbik_gemm_rowmajor_b_pays(rows, N, K, leaf_k):
+        return B, s0, 1
+    return _weight_operand(B, rows, True)
 
 
 # --------------------------------------------------------------------------------------------
@@ -213,7 +229,7 @@ def _gemm_tree_impl(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tenso
     M, K = A.shape
     N = B.shape[1]
     a, lda = _rows16(A)
-    w, ldb_k, ldb_n = _weight_operand(B, M, leaf_k)
+    w, ldb_k, ldb_n = _tree_operand(B, M, leaf_k)
     b = None if bias is None else bias.contiguous()
     f16 = _is_f16(A, B, bias)
     C = torch.empty((M, N), device=A.device, dtype=A.dtype)
@@ -311,8 +327,8 @@ def _(parts):
 # --------------------------------------------------------------------------------------------
 # batch-invariant ops
 # --------------------------------------------------------------------------------------------
-def _bi_gemm_kmajor(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """bf16 A @ B with a row-major B (and, in a weight gradient, an A whose columns are contiguous) read in place; None
+def _bi_gemm_kmajor(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor], f16: bool) -> Optional[torch.Tensor]:
+    """A @ B in 16 bits with a row-major B (and, in a weight gradient, an A whose columns are contiguous) read in place; None
     where the library prefers copies or an operand lies otherwise.  Same bits either way."""
     (M, K), N = A.shape, B.shape[1]
     across = _k_across(A)
@@ -325,8 +341,10 @@ def _bi_gemm_kmajor(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tenso
         return None
     b = None if bias is None else bias.contiguous()
     C = torch.empty((M, N), device=A.device, dtype=A.dtype)
-    rc = _lib.lib().bi_gemm_kmajor_bf16(A.data_ptr(), lda, int(across), B.data_ptr(), ldb, C.data_ptr(), C.stride(0), M, N, K,
-                                        None if b is None else b.data_ptr(), _stream(A))
+    L = _lib.lib()
+    rc = (L.bi_gemm_kmajor_f16 if f16 else L.bi_gemm_kmajor_bf16)(
+        A.data_ptr(), lda, int(across), B.data_ptr(), ldb, C.data_ptr(), C.stride(0), M, N, K,
+        None if b is None else b.data_ptr(), _stream(A))
     if rc == _lib.TBIK_ERR_UNSUPPORTED:
         return None
     _lib.check(rc, "bi_gemm_kmajor")
@@ -340,8 +358,8 @@ def _bi_gemm_impl(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]
     M, K = A.shape
     N = B.shape[1]
     f16 = _is_f16(A, B, bias)
-    if not f16 and B.stride(1) == 1 and N % 8 == 0:
-        C = _bi_gemm_kmajor(A, B, bias)
+    if B.stride(1) == 1 and N % 8 == 0:
+        C = _bi_gemm_kmajor(A, B, bias, f16)
         if C is not None:
             return C
     if K % 8 != 0 or (K % 64 != 0 and _k_across(A) and _k_across(B.t())):
@@ -354,7 +372,7 @@ def _bi_gemm_impl(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch.Tensor]
         ldb_k = 1
     else:
         a, lda = _rows16(A)
-        w, ldb_k, ldb_n = _weight_operand(B, M, None)
+        w, ldb_k, ldb_n = _weight_operand(B, M, False)
     b = None if bias is None else bias.contiguous()
     C = torch.empty((M, N), device=A.device, dtype=A.dtype)
     L = _lib.lib()
@@ -748,7 +766,7 @@ def gemm_tree_add_rmsnorm(A: torch.Tensor, B: torch.Tensor, bias: Optional[torch
                and not torch.compiler.is_compiling() and ("tree_norm", M, N, K, leaf_k) not in _declined)
     if fusable:
         a, lda = _rows16(A)
-        w, ldb_k, ldb_n = _weight_operand(B, M, leaf_k)
+        w, ldb_k, ldb_n = _tree_operand(B, M, leaf_k)
         if ldb_k == 1:
             L = _lib.lib()
             b = None if bias is None else bias.contiguous()

@@ -15,14 +15,14 @@ ONE = [(1, 64, 8), (1, 4096, 4096), (16, 4096, 24576), (40, 128, 1000), (127, 19
 BOTH = [(8, 1, 8), (8, 63, 264), (136, 64, 1000), (264, 65, 4096), (1024, 127, 1032), (2048, 200, 2048), (1000, 129, 40), (4096, 33, 8192)]
 
 
-def _operand(g, rows, cols, extra=0):
-    t = torch.randn(rows, cols + extra, device="cuda", generator=g).to(torch.bfloat16)
+def _operand(g, rows, cols, extra=0, dt=torch.bfloat16):
+    t = torch.randn(rows, cols + extra, device="cuda", generator=g).to(dt)
     return t[:, :cols]
 
 
 def _check(A, B, bias, in_place):
     """in_place: the size is one that the library takes so (None: either way)."""
-    direct = ops._bi_gemm_kmajor(A, B, bias)
+    direct = ops._bi_gemm_kmajor(A, B, bias, A.dtype is torch.float16)
     if in_place is not None:
         assert (direct is not None) == in_place
     want = ops.bi_gemm(A.contiguous(), B.t().contiguous().t(), bias)
@@ -33,24 +33,26 @@ def _check(A, B, bias, in_place):
     return want
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N", ONE)
 @pytest.mark.parametrize("extra", [0, 24])
-def test_row_major_right_operand(M, K, N, extra):
+def test_row_major_right_operand(M, K, N, extra, dt):
     g = torch.Generator(device="cuda").manual_seed(M + K + N)
-    A, B = _operand(g, M, K, extra), _operand(g, K, N, extra)
-    bias = _operand(g, 1, N)[0] if extra else None
+    A, B = _operand(g, M, K, extra, dt), _operand(g, K, N, extra, dt)
+    bias = _operand(g, 1, N, 0, dt)[0] if extra else None
     want = _check(A, B, bias, True)
-    # one rounding to bf16 (2^-8) of a sum whose own error is at most K rounding steps of 2^-24 of the sum of magnitudes
+    # one rounding to the type (2^-8, 2^-11) of a sum whose own error is at most K rounding steps of 2^-24 of the sum of magnitudes
     ref = A.double() @ B.double() + (0 if bias is None else bias.double())
     mag = A.double().abs() @ B.double().abs()
-    assert ((want.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + mag * (K + 1) * 2.0 ** -24).all()
+    assert ((want.double() - ref).abs() <= ref.abs() * 2.0 ** (-11 if dt is torch.float16 else -8) + mag * (K + 1) * 2.0 ** -24).all()
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,K,N", BOTH)
 @pytest.mark.parametrize("extra", [0, 8])
-def test_both_operands_k_major(M, K, N, extra):
+def test_both_operands_k_major(M, K, N, extra, dt):
     g = torch.Generator(device="cuda").manual_seed(M + K + N)
-    At, B = _operand(g, K, M, extra), _operand(g, K, N, extra)
+    At, B = _operand(g, K, M, extra, dt), _operand(g, K, N, extra, dt)
     _check(At.t(), B, None, None if K == 1 else True)
     At[-1, 0], B[-1, -1] = float("inf"), float("nan")    # the last row is what stands in for the rows behind K
     _check(At.t(), B, None, None if K == 1 else True)
@@ -107,3 +109,17 @@ def test_tree_row_major_against_the_oracle():
     x, w = O.integer_bf16((70, 3072), -9, 9, 0), O.integer_bf16((200, 3072), -7, 7, 1)
     B = w.t().contiguous()
     assert torch.equal(matmul_tp_persistent(x.cuda(), B.cuda(), leaf_k=256).cpu(), O.matmul_tree(x, B, leaf=256))
+
+
+# one row of tiles of every width, grids of one round and of several (128x256, 256x256 and 192x192 tiles), ends in rows and columns
+@pytest.mark.parametrize("M,K,N", [(33, 64, 4096), (64, 4096, 768), (65, 128, 6144), (128, 192, 24576), (129, 256, 1030), (384, 128, 24576),
+                                   (1000, 320, 6150), (2048, 64, 8192), (2100, 128, 8190), (4096, 128, 5000)])
+def test_fp16_rows_in_blocks(M, K, N):
+    """fp16 batches on the large tiles: the bits of 32 rows at a time, which run on another kernel."""
+    print("case fp16", M, K, N, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    A, W = _operand(g, M, K, 8, torch.float16), _operand(g, N, K, 0, torch.float16)
+    bias = _operand(g, 1, N, 0, torch.float16)[0]
+    for b in (None, bias):
+        want = torch.cat([ops.bi_gemm(A[i:i + 32], W.t(), b) for i in range(0, M, 32)])
+        assert torch.equal(ops.bi_gemm(A, W.t(), b), want)
