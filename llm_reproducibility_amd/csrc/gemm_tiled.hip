@@ -848,12 +848,15 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
     // chain per element, so the same bits as the tiled kernel)
     const int64_t wide_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
     // 33..128 rows: one row of 128-row tiles whose width balances the grid, when such a grid exists (same MFMA chain
-    // per element again; measured faster than the streaming kernel from 33 rows on)
+    // per element again)
     const bool narrow_n = N < 4096;   // no one-row grid of at least 128 tiles, whatever their width
     // fp16 takes all of these since they were built for it: [128,12288]x[12288,4096] 117 -> 49 us, [512,4096]x[4096,6144] 61 -> 34,
-    // [2048,4096]x[4096,24576] 492 -> 296, [4096,12288]x[12288,4096] 463 -> 275 against the tiled kernel; up to 64 rows of a
-    // wide matrix the ring kernel stays ([33,4096]x[4096,24576] 39 against 42, [48,12288]x[12288,4096] 43.5 against 46)
-    if ((!f16 || M > 64 || narrow_n) && M > 32 && M <= 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
+    // [2048,4096]x[4096,24576] 492 -> 296, [4096,12288]x[12288,4096] 463 -> 275 against the tiled kernel.
+    // Up to 48 rows, and up to 64 of more columns than 8192, the ring kernel is ahead of one row of tiles wherever its slices of 128
+    // divide K ([33,4096]x[4096,24576] 46.1 -> 39.7 us, [64,4096]x[4096,24576] 47.0 -> 41.9, [33,4096]x[4096,12288] 27.0 -> 20.5,
+    // [40,5120]x[5120,10240] 35.4 -> 27.1; level at 6144 columns; [64,12288]x[12288,4096] in fp16 49 against 45 on the tiles)
+    const bool ring = M <= (N > 8192 ? 64 : 48) && (K & 127) == 0;
+    if ((narrow_n || !ring) && M > 32 && M <= 128 && (K & 63) == 0 && lda < (1 << 22) && ldb_n < (1 << 22)) {
       QuadArgs qa{a.X, a.W, a.C, a.bias, a.ldx, a.ldw, a.ldc, M, N, K, a.vec_store};
       qa.f16 = f16;
       if (!narrow_n) {
