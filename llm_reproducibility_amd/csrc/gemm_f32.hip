@@ -218,6 +218,164 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(const GemmF32Arg
   }
 }
 
+// The tree of few rows.  One chain over all of K is what a call of few rows waits for above, whatever the tile (31 us at K =
+// 4096, 84 at 12288, where the weights need 11 and 32); a tree's leaves are independent, so here K is cut over the NW waves
+// of a work-group of 16 columns, each an aligned subtree with a ring of its own in the LDS (no barrier until the end), and the
+// waves' roots are added in adjacent pairs through the LDS: the same nodes, hence the same bits.  Rings of NS slices, so
+// that eight waves are on a CU: one work-group of eight, or two of four; grid.y counts blocks of RX rows.
+// [1,4096]x[4096,4096] 38.9 -> 13.3 us, [16,12288]x[12288,4096] 105 -> 41.5, [32,8192]x[8192,5120] 72 -> 61, [8,6144]x[6144,2048]
+// 53 -> 15, weights from memory; at 33 rows and more a second block per strip costs what the tiles do (4096x4096 38, 12288x4096
+// 106) unless all blocks are one round ([64,6144]x[6144,2048] 54 -> 27).
+template <int TM, int NW, int NS>
+__global__ __launch_bounds__(64 * NW) void gemm_f32_strip_kernel(const GemmF32Args p) {
+  constexpr int RX = TM * 16, STAGE = (RX + 16) * 128, NI = (RX + 16) / 8;
+  static_assert(NS >= 3 && (NS - 1) * NI < 64 && NW * NS * STAGE <= 160 * 1024 && TM <= NW, "ring");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = xcd_contiguous_tile(blockIdx.x, gridDim.x) * 16, m0 = blockIdx.y * RX;
+  const int r16 = lane & 15, g = lane >> 4;
+  const int kw = p.K / NW, nslices = kw / F32_SLICE;  // this wave's k, a multiple of 128
+  int lb = p.lb;
+  for (int w = NW; w > 1; w >>= 1) lb--;
+  const uint8_t* xbase = reinterpret_cast<const uint8_t*>(p.X + (int64_t)m0 * p.ldx + wave * kw);
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(p.W + (int64_t)n0 * p.ldw + wave * kw);
+  const int lrow = lane >> 3, lchunk = (lane & 7) ^ lrow;
+  uint32_t voff[NI];
+#pragma unroll
+  for (int i = 0; i < NI; i++) {
+    const int row = i * 8 + lrow;  // X rows, then weight rows; rows past the edge are clamped
+    if (row < RX) voff[i] = (uint32_t)((int64_t)(min(m0 + row, p.M - 1) - m0) * p.ldx * 4) + lchunk * 16;
+    else voff[i] = (uint32_t)((int64_t)(min(n0 + row - RX, p.N - 1) - n0) * p.ldw * 4) + lchunk * 16;
+  }
+  uint8_t* ring = smem + wave * (NS * STAGE);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)ring;
+  auto load_slice = [&](int s, int slot) __attribute__((always_inline)) {
+    const int64_t at = (int64_t)min(s, nslices - 1) * (F32_SLICE * 4);  // past the end the last one again: the count in flight stays
+#pragma unroll
+    for (int i = 0; i < NI; i++) dma16(lds0 + slot * STAGE + i * 1024, voff[i], (i * 8 < RX ? xbase : wbase) + at);
+  };
+  const uint32_t frag = r16 * 128 + ((g ^ (r16 & 7)) << 4);
+  f32x4 fx[2][2][TM], fw[2][2];
+  auto read_frags = [&](int buf, int slot) __attribute__((always_inline)) {
+    const uint8_t* st = ring + slot * STAGE;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+#pragma unroll
+      for (int a = 0; a < TM; a++) fx[buf][c][a] = *reinterpret_cast<const f32x4*>(st + (frag ^ (c * 64)) + a * 2048);
+      fw[buf][c] = *reinterpret_cast<const f32x4*>(st + (frag ^ (c * 64)) + RX * 128);
+    }
+  };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[TM], s0[TM], sb[F32_LBMAX][TM];
+#pragma unroll
+  for (int a = 0; a < TM; a++) acc[a] = zero;
+
+#pragma unroll
+  for (int s = 0; s < NS - 1; s++) load_slice(s, s);
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NS - 2) * NI) : "memory");
+  read_frags(0, 0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  int slot = 0, c0 = 0, grp = 0;
+  for (int j = 0; j < nslices / 4; j++) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int s = 4 * j + i, buf = i & 1;
+      const int next = slot + 1 == NS ? 0 : slot + 1, prev = slot == 0 ? NS - 1 : slot - 1;
+      // the slot of slice s - 1, whose fragments arrived a slice ago, takes slice s + NS - 1; then slice s + 1 has to be there
+      load_slice(s + NS - 1, prev);
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NS - 2) * NI) : "memory");
+      read_frags(buf ^ 1, next);
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int a = 0; a < TM; a++) acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[buf][c][e], fx[buf][c][a][e], acc[a], 0, 0, 0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      slot = next;
+    }
+    // the leaf is done: binary-counter merge (all conditions are uniform)
+    f32x4 t[TM];
+#pragma unroll
+    for (int a = 0; a < TM; a++) {
+      t[a] = c0 != 0 ? s0[a] + acc[a] : acc[a];
+      acc[a] = zero;
+    }
+    if (++c0 < p.flb) {
+#pragma unroll
+      for (int a = 0; a < TM; a++) s0[a] = t[a];
+    } else {
+      c0 = 0;
+      bool parked = false;
+#pragma unroll
+      for (int l = 0; l < F32_LBMAX; l++) {
+        if (!parked && l < lb) {
+          if ((grp >> l) & 1) {
+#pragma unroll
+            for (int a = 0; a < TM; a++) t[a] = sb[l][a] + t[a];
+          } else {
+#pragma unroll
+            for (int a = 0; a < TM; a++) sb[l][a] = t[a];
+            parked = true;
+          }
+        }
+      }
+      grp++;
+      if (!parked) {  // the wave's root, behind its last leaf
+#pragma unroll
+        for (int a = 0; a < TM; a++) s0[a] = t[a];
+      }
+    }
+  }
+
+  // roots of the waves, in the place of each wave's ring (its loads past the end of K have landed): adjacent pairs
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int a = 0; a < TM; a++) *reinterpret_cast<f32x4*>(ring + a * 1024 + lane * 16) = s0[a];
+  __syncthreads();
+  if (wave >= TM) return;  // wave a finishes tile a
+  f32x4 v[NW];
+#pragma unroll
+  for (int w = 0; w < NW; w++) v[w] = *reinterpret_cast<const f32x4*>(smem + w * (NS * STAGE) + wave * 1024 + lane * 16);
+#pragma unroll
+  for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+    for (int w = 0; w < NW; w += 2 * d) v[w] = v[w] + v[w + d];
+  const int m = m0 + wave * 16 + r16, n = n0 + 4 * g;
+  if (m >= p.M || n >= p.N) return;
+  float* dst = p.C + (int64_t)m * p.ldc + n;
+#pragma unroll
+  for (int e = 0; e < 4; e++) v[0][e] += p.bias && n + e < p.N ? p.bias[n + e] : 0.f;
+  if (p.vec_store && n + 3 < p.N) {
+    *reinterpret_cast<f32x4*>(dst) = v[0];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (n + e < p.N) dst[e] = v[0][e];
+  }
+}
+
+template <int TM, int NW, int NS>
+static int f32_strip_launch(const GemmF32Args& a, hipStream_t stream) {
+  constexpr int smem = NW * NS * (TM * 16 + 16) * 128;
+  auto kern = gemm_f32_strip_kernel<TM, NW, NS>;
+  static std::atomic<uint64_t> done{0};
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + 15) / 16), (unsigned)((a.M + TM * 16 - 1) / (TM * 16))), dim3(64 * NW), smem, stream, a);
+  return hip_code(hipGetLastError());
+}
+
+// TBIK_ERR_UNSUPPORTED (nothing launched) where the tiles above serve the call
+static int f32_strip(const GemmF32Args& a, hipStream_t stream) {
+  const int64_t strips = ((int64_t)a.N + 15) / 16, blocks = ((int64_t)a.M + 31) / 32;
+  if ((blocks > 1 && (strips * blocks > 256 || a.lb < 3)) || a.lb < 2 || a.ldx >= (1 << 24) || a.ldw >= (1 << 24)) return TBIK_ERR_UNSUPPORTED;  // 32-bit byte offsets
+  const bool eight = a.lb >= 3 && strips <= 256;   // one round of work-groups of eight waves
+  if (a.M <= 16) return eight ? f32_strip_launch<1, 8, 5>(a, stream) : f32_strip_launch<1, 4, 5>(a, stream);
+  return eight ? f32_strip_launch<2, 8, 3>(a, stream) : f32_strip_launch<2, 4, 3>(a, stream);
+}
+
 template <int WM, int WN, int TM, int TN, int NS, bool TREE>
 static int f32_launch(const GemmF32Args& a, hipStream_t stream) {
   typedef F32Shape<WM, WN, TM, TN, NS> S;
@@ -316,6 +474,8 @@ int gemm_f32_dispatch(bool tree, const void* A, int64_t lda, const void* B, int6
     if (level_k - 1 > F32_LBMAX) return TBIK_ERR_UNSUPPORTED;
     a.flb = flb;
     a.lb = level_k - 1;
+    const int rc = f32_strip(a, stream);
+    if (rc != TBIK_ERR_UNSUPPORTED) return rc;
   }
   const int cfg = f32_pick(M, N, K, tree);
   return tree ? f32_run_reaching<true>(a, cfg, stream) : f32_run_reaching<false>(a, cfg, stream);
