@@ -224,8 +224,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(const GemmF32Arg
 // waves' roots are added in adjacent pairs through the LDS: the same nodes, hence the same bits.  Rings of NS slices, so
 // that eight waves are on a CU: one work-group of eight, or two of four; grid.y counts blocks of RX rows.
 // [1,4096]x[4096,4096] 38.9 -> 13.3 us, [16,12288]x[12288,4096] 105 -> 41.5, [32,8192]x[8192,5120] 72 -> 61, [8,6144]x[6144,2048]
-// 53 -> 15, weights from memory; at 33 rows and more a second block per strip costs what the tiles do (4096x4096 38, 12288x4096
-// 106) unless all blocks are one round ([64,6144]x[6144,2048] 54 -> 27).
+// 53 -> 15, weights from memory.  More rows as long as the blocks make at most two rounds ([64,6144]x[6144,2048] 54 -> 23,
+// [128,6144]x[6144,2048] 55 -> 39, [64,4096]x[4096,4096] 38 -> 30, [64,12288]x[12288,4096] 106 -> 93); three rounds lose to the tiles.
 template <int TM, int NW, int NS>
 __global__ __launch_bounds__(64 * NW) void gemm_f32_strip_kernel(const GemmF32Args p) {
   constexpr int RX = TM * 16, STAGE = (RX + 16) * 128, NI = (RX + 16) / 8;
@@ -370,7 +370,7 @@ static int f32_strip_launch(const GemmF32Args& a, hipStream_t stream) {
 // TBIK_ERR_UNSUPPORTED (nothing launched) where the tiles above serve the call
 static int f32_strip(const GemmF32Args& a, hipStream_t stream) {
   const int64_t strips = ((int64_t)a.N + 15) / 16, blocks = ((int64_t)a.M + 31) / 32;
-  if ((blocks > 1 && (strips * blocks > 256 || a.lb < 3)) || a.lb < 2 || a.ldx >= (1 << 24) || a.ldw >= (1 << 24)) return TBIK_ERR_UNSUPPORTED;  // 32-bit byte offsets
+  if ((blocks > 1 && (strips * blocks > 512 || a.lb < 3)) || a.lb < 2 || a.ldx >= (1 << 24) || a.ldw >= (1 << 24)) return TBIK_ERR_UNSUPPORTED;  // 32-bit byte offsets
   const bool eight = a.lb >= 3 && strips <= 256;   // one round of work-groups of eight waves
   if (a.M <= 16) return eight ? f32_strip_launch<1, 8, 5>(a, stream) : f32_strip_launch<1, 4, 5>(a, stream);
   return eight ? f32_strip_launch<2, 8, 3>(a, stream) : f32_strip_launch<2, 4, 3>(a, stream);
