@@ -42,6 +42,11 @@ bool half(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.sc
 int code(const at::Tensor& t) {
   return t.scalar_type() == at::kFloat ? 0 : t.scalar_type() == at::kBFloat16 ? 1 : t.scalar_type() == at::kHalf ? 2 : -1;
 }
+// a flag that is Python's own bool; whatever else counts as true or false there (0, 1, a numpy bool) goes the long way
+bool flag(PyObject* o, bool* v) {
+  *v = o == Py_True;
+  return PyBool_Check(o);
+}
 void* stream_of(int dev) { return static_cast<void*>(c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream()); }
 
 // the launch, other Python threads free to run meanwhile (it may wait for room in the queue)
@@ -144,14 +149,15 @@ PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // mean_last(x, keepdim): the mean over the last dimension of a contiguous tensor
 PyObject* mean_last(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 2) Py_RETURN_NONE;
+  bool keepdim;
+  if (n != 2 || !flag(a[1], &keepdim)) Py_RETURN_NONE;
   return or_none([&](int dev) -> at::Tensor {
     if (!plain(a[0], dev)) return {};
     const at::Tensor& t = THPVariable_Unpack(a[0]);
     if (t.dim() < 1 || !t.is_contiguous() || t.numel() == 0 || code(t) < 0) return {};
     const int64_t cols = t.size(-1), rows = t.numel() / cols;
     c10::SmallVector<int64_t, 6> shape(t.sizes().begin(), t.sizes().end() - 1);
-    if (a[1] == Py_True) shape.push_back(1);
+    if (keepdim) shape.push_back(1);
     at::Tensor out = at::empty(shape, t.options());
     void *o = out.data_ptr(), *st = stream_of(dev);
     const void* in = t.data_ptr();
@@ -162,19 +168,19 @@ PyObject* mean_last(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // log_softmax(x, write_softmax, to_float) over the rows of a matrix
 PyObject* log_softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 3) Py_RETURN_NONE;
+  bool soft, to_float;
+  if (n != 3 || !flag(a[1], &soft) || !flag(a[2], &to_float)) Py_RETURN_NONE;
   return or_none([&](int dev) -> at::Tensor {
     if (!plain(a[0], dev)) return {};
     const at::Tensor& t = THPVariable_Unpack(a[0]);
     if (t.dim() != 2 || t.numel() == 0 || code(t) < 0 || t.stride(1) != 1 || (t.size(0) > 1 && t.stride(0) < t.size(1))) return {};
     const int64_t rows = t.size(0), cols = t.size(1);
-    at::Tensor out = at::empty({rows, cols}, a[2] == Py_True ? t.options().dtype(at::kFloat) : t.options());
+    at::Tensor out = at::empty({rows, cols}, to_float ? t.options().dtype(at::kFloat) : t.options());
     const size_t need = bi_log_softmax_workspace_bytes(rows, cols);
     at::Tensor ws;
     if (need) ws = at::empty({static_cast<int64_t>((need + 3) / 4)}, t.options().dtype(at::kFloat));
     void *o = out.data_ptr(), *st = stream_of(dev), *wp = need ? ws.data_ptr() : nullptr;
     const void* in = t.data_ptr();
-    const bool soft = a[1] == Py_True;
     const int rc = launch([&] { return bi_log_softmax(in, rows > 1 ? t.stride(0) : cols, code(t), o, cols, code(out), rows, cols, wp, need, soft, st); });
     return rc == TBIK_OK ? out : at::Tensor();
   });

@@ -1,5 +1,6 @@
 """The row-wise operators by the extension's short way and by the long one: the same results, and the same refusals, over the
 forms of input that the long way takes."""
+import numpy as np
 import pytest
 import torch
 
@@ -96,3 +97,17 @@ def test_on_another_stream_and_in_a_graph(dev):
         x.normal_()
         g.replay()
         assert torch.equal(out, ops._bi_rmsnorm_impl(x, w, 1e-6)), k
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_flags_that_are_no_bool(dev, dt):
+    """0, 1, None and numpy's bools count as what they are true for, as on the long way."""
+    x = torch.randn((5, 256), generator=torch.Generator(device=dev).manual_seed(4), device=dev).to(dt)
+    for one in (0, 1, 2, np.bool_(False), np.bool_(True), None):
+        truth = bool(one)
+        assert _same(_outcome(lambda: ops.bi_mean_dim(x, -1, one)), _outcome(lambda: ops.bi_mean_dim(x, -1, truth)))
+        assert _same(_outcome(lambda: ops.bi_log_softmax(x, False, one)), _outcome(lambda: ops.bi_log_softmax(x, False, truth)))
+        want = _outcome(lambda: ops._bi_log_softmax_impl(x, one, False))    # (None is a TypeError there)
+        assert _same(_outcome(lambda: ops.bi_log_softmax(x, one)), want)
+        if one is not None:
+            assert _same(want, _outcome(lambda: ops.bi_log_softmax(x, truth)))
