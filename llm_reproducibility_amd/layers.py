@@ -125,8 +125,8 @@ class SimulatedTPRowLinear(nn.Module):
         in launches of their own their work-groups keep step, 1 - 5 % ([2048,12288]x[12288,4096] in four ranks 247 us in one
         grid, 234 in four, in two 220 and 221; fp16 [2048,8192]x[8192,5120] in two 224 and 213, bf16 206 and 220)."""
         tp, K = self.tp_size, self.weight.shape[1]
-        if not (2 <= tp <= 32 and tp & (tp - 1) == 0 and x2.is_cuda and x2.shape[1] == K and x2.dtype == self.weight.dtype
-                and x2.dtype in (torch.bfloat16, torch.float16) and K % (tp * self.leaf_k) == 0):
+        if not (2 <= tp <= 32 and tp & (tp - 1) == 0 and x2.is_cuda and x2.device == self.weight.device and x2.shape[1] == K
+                and x2.dtype == self.weight.dtype and x2.dtype in (torch.bfloat16, torch.float16) and K % (tp * self.leaf_k) == 0):
             return False
         tiles = -(-x2.shape[0] // 128) * -(-self.weight.shape[0] // 256)
         full = 256 <= tiles < 512 if x2.dtype is torch.float16 else tiles == 256

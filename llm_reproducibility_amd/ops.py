@@ -260,7 +260,16 @@ def _(A, B, bias, leaf_k):
     return A.new_empty((A.shape[0], B.shape[1]))
 
 
+def _check_sharded(A: torch.Tensor, W: torch.Tensor) -> None:
+    """K is taken from A alone: a W of other columns would be read in part, or behind its rows."""
+    if A.dim() != 2 or W.dim() != 2 or A.shape[1] != W.shape[1]:
+        raise ValueError(f"gemm_tree_sharded takes A [M,K] and W [N,K], got {tuple(A.shape)} and {tuple(W.shape)}")
+    if A.device != W.device:
+        raise ValueError(f"gemm_tree_sharded takes operands on one device, got {A.device} and {W.device}")
+
+
 def _gemm_tree_sharded_impl(A: torch.Tensor, W: torch.Tensor, leaf_k: int, shards: int) -> torch.Tensor:
+    _check_sharded(A, W)
     _require_gpu(A, W)
     M, K = A.shape
     N = W.shape[0]
@@ -290,6 +299,7 @@ def gemm_tree_sharded(A: torch.Tensor, W: torch.Tensor, leaf_k: int, shards: int
 
 @_gemm_tree_sharded_op.register_fake
 def _(A, W, leaf_k, shards):
+    _check_sharded(A, W)
     return A.new_empty((A.shape[0], W.shape[0]))
 
 

@@ -331,3 +331,21 @@ def test_tree_all_reduce_wrapper_contract(monkeypatch):
     for q in partials[1:8]:
         seq = seq + q
     assert not torch.equal(seq, O.tree_combine(partials))
+
+
+def test_sharded_product_refuses_operands_that_do_not_match():
+    """K comes from the left operand: a weight of more or fewer columns, a narrower view of a wider buffer among them (whose row stride
+    would pass the library's check), is refused before any pointer is taken, eagerly and while tracing."""
+    from torch._subclasses import FakeTensorMode
+    x, wide = torch.zeros((4, 1024), dtype=torch.bfloat16), torch.zeros((64, 2048), dtype=torch.bfloat16)
+    for w in (wide, wide[:, 512:1024], wide[:, 1536:], wide[0], wide[:, :1024].unsqueeze(0)):
+        with pytest.raises(ValueError):
+            ops.gemm_tree_sharded(x, w, 256, 2)
+    with pytest.raises(ValueError):
+        ops.gemm_tree_sharded(x[0], wide[:, :1024], 256, 2)
+    with FakeTensorMode():
+        a, w = (torch.empty(s, dtype=torch.bfloat16, device="cuda") for s in ((4, 1024), (64, 2048)))
+        assert ops._gemm_tree_sharded_op(a, w[:, :1024], 256, 2).shape == (4, 64)
+        for bad in (w, w[:, :512], w[:, :1024].cpu()):
+            with pytest.raises(ValueError):
+                ops._gemm_tree_sharded_op(a, bad, 256, 2)
