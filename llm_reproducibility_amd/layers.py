@@ -128,6 +128,8 @@ class SimulatedTPRowLinear(nn.Module):
         if not (2 <= tp <= 32 and tp & (tp - 1) == 0 and x2.is_cuda and x2.device == self.weight.device and x2.shape[1] == K
                 and x2.dtype == self.weight.dtype and x2.dtype in (torch.bfloat16, torch.float16) and K % (tp * self.leaf_k) == 0):
             return False
+        if self.weight.stride(1) != 1:   # the one grid would copy all of it, a rank's matmul reads its rows in place
+            return False
         tiles = -(-x2.shape[0] // 128) * -(-self.weight.shape[0] // 256)
         full = 256 <= tiles < 512 if x2.dtype is torch.float16 else tiles == 256
         return not (full and self.leaf_k == 256 and K // tp >= 3072)

@@ -349,3 +349,15 @@ def test_sharded_product_refuses_operands_that_do_not_match():
         for bad in (w, w[:, :512], w[:, :1024].cpu()):
             with pytest.raises(ValueError):
                 ops._gemm_tree_sharded_op(a, bad, 256, 2)
+
+
+def test_simulated_ranks_read_a_weight_of_contiguous_columns_in_place():
+    """Ranks share one grid only on a K-contiguous weight: the other way round each rank's matmul reads its rows of it in place,
+    where the one grid would copy the whole weight on every call."""
+    from torch._subclasses import FakeTensorMode
+    from llm_reproducibility_amd.layers import SimulatedTPRowLinear
+    with FakeTensorMode():
+        x, w = torch.empty((200, 6144), dtype=torch.bfloat16, device="cuda"), torch.empty((2048, 6144), dtype=torch.bfloat16, device="cuda")
+        across = torch.empty((6144, 2048), dtype=torch.bfloat16, device="cuda").t()
+        assert SimulatedTPRowLinear(w, 4)._one_grid(x)
+        assert not SimulatedTPRowLinear(across, 4)._one_grid(x)
