@@ -137,6 +137,9 @@ int tbik_gemm_bf16_static(const void* A, int64_t lda,
  * Replaces: the simulated tensor parallelism of the reference, simple_matmul.py:16-43 (one matmul per rank, then the tree).
  */
 size_t tbik_gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, int f16);
+/* 0 where a tbik_gemm_bf16 / _f16 per rank and tbik_tree_combine_bf16 / _f16 are estimated to be at least 5 % faster than that one grid, else 1
+ * (invalid arguments too: the call itself refuses them).  Either way gives the same bits. */
+int tbik_gemm_sharded_pays(int M, int N, int K, int leaf_k, int shards, int f16);
 int tbik_gemm_sharded(const void* A, int64_t lda,
                       const void* B, int64_t ldb_n,
                       void* C, int64_t ldc,

@@ -11,7 +11,7 @@ import os
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libtbik_hip.so")
 
-ABI_VERSION = 22
+ABI_VERSION = 23
 TBIK_OK = 0
 TBIK_ERR_INVALID = 1
 TBIK_ERR_ALIGNMENT = 2
@@ -28,7 +28,7 @@ EXPORTS = (
     "tbik_gemm_bf16_static", "bi_log_softmax", "tbik_gemm_workspace_bytes_rowmajor_b", "tbik_gemm_rowmajor_b_pays", "tbik_gemm_plan_info",
     "bi_rmsnorm_gemm_bf16", "tbik_gemm_silu_mul_bf16", "bi_argmax_advance_bf16",
     "tbik_gemm_rmsnorm_bf16", "tbik_tree_combine_rmsnorm_bf16", "bi_attention_decode_qkv_bf16", "bi_gemm_silu_mul_bf16",
-    "tbik_gemm_sharded", "tbik_gemm_sharded_workspace_bytes", "bi_transpose", "bi_gemm_kmajor_bf16", "bi_gemm_kmajor_f16", "bi_attention_workspace_bytes", "bi_attention_ws_bf16", "bi_attention_decode_qkv_ws_bf16",
+    "tbik_gemm_sharded", "tbik_gemm_sharded_workspace_bytes", "tbik_gemm_sharded_pays", "bi_transpose", "bi_gemm_kmajor_bf16", "bi_gemm_kmajor_f16", "bi_attention_workspace_bytes", "bi_attention_ws_bf16", "bi_attention_decode_qkv_ws_bf16",
 )
 
 _lib = None
@@ -54,6 +54,8 @@ def lib() -> ctypes.CDLL:
     pi32 = ctypes.POINTER(ctypes.c_int)
     L.tbik_gemm_sharded_workspace_bytes.argtypes = [i32] * 6
     L.tbik_gemm_sharded_workspace_bytes.restype = sz
+    L.tbik_gemm_sharded_pays.argtypes = [i32] * 6
+    L.tbik_gemm_sharded_pays.restype = i32
     L.tbik_gemm_sharded.argtypes = [vp, i64, vp, i64, vp, i64, i32, i32, i32, i32, i32, i32, vp, vp, sz, vp]
     L.tbik_gemm_sharded.restype = i32
     L.tbik_abi_version.argtypes = []

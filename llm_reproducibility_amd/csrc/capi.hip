@@ -8,6 +8,7 @@ int gemm_dispatch(bool tree, bool f16, const void* A, int64_t lda, const void* B
                   hipStream_t stream);
 size_t gemm_workspace_bytes(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b = false);
 size_t gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, bool f16);
+bool gemm_sharded_pays(int M, int N, int K, int leaf_k, int shards, bool f16);
 bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
 int gemm_kmajor_dispatch(bool f16, const void* A, int64_t lda, bool a_kmajor, const void* B, int64_t ldb, void* C, int64_t ldc, int M,
                          int N, int K, const void* bias, hipStream_t stream);
@@ -60,7 +61,7 @@ int gemm_tree_gated_dispatch(const void* gate, const void* up, int64_t ld, const
 
 extern "C" {
 
-int tbik_abi_version(void) { return 22; }
+int tbik_abi_version(void) { return 23; }
 
 const char* tbik_error_string(int code) {
   switch (code) {
@@ -106,6 +107,10 @@ int tbik_gemm_bf16(const void* A, int64_t lda, const void* B, int64_t ldb_k, int
 
 size_t tbik_gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards, int f16) {
   return tbik::gemm_sharded_workspace_bytes(M, N, K, leaf_k, shards, f16 != 0);
+}
+
+int tbik_gemm_sharded_pays(int M, int N, int K, int leaf_k, int shards, int f16) {
+  return tbik::gemm_sharded_pays(M, N, K, leaf_k, shards, f16 != 0) ? 1 : 0;
 }
 
 int tbik_gemm_sharded(const void* A, int64_t lda, const void* B, int64_t ldb_n, void* C, int64_t ldc, int M, int N, int K, int leaf_k,

@@ -756,6 +756,25 @@ size_t gemm_sharded_workspace_bytes(int M, int N, int K, int leaf_k, int shards,
   return ranks_ok(K, leaf_k, shards) && tree_plan(M, N, K, leaf_k, f16, false, true, &tp, shards) ? tp.bytes : 0;
 }
 
+// Whether the grid of all ranks is estimated less than 5 % behind a launch per rank and the combine of their products.  It
+// is nearly always ahead, level where the ranks fill whole rounds by themselves; only a rank cut into column regions, which the one
+// grid cannot be, may finish the tiles behind its last whole round sooner (two ranks whose tiles are a few more than 256 or
+// 512).  One grid against a launch per rank, us: [2171,12288]x[12288,4096] in two 280 against 257 (estimated 303 and 277), in four
+// 273 against 304; [2043,...] in two 225 against 227, in four 239 and 240; [1403,12288]x[12288,6144] in two 291 against 267;
+// [3323,8192]x[8192,5120] in two 361 against 346, [2043,...] 206 against 219.  fp16 within 2 % of the same.
+bool gemm_sharded_pays(int M, int N, int K, int leaf_k, int shards, bool f16) {
+  TreePlan one, rank;
+  if (!ranks_ok(K, leaf_k, shards) || !tree_plan(M, N, K, leaf_k, f16, false, true, &one, shards) || one.path != PATH_SINGLE || !one.single.wide ||
+      !tree_plan(M, N, K / shards, leaf_k, f16, false, true, &rank) || rank.path != PATH_REGIONS)
+    return true;
+  int T, flb, level_k, split;
+  if (tbik_tree_params(K / shards, leaf_k, &T, &flb, &level_k) != TBIK_OK) return true;
+  const int na = rank.regions.na, lb = level_k - 1;
+  const double one_grid = wide_cost_us(M, N, K, leaf_k, f16, flb, lb, &split, shards);
+  const double a_rank = wide_cost_us(M, na, K / shards, leaf_k, f16, flb, lb, &split) + wide_cost_us(M, N - na, K / shards, leaf_k, f16, flb, lb, &split);
+  return one_grid < 1.05 * (shards * a_rank + 4.0 + (double)(shards + 1) * M * N * 2.0 / 5.0e6);
+}
+
 // What tree_plan() chose for a shape, for callers and tests that want to know (no effect on any result):
 // out[0] path (TreePath), out[1] K split (of the first region for path 2; waves per strip for path 0), out[2] columns of
 // the first region (path 2, else 0), out[3] K split of the second region (path 2, else 0), out[4] for path 2: 1 when the

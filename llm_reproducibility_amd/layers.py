@@ -119,20 +119,13 @@ class SimulatedTPRowLinear(nn.Module):
         return out.reshape(*lead, out.shape[-1])
 
     def _one_grid(self, x2: torch.Tensor) -> bool:
-        """Whether the ranks' products and the shard tree go out as one grid and its combine (ops.gemm_tree_sharded: 1.2 - 7
-        times as fast up to 500 rows, level to 1.4 times beyond); calls that the per-rank form takes in other ways, or
-        refuses, stay with it.  So do ranks that fill a round of the chip with 128x256 tiles by themselves and have a long K:
-        in launches of their own their work-groups keep step, 1 - 5 % ([2048,12288]x[12288,4096] in four ranks 247 us in one
-        grid, 234 in four, in two 220 and 221; fp16 [2048,8192]x[8192,5120] in two 224 and 213, bf16 206 and 220)."""
+        """Whether the ranks' products and the shard tree go out as one call (ops.gemm_tree_sharded: 1.2 - 7 times as fast up to
+        500 rows, level to 1.4 times beyond); calls that the per-rank form takes in other ways, or refuses, stay with it."""
         tp, K = self.tp_size, self.weight.shape[1]
         if not (2 <= tp <= 32 and tp & (tp - 1) == 0 and x2.is_cuda and x2.device == self.weight.device and x2.shape[1] == K
                 and x2.dtype == self.weight.dtype and x2.dtype in (torch.bfloat16, torch.float16) and K % (tp * self.leaf_k) == 0):
             return False
-        if self.weight.stride(1) != 1:   # the one grid would copy all of it, a rank's matmul reads its rows in place
-            return False
-        tiles = -(-x2.shape[0] // 128) * -(-self.weight.shape[0] // 256)
-        full = 256 <= tiles < 512 if x2.dtype is torch.float16 else tiles == 256
-        return not (full and self.leaf_k == 256 and K // tp >= 3072)
+        return self.weight.stride(1) == 1   # else the one grid would copy all of it, a rank's matmul reads its rows in place
 
     def forward_add_norm(self, x: torch.Tensor, residual: Optional[torch.Tensor], norm_weight: Optional[torch.Tensor], eps: float):
         """(rms_norm(forward(x) [+ residual]) * norm_weight, new residual or None): the add-RMSNorm that follows a

@@ -273,11 +273,14 @@ def _gemm_tree_sharded_impl(A: torch.Tensor, W: torch.Tensor, leaf_k: int, shard
     _require_gpu(A, W)
     M, K = A.shape
     N = W.shape[0]
+    f16 = _is_f16(A, W)
+    L = _lib.lib()
+    if not L.tbik_gemm_sharded_pays(M, N, K, leaf_k, shards, int(f16)):
+        ks = K // shards
+        return _tree_combine_impl([_gemm_tree_impl(A[:, r * ks:(r + 1) * ks], W[:, r * ks:(r + 1) * ks].t(), None, leaf_k) for r in range(shards)])
     a, lda = _rows16(A)
     w, ldw = _rows16(W)
-    f16 = _is_f16(A, W)
     C = torch.empty((M, N), device=A.device, dtype=A.dtype)
-    L = _lib.lib()
     ws_bytes = L.tbik_gemm_sharded_workspace_bytes(M, N, K, leaf_k, shards, int(f16))
     ws = torch.empty(ws_bytes, device=A.device, dtype=torch.uint8) if ws_bytes else None
     rc = L.tbik_gemm_sharded(a.data_ptr(), lda, w.data_ptr(), ldw, C.data_ptr(), C.stride(0), M, N, K, leaf_k, shards, int(f16), None,
@@ -291,7 +294,7 @@ _gemm_tree_sharded_op = torch.library.custom_op("tbik::gemm_tree_sharded", _gemm
 
 def gemm_tree_sharded(A: torch.Tensor, W: torch.Tensor, leaf_k: int, shards: int) -> torch.Tensor:
     """The products of all `shards` ranks of a row-split layer (weight W [N,K], 16 bits) and the shard tree over them: one grid
-    and one combine, the bits of a `gemm_tree` per rank and `tree_combine`.  shards: a power of two up to 32."""
+    and one combine, or, where the library expects more of it, a `gemm_tree` per rank and `tree_combine`; the same bits.  shards: a power of two up to 32."""
     if torch.compiler.is_compiling():
         return _gemm_tree_sharded_op(A, W, leaf_k, shards)
     return _gemm_tree_sharded_impl(A, W, leaf_k, shards)

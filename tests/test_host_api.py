@@ -361,3 +361,19 @@ def test_simulated_ranks_read_a_weight_of_contiguous_columns_in_place():
         across = torch.empty((6144, 2048), dtype=torch.bfloat16, device="cuda").t()
         assert SimulatedTPRowLinear(w, 4)._one_grid(x)
         assert not SimulatedTPRowLinear(across, 4)._one_grid(x)
+
+
+@pytest.mark.parametrize("f16", [0, 1])
+def test_ranks_in_one_grid_or_one_by_one_follows_the_estimate(f16):
+    """The choice between one grid of all ranks and a launch per rank turns on the estimated rounds, not on a tile count of its own: one grid
+    where the ranks fill whole rounds or are far from it, for every type alike; one by one where two ranks have a few tiles
+    more than whole rounds (each of them in column regions); and one grid for what the call itself refuses."""
+    pays = lambda M, N, K, leaf, tp: _lib.lib().tbik_gemm_sharded_pays(M, N, K, leaf, tp, f16)  # noqa: E731
+    for M in (1, 64, 500, 1024, 1900, 1921, 2048, 2560, 3072, 3968, 4096, 6144):
+        for tp in (2, 4):
+            assert pays(M, 4096, 12288, 256, tp) == 1, (M, tp)
+    for M in (2049, 2100, 2171):
+        assert pays(M, 4096, 12288, 256, 2) == 0 and pays(M, 4096, 12288, 256, 4) == 1
+    assert pays(1403, 6144, 12288, 256, 2) == 0 and pays(3323, 5120, 8192, 256, 2) == 0
+    for bad in ((4, 64, 1536, 256, 3), (4, 64, 1536, 256, 4), (4, 64, 1536, 64, 2), (0, 64, 1536, 256, 2)):
+        assert pays(*bad) == 1
