@@ -473,6 +473,12 @@ static int ring_waves(int mb, int64_t strips, int K, bool gated) {
   return best;
 }
 
+// The waves of the ring kernel's work-groups for this call, 0 where it does not take it.
+static int ring_waves_of(const StreamArgs& a, int mb, bool gated) {
+  if (a.ldx >= (1 << 22) || a.ldw >= (1 << 22)) return 0;  // the ring kernel's 32-bit byte offsets
+  return ring_waves(mb, ((int64_t)a.N + 15) / 16, a.K, gated);
+}
+
 template <int MB, bool F16, bool GATED>
 static int ring_launch(const StreamArgs& a, int waves, hipStream_t stream) {
   switch (waves) {
@@ -513,11 +519,8 @@ static int stream_launch(const StreamArgs& a, hipStream_t stream) {
   // four (two on every second CU), 41.2 us as 256 groups of six; [32,4096]x[4096,18432] 48.6 -> 35.4; lm_head (9496
   // strips, ten rounds of groups of four) is within 2 % for three, four and six.
   const int64_t strips = ((int64_t)a.N + 15) / 16;
-  const bool near_rows = a.ldx < (1 << 22) && a.ldw < (1 << 22);  // the ring kernel's 32-bit byte offsets
-  if (near_rows) {
-    const int waves = ring_waves(MB, strips, a.K, GATED);
-    if (waves) return ring_launch<MB, F16, GATED>(a, waves, stream);
-  }
+  const int waves = ring_waves_of(a, MB, GATED);
+  if (waves) return ring_launch<MB, F16, GATED>(a, waves, stream);
   // grids of many rounds do not run in rounds: the last one matters little there, the restaging of X more
   if (strips > 4 * 1024) return MB >= 3 ? stream_launch_nw<MB, WS, 8, F16, GATED>(a, stream) : stream_launch_nw<MB, WS, 4, F16, GATED>(a, stream);
   static const int cand[5] = {8, 6, 4, 3, 2};
@@ -559,14 +562,13 @@ static int stream_rows_launch(const StreamArgs& a, hipStream_t stream, const Str
 // share of CU slots that the last round of work-groups leaves used (measured: gate_up of an 8B model, 1536 strips, 41 us
 // as 384 groups of four, 37 us as 512 groups of three).  One strip per work-group restages X for every strip and is only
 // considered while X is small; two strips per work-group measured worse than either neighbour throughout.
+static double rows_fill(const StreamArgs& a, int nw) {
+  const int64_t groups = (((int64_t)a.N + 15) / 16 + nw - 1) / nw;
+  return (double)groups / (double)(((groups + 255) / 256) * 256);
+}
 static int stream_rows_waves(const StreamArgs& a) {
-  const int64_t strips = ((int64_t)a.N + 15) / 16;
-  auto score = [&](int nw, double weight) {
-    const int64_t groups = (strips + nw - 1) / nw;
-    return weight * (double)groups / (double)(((groups + 255) / 256) * 256);
-  };
-  const double s3 = score(3, 1.0), s4 = score(4, 0.98);
-  const double s1 = a.M * a.K <= ROWS_MAX_ELEMS / 4 ? score(1, 0.95) : 0.0;
+  const double s3 = rows_fill(a, 3), s4 = 0.98 * rows_fill(a, 4);
+  const double s1 = a.M * a.K <= ROWS_MAX_ELEMS / 4 ? 0.95 * rows_fill(a, 1) : 0.0;
   if (s1 > s3 && s1 > s4) return 1;
   return s3 >= s4 ? 3 : 4;
 }
@@ -598,13 +600,25 @@ int gemm_single_acc_stream_norm_launch(const StreamArgs& a, const StreamNormArgs
 // while X is small; it loses from a few thousand elements of X on -- [4,4096] x [4096,6144] 16.7 against 13.0 us,
 // [2,8192] x [8192,5120] 29.2 against 22.8, [1,12288] x [12288,4096] 38.3 against 29.9, [8,2048] x [2048,4096] 10.1
 // against 7.2 -- the earlier the more strips there are.
+// From 10240 columns on the ring kernel, which is ahead of both, takes the call where it can (K a multiple of 128, from 1024 on).  Of what
+// it leaves, the whole-X kernel keeps a K that is no multiple of 128 and rows too far apart for the ring; of a short K (512 .. 896) only
+// more than 65536 columns, where the windowed kernel makes groups of four whatever they fill, and only if its own groups of three
+// or four fill their rounds: windowed against whole-X, [4,896] x [896,81920] 38.8 and 34.5 us, [16,896] x [896,81920] 41.0 and 37.1 (all slots
+// used), [4,896] x [896,128256] 55.2 and 50.0 (98 %), [4,896] x [896,151936] 65.1 and 60.2 (95 %; 16 rows of 768 58.0 and 60.0), but
+// [8,896] x [896,100000] 47.8 and 53.2 (90 %), [8,640] x [640,65552] 21.6 and 24.3 (89 %).  Up to 65536 columns the windowed kernel is level up to two
+// rows and ahead from four on ([4,640] x [640,12288] 6.2 against 6.5, [8,768] x [768,24576] 10.9 and 11.3, [16,512] x [512,51200]
+// 13.8 and 19.4).
 static bool stream_rows_pays(const StreamArgs& a) {
 #ifdef TBIK_STREAM_ROWS_ALWAYS
   return true;
 #endif
   const int64_t xe = (int64_t)a.M * a.K;
   if (a.K < 512) return true;   // shorter than one window: nothing to stage behind
-  if (a.N >= 10240 && a.K % ring::BK != 0) return true;   // (the ring kernel is ahead of both, but does not take it)
+  if (a.N >= 10240 && !ring_waves_of(a, (a.M + 15) / 16, false)) {
+    if (a.K % ring::BK != 0 || a.K >= 1024) return true;
+    const int nw = stream_rows_waves(a);
+    if (a.N > 65536 && nw > 1 && rows_fill(a, nw) >= (a.M <= 8 ? 0.93 : 0.97)) return true;
+  }
   return xe <= 2048 || (xe <= 4096 && a.N <= 4096) || (xe <= 8192 && a.N <= 3072);
 }
 

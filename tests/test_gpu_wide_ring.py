@@ -38,3 +38,18 @@ def test_gated_widths(inter, K):
         x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
         both = torch.cat([ops.bi_gemm(x, W[i:i + 1024].t(), None) for i in range(0, 2 * inter, 1024)], dim=1)
         assert torch.equal(ops.gemm_silu_mul(x, W), ops.bi_silu_mul(both))
+
+
+# a short K that the ring kernel leaves on very wide matrices: both sides of the rows, the columns and the fill of the rounds from which on
+# all of X is staged at once, a last group that ends early
+@pytest.mark.parametrize("N", [65536, 65552, 81920, 100000, 128255])
+@pytest.mark.parametrize("K", [512, 896])
+def test_short_k_of_a_very_wide_matrix(N, K):
+    print("case short k", N, K, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    W = (torch.randn(N, K, device="cuda", generator=g) * 0.05).to(torch.bfloat16)
+    for M in (3, 8, 9):
+        x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+        got = ops.bi_gemm(x, W.t(), None)
+        want = torch.cat([ops.bi_gemm(x, W[i:i + 2048].t(), None) for i in range(0, N, 2048)], dim=1)
+        assert torch.equal(got, want)
