@@ -17,8 +17,14 @@
 // of N = 64 .. 51200 and K = 256 .. 32768 8 % faster on average, 8 % of them more than 4 % slower: a few rows on tiny
 // matrices (0.4 .. 1 us) and N = 16384 and more on a K cut in two ([32,12288]x[12288,16384] 80 -> 97).
 //
-// The weights are loaded with the non-temporal hint (dma16_once): [16,25600]x[25600,5120] 54.5 -> 48.4 us (5.4 TB/s),
-// [32,12288]x[12288,4096] 24.9 -> 22.7, [8,4096]x[4096,4096] 11.8 -> 10.9; at 64 rows level.
+// Weights of 64 MB and more are loaded with the non-temporal hint (dma16_once) up to 32 rows, as a model's are in decode: from
+// memory on every call.  Without it -> with it, us, weights from memory / the same ones again and again / copied into place just before:
+//   [16,25600]x[25600,5120] 52.9 -> 47.4 / 44.1 -> 46.2 / 54.2 -> 59.8;  [16,12288]x[12288,4096] 24.1 -> 21.9 / 20.4 -> 20.0 / 22.4 -> 22.1;
+//   [32,12288]x[12288,4096] 25.1 -> 22.9 / 21.6 -> 21.3 / 24.0 -> 23.8;  [32,8192]x[8192,5120] 20.7 -> 19.6 / 18.7 -> 18.2 / 21.0 -> 20.5.
+// It is off where it gives little from memory or takes more from weights that the 256 MB cache holds: smaller ones ([8,4096]x[4096,4096]
+// 11.3 -> 10.9 / 8.4 -> 8.7 / 13.4 -> 13.3) and more rows ([49,25600]x[25600,5120] 58.7 -> 58.3 / 55.9 -> 56.4 / 66.2 -> 64.5, written in place
+// just before 64.0 -> 72.7; [64,8192]x[8192,5120] 25.4 -> 25.6 / 22.0 -> 21.9 / 24.5 -> 31.6; [49,12288]x[12288,4096] 26.5 -> 24.5 / 23.2 ->
+// 23.1 / 25.5 -> 30.8).
 //
 // The arithmetic per element is that of gemm_tiled.hip: one chain of 16x16x32 MFMAs over ascending k per leaf, one
 // rounding per leaf, left to right over the leaves of a group, adjacent pairs above, every node rounded; the whole tree
@@ -48,8 +54,8 @@ struct Shape {
 };
 }  // namespace few
 
-// MT: 16-row tiles; NW: waves, 32 columns each; LS: slices per leaf
-template <int MT, int NW, int LS, bool F16>
+// MT: 16-row tiles; NW: waves, 32 columns each; LS: slices per leaf; ONCE: weights with the non-temporal hint
+template <int MT, int NW, int LS, bool F16, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void gemm_tree_few_kernel(const WideArgs p) {
   using namespace few;
   using Num = Num16<F16>;
@@ -88,7 +94,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_tree_few_kernel(const WideArgs p
 #pragma unroll
     for (int i = 0; i < XDMA; i++) dma16(base + dst[i], voff[i], xbase + (int64_t)s * (BK * 2));
 #pragma unroll
-    for (int i = XDMA; i < NDMA; i++) dma16_once(base + dst[i], voff[i], wbase + (int64_t)s * (BK * 2));
+    for (int i = XDMA; i < NDMA; i++) {
+      if (ONCE) dma16_once(base + dst[i], voff[i], wbase + (int64_t)s * (BK * 2));
+      else dma16(base + dst[i], voff[i], wbase + (int64_t)s * (BK * 2));
+    }
   };
 
   const int frow = lane & 15, fchk = lane >> 4;
@@ -203,27 +212,28 @@ __global__ __launch_bounds__(NW * 64) void gemm_tree_few_kernel(const WideArgs p
   }
 }
 
-template <int MT, int NW, int LS, bool F16>
+template <int MT, int NW, int LS, bool F16, bool ONCE>
 static int few_launch(const WideArgs& a, int split, hipStream_t stream) {
   using namespace few;
   using S = Shape<MT, NW>;
   constexpr int smem = S::NSLOT * S::STAGE_BYTES;
   static_assert(smem <= 160 * 1024 && (S::NSLOT - 1) * S::NDMA < 64, "ring does not fit the LDS or the wait counter");
   static std::atomic<uint64_t> done{0};
-  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tree_few_kernel<MT, NW, LS, F16>), smem, done);
+  hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(gemm_tree_few_kernel<MT, NW, LS, F16, ONCE>), smem, done);
   if (e != hipSuccess) return hip_code(e);
   const unsigned tiles = (unsigned)((a.N + S::BN - 1) / S::BN);
-  hipLaunchKernelGGL((gemm_tree_few_kernel<MT, NW, LS, F16>), dim3(tiles, (unsigned)split), dim3(NW * 64), smem, stream, a);
+  hipLaunchKernelGGL((gemm_tree_few_kernel<MT, NW, LS, F16, ONCE>), dim3(tiles, (unsigned)split), dim3(NW * 64), smem, stream, a);
   return hip_code(hipGetLastError());
 }
 
 template <int LS, bool F16>
 static int few_by_shape(const WideArgs& a, int waves, int split, hipStream_t stream) {
+  const bool once = (int64_t)a.N * a.K * split * 2 >= 64000000;
   auto rows = [&](auto nw) {
     constexpr int NW = decltype(nw)::value;
-    if (a.M <= 16) return few_launch<1, NW, LS, F16>(a, split, stream);
-    if (a.M <= 32) return few_launch<2, NW, LS, F16>(a, split, stream);
-    return few_launch<4, NW, LS, F16>(a, split, stream);
+    if (a.M <= 16) return once ? few_launch<1, NW, LS, F16, true>(a, split, stream) : few_launch<1, NW, LS, F16, false>(a, split, stream);
+    if (a.M <= 32) return once ? few_launch<2, NW, LS, F16, true>(a, split, stream) : few_launch<2, NW, LS, F16, false>(a, split, stream);
+    return few_launch<4, NW, LS, F16, false>(a, split, stream);
   };
   switch (waves) {
     case 2: return rows(std::integral_constant<int, 2>{});

@@ -49,3 +49,18 @@ def test_three_levels_inside_a_shard(dev, N, K):
     for M in (6, 25, 61):
         print("case few levels", M, N, K, flush=True)
         assert torch.equal(matmul_tp_persistent(x[:M], w.t()), big[:M])
+
+
+# both sides of the size from which on the weights are loaded with the non-temporal hint (64 MB), which the last rows of a matrix do too
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("leaf", [128, 256])
+@pytest.mark.parametrize("N", [3906, 3907])
+def test_weights_around_the_size_of_the_hint(dev, N, leaf, f16):
+    print("case few hint", N, leaf, f16, flush=True)
+    dt, K = torch.float16 if f16 else torch.bfloat16, 8192
+    gen = torch.Generator(device=dev).manual_seed(N)
+    x = torch.randn((300, K), generator=gen, device=dev).to(dt)
+    w = (torch.randn((N, K), generator=gen, device=dev) * 0.02).to(dt)
+    big = matmul_tp_persistent(x, w.t(), leaf_k=leaf)
+    for M in (5, 16, 17, 32, 33, 64):
+        assert torch.equal(matmul_tp_persistent(x[:M], w.t(), leaf_k=leaf), big[:M])
