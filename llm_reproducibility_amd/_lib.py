@@ -34,6 +34,12 @@ EXPORTS = (
 _lib = None
 
 
+def fast_built_for() -> str:
+    """What the host extension (csrc_host/fast_ops.cpp) is compiled against, as it has to say of itself to be used."""
+    import torch
+    return f"tbik ABI {ABI_VERSION}, torch {torch.__version__}"
+
+
 class TbikError(RuntimeError):
     def __init__(self, code: int, where: str):
         self.code = code

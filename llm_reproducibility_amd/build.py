@@ -1,9 +1,9 @@
-"""Builds libtbik_hip.so (the gfx950 kernels + their C ABI) in-tree with hipcc, beside it _fast.so (a Python extension with the
-common calls of the row-wise operators, host code only) and measure/libtbik_measure.so (the benchmark's machine probes,
+"""Builds libtbik_hip.so (the gfx950 kernels + their C ABI) in-tree with hipcc, beside it _fast.<python tag>.so (a Python extension
+with the common calls of the row-wise operators, host code only) and measure/libtbik_measure.so (the benchmark's machine probes,
 which are not part of the product library).
 
     python -m llm_reproducibility_amd.build            # compile every source, link
-    python -m llm_reproducibility_amd.build --if-stale # only when a source is newer than the library
+    python -m llm_reproducibility_amd.build --if-stale # only when a source is newer than what is built, or torch is another
 
 hipcc cross-compiles for gfx950 without a GPU, so this runs anywhere ROCm is installed.
 """
@@ -15,13 +15,16 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
+
+from . import _lib
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libtbik_hip.so")
 FAST_SRC = os.path.join(PKG_DIR, "csrc_host", "fast_ops.cpp")
-FAST_PATH = os.path.join(PKG_DIR, "_fast.so")
+FAST_PATH = os.path.join(PKG_DIR, "_fast" + sysconfig.get_config_var("EXT_SUFFIX"))
 MEASURE_DIR = os.path.join(PKG_DIR, "measure")
 MEASURE_LIB_PATH = os.path.join(MEASURE_DIR, "libtbik_measure.so")
 OBJ_DIR = os.path.join(PKG_DIR, "build")
@@ -65,6 +68,9 @@ def is_stale() -> bool:
     built = (LIB_PATH, MEASURE_LIB_PATH, FAST_PATH)
     if not all(os.path.exists(p) for p in built):
         return True
+    with open(FAST_PATH, "rb") as f:
+        if _lib.fast_built_for().encode() + b"\0" not in f.read():   # another torch, or another ABI of the library
+            return True
     t = min(os.path.getmtime(p) for p in built)
     return any(os.path.getmtime(d) > t for d in _deps())
 
@@ -95,15 +101,13 @@ def _link(objs, path: str) -> None:
 
 
 def _compile_fast() -> str:
-    import sysconfig
-
     import torch
     from torch.utils import cpp_extension
 
     obj = os.path.join(OBJ_DIR, "fast_ops.o")
     includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[a for p in includes for a in ("-isystem", p)],
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTBIK_BUILT_FOR="{_lib.fast_built_for()}"', *[a for p in includes for a in ("-isystem", p)],
            "-c", FAST_SRC, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

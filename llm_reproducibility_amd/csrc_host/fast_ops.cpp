@@ -192,4 +192,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fast", "common calls of the row-w
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fast(void) { return PyModule_Create(&module); }
+// built_for (TBIK_BUILT_FOR, from build.py): the library's ABI and the torch this was compiled against; ops.py compares it with what
+// it runs with before the first call
+PyMODINIT_FUNC PyInit__fast(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", TBIK_BUILT_FOR) != 0) Py_CLEAR(m);
+  return m;
+}

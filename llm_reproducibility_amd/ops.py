@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import warnings
 from typing import List, Optional
 
 import torch
@@ -35,17 +36,31 @@ def _stream(t: torch.Tensor) -> int:
 _fast_module = None
 
 
+class _NoFast:
+    """Stands in for the extension where there is none to use: every call goes the way written out here."""
+    rms_norm = add_rms_norm = silu_mul = mean_last = log_softmax = staticmethod(lambda *args: None)
+
+
 def _fast():
     """The extension with the common calls of the row-wise operators (csrc_host/fast_ops.cpp): each gives the result, or None
-    for a call that is not the plain case, which then goes the way written out here."""
+    for a call that is not the plain case, which then goes the way written out here.  The same kernels run either way, so
+    one that is missing, or built for another library or torch, costs host time only: a warning, once."""
     global _fast_module
     if _fast_module is None:
         _lib.lib()   # a missing library is reported as such
+        why = None
         try:
             from . import _fast as module
         except ImportError as e:
-            raise RuntimeError("llm_reproducibility_amd/_fast.so is missing or does not load: run "
-                               "`python -m llm_reproducibility_amd.build`") from e
+            why = f"does not load ({e})"
+        else:
+            built_for = getattr(module, "built_for", "nothing it tells")
+            if built_for != _lib.fast_built_for():
+                why = f"was built for {built_for}, this is {_lib.fast_built_for()}"
+        if why:
+            warnings.warn(f"the host extension llm_reproducibility_amd._fast {why}: row-wise operators take a slower way to the same "
+                          "kernels; run `python -m llm_reproducibility_amd.build`", RuntimeWarning, stacklevel=2)
+            module = _NoFast
         _fast_module = module
     return _fast_module
 

@@ -377,3 +377,34 @@ def test_ranks_in_one_grid_or_one_by_one_follows_the_estimate(f16):
     assert pays(1403, 6144, 12288, 256, 2) == 0 and pays(3323, 5120, 8192, 256, 2) == 0
     for bad in ((4, 64, 1536, 256, 3), (4, 64, 1536, 256, 4), (4, 64, 1536, 64, 2), (0, 64, 1536, 256, 2)):
         assert pays(*bad) == 1
+
+
+def test_host_extension_is_for_this_library_and_torch(monkeypatch):
+    """The extension says what it was built for.  Without one, or with one for another library or torch, a warning and the way
+    written out in ops.py, which needs the library alone."""
+    import sys
+    import types
+    import warnings
+    from llm_reproducibility_amd import build
+    name = pkg.__name__ + "._fast"
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert ops._fast().built_for == _lib.fast_built_for()
+    monkeypatch.setattr(build, "_deps", lambda: [])              # whatever the sources' times
+    assert not build.is_stale() and f"cpython-{sys.version_info.major}{sys.version_info.minor}" in os.path.basename(build.FAST_PATH)
+    other = types.ModuleType(name)
+    older = types.ModuleType(name)
+    older.built_for = _lib.fast_built_for().replace(f"ABI {_lib.ABI_VERSION}", "ABI 1")
+    for module in (None, other, older):
+        monkeypatch.setattr(ops, "_fast_module", None)
+        monkeypatch.setitem(sys.modules, name, module)
+        monkeypatch.delattr(pkg, "_fast", raising=False)
+        if module is not None:
+            monkeypatch.setattr(pkg, "_fast", module, raising=False)
+        with pytest.warns(RuntimeWarning, match="host extension"):
+            fast = ops._fast()
+        assert fast is ops._fast() and fast.rms_norm(None, None, 0.0) is None and fast.mean_last(None, True) is None
+        with pytest.raises(RuntimeError, match="GPU only"):      # the long way's refusal, not the extension's absence
+            ops.bi_rmsnorm(torch.zeros((2, 64), dtype=torch.bfloat16), None, 1e-6)
+    monkeypatch.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)
+    assert build.is_stale()
