@@ -987,10 +987,23 @@ static void group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int
     else TBIK_ATTN_GROUP(1, true, 0, ALL_CHUNKS);
   } else {
     constexpr int LOADERS = G == 1 ? 1280 : G == 2 ? 1024 : 512, SINGLE = G == 4 ? 768 : 0, QB = G == 8 ? 1 : 2;
-    if (groups <= 512) TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS);
-    else if (groups <= LOADERS) TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS, 1);
-    else if (groups <= SINGLE) TBIK_ATTN_GROUP(1, false, 0, ALL_CHUNKS);
-    else TBIK_ATTN_GROUP(QB, false, 0, ALL_CHUNKS);
+    if (groups <= 512) {
+      TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS);
+      return;
+    }
+    if constexpr (LOADERS > 512) {
+      if (groups <= LOADERS) {
+        TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS, 1);
+        return;
+      }
+    }
+    if constexpr (SINGLE > 0) {
+      if (groups <= SINGLE) {
+        TBIK_ATTN_GROUP(1, false, 0, ALL_CHUNKS);
+        return;
+      }
+    }
+    TBIK_ATTN_GROUP(QB, false, 0, ALL_CHUNKS);
   }
 #undef TBIK_ATTN_GROUP
 }
