@@ -57,15 +57,19 @@ int tbik_tree_params(int K, int leaf_k, int* T, int* flb, int* level_k);
  *   B: element (k,n) at B[k*ldb_k + n*ldb_n], as the reference passes B's strides to its kernel
  *      (src/tbik/tree_based_matmul.py:259-264).  ldb_k == 1 (the nn.Linear weight [N,K], i.e. weight.t()) is the
  *      native layout of every kernel; ldb_n == 1 (row-major [K,N], what simple_matmul.py:11-14 hands over) is
- *      consumed in place by the tiled kernels, which transpose 8x8 blocks in registers on the way to LDS -- same
- *      MFMA chain, same bits, no copy (the large-M pipelines are built for [N,K] only: measured on MI355X,
- *      [M,12288] x [12288,4096] row-major takes 60 / 762 us at M = 128 / 2048 against 32 / 200 us for the [N,K]
- *      form, so a caller with many rows should hand over [N,K]; the Python wrappers repack, with bi_transpose,
- *      where that is the faster way).  The contiguous dimension's partner stride must be a multiple of 8 elements;
- *      neither stride equal to 1 returns TBIK_ERR_UNSUPPORTED.
+ *      consumed in place, same MFMA chain, same bits, no copy: with leaves of 256 and N a multiple of 8 on 128x128 tiles
+ *      that read it K-major through transposing LDS reads, else on 64-row tiles that transpose 8x8 blocks in registers on
+ *      the way to LDS.  The kernels of many rows are built for [N,K] only (measured on MI355X, [M,12288] x [12288,4096]
+ *      row-major takes 25 / 30 / 132 / 354 us at M = 16 / 128 / 700 / 2048 against 23 / 29 / 103 / 200 us for the [N,K]
+ *      form), so a caller with many rows should hand over [N,K]; tbik_gemm_rowmajor_b_pays says where, and the Python
+ *      wrappers repack there, with bi_transpose.  The contiguous dimension's partner stride must be a multiple of 8
+ *      elements; neither stride equal to 1 returns TBIK_ERR_UNSUPPORTED.
  *      For ldb_n == 1 the workspace size is tbik_gemm_workspace_bytes_rowmajor_b(M,N,K,leaf_k,f16).
  *   C: element (m,n) at C[m*ldc + n]
- *   workspace: at least tbik_gemm_workspace_bytes(M,N,K,leaf_k) bytes, 16-byte aligned (may be NULL when 0)
+ *   workspace: at least tbik_gemm_workspace_bytes(M,N,K,leaf_k) bytes, 16-byte aligned (may be NULL when 0); fewer return
+ *      TBIK_ERR_WORKSPACE before anything is launched.  A row-major B alone has a second way: with fewer bytes than its
+ *      size above the 128x128 tiles give way to the 64-row tiles, which need less or none (and take longer), and only what
+ *      does not suffice for those either is refused.
  * Replaces: matmul_tp_persistent + matmul_kernel_tp_persistent,
  *           src/tbik/tree_based_matmul.py:190-277 and :50-187.
  */
@@ -111,7 +115,7 @@ int tbik_gemm_plan_info(int M, int N, int K, int leaf_k, int f16, int rowmajor_b
  * harnesses that forbid hipMalloc.  Same arguments (without the workspace), same kernels, same bits; the workspace is
  * a fixed array of TBIK_STATIC_SCRATCH_BYTES inside the library, one copy per GPU, held until the process ends.  A
  * problem whose tbik_gemm_workspace_bytes() exceeds that size returns TBIK_ERR_SCRATCH_LIMIT before anything is
- * launched (decode- and mid-sized batches fit, and so does the 2048-row benchmark shape, whose two parked tree levels
+ * launched (a row-major B only if the 64-row tiles, its second way, exceed it as well; decode- and mid-sized batches fit, and so does the 2048-row benchmark shape, whose two parked tree levels
  * are 32 MiB; the 4096-row shapes of the 32B configuration do not).  The call allocates and frees
  * nothing.  The first call on a device resolves the array's device address (hipGetSymbolAddress): make that call
  * outside a graph capture.  Every call on a GPU uses that GPU's one array, whose contents are scratch (written

@@ -866,8 +866,9 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
     // large problems whose K is a whole number of 64-wide slices take the one-wave-per-SIMD pipeline (same MFMA
     // chain per element, so the same bits as the tiled kernel)
     const int64_t wide_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
-    // 33..128 rows: one row of 128-row tiles whose width balances the grid, when such a grid exists (same MFMA chain
-    // per element again)
+    // 49..128 rows (33..128 of fewer than 4096 columns or a K that is no multiple of 128, 65..128 of more than 8192): one row of
+    // 128-row tiles whose width balances the grid, when such a grid exists (same MFMA chain per element again); the fewer
+    // rows go to the ring kernel, `ring` below
     const bool narrow_n = N < 4096;   // no one-row grid of at least 128 tiles, whatever their width
     // fp16 takes all of these since they were built for it: [128,12288]x[12288,4096] 117 -> 49 us, [512,4096]x[4096,6144] 61 -> 34,
     // [2048,4096]x[4096,24576] 492 -> 296, [4096,12288]x[12288,4096] 463 -> 275 against the tiled kernel.

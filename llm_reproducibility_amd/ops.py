@@ -188,10 +188,13 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
 #   single-accumulator mm: in place cannot cut K, so a call takes as long as one chain per round of 512 work-groups (two on
 #     a CU), whatever it fills them with; narrow matrices are repacked (4096 x 4096: 88 against 27 at one row, 77 against 34 at
 #     64), wide ones not while they are one round (12288 x 16384: 220 against 273 at 64 rows, 248 against 318 at 256; 4096 x
-#     24576: 93 against 123 at 128 rows, 158 against 138 at 160).  K, the type (fp16 has slower tiles above 64 rows:
-#     12288 x 10240 at 256 rows 182 against 244, bf16 201 against 201) and the rounds move the line, so both times are estimated.
-#     Over 4,862 points of 1 .. 3072 rows, K = 512 .. 25600, N = 512 .. 151936 in both types the choice is 0.25 % from the
-#     better of the two on average and 23 % at worst.
+#     24576: 93 against 123 at 128 rows, 158 against 138 at 160).  K, the rounds and, for a K that is no multiple of 64, the type (fp16
+#     has the large tiles of bf16 for whole slices only) move the line, so both times are estimated.
+#   Both estimates are of whole column tiles (N a multiple of 128, of 64 up to 16 rows).  Of the operands that come here, 1 .. 3072
+#     rows, K = 512 .. 25600, N = 512 .. 48000 in both types: on whole tiles the choice is 0.5 % from the better of the two on average
+#     and 12 % at worst for the mm (62 points), 3 % and 32 % for the tree (33).  A last tile that is not whole costs the 64-row
+#     tiles two to four times the time, which the estimates do not know: where such an operand stays in place (118 of 655 points
+#     of the mm, 119 of 171 of the tree) a repack would nearly always be ahead, 1.7 times on average.
 _TREE_IN_PLACE_MACS = 416 * 2048 * 1536
 
 
