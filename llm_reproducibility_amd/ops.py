@@ -194,7 +194,7 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
 #     rows, K = 512 .. 25600, N = 512 .. 48000 in both types: on whole tiles the choice is 0.5 % from the better of the two on average
 #     and 12 % at worst for the mm (62 points), 3 % and 32 % for the tree (33).  A last tile that is not whole costs the 64-row
 #     tiles two to four times the time, which the estimates do not know: where such an operand stays in place (118 of 655 points
-#     of the mm, 119 of 171 of the tree) a repack would nearly always be ahead, 1.7 times on average.
+#     of the mm, 119 of 171 of the tree) a repack would nearly always be ahead, 1.8 times on average.
 _TREE_IN_PLACE_MACS = 416 * 2048 * 1536
 
 
