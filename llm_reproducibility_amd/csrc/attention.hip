@@ -2,8 +2,8 @@
 // lanes {j, j+16, j+32, j+48} of one wavefront; three kernels differ in what else the wavefront and its work-group hold:
 //   attention_kernel        one wavefront per (16 consecutive queries of a sequence, query head), operands from global
 //                           memory (any cache length);
-//   attention_group_kernel  the G query heads of a KV head as the G wavefronts of a work-group, K/V tiles staged in LDS
-//                           once for all of them (prefill and chunked prefill);
+//   attention_group_kernel  the G query heads of a KV head times one or two blocks of 16 queries in the wavefronts of a
+//                           work-group, keys and values staged in LDS once for all of them (prefill and chunked prefill);
 //   attention_decode_kernel the few new queries of a sequence times the G heads as the 16 rows of ONE tile, the output
 //                           channels split over four wavefronts, four more wavefronts bringing the tiles in (decode).
 //
@@ -44,7 +44,7 @@ struct AttnArgs {
 
 constexpr int HD = 128;
 constexpr int CHUNK_TILES = 16;           // key tiles per chunk: 512 keys
-constexpr float kNoKey = -__FLT_MAX__;    // reference point of an empty state: no finite score lies below it (see softmax_tile)
+constexpr float kNoKey = -__FLT_MAX__;    // reference point of an empty state: no finite score lies below it (see move_reference)
 
 // Where the chunks of a row go when different work-groups compute them (SPLIT): slot (sequence * q_rows + query) *
 // q_heads + head of [nchunks] states.  q_rows are the queries per sequence that the kernels' tiles have room for and not
@@ -69,61 +69,67 @@ struct QkvArgs {
   float eps;
 };
 
-// One online-softmax update of a query row for a tile of 32 keys, shared by all kernels of this file (one body: the same
-// bits).  Lane (j, g) holds the scores of query j for keys k0 + 16u + 4g + i in s[u][i]; on return p holds the four packed
-// probability pairs of the lane (the B operand of the P*V MFMA) and alpha the factor for the output accumulators of the
-// row (exactly 1.0 when the reference point of the exponentials did not move).  MASK: apply the causal mask (needed only for tiles that
-// reach beyond some row's horizon; the values are the same either way for the others).
-// 2^x is the hardware exponential: the arguments are <= 0, and a result below 2^-126 is dropped, which neither the
-// denominator (>= 1: the row's maximum contributes 2^0) nor a bf16 probability can show.
-template <bool MASK>
-__device__ __forceinline__ void softmax_tile(const f32x4 (&s)[2], int k0, int g, int qpos, float scale_log2, float& m, float& l,
-                                             float& alpha, bf16x8& p) {
-  // every product and sum below is rounded on its own, except where a fused multiply-add is written out: left to the
-  // compiler, a multiplication could be fused with the next addition in one instantiation and not in another, and the
-  // kernels would no longer agree bit for bit
-#pragma clang fp contract(off)
-  float sv[8];
+// One online-softmax update of a query row for a tile of 32 keys, in the pieces that the kernels of this file put together (the
+// same bits in all).  Row 4g + i of the 16-row sub-tile u of a key tile is key 8g + 4u + i (key_row), so lane (j, g) holds the
+// scores of query j for the eight consecutive keys k0 + 8g .. +7 in s[0], s[1], and its probabilities are the B operand of a
+// P*V MFMA whose A operand is eight consecutive keys of a channel: 16 bytes of the V^T cache as they lie.
+// Every product and sum below is rounded on its own, except where a fused multiply-add is written out: left to the
+// compiler, a multiplication could be fused with the next addition in one instantiation and not in another, and the
+// kernels would no longer agree bit for bit.
+__device__ __forceinline__ int key_row(int u, int r) { return 8 * (r >> 2) + 4 * u + (r & 3); }
+
+// the causal mask (needed only for tiles that reach beyond some row's horizon; the others' values do not change)
+__device__ __forceinline__ void mask_scores(f32x4 (&s)[2], int k0, int g, int qpos) {
 #pragma unroll
   for (int u = 0; u < 2; u++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      float v = s[u][i];
-      if (MASK) v = (k0 + 16 * u + 4 * g + i <= qpos) ? v : -INFINITY;
-      sv[4 * u + i] = v;
-    }
-  // the maximum is taken over the raw scores and scaled once (the scale is positive and rounding is monotonic, so this
-  // is the maximum of the scaled scores); 2^(score * scale - maximum) is then one fused multiply-add and one exponential
-  // (NaN-propagating maxima: a NaN score makes the row NaN, as it would through the sum)
-  float tmax = LaneMaxNaN::f(LaneMaxNaN::f(LaneMaxNaN::f(sv[0], sv[1]), LaneMaxNaN::f(sv[2], sv[3])),
-                             LaneMaxNaN::f(LaneMaxNaN::f(sv[4], sv[5]), LaneMaxNaN::f(sv[6], sv[7])));
-  tmax = xor_step<16, LaneMaxNaN>(tmax);
+    for (int i = 0; i < 4; i++) s[u][i] = (k0 + 8 * g + 4 * u + i <= qpos) ? s[u][i] : -INFINITY;
+}
+// The largest of the lane's eight raw scores; scaled, it is the largest of the scaled ones (the scale is positive and
+// rounding is monotonic).  NaN-propagating: a NaN score makes the row NaN, as it would through the sum.
+__device__ __forceinline__ float lane_max(const f32x4 (&s)[2]) {
+  return LaneMaxNaN::f(LaneMaxNaN::f(LaneMaxNaN::f(s[0][0], s[0][1]), LaneMaxNaN::f(s[0][2], s[0][3])),
+                       LaneMaxNaN::f(LaneMaxNaN::f(s[1][0], s[1][1]), LaneMaxNaN::f(s[1][2], s[1][3])));
+}
+// The reference point of the exponentials moves lazily: only when a score of this tile exceeds it by more than 2^kLazy
+// (probabilities then stay below 2^kLazy instead of 1: no loss in fp32 sums or in the relative precision of a bf16
+// probability, and out = o / l is the same quotient).  After the first tiles of a chunk it practically never moves.  The rule
+// looks at a row's own scores in its fixed tile order only, so it is the same for prefill, chunked prefill and decode; and
+// while no lane of a wavefront has a score that far up (score_exceeds), move_reference would leave every row where it is
+// and return exactly 1.0 -- the grouped kernel asks that first and skips the exchange between a row's lanes, the
+// exponential and the rescale.
+// A row's first key of a chunk moves it from kNoKey to a score; in a tile that lies entirely behind the horizon it stays
+// where it is (kNoKey is finite, so kNoKey - kNoKey is 0 and not NaN) and every probability is 2^-inf = 0.
+constexpr float kLazy = 8.0f;
+__device__ __forceinline__ bool score_exceeds(float lmax, float scale_log2, float m) {
+#pragma clang fp contract(off)
+  return lmax * scale_log2 > m + kLazy;
+}
+// returns the factor for the row's accumulators and (applied here) denominator
+__device__ __forceinline__ float move_reference(float lmax, float scale_log2, float& m, float& l) {
+#pragma clang fp contract(off)
+  float tmax = xor_step<16, LaneMaxNaN>(lmax);
   tmax = xor_step<32, LaneMaxNaN>(tmax);
-  // The reference point of the exponentials moves lazily: only when a score of this tile exceeds it by more than 2^kLazy
-  // (probabilities then stay below 2^kLazy instead of 1: no loss in fp32 sums or in the relative precision of a bf16
-  // probability, and out = o / l is the same quotient).  After the first tiles of a row it practically never moves, so
-  // the rescale of the output accumulators is skipped for whole rows of tiles.  The rule looks at a row's own scores
-  // in its fixed tile order only, so it is the same for prefill, chunked prefill and decode.
-  // A row's first key of a chunk moves it from kNoKey to a score; in a tile that lies entirely behind the horizon it stays
-  // where it is (kNoKey is finite, so kNoKey - kNoKey is 0 and not NaN) and every probability is 2^-inf = 0.
-  constexpr float kLazy = 8.0f;
   const float cand = tmax * scale_log2;
   const float m_new = cand > m + kLazy ? cand : m;
-  alpha = __builtin_amdgcn_exp2f(m - m_new);        // exactly 1.0 when the reference point did not move
+  const float alpha = __builtin_amdgcn_exp2f(m - m_new);        // exactly 1.0 when the reference point did not move
+  m = m_new;
+  l = l * alpha;
+  return alpha;
+}
+// The lane's eight probabilities, 2^(score * scale - m) as one fused multiply-add and one hardware exponential each (the
+// arguments are <= kLazy, and a result below 2^-126 is dropped, which neither the denominator nor a bf16 probability can
+// show).  The denominator is kept per lane and summed over a row's four lanes where a chunk ends (row_sum).
+__device__ __forceinline__ bf16x8 probabilities(const f32x4 (&s)[2], float scale_log2, float m, float& l) {
+#pragma clang fp contract(off)
   float pv[8];
 #pragma unroll
-  for (int e = 0; e < 8; e++) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[e], scale_log2, -m_new));
-  float psum = pv[0];
-#pragma unroll
-  for (int e = 1; e < 8; e++) psum += pv[e];
-  psum = xor_step<16, LaneSum>(psum);
-  psum = xor_step<32, LaneSum>(psum);
-  l = __builtin_fmaf(l, alpha, psum);
-  m = m_new;
-  // P as the MFMA "B" operand: k slots 0..3 = keys k0+4g.., slots 4..7 = keys k0+16+4g..
-  p = __builtin_bit_cast(bf16x8, u32x4{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3]), pack_bf16x2(pv[4], pv[5]),
-                                       pack_bf16x2(pv[6], pv[7])});
+  for (int e = 0; e < 8; e++) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e >> 2][e & 3], scale_log2, -m));
+  l = l + (((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7])));
+  return __builtin_bit_cast(bf16x8, u32x4{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3]), pack_bf16x2(pv[4], pv[5]),
+                                          pack_bf16x2(pv[6], pv[7])});
 }
+__device__ __forceinline__ float row_sum(float l) { return xor_step<32, LaneSum>(xor_step<16, LaneSum>(l)); }
 
 // The merge of a row's next chunk (m, l, and below each accumulator) into its state so far (M, L): both are brought to the
 // larger reference point, rounded as written in every kernel (no contraction).
@@ -174,6 +180,7 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
   float mt = 0.f, lt = 0.f;
   // chunk `c` is complete: merged into the rows that see it, and an empty state for the next
   auto end_chunk = [&](int c) {
+    l = row_sum(l);
     if (c == 0) {
       mt = m, lt = l;
 #pragma unroll
@@ -195,11 +202,11 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
   for (int tile = 0; tile < ntiles; tile++) {
     const int k0 = tile * 32;
     if (tile != 0 && tile % CHUNK_TILES == 0) end_chunk(tile / CHUNK_TILES - 1);
-    // ---- scores: two 16-key sub-tiles; lane (j, g) receives keys k0 + 16u + 4g + i of query j
+    // ---- scores: two sub-tiles of 16 keys; lane (j, g) receives keys k0 + 8g + 4u + i of query j
     f32x4 s[2];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      const int krow = min(k0 + 16 * u + j, a.max_len - 1);
+      const int krow = min(k0 + key_row(u, j), a.max_len - 1);
       const uint16_t* kp = kbase + (int64_t)krow * HD + g * 8;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -209,12 +216,12 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
       }
       s[u] = acc;
     }
-    float alpha;
-    bf16x8 pf;
-    softmax_tile<true>(s, k0, g, qpos, a.scale_log2, m, l, alpha, pf);
-    // ---- out^T += V^T * P: "A" operand lane (j, g) holds channel 16t + j, the same 8 key slots
-    const int kv0 = min(k0 + 4 * g, a.max_len - 4);
-    const int kv1 = min(k0 + 16 + 4 * g, a.max_len - 4);
+    mask_scores(s, k0, g, qpos);
+    const float alpha = move_reference(lane_max(s), a.scale_log2, m, l);
+    const bf16x8 pf = probabilities(s, a.scale_log2, m, l);
+    // ---- out^T += V^T * P: "A" operand lane (j, g) holds channel 16t + j, the same 8 keys
+    const int kv0 = min(k0 + 8 * g, a.max_len - 4);
+    const int kv1 = min(k0 + 8 * g + 4, a.max_len - 4);
 #pragma unroll
     for (int t = 0; t < 8; t++) {
       const uint16_t* vp = vbase + (int64_t)(16 * t + j) * a.max_len;
@@ -237,278 +244,284 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
   }
 }
 
+// Key tiles in LDS.  A direct load puts lane l's 16 bytes at (wave-uniform address) + 16 l, so the layout is made on the global
+// side: each lane fetches the 16-byte chunk that belongs at its place.
+//   K rows [keys][256 bytes]: position pc of key row kr holds chunk pc ^ k_swizzle(kr);
+//   V^T rows [128 channels][KEYS * 2 bytes]: position pc of channel row r holds chunk pc ^ v_swizzle<KEYS>(r).
+// A 16-byte read is served for lanes {0-7, 16-23} together (then {8-15, 24-31}, ...): the eight rows and two neighbouring
+// chunks of such a pass cover all 64 banks in both.
+__device__ __forceinline__ int k_swizzle(int kr) { return 2 * ((kr & 3) + 4 * ((kr >> 3) & 1)); }
+template <int KEYS>
+__device__ __forceinline__ int v_swizzle(int r) { return KEYS == 64 ? 2 * ((r >> 1) & 3) : 2 * ((r >> 2) & 1); }
+// byte offsets of lane (j, g)'s fragments: chunk c of key key_row(0, j) (sub-tile 1 lies four rows = 1024 bytes on), and chunk c
+// = eight keys of channel row j (sixteen channels are 16 rows on)
+__device__ __forceinline__ uint32_t k_fragment(int j, int c) { return key_row(0, j) * 256 + ((c ^ k_swizzle(key_row(0, j))) << 4); }
+template <int KEYS>
+__device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * (KEYS * 2) + ((c ^ v_swizzle<KEYS>(j)) << 4); }
+
 // ------------------------------------------------------------------------------------------------
-// Grouped variant: one work-group per (16 * QB consecutive queries, KV head, sequence); its G * QB wavefronts are the G
-// query heads that share the KV head, for each of the QB blocks of 16 queries.  Each 32-key tile of K and of V^T is fetched from global memory ONCE per group with
-// coalesced 16-byte loads, staged in LDS (double buffered; K rows XOR-swizzled against bank conflicts, V^T rows stored in
-// fragment order) and read from there
-// by every wave.  A row's arithmetic -- the lanes that own it, the MFMA chain, the order of the softmax updates --
-// is exactly that of attention_kernel above, so both kernels produce the same bits; this one just moves 1/G of
-// the bytes and hides the load latency behind the previous tile.
-// NLD > 0: that many more wavefronts in the work-group do all the staging (loads, LDS writes) at the same barriers and
-// the G computing waves none of it: for launches that leave the chip short of work-groups, where a work-group's time is
-// its own chain of tiles rather than its share of a CU.
-// SPLIT: a work-group takes one chunk of the keys (blockIdx.z) and leaves its state in the workspace for
-// attention_merge_kernel: a few new tokens against a long cache are a handful of work-groups otherwise
-// (55 tokens at 8192 keys 133 -> 24 us, 16 tokens of two sequences at 16384 keys 227 -> 30).
+// Grouped variant: one work-group of NW = G * WQ wavefronts per (16 * QB * WQ consecutive queries, KV head, sequence).  A
+// wavefront holds one of the G query heads that share the KV head and QB blocks of 16 queries; the keys are brought in 64 at
+// a time (K and V^T, 32 KiB) by direct loads into an LDS ring of NS slots, once for the whole work-group, and every fragment
+// read from there serves the wavefront's QB blocks.  A row's arithmetic -- the lanes that own it, the MFMA chain, the order of
+// the softmax updates -- is exactly that of attention_kernel above, so the kernels produce the same bits.
+// SPLIT_CHUNKS: a work-group takes one chunk of the keys (blockIdx.z) and leaves its state in the workspace for
+// attention_merge_kernel: a few new tokens against a long cache are a handful of work-groups otherwise.
+// What bounds it: vector issue and matrix pipes together.  8192 tokens of 32 heads on two blocks (503 us, 1.09 PFLOP/s; 599 before):
+// per 32 queries x 32 keys of a wavefront 512 cycles of MFMA (busy 51 % of the SIMD's cycles), some 100 vector instructions
+// and 16 exponentials (47 %), no bank conflict, the LDS read port busy a quarter of the time.  One fragment read per 16
+// queries made it the LDS and the L2 (a 64-byte half of a V^T line per load and tile: 8.4 TB/s) instead; in work-groups of
+// 64 queries, which halve the key traffic once more, it takes the same time (532), and so does forming a tile's scores ahead.
+// Launches that leave CUs short of work-groups are a chain of 0.53 us per tile, a third of it the slot's barrier and waits.
 // ------------------------------------------------------------------------------------------------
-// chunks: the cache has a single one / a work-group walks them all / a work-group takes one (SPLIT)
+// chunks: the cache has a single one / a work-group walks them all / a work-group takes one
 enum { ONE_CHUNK, ALL_CHUNKS, SPLIT_CHUNKS };
-template <int G, int QB, bool DEEP, int NLD, int CHUNKS, int AHEAD>
-__global__ __launch_bounds__(64 * (G * QB + NLD)) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
+constexpr int UNIT = 64, UNIT_BYTES = 4 * UNIT * HD;  // keys of a ring slot; 16 KiB of K, 16 KiB of V^T
+template <int G, int WQ, int QB, int NS, int CHUNKS>
+__global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
   constexpr bool SPLIT = CHUNKS == SPLIT_CHUNKS;
-  constexpr int NW = G * QB;   // computing wavefronts
-  // The merged chunks (32 registers a lane, touched once in sixteen tiles) would cost work-groups of eight wavefronts the
-  // second one of a CU: half of them lie in LDS there, which two such work-groups have to spare (64 of 80 KiB), and four
-  // wavefronts fit a SIMD again (144 -> 124 registers).
-  constexpr int PARK = CHUNKS == ALL_CHUNKS && NW == 8 && NLD == 0 ? 4 : 0;
-  __shared__ f32x4 parked[PARK ? PARK : 1][PARK ? 64 * NW : 1];
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2][16384];  // per buffer: K tile [32][128] (8 KiB), V^T tile [128][32] (8 KiB)
+  constexpr int NW = G * WQ, ROWS = 16 * QB * WQ;
+  constexpr int PI = 16 / NW;                           // load instructions per slot, operand and wavefront
+  constexpr int CHUNK_UNITS = CHUNK_TILES * 32 / UNIT;
+  static_assert((NW == 4 || NW == 8) && CHUNK_UNITS % NS == 0 && NS >= 2, "work-group shape");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int b = blockIdx.y;
   // Work-groups are dealt to the eight XCDs round robin, each with an L2 of its own: with the KV head as the fastest
-  // index every XCD serves the query blocks of the same few KV heads, and the key tiles those blocks share (every block
+  // index every XCD serves the query blocks of the same few KV heads, and the keys those blocks share (every block
   // of a head walks the same keys) stay in ITS L2 instead of being fetched by all eight.
   // Causal attention: the last query blocks have the most keys, so they are dispatched first (longest work first
   // keeps the tail of the launch short); which work-group computes a block has no numeric effect.
   const int kvh = blockIdx.x % a.kv_heads;
   const int qb = gridDim.x / a.kv_heads - 1 - blockIdx.x / a.kv_heads;
   const int qlen = a.q_len[b];
-  if (qb * (16 * QB) >= qlen) return;  // uniform over the work-group
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int h = kvh * G + (QB == 1 ? wave : wave % G);
+  if (qb * ROWS >= qlen) return;  // uniform over the work-group
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = kvh * G + wave % G;
   const int j = lane & 15;
   const int g = lane >> 4;
   const int ctx = a.ctx_len[b];
-  const int qrow = qb * (16 * QB) + (QB == 1 ? 0 : wave / G * 16) + j;
-  const bool qvalid = qrow < qlen;
-  const int qpos = ctx - qlen + min(qrow, qlen - 1);
-  const int last_pos = ctx - qlen + min(qb * (16 * QB) + (16 * QB - 1), qlen - 1);
+  const int row0 = qb * ROWS + wave / G * (16 * QB);   // this wavefront's first query
+  // the tiles of 32 keys that the work-group's queries see, and this wavefront's; SPLIT: up to the end of chunk blockIdx.z
+  const int tile0 = SPLIT ? (int)blockIdx.z * CHUNK_TILES : 0;
+  const int all_tiles = (ctx - qlen + min(qb * ROWS + ROWS - 1, qlen - 1)) / 32 + 1;
+  const int ntiles = SPLIT ? min(all_tiles, tile0 + CHUNK_TILES) : all_tiles;
+  if (SPLIT && tile0 >= ntiles) return;  // uniform over the work-group
+  const int wave_tiles = min(ntiles, (ctx - qlen + min(row0 + 16 * QB - 1, qlen - 1)) / 32 + 1);
+  const int unit0 = tile0 / 2, nunits = (ntiles + 1) / 2;
 
+  int qpos[QB];
+  bf16x8 qf[QB][4];
+#pragma unroll
+  for (int q = 0; q < QB; q++) {
+    const int qrow = min(row0 + 16 * q + j, qlen - 1);
+    qpos[q] = ctx - qlen + qrow;
+    const uint16_t* qp = a.q + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
+#pragma unroll
+    for (int c = 0; c < 4; c++) qf[q][c] = *reinterpret_cast<const bf16x8*>(qp + c * 32 + g * 8);
+  }
+
+  // ---- staging: load instruction n of the sixteen of a slot covers key rows 4n .. 4n+3 / channel rows 8n .. 8n+7 (whole
+  // 128-byte lines of the V^T cache); this wavefront issues the instructions wave, wave + NW, ...
+  // A cache whose length is an odd number of tiles ends in the middle of the last slot: K instructions behind its end fetch
+  // the last rows again, and V^T lanes of the second half what those of the first half do (rows that nobody sees).
   const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.k_cache + ((int64_t)b * a.kv_heads + kvh) * a.max_len * HD);
   const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vt_cache + ((int64_t)b * a.kv_heads + kvh) * (int64_t)HD * a.max_len);
-
-  // cooperative staging: 512 16-byte chunks per tile and operand, NCH per thread
-  // (NLD loader waves, where the kernel has them, do all of it; the computing waves then neither load nor store tiles)
-  constexpr int NT = NLD ? 64 * NLD : 64 * NW;
-  const int stid = NLD ? tid - 64 * NW : tid;   // staging thread
-  constexpr int NCH = (512 + NT - 1) / NT;
-  // Key tiles are fetched DEPTH tiles ahead into DEPTH register sets (set = tile % DEPTH).  DEEP is for decode: a
-  // single block of queries per sequence makes the kernel a chain of memory round trips, and one tile of arithmetic
-  // hides none of them.  Prefill has arithmetic to overlap and prefers the registers (more waves per SIMD), and so does
-  // decode where they decide about the second work-group of a CU (8 heads, 128 sequences of 1000 keys 151 -> 116 us).
-  // Loader waves without DEEP fetch AHEAD tiles ahead: with one, a tile is stored in the iteration that asked for it and the
-  // barrier waits for the memory (0.8 us per tile where several sequences share an L2 and read their own keys).
-  constexpr int DEPTH = !DEEP ? AHEAD : PARK ? 2 : (NCH <= 2 ? 4 : (NCH <= 4 ? 2 : 1));
-  u32x4 kregs[DEPTH][NCH], vregs[DEPTH][NCH];
-  // A K tile is 8 KiB of consecutive bytes (32 rows of 256), chunk ch at byte 16 ch; a V^T tile is 128 rows of 64 bytes,
-  // max_len elements apart.  Per-thread byte offsets inside a tile (global and LDS side) are formed once; per tile only
-  // a wave-uniform base moves, so the loads take a scalar base and the loop spends no vector instruction on addresses.
-  uint32_t vsrc[NCH], kdst[NCH], vdst0[NCH], vdst1[NCH];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+  const int64_t vstep = (int64_t)a.max_len * 16;   // bytes of eight channel rows
+  const int vchunk = (lane & 7) ^ v_swizzle<64>(lane >> 3);
+  const uint32_t vrow = (uint32_t)(lane >> 3) * (uint32_t)a.max_len * 2u;
+  auto load_unit = [&](int unit, int slot) __attribute__((always_inline)) {
+    const int k0 = min(unit * UNIT, a.max_len - 32);   // max_len is a multiple of 32
+    const uint32_t voff = vrow + ((k0 + UNIT <= a.max_len ? vchunk : vchunk & 3) << 4);
 #pragma unroll
-  for (int i = 0; i < NCH; i++) {
-    const int ch = min(max(stid, 0) + i * NT, 511);
-    const int kr = ch >> 4, kc = ch & 15;   // key row, 16-byte chunk of its 256 bytes
-    kdst[i] = kr * 256 + ((kc ^ (2 * (kr & 7))) << 4);
-    // V^T: channel row vr (64 bytes = 32 keys), 16-byte chunk vc = keys 8vc .. 8vc+7.  The keys of a row are stored
-    // in the order a P*V fragment wants them -- lane group g takes keys 4g..4g+3 and 16+4g..16+4g+3 -- so that a
-    // fragment is ONE 16-byte read at byte 16g of the row: keys 4a..4a+3 live in the 8-byte slot 2 (a & 3) + (a >> 2).
-    // A 16-byte read is served for lanes {0-7, 16-23} together (then {8-15, 24-31}, ...): rows j and j + 4 of a 64-byte
-    // pitch meet in the same banks, so rows with bit 2 set keep their chunks in the other half of the row (chunk ^ 2,
-    // i.e. 8-byte slot ^ 4) and the sixteen lanes of a phase cover all 64 banks.
-    const int vr = ch >> 2, vc = ch & 3;
-    const int vx = 4 * ((vr >> 2) & 1);
-    vsrc[i] = (uint32_t)vr * (uint32_t)a.max_len * 2u + vc * 16;
-    vdst0[i] = 8192 + vr * 64 + ((2 * ((2 * vc) & 3) + (vc >> 1)) ^ vx) * 8;
-    vdst1[i] = 8192 + vr * 64 + ((2 * ((2 * vc + 1) & 3) + (vc >> 1)) ^ vx) * 8;
-  }
-  // this (sequence, KV head)'s slice of each cache as a raw buffer (no stride, extent in bytes; the dispatcher keeps
-  // max_len small enough for 32-bit offsets)
-  const __amdgpu_buffer_rsrc_t krsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(kbase), 0, a.max_len * (HD * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t vrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(vbase), 0, a.max_len * (HD * 2), 0x00020000);
-  auto load_tile = [&](int tile, int set) __attribute__((always_inline)) {
-    u32x4* kreg = kregs[set];
-    u32x4* vreg = vregs[set];
-    const int k0 = min(tile * 32, a.max_len - 32);  // max_len is a multiple of 32: never past the cache
-    // buffer loads: the descriptors (one per cache, in scalar registers) and the tile's byte offset are wave-uniform,
-    // the per-thread offsets are the constants formed above -- no vector instruction per load
-    const int ks = k0 * (HD * 2), vs = k0 * 2;
-#pragma unroll
-    for (int i = 0; i < NCH; i++) {
-      if (512 % NT == 0 || stid + i * NT < 512) {
-        kreg[i] = __builtin_amdgcn_raw_buffer_load_b128(krsrc, (stid + i * NT) * 16, ks, 0);
-        vreg[i] = __builtin_amdgcn_raw_buffer_load_b128(vrsrc, (int)vsrc[i], vs, 0);
-      }
-    }
-  };
-  auto store_tile = [&](int buf, int set) __attribute__((always_inline)) {
-    const u32x4* kreg = kregs[set];
-    const u32x4* vreg = vregs[set];
-#pragma unroll
-    for (int i = 0; i < NCH; i++) {
-      if (512 % NT == 0 || stid + i * NT < 512) {
-        *reinterpret_cast<u32x4*>(&lds[buf][kdst[i]]) = kreg[i];
-        *reinterpret_cast<uint2*>(&lds[buf][vdst0[i]]) = make_uint2(vreg[i][0], vreg[i][1]);
-        *reinterpret_cast<uint2*>(&lds[buf][vdst1[i]]) = make_uint2(vreg[i][2], vreg[i][3]);
-      }
+    for (int i = 0; i < PI; i++) {
+      const int n = wave + i * NW;
+      const int kr = 4 * n + (lane >> 4);
+      const uint32_t koff = (uint32_t)((lane >> 4) * 256 + (((lane & 15) ^ k_swizzle(kr)) << 4));
+      dma16(lds0 + slot * UNIT_BYTES + n * 1024, koff, kbase + (int64_t)min(k0 + 4 * n, a.max_len - 4) * (HD * 2));
+      dma16(lds0 + slot * UNIT_BYTES + UNIT * HD * 2 + n * 1024, voff, vbase + (int64_t)k0 * 2 + n * vstep);
     }
   };
 
-  // the tiles of this work-group: all of them, or (SPLIT) those of chunk blockIdx.z
-  const int tile0 = SPLIT ? (int)blockIdx.z * CHUNK_TILES : 0;
-  const int ntiles = SPLIT ? min(last_pos / 32 + 1, tile0 + CHUNK_TILES) : last_pos / 32 + 1;
-  if (SPLIT && tile0 >= ntiles) return;  // uniform over the work-group
-  constexpr int UNROLL = DEPTH < 2 ? 2 : DEPTH;
-  if (NLD && stid >= 0) {
-    // ---- loader waves: the staging half of the loop below, at the same barriers
+  f32x4 o[QB][8], ot[QB][8];   // this chunk's accumulators, and the merged chunks so far
+  float m[QB], l[QB], mt[QB], lt[QB];
+  auto empty_state = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_tile(tile0 + d, d);
-    store_tile(0, 0);
-    __syncthreads();
-    for (int t0 = tile0; t0 < ntiles; t0 += UNROLL) {
+    for (int q = 0; q < QB; q++) {
+      m[q] = kNoKey, l[q] = 0.f;
 #pragma unroll
-      for (int d = 0; d < UNROLL; d++) {
-        const int tile = t0 + d;
-        if (tile >= ntiles) break;
-        load_tile(tile + DEPTH, d % DEPTH);
-        if (tile + 1 < ntiles) store_tile((d & 1) ^ 1, (d + 1) % DEPTH);
-        __syncthreads();
-      }
+      for (int t = 0; t < 8; t++) o[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    return;
-  }
-  const uint16_t* qp = a.q + ((int64_t)(a.q_start[b] + min(qrow, qlen - 1)) * a.q_heads + h) * HD;
-  bf16x8 qf[4];
-#pragma unroll
-  for (int c = 0; c < 4; c++) qf[c] = *reinterpret_cast<const bf16x8*>(qp + c * 32 + g * 8);
-
-  f32x4 o[8];
-#pragma unroll
-  for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = kNoKey;
-  float l = 0.f;
-  // The merged chunks so far.  (All of them parked in scratch memory cost 25 %: 557 MB of it for a prompt of 4096.)
-  f32x4 ot[8 - PARK];
-  auto merged = [&](int t) __attribute__((always_inline)) { return t < 8 - PARK ? ot[t] : parked[t - (8 - PARK)][tid]; };
-  auto set_merged = [&](int t, f32x4 v) __attribute__((always_inline)) {
-    if (t < 8 - PARK) ot[t] = v;
-    else parked[t - (8 - PARK)][tid] = v;
   };
-  float mt = 0.f, lt = 0.f;
+  empty_state();
+#pragma unroll
+  for (int q = 0; q < QB; q++) mt[q] = lt[q] = 0.f;
   // chunk `c` is complete: merged into the rows that see it; after the last one the result stays in m, l and o,
   // otherwise an empty state follows
   auto end_chunk = [&](int c, bool last) __attribute__((always_inline)) {
-    if (c != 0) {
-      if (qpos >= c * CHUNK_TILES * 32) {
-        float fa, fb;
-        merge_chunk(mt, lt, m, l, fa, fb);
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-          f32x4 u = merged(t);
+    for (int q = 0; q < QB; q++) {
+      l[q] = row_sum(l[q]);
+      if (c != 0) {
+        if (qpos[q] >= c * CHUNK_TILES * 32) {
+          float fa, fb;
+          merge_chunk(mt[q], lt[q], m[q], l[q], fa, fb);
 #pragma unroll
-          for (int i = 0; i < 4; i++) u[i] = merge_acc(u[i], fa, o[t][i], fb);
-          set_merged(t, u);
+          for (int t = 0; t < 8; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) ot[q][t][i] = merge_acc(ot[q][t][i], fa, o[q][t][i], fb);
         }
+      } else {
+        mt[q] = m[q], lt[q] = l[q];
+#pragma unroll
+        for (int t = 0; t < 8; t++) ot[q][t] = o[q][t];
       }
-    } else {
-      mt = m, lt = l;
+      if (last) {
+        l[q] = lt[q];
 #pragma unroll
-      for (int t = 0; t < 8; t++) set_merged(t, o[t]);
+        for (int t = 0; t < 8; t++) o[q][t] = ot[q][t];
+      }
     }
-    if (last) {
-      l = lt;
-#pragma unroll
-      for (int t = 0; t < 8; t++) o[t] = merged(t);
-    } else {
-      m = kNoKey, l = 0.f;
-#pragma unroll
-      for (int t = 0; t < 8; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    if (!last) empty_state();
   };
 
-  // LDS offsets of this lane's fragments inside a tile buffer, formed once: key row 16u + j of the K tile (256 bytes a
-  // row, 16-byte chunk c*4 + g swizzled by the row; u adds 4096), channel row 16t + j of the V^T tile (64 bytes a row,
-  // the lane group's eight keys are the 16-byte chunk g, or g ^ 2 in rows with bit 2 set; t adds 1024)
-  uint32_t kofs[4];
+  // fragment addresses in the first slot; every other slot, sub-tile and channel tile is an immediate offset from them
+  typedef __attribute__((address_space(3))) const uint8_t lds_byte;
+  typedef __attribute__((address_space(3))) const bf16x8 lds_fragment;
+  lds_byte *kp[4], *vp[2];
 #pragma unroll
-  for (int c = 0; c < 4; c++) kofs[c] = j * 256 + (((c * 4 + g) ^ (2 * (j & 7))) << 4);
-  const uint32_t vofs = 8192 + j * 64 + (g ^ (2 * ((j >> 2) & 1))) * 16;
-
-  // loads past the last tile are clamped to a valid address and never used: issuing them unconditionally keeps the
-  // number of loads in flight static, so the waits below can leave the newer tiles in flight
-  if (!NLD) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_tile(tile0 + d, d);
-    store_tile(0, 0);
+  for (int c = 0; c < 4; c++) {
+    kp[c] = (lds_byte*)lds + k_fragment(j, c * 4 + g);
+    asm volatile("" : "+v"(kp[c]));   // (the sum with the base of the LDS is formed once, not at every use)
   }
-  __syncthreads();
-  // the loop body covers UNROLL (an even number of) tiles, so that the LDS buffer of each is a compile-time constant and
-  // every LDS address is a per-thread offset plus an immediate
-  static_assert(CHUNK_TILES % UNROLL == 0, "a chunk is a whole number of loop bodies");
-  for (int c0 = tile0; c0 < ntiles; c0 += CHUNK_TILES) {
-  const int ce = min(c0 + CHUNK_TILES, ntiles);
-  for (int t0 = c0; t0 < ce; t0 += UNROLL) {
 #pragma unroll
-   for (int d = 0; d < UNROLL; d++) {
-    const int tile = t0 + d;
-    if (tile >= ce) break;
-    const int cur = d & 1;
-    if (!NLD) load_tile(tile + DEPTH, d % DEPTH);  // that set held this tile and went to LDS a tile ago
-    const int k0 = tile * 32;
-    const uint8_t* tb = &lds[cur][0];
-    f32x4 s[2];
+  for (int hf = 0; hf < 2; hf++) {
+    vp[hf] = (lds_byte*)lds + UNIT * HD * 2 + v_fragment<64>(j, hf * 4 + g);
+    asm volatile("" : "+v"(vp[hf]));
+  }
+  // tile hf of the two in a slot.  All fragments of an operand are asked for before the first MFMA that takes one (the
+  // scheduling barrier keeps the compiler from moving each read to its use, where the wave would wait out the LDS latency once
+  // per fragment).
+  auto read_keys = [&](int slot, int hf, bf16x8 (&kf)[4][2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-      f32x4 acc;
+    for (int c = 0; c < 4; c++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(tb + kofs[c] + u * 4096);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[c], c == 0 ? zero : acc, 0, 0, 0);
+      for (int u = 0; u < 2; u++) kf[c][u] = *(lds_fragment*)(kp[c] + slot * UNIT_BYTES + hf * 8192 + u * 1024);
+  };
+  auto read_values = [&](int slot, int hf, bf16x8 (&vf)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 8; t++) vf[t] = *(lds_fragment*)(vp[hf] + slot * UNIT_BYTES + t * 2048);
+  };
+  auto scores = [&](const bf16x8 (&kf)[4][2], int q, f32x4 (&s)[2]) __attribute__((always_inline)) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int u = 0; u < 2; u++) s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[c][u], qf[q][c], c == 0 ? zero : s[u], 0, 0, 0);
+  };
+  // mask and reference point of tile `tile`; the conditions are uniform over the wave
+  auto reference = [&](int tile, int q, f32x4 (&s)[2]) __attribute__((always_inline)) {
+    if (tile * 32 + 31 > ctx - qlen + row0 + 16 * q) mask_scores(s, tile * 32, g, qpos[q]);   // (beyond the block's first query)
+    const float lmax = lane_max(s);
+    if (__builtin_amdgcn_ballot_w64(score_exceeds(lmax, a.scale_log2, m[q])) != 0) {
+      const float alpha = move_reference(lmax, a.scale_log2, m[q], l[q]);
+#pragma unroll
+      for (int t = 0; t < 8; t++) o[q][t] = f32x4{o[q][t][0] * alpha, o[q][t][1] * alpha, o[q][t][2] * alpha, o[q][t][3] * alpha};
+    }
+  };
+  auto accumulate = [&](const bf16x8 (&vf)[8], int q, bf16x8 pf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 8; t++) o[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pf, o[q][t], 0, 0, 0);
+  };
+  // eight MFMAs of one block beside the exponentials of another: an MFMA holds the matrix pipe for 16 cycles and takes one
+  // of its wave's issue slots, so three or four vector instructions fit behind each
+  auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);   // VALU
+      __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);   // transcendental
+    }
+  };
+  // formed here, and not behind the next branch where the compiler would sink it
+  auto pin = [&](bf16x8& p, float& sum) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(p), "+v"(sum));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto do_tile = [&](int tile, int slot, int hf) __attribute__((always_inline)) {
+    f32x4 s[QB][2];
+    bf16x8 kf[4][2], vf[8], pf[QB];
+    read_keys(slot, hf, kf);
+    __builtin_amdgcn_sched_barrier(0);
+    scores(kf, 0, s[0]);
+    reference(tile, 0, s[0]);
+#pragma unroll
+    for (int q = 0; q < QB; q++) {
+      if (q + 1 < QB) scores(kf, q + 1, s[q + 1]);
+      else if (q > 0) accumulate(vf, q - 1, pf[q - 1]);
+      if (q + 1 == QB - 1 || QB == 1) read_values(slot, hf, vf);
+      pf[q] = probabilities(s[q], a.scale_log2, m[q], l[q]);
+      interleave();
+      pin(pf[q], l[q]);
+      if (q + 1 < QB) reference(tile, q + 1, s[q + 1]);
+    }
+    accumulate(vf, QB - 1, pf[QB - 1]);
+  };
+
+#pragma unroll
+  for (int i = 0; i < NS - 1; i++)
+    if (unit0 + i < nunits) load_unit(unit0 + i, i);
+  // The queries are in their registers from here on.  (The compiler does not see the direct loads: left to the first use, its
+  // wait for the queries would stand in the loop and drain every load in flight.)
+#pragma unroll
+  for (int q = 0; q < QB; q++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) asm volatile("" : "+v"(qf[q][c]));
+  for (int c0 = unit0; c0 < nunits; c0 += CHUNK_UNITS) {
+    const int ce = min(c0 + CHUNK_UNITS, nunits);
+    for (int u0 = c0; u0 < ce; u0 += NS) {
+#pragma unroll
+      for (int d = 0; d < NS; d++) {   // slot d: a chunk is a whole number of rings
+        const int unit = u0 + d;
+        if (unit >= ce) break;
+        // the slot has landed for every wave, and every wave is done with what it read from the slot before, which the
+        // loads behind the barrier refill; up to NS - 2 slots stay in flight
+        wait_slices<2 * PI, NS - 2>(min(NS - 2, nunits - 1 - unit));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (unit + NS - 1 < nunits) load_unit(unit + NS - 1, (d + NS - 1) % NS);
+        if (2 * unit < wave_tiles) do_tile(2 * unit, d, 0);
+        if (2 * unit + 1 < wave_tiles) do_tile(2 * unit + 1, d, 1);
       }
-      s[u] = acc;
     }
-    // only the tiles on the causal diagonal need the mask: when every key of the tile is visible to every query of
-    // this wave (a uniform condition) the selects are skipped; the values are the same either way.  Prefill only:
-    // in decode the tile loop is one dependent chain and a branch on a freshly computed value lengthens it.
-    float alpha;
-    bf16x8 pf;
-    if (!DEEP && __builtin_amdgcn_ballot_w64(k0 + 31 > qpos) == 0) softmax_tile<false>(s, k0, g, qpos, a.scale_log2, m, l, alpha, pf);
-    else softmax_tile<true>(s, k0, g, qpos, a.scale_log2, m, l, alpha, pf);
-    // rescale the output accumulators only when some row's reference point moved (uniform over the wave): x * 1.0f is x bit
-    // for bit, and after the first tiles of a long row the maximum rarely moves (prefill only, as above)
-    if (DEEP || __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    if (CHUNKS == ALL_CHUNKS && nunits > CHUNK_UNITS) end_chunk(c0 / CHUNK_UNITS, ce == nunits);
+  }
+  if (CHUNKS != ALL_CHUNKS || nunits <= CHUNK_UNITS) {
 #pragma unroll
-      for (int t = 0; t < 8; t++) o[t] = f32x4{o[t][0] * alpha, o[t][1] * alpha, o[t][2] * alpha, o[t][3] * alpha};
+    for (int q = 0; q < QB; q++) l[q] = row_sum(l[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < QB; q++) {
+    const int qrow = row0 + 16 * q + j;
+    if (qrow >= qlen) continue;
+    if (SPLIT && qpos[q] >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete here)
+      const int64_t at = ((int64_t)(b * sp.q_rows + qrow) * a.q_heads + h) * sp.nchunks + blockIdx.z;
+#pragma unroll
+      for (int t = 0; t < 8; t++) *reinterpret_cast<f32x4*>(sp.o + at * HD + 16 * t + 4 * g) = o[q][t];
+      if (g == 0) *reinterpret_cast<f32x2*>(sp.ml + at * 2) = f32x2{m[q], l[q]};
+      continue;
     }
+    if (SPLIT && blockIdx.z != 0) continue;
+    const float inv = 1.0f / l[q];
+    uint16_t* op = a.out + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
 #pragma unroll
     for (int t = 0; t < 8; t++) {
-      const bf16x8 vf = *reinterpret_cast<const bf16x8*>(tb + vofs + t * 1024);
-      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[t], 0, 0, 0);
+      const uint32_t lo = pack_bf16x2(o[q][t][0] * inv, o[q][t][1] * inv);
+      const uint32_t hi = pack_bf16x2(o[q][t][2] * inv, o[q][t][3] * inv);
+      *reinterpret_cast<uint2*>(op + 16 * t + 4 * g) = make_uint2(lo, hi);
     }
-    if (!NLD && tile + 1 < ntiles) store_tile(cur ^ 1, (d + 1) % DEPTH);
-    __syncthreads();
-   }
-  }
-  if (CHUNKS == ALL_CHUNKS && ntiles > CHUNK_TILES) end_chunk(c0 / CHUNK_TILES, ce == ntiles);
-  }
-  if (!qvalid) return;
-  if (SPLIT && qpos >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete here)
-    const int64_t at = ((int64_t)(b * sp.q_rows + qrow) * a.q_heads + h) * sp.nchunks + blockIdx.z;
-#pragma unroll
-    for (int t = 0; t < 8; t++) *reinterpret_cast<f32x4*>(sp.o + at * HD + 16 * t + 4 * g) = o[t];
-    if (g == 0) *reinterpret_cast<f32x2*>(sp.ml + at * 2) = f32x2{m, l};
-    return;
-  }
-  if (SPLIT && blockIdx.z != 0) return;
-  const float inv = 1.0f / l;
-  uint16_t* op = a.out + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
-#pragma unroll
-  for (int t = 0; t < 8; t++) {
-    const uint32_t lo = pack_bf16x2(o[t][0] * inv, o[t][1] * inv);
-    const uint32_t hi = pack_bf16x2(o[t][2] * inv, o[t][3] * inv);
-    *reinterpret_cast<uint2*>(op + 16 * t + 4 * g) = make_uint2(lo, hi);
   }
 }
 
@@ -525,11 +538,7 @@ __global__ __launch_bounds__(64 * (G * QB + NLD)) void attention_group_kernel(co
 //     piece of that chain.  Loader i issues two of the eight 1 KiB load instructions of every K tile and V^T tile.
 // A direct load puts lane l's 16 bytes at (wave-uniform address) + 16 l, so the LDS layout is made on the global side:
 // each lane fetches the chunk that belongs at its fixed place.
-//   K tile [32 keys][256 bytes]: chunk position pc of key row kr holds chunk pc ^ 2 (kr & 7) (the swizzle of the grouped
-//     kernel, read the same way);
-//   V^T tile [128 channels][64 bytes = 32 keys]: chunk position pc of channel row r holds chunk pc ^ ((r >> 2) & 3); a
-//     P*V fragment (keys 4g .. 4g+3 and 16+4g .. 16+4g+3 of channel row 16t + j) is two 8-byte reads, and the sixteen
-//     rows x two lane groups of a read pass cover all 64 banks.
+// The rows lie as k_swizzle and v_swizzle<32> say.
 // K tiles and V^T tiles have rings of NS slots each.  Iteration t reads K tile t + 1 and V^T tile t; the loaders request
 // K tile t + NS (slot t % NS, read during iteration t - 1) and V^T tile t + NS - 1 (slot (t - 1) % NS, likewise), wait
 // until what they requested NS - 2 iterations ago has landed (K tile t + 2, V^T tile t + 1: what iteration t + 1 reads),
@@ -585,8 +594,8 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
     for (int i = 0; i < PI; i++) {
       const int q = li * PI + i;
       const int kr = 4 * q + (lane >> 4), pc = lane & 15;
-      const int r = 16 * q + (lane >> 2), vc = (lane & 3) ^ ((lane >> 4) & 3);
-      kvoff[i] = (uint32_t)(kr * 256 + ((pc ^ (2 * (kr & 7))) << 4));
+      const int r = 16 * q + (lane >> 2), vc = (lane & 3) ^ v_swizzle<32>(r);
+      kvoff[i] = (uint32_t)(kr * 256 + ((pc ^ k_swizzle(kr)) << 4));
       vvoff[i] = (uint32_t)r * (uint32_t)a.max_len * 2u + vc * 16;
     }
     const uint32_t lk = (uint32_t)(uintptr_t)&lds_k[0][0] + li * PI * 1024;
@@ -714,20 +723,18 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   const int lt = pos >> 5, pr = pos & 31;
   auto patch_k = [&](int slot) __attribute__((always_inline)) {
     if (lane < 16)
-      *reinterpret_cast<u32x4*>(&lds_k[slot][pr * 256 + ((lane ^ (2 * (pr & 7))) << 4)]) = *reinterpret_cast<const u32x4*>(hs + G * HD + lane * 8);
+      *reinterpret_cast<u32x4*>(&lds_k[slot][pr * 256 + ((lane ^ k_swizzle(pr)) << 4)]) = *reinterpret_cast<const u32x4*>(hs + G * HD + lane * 8);
   };
   auto patch_v = [&](int slot) __attribute__((always_inline)) {
     if (lane < 16 * CT) {
       const int ch = 16 * CT * wv + lane;
-      *reinterpret_cast<uint16_t*>(&lds_v[slot][ch * 64 + (((pr >> 3) ^ ((ch >> 2) & 3)) << 4) + (pr & 7) * 2]) = hs[(G + 1) * HD + ch];
+      *reinterpret_cast<uint16_t*>(&lds_v[slot][ch * 64 + (((pr >> 3) ^ v_swizzle<32>(ch)) << 4) + (pr & 7) * 2]) = hs[(G + 1) * HD + ch];
     }
   };
   uint32_t kofs[4];
 #pragma unroll
-  for (int c = 0; c < 4; c++) kofs[c] = j * 256 + (((c * 4 + g) ^ (2 * (j & 7))) << 4);
-  const int vsw = (j >> 2) & 3;
-  const uint32_t vofs0 = (CT * wv) * 1024 + j * 64 + (((g >> 1) ^ vsw) << 4) + (g & 1) * 8;
-  const uint32_t vofs1 = (CT * wv) * 1024 + j * 64 + (((2 + (g >> 1)) ^ vsw) << 4) + (g & 1) * 8;
+  for (int c = 0; c < 4; c++) kofs[c] = k_fragment(j, c * 4 + g);
+  const uint32_t vofs = CT * wv * 1024 + v_fragment<32>(j, g);
   auto scores = [&](int slot, f32x4 (&s)[2]) __attribute__((always_inline)) {
     const uint8_t* tb = &lds_k[slot][0];
 #pragma unroll
@@ -736,7 +743,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       f32x4 acc;
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(tb + kofs[c] + u * 4096);
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(tb + kofs[c] + u * 1024);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[c], c == 0 ? zero : acc, 0, 0, 0);
       }
       s[u] = acc;
@@ -763,17 +770,12 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
         if (FUSED && tile_of(t0 + d + 1) == lt) patch_k((d + 1) % NS);
         bf16x8 vf[CT];
 #pragma unroll
-        for (int i = 0; i < CT; i++) {
-          const uint2 va = *reinterpret_cast<const uint2*>(&lds_v[d][vofs0 + i * 1024]);
-          const uint2 vb = *reinterpret_cast<const uint2*>(&lds_v[d][vofs1 + i * 1024]);
-          vf[i] = __builtin_bit_cast(bf16x8, u32x4{va.x, va.y, vb.x, vb.y});
-        }
+        for (int i = 0; i < CT; i++) vf[i] = *reinterpret_cast<const bf16x8*>(&lds_v[d][vofs + i * 1024]);
         f32x4 s_next[2];
         scores((d + 1) % NS, s_next);
-        float alpha;
-        bf16x8 pf;
-        if (tile < nfull) softmax_tile<false>(s_cur, tile * 32, g, qpos, a.scale_log2, m, l, alpha, pf);
-        else softmax_tile<true>(s_cur, tile * 32, g, qpos, a.scale_log2, m, l, alpha, pf);
+        if (tile >= nfull) mask_scores(s_cur, tile * 32, g, qpos);
+        const float alpha = move_reference(lane_max(s_cur), a.scale_log2, m, l);
+        const bf16x8 pf = probabilities(s_cur, a.scale_log2, m, l);
 #pragma unroll
         for (int i = 0; i < CT; i++) o[i] = f32x4{o[i][0] * alpha, o[i][1] * alpha, o[i][2] * alpha, o[i][3] * alpha};
 #pragma unroll
@@ -785,6 +787,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
     }
     // the chunk is complete
     const int chunk = tile_of(c0) / CHUNK_TILES;
+    l = row_sum(l);
     if (SPLIT && qpos >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete with it)
       if (qvalid) {
         const int64_t at = ((int64_t)(b * sp.q_rows + qi) * a.q_heads + h) * sp.nchunks + chunk;
@@ -939,72 +942,54 @@ static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max
   return hip_code(hipGetLastError());
 }
 
-template <int G, int QB, bool DEEP, int NLD, int CHUNKS, int AHEAD = NLD ? 2 : 1>
-static void group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_q_len, hipStream_t stream) {
-  const int64_t blocks = ((int64_t)max_q_len + 16 * QB - 1) / (16 * QB);
+template <int G, int WQ, int QB, int NS, int CHUNKS>
+static int group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_q_len, hipStream_t stream) {
+  constexpr int ROWS = 16 * QB * WQ, LDS = NS * UNIT_BYTES;
+  const int64_t blocks = ((int64_t)max_q_len + ROWS - 1) / ROWS;
   const dim3 grid((unsigned)(blocks * a.kv_heads), (unsigned)batch, CHUNKS == SPLIT_CHUNKS ? (unsigned)sp.nchunks : 1u);
-  hipLaunchKernelGGL((attention_group_kernel<G, QB, DEEP, NLD, CHUNKS, AHEAD>), grid, dim3(64 * (G * QB + NLD)), 0, stream, a, sp);
+  static std::atomic<uint64_t> done{0};
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_group_kernel<G, WQ, QB, NS, CHUNKS>), LDS, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL((attention_group_kernel<G, WQ, QB, NS, CHUNKS>), grid, dim3(64 * G * WQ), LDS, stream, a, sp);
+  return hip_code(hipGetLastError());
 }
 
 // The form of the grouped kernel, same bits in all.  Lengths are the device's, so what is known is the number of
-// work-groups of one block of 16 queries and the cache length.
-// Two more waves per work-group that only stage the tiles (NLD = 2) take the loads and LDS writes out of the computing
-// waves' instruction streams.  That pays while the launch leaves CUs short of work-groups (a chunk of a prompt, a few
-// sequences: up to two work-groups per CU: 3 - 18 % faster) and costs once the chip is full, where the extra waves
-// take the place of a whole work-group (from three per CU on: 35 % slower).
-// In a cache of several chunks the accumulators of the merged chunks take a wavefront per SIMD from the others, and a
-// block of 16 queries at a time is 7 - 40 % slower than a walk without chunks is.  There two blocks share a work-group
-// (one of eight heads has eight wavefronts by itself) once a launch of that form fills the chip; before that, four
-// heads have a range in which one block without loader waves is ahead, and one or two heads keep the loader waves for as
-// long as all their work-groups are resident at once.  Measured on MI355X, us, a walk without chunks / one block / the form
-// chosen here:
-//   4 heads: 3 prompts of 4096, 3136 and 2176 tokens 327 / 347 / 308, 1 of 8192 655 / 705 / 615, 32 chunks of 64 tokens at
-//     4000 keys 206 / 273 / 182, 16 prompts of 400 in a cache of 8192 47.1 / 48.2 / 50.0; 1040 tokens (520 blocks) 24.6 /
-//     26.6 / 26.6, against 30.1 with two blocks and 24.7 with loader waves (which take 123 against 103 where 4000 keys are
-//     cached already); at 1024 blocks 2 prompts of 1020 35.6 / 35.3 / 40.2 but 8 chunks of 250 at 800 keys 39 / 45.5 / 37.7;
-//   8 heads: prompt of 4096 298 / 420 / 310, 16 of 400 87 / 111 / 87;   2 heads: 125 / 130 / 102, 1040 tokens 22.6 / 26.3 / 20.8;
-//   1 head: 217 / 225 / 126, 1040 tokens 27.0 / 28.2 / 20.8.
-// Up to 512 work-groups the loader waves fetch two tiles ahead: 4 sequences of 128 tokens at 8000 keys 194 -> 142 us, 2 of 196 at 4251
-// 105 -> 76, 2 heads 16 of 20 at 8000 207 -> 143, 1 head 4 of 64 at 1500 40 -> 27; one sequence alone, whose keys wait in the L2, 34.2 ->
-// 32.1 (405 tokens at 1633).  Beyond that the registers cost one or two heads work-groups of a CU (1 head 2 of 600 at 1870 58 -> 66).
-// What is left of the cost of the chunks is their merge, where a launch is a chain (520 tokens 12.6 -> 13.7) or its rounds
-// are few.
+// work-groups, the queries of the longest sequence and the cache length.
+//   one block of 16 queries per wavefront, two slots: two to four work-groups share a CU and fill each other's waits;
+//   the same with four slots (one work-group per CU, 96 KiB of keys on their way): a few new tokens of several sequences, whose
+//     work-groups stream keys that no other one has brought into the L2;
+//   two blocks per wavefront, two slots: half the fragment reads and half the key traffic per query, for launches that fill
+//     the chip in twice as large pieces.  That takes more work-groups where the longest sequence is as long as the cache: with
+//     nothing cached before it, its work-groups are of all lengths, and few large ones leave the chip with a tail.
+// Measured on MI355X, us, the three forms in this order (parentheses: the kernel with register staging and 16 queries per
+// fragment read that these replace):
+//   4 heads per KV head: 8192 tokens 629 / 961 / 503 (599), prompts of 4096, 3136 and 2176 321 / 488 / 256 (323), 1900 tokens at
+//     9000 keys 297 / 456 / 256 (299), 4 x 500 at 3000 116 / 170 / 100 (118), 32 x 64 at 4000 195 / 245 / 164 (182), 2 prompts of
+//     1020 29.6 / 43 / 37 (41), 526 at 3526 59 / 93 / 73 (75), 2 x 196 at 4251 62 / 66 / 88 (76), 8 x 60 at 8000
+//     130 / 118 / 161 (146), 24 x 16 at 4000 94 / 76 / 99 (80), 300 tokens 8.2 / 8.5 / 11.0 (8.8);
+//   8 heads: 4096 tokens 159 / 168 / 138 (175), 16 prompts of 400 43 / 57 / 52 (48), 32 x 64 at 4000 170 / 168 / 141 (191);
+//   2 heads: 8 x 400 at 4000 147 / 225 / 124 (184), 16 x 20 at 8000 154 / 125 / 165 (133);   1 head: 4096 tokens 91 / 136 / 95 (133).
 template <int G>
-static void group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
-  const bool deep = max_q_len <= 16;  // decode: one block of queries per sequence
-  const int64_t groups = ((int64_t)max_q_len + 15) / 16 * a.kv_heads * batch;
-#define TBIK_ATTN_GROUP(...) group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
-  if (split) {
-    if (deep) TBIK_ATTN_GROUP(1, true, 2, SPLIT_CHUNKS);
-    else TBIK_ATTN_GROUP(1, false, 2, SPLIT_CHUNKS);
-  } else if (chunks_of(a.max_len) == 1) {
-    if (groups <= 512 && deep) TBIK_ATTN_GROUP(1, true, 2, ONE_CHUNK);
-    else if (groups <= 512) TBIK_ATTN_GROUP(1, false, 2, ONE_CHUNK);
-    else if (deep) TBIK_ATTN_GROUP(1, true, 0, ONE_CHUNK);
-    else TBIK_ATTN_GROUP(1, false, 0, ONE_CHUNK);
-  } else if (deep) {
-    if (groups <= 512) TBIK_ATTN_GROUP(1, true, 2, ALL_CHUNKS);
-    else TBIK_ATTN_GROUP(1, true, 0, ALL_CHUNKS);
-  } else {
-    constexpr int LOADERS = G == 1 ? 1280 : G == 2 ? 1024 : 512, SINGLE = G == 4 ? 768 : 0, QB = G == 8 ? 1 : 2;
-    if (groups <= 512) {
-      TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS);
-      return;
+static int group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
+  constexpr int WQ = G >= 4 ? 1 : 4 / G;   // at least four wavefronts per work-group
+  const int64_t wgs = ((int64_t)max_q_len + 16 * WQ - 1) / (16 * WQ) * a.kv_heads * batch;
+  const bool one_chunk = chunks_of(a.max_len) == 1;
+  const bool prompts = (int64_t)max_q_len * 4 > (int64_t)a.max_len * 3;
+  // (work-groups of eight wavefronts: two of them share a CU with one block each and one chunk only)
+  const int64_t few = G == 8 ? (one_chunk ? INT64_MAX : prompts ? 768 : 448) : prompts ? 1152 : 640;
+  const bool two_blocks = max_q_len > 16 && wgs > few;
+#define TBIK_ATTN_GROUP(...) return group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
+  if (split) TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS);
+  if (one_chunk) {
+    if constexpr (G != 8) {
+      if (two_blocks) TBIK_ATTN_GROUP(WQ, 2, 2, ONE_CHUNK);
     }
-    if constexpr (LOADERS > 512) {
-      if (groups <= LOADERS) {
-        TBIK_ATTN_GROUP(1, false, 2, ALL_CHUNKS, 1);
-        return;
-      }
-    }
-    if constexpr (SINGLE > 0) {
-      if (groups <= SINGLE) {
-        TBIK_ATTN_GROUP(1, false, 0, ALL_CHUNKS);
-        return;
-      }
-    }
-    TBIK_ATTN_GROUP(QB, false, 0, ALL_CHUNKS);
+    TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK);
   }
+  if (two_blocks) TBIK_ATTN_GROUP(WQ, 2, 2, ALL_CHUNKS);
+  if (wgs <= 256 && max_q_len <= 64) TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS);
+  TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS);
 #undef TBIK_ATTN_GROUP
 }
 
@@ -1037,10 +1022,11 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
     const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len) : 0;
     const bool split = need != 0 && ws_bytes >= need;
     const SplitArgs sp = split ? split_args(ws, batch, max_q_len, q_heads, kv_heads, max_len) : SplitArgs{};
-    if (G == 1) group_launch<1>(a, sp, split, batch, max_q_len, stream);
-    else if (G == 2) group_launch<2>(a, sp, split, batch, max_q_len, stream);
-    else if (G == 4) group_launch<4>(a, sp, split, batch, max_q_len, stream);
-    else group_launch<8>(a, sp, split, batch, max_q_len, stream);
+    const int code = G == 1 ? group_launch<1>(a, sp, split, batch, max_q_len, stream)
+                   : G == 2 ? group_launch<2>(a, sp, split, batch, max_q_len, stream)
+                   : G == 4 ? group_launch<4>(a, sp, split, batch, max_q_len, stream)
+                            : group_launch<8>(a, sp, split, batch, max_q_len, stream);
+    if (code != TBIK_OK) return code;
     if (split) merge_launch<false>(a, sp, batch, stream);
   } else {
     const dim3 grid((unsigned)((max_q_len + 15) / 16), (unsigned)q_heads, (unsigned)batch);

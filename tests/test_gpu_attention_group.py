@@ -1,0 +1,48 @@
+"""The forms of the grouped attention kernel (one or two blocks of queries per wavefront, two or four slots of 64 keys, a chunk
+per work-group) at caches that end in the middle of a slot: the bits of the one-wave kernel, and the float64 oracle's values."""
+import math
+
+import pytest
+import torch
+
+from llm_reproducibility_amd import ops
+from oracle import tbik_oracle as O
+
+pytestmark = pytest.mark.gpu
+D, SCALE = 128, 1.0 / math.sqrt(128)
+
+
+def _at_end_of_nan(t):
+    """The tensor in memory that goes on with NaNs: a kernel that took a key behind the cache would show it."""
+    buf = torch.full((t.numel() + 4096,), math.nan, dtype=t.dtype, device=t.device)
+    buf[: t.numel()] = t.reshape(-1)
+    return buf[: t.numel()].view(t.shape)
+
+
+# query heads, KV heads, sequences, longest number of new tokens, cache length
+@pytest.mark.parametrize("hq,hkv,B,new,L", [
+    (32, 8, 28, 33, 96), (32, 8, 28, 33, 1120), (16, 8, 41, 33, 96), (16, 8, 41, 33, 1120), (8, 8, 41, 70, 96), (8, 8, 41, 70, 1120),
+    (64, 8, 20, 33, 1120),                                                            # two blocks of queries per wavefront
+    (64, 8, 20, 33, 96), (32, 8, 3, 100, 1120), (16, 8, 2, 40, 160), (4, 4, 2, 20, 32),   # one
+    (32, 8, 5, 50, 1120), (16, 8, 10, 50, 1120), (4, 4, 33, 64, 1120),                # one, four slots
+    (32, 8, 1, 40, 1120), (3, 3, 2, 20, 1568), (64, 8, 1, 17, 1120),                  # a chunk per work-group
+])
+def test_forms_at_odd_cache_lengths(dev, hq, hkv, B, new, L):
+    print("case group forms", hq, hkv, B, new, L, flush=True)
+    gen = torch.Generator(device=dev).manual_seed(hq + B + L)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    new = min(new, L)
+    qlens = [(new, 1, min(17, new), min(33, new), max(new - 1, 1))[b % 5] for b in range(B)]
+    ctxs = [max(n, (L, L - 31, L - 32, L // 2 + 1, 64, L - 63)[b % 6]) for b, n in enumerate(qlens)]
+    ctxs[-1] = L
+    starts = [sum(qlens[:i]) for i in range(B)]
+    q, kc, vt = rnd(sum(qlens), hq, D), _at_end_of_nan(rnd(B, hkv, L, D)), _at_end_of_nan(rnd(B, hkv, D, L))
+    args = (i32(starts), i32(qlens), i32(ctxs), new, SCALE)
+    got = ops.bi_attention_bf16(q, kc, vt, *args)
+    pad = torch.nn.functional.pad
+    assert torch.equal(ops.bi_attention_bf16(q, pad(kc, (0, 0, 0, 4)), pad(vt, (0, 4)), *args), got)   # the one-wave kernel
+    for b in {0, B - 1}:
+        k, v = kc[b, :, : ctxs[b]].transpose(0, 1).cpu(), vt[b, :, :, : ctxs[b]].permute(2, 0, 1).cpu()
+        mine = slice(starts[b], starts[b] + qlens[b])
+        assert not O.outside_tolerance(got[mine].cpu(), O.causal_attention(q[mine].cpu(), k, v, SCALE).to(torch.bfloat16)).any()
