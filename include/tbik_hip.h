@@ -57,7 +57,7 @@ int tbik_tree_params(int K, int leaf_k, int* T, int* flb, int* level_k);
  *   B: element (k,n) at B[k*ldb_k + n*ldb_n], as the reference passes B's strides to its kernel
  *      (src/tbik/tree_based_matmul.py:259-264).  ldb_k == 1 (the nn.Linear weight [N,K], i.e. weight.t()) is the
  *      native layout of every kernel; ldb_n == 1 (row-major [K,N], what simple_matmul.py:11-14 hands over) is
- *      consumed in place, same MFMA chain, same bits, no copy: with leaves of 256 and N a multiple of 8 on 128x128 tiles
+ *      consumed in place, same MFMA chain, same bits, no copy: with N a multiple of 8 on tiles of 128 rows by 128 or 64 columns
  *      that read it K-major through transposing LDS reads, else on 64-row tiles that transpose 8x8 blocks in registers on
  *      the way to LDS.  The kernels of many rows are built for [N,K] only (measured on MI355X, [M,12288] x [12288,4096]
  *      row-major takes 25 / 30 / 132 / 354 us at M = 16 / 128 / 700 / 2048 against 23 / 29 / 103 / 200 us for the [N,K]
@@ -91,7 +91,7 @@ size_t tbik_gemm_workspace_bytes(int M, int N, int K, int leaf_k);
 /* The same for a row-major B[K,N] (ldb_n == 1); f16 != 0: for tbik_gemm_f16. */
 size_t tbik_gemm_workspace_bytes_rowmajor_b(int M, int N, int K, int leaf_k, int f16);
 
-/* 1 where the kernel that reads a row-major B K-major in place (ldb_n == 1; leaves of 256, N a multiple of 8) takes the problem and beats a
+/* 1 where the kernel that reads a row-major B K-major in place (ldb_n == 1; N a multiple of 8) takes the problem and beats a
  * copy as [N,K] (bi_transpose) and that product.  Either way gives the same bits. */
 int tbik_gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
 /*

@@ -40,7 +40,9 @@ int gemm_tree_deep_pair_launch(const WidePair& a, hipStream_t stream);
 
 // gemm_tree_quad.hip: tree-ordered bf16 GEMM with leaves of 256 on 128x128 tiles (one wave per SIMD, the tree of a shard
 // in registers: a.lb <= 1, a.ws unused); grid.y = split as for the kernels above
-int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream, bool w_kmajor = false);
+int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream);
+// the right operand [K,N] (a.ldw its row stride, N a multiple of 8), read in place, on tiles of 128 or 64 columns; leaves of 256 or 128
+int gemm_tree_quad_kmajor_launch(const WideArgs& a, int leaf_k, bool f16, int tile_cols, int split, hipStream_t stream);
 // gemm_tree_few.hip: up to 64 rows, bf16 / fp16, tiles of `waves` (2 .. 6) times 32 columns, shards of at most
 // TREE_FEW_LEVELS binary levels; no parked levels (a.ws is not used)
 constexpr int TREE_FEW_LEVELS = 3;

@@ -416,7 +416,7 @@ struct Plan {
   int split;       // power of two, divides 2^lb
   int T, flb, lb;  // tree of ONE shard
   size_t partial_bytes, parked_bytes;
-  bool kmajor;     // a row-major B on the 128x128 tiles of gemm_tree_quad.hip (kmajor_plan)
+  int kmajor;      // a row-major B on the tiles of gemm_tree_quad.hip of that many columns (kmajor_plan), 0: other kernels
 };
 
 // Which of the two 128x256-tile kernels runs a shard whose tree has groups of `flb` leaves and `lb` binary levels.  The
@@ -523,7 +523,7 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
   const int64_t wide_tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256);
   int split = shards;
   bool wide = false;
-  pl->kmajor = false;
+  pl->kmajor = 0;
   if (M >= 64 && !rowmajor_b) {  // the wide kernels exist for [N,K] weights only
     wide_cost_us(M, N, K, leaf_k, f16, flb, lb, &split, shards);
     // exactly 64 rows fit one 64-row tile of the tiled kernel, which half-empty 128-row tiles only beat on a grid that
@@ -551,32 +551,42 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
   return true;
 }
 
-// A row-major B with leaves of 256 and columns in whole chunks of eight: in place on the 128x128 tiles of gemm_tree_quad.hip,
-// which take it K-major (kmajor.h).  K is cut until at most two groups of leaves are left to a shard (the tree that kernel
-// holds), once or not at all beyond that: the cheaper by 3 us, 0.3 us + 12.3 ns per k of a shard for every round of 256
-// work-groups, and the combine.  Returns that time in us, 0 where the kernel does not apply.  Measured on MI355X against the 64-row
-// tiles, the other kernels that read a row-major B, over M = 1 .. 2048, K = 512 .. 12288, N = 2048 .. 16384 in both types: faster
-// everywhere, [1,4096]x[4096,4096] 16.8 -> 13.4 us, [16,12288]x[12288,16384] 154 -> 85, [100,12288]x[12288,4096] 68 -> 30,
-// [1024,1536]x[1536,2048] 33.8 -> 16.7, [2048,2048]x[2048,4096] 137 -> 64.
+// A row-major B with columns in whole chunks of eight: in place on the tiles of gemm_tree_quad.hip, which take it K-major
+// (kmajor.h), 128 rows by 128 or 64 columns.  K is cut until at most two groups of leaves are left to a shard (the tree that
+// kernel holds), once or not at all beyond that.  The cheaper of all these, in us (returned; 0 where the kernel does not apply):
+//   128 columns, one work-group per CU: 3, and 0.3 + 12.3 ns per k of a shard (14.2 with leaves of 128) for every round of 256;
+//   64 columns, two per CU: 4.2, and per k of a shard 6.3 ns while the CUs are mostly idle, 2.6 + 11.5 ns per 512 work-groups
+//     beyond (a third more with leaves of 128): direct loads at some 15 TB/s from the L2s;
+//   and for a cut 3 us (7 behind tiles of 64 columns) and the combine's traffic.
+// Measured on MI355X over M = 16 .. 4096 and 26 shapes of K and N in both types (1.5 % from the best of the four on average),
+// against the 128-column tiles alone 7 % ahead on average with leaves of 256: [1024,1536]x[1536,2048] 19.0 -> 14.3 us,
+// [1024,1024]x[1024,5120] 28 -> 21.7, [16,1024]x[1024,4096] 15.9 -> 10.4; level at several rounds of a cut K, where
+// the 128-column tiles stay.  Leaves of 128 had the 64-row tiles of the tiled kernel or a
+// transposing copy before: [8,6400]x[6400,5120] 67 -> 35, [212,6400]x[6400,5120] 82 -> 50, [128,25600]x[25600,5120] 206 -> 90.
 static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
   int T, flb, level_k;
-  if (leaf_k != 256 || (N & 7) || M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return 0.0;
+  if ((N & 7) || M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return 0.0;
   const int lb = level_k - 1;
-  const int64_t tiles = (((int64_t)N + 127) / 128) * (((int64_t)M + 127) / 128);
+  const double slow = leaf_k == 128 ? 1.3 : 1.0;
   double best = 0.0;
-  for (int ls = lb > 1 ? lb - 1 : 0; ls <= lb && ls <= 5; ls++) {
-    const int sp = 1 << ls;
-    const double t = 3.0 + (double)((tiles * sp + 255) / 256) * (0.3 + 0.0123 * (K / sp)) +
-                     (sp > 1 ? 3.0 + (double)(sp + 1) * M * N * 2.0 / 5.0e6 : 0.0);
-    if (best > 0.0 && t >= best) continue;
-    best = t;
-    *pl = Plan{};
-    pl->kmajor = true;
-    pl->split = sp;
-    pl->T = T >> ls;
-    pl->flb = flb;
-    pl->lb = lb - ls;
-    pl->partial_bytes = sp > 1 ? (((size_t)sp * M * N * sizeof(uint16_t) + 255) & ~(size_t)255) : 0;
+  for (int cols = 128; cols >= 64; cols -= 64) {
+    const int64_t tiles = (((int64_t)N + cols - 1) / cols) * (((int64_t)M + 127) / 128);
+    for (int ls = lb > 1 ? lb - 1 : 0; ls <= lb && ls <= 5; ls++) {
+      const int sp = 1 << ls;
+      const double k = K / sp;
+      double t = cols == 128 ? 3.0 + (double)((tiles * sp + 255) / 256) * (0.3 + (leaf_k == 128 ? 0.0142 : 0.0123) * k)
+                             : 4.2 + k * slow * std::max(leaf_k == 128 ? 0.0070 : 0.0063, 0.0026 + 0.0115 * (double)(tiles * sp) / 512.0);
+      if (sp > 1) t += (cols == 128 ? 3.0 : 7.0) + (double)(sp + 1) * M * N * 2.0 / 5.0e6;
+      if (best > 0.0 && t >= best) continue;
+      best = t;
+      *pl = Plan{};
+      pl->kmajor = cols;
+      pl->split = sp;
+      pl->T = T >> ls;
+      pl->flb = flb;
+      pl->lb = lb - ls;
+      pl->partial_bytes = sp > 1 ? (((size_t)sp * M * N * sizeof(uint16_t) + 255) & ~(size_t)255) : 0;
+    }
   }
   return best;
 }
@@ -584,12 +594,14 @@ static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
 // Whether a row-major B is better read by those tiles than through a transposing copy (23 us for 4096 x 4096, 45 us for 12288 x
 // 4096) and the kernels for [N,K] weights: the estimate above against the copy's two passes at 4.1 TB/s and the product at 1.1
 // PFLOP/s (700 rows: 4096 x 4096 51 us against 57, 8192 x 5120 128 against 107, 12288 x 4096 133 against 137; 0.4 % from the
-// better of the two on average over 99 shapes of the sweep above, 15 % at worst).
+// better of the two on average over 99 shapes on tiles of 128 columns, 15 % at worst; the estimate for those stands 10 % high).
+// Tiles of 64 columns count in full: 1024 rows of 12288 x 4096 take 187 us on them and 153 through the copy.  With leaves of
+// 128 the product behind the copy takes 20 us more (500 rows of 3200 x 5120 66 us through the copy, 44 in place).
 bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k) {
   Plan pl;
   const double mkn = (double)M * K * N;
   const double in_place = kmajor_plan(M, N, K, leaf_k, &pl);
-  return in_place > 0.0 && 0.9 * in_place < 9.0 + (double)K * N * 4.0 / 4.1e6 + std::max(mkn / 0.55e9, 3.0 + (double)K * N * 2.0 / 5.0e6);
+  return in_place > 0.0 && (pl.kmajor == 128 ? 0.9 : 1.0) * in_place < (leaf_k == 128 ? 29.0 : 9.0) + (double)K * N * 4.0 / 4.1e6 + std::max(mkn / 0.55e9, 3.0 + (double)K * N * 2.0 / 5.0e6);
 }
 
 // Short shards, leaves of 256: where K cannot be cut into long enough pieces, tiles of 128x256 leave half of the chip idle
@@ -1042,7 +1054,7 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
     if (pl.kmajor && lda < (1 << 22) && ldw < (1 << 22)) {  // else rows too far apart for 32-bit offsets: the 64-row tiles on the same shards
       const WideArgs w{a.X, a.W, a.C, a.bias, nullptr, a.ldx, a.ldw, a.ldc, M, N, a.K, a.T, a.flb, a.lb, a.vec_store, a.k_shard,
                        pl.split > 1 ? a.c_shard : 0};
-      rc = gemm_tree_quad_launch(w, f16, pl.split, stream, true);
+      rc = gemm_tree_quad_kmajor_launch(w, leaf_k, f16, pl.kmajor, pl.split, stream);
     } else
     if (f16) rc = leaf_k == 256 ? launch_rowmajor_b<4, 6, true, true>(a, pl.split, stream) : launch_rowmajor_b<2, 6, true, true>(a, pl.split, stream);
     else rc = leaf_k == 256 ? launch_rowmajor_b<4, 6, true, false>(a, pl.split, stream) : launch_rowmajor_b<2, 6, true, false>(a, pl.split, stream);

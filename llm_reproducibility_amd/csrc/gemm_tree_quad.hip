@@ -21,8 +21,8 @@
 // costs 0.59 us against 0.385 us in the single-accumulator kernel with the same tile: the tree's two to three vector
 // instructions per MFMA do not fit behind the MFMAs of ONE wave per SIMD ([512,8192]x[8192,5120] uncut on 128x96 tiles
 // 75 us against 70 us for the 128x256-tile kernels with their K split; [256,K]x[K,N] 10-20 % slower from K = 6144 on),
-// which is why the tile widths of 32, 64 and 96 columns, the deeper rings and the leaves of 128 that this pipeline
-// also allows were measured and are not built.
+// which is why, for [N,K] operands, the tile widths of 32, 64 and 96 columns, the deeper rings and the leaves of 128 that this
+// pipeline also allows were measured and are not built (a row-major operand has 64 columns and leaves of 128 as well: kmajor_plan).
 // An uncut product of a short K (the shard of a tensor-parallel rank) gains most: no pass over partial results and twice
 // the work-groups ([1024,1536]x[1536,4096] 24.9 -> 19.6 us; the rule of the dispatch and its figures stand at narrow_plan in
 // gemm_tiled.hip).  fp16 merges a register with one packed addition.
@@ -343,9 +343,20 @@ static int tq_launch(const WideArgs& a, int split, hipStream_t stream) {
 
 // a ring of four slices (128 KiB): 2-5 % ahead of three on half of the shapes measured, level with it on the rest; five
 // are no better than three
-int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream, bool w_kmajor) {
-  if (w_kmajor) return f16 ? tq_launch<4, 4, 4, true, true>(a, split, stream) : tq_launch<4, 4, 4, false, true>(a, split, stream);
+int gemm_tree_quad_launch(const WideArgs& a, bool f16, int split, hipStream_t stream) {
   return f16 ? tq_launch<4, 4, 4, true>(a, split, stream) : tq_launch<4, 4, 4, false>(a, split, stream);
+}
+
+// K-major right operands, leaves of 256 or 128: tiles of 64 columns have a ring of three slices (72 KiB), so that two work-groups
+// share a CU and one's merges run beside the other's MFMAs; with six slices and one work-group per CU they are level on grids
+// of up to 256 and a third slower beyond ([1024,3072]x[3072,2048] 25.9 against 32.1 us)
+template <int LS, bool F16>
+static int kmajor_launch(const WideArgs& a, int tile_cols, int split, hipStream_t stream) {
+  return tile_cols == 128 ? tq_launch<4, 4, LS, F16, true>(a, split, stream) : tq_launch<2, 3, LS, F16, true>(a, split, stream);
+}
+int gemm_tree_quad_kmajor_launch(const WideArgs& a, int leaf_k, bool f16, int tile_cols, int split, hipStream_t stream) {
+  if (leaf_k == 256) return f16 ? kmajor_launch<4, true>(a, tile_cols, split, stream) : kmajor_launch<4, false>(a, tile_cols, split, stream);
+  return f16 ? kmajor_launch<2, true>(a, tile_cols, split, stream) : kmajor_launch<2, false>(a, tile_cols, split, stream);
 }
 
 }  // namespace tbik

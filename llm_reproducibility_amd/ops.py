@@ -177,8 +177,8 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
     return out if len(shape) == 2 else out.reshape(shape)
 
 
-# Where a row-major [K,N] operand that the K-major kernels do not take (`_bi_gemm_kmajor`, `_tree_operand`: odd columns, leaves of
-# 128, a K that is no multiple of 64) is repacked into the native [N,K] layout instead of being consumed in place.  In place
+# Where a row-major [K,N] operand that the K-major kernels do not take (`_bi_gemm_kmajor`, `_tree_operand`: odd columns, a K
+# that is no multiple of 64) or not at a gain is repacked into the native [N,K] layout instead of being consumed in place.  In place
 # it runs on the 64-row tiled kernels; a repack is one pass of the transposing copy kernel (23 us for 4096 x 4096 in 16 bits,
 # 45 us for 12288 x 4096) and then whatever kernel is best.  Same bits either way.  Measured on MI355X, us in place against repacked:
 #   tree matmul: in place cuts K and holds out until its 64-row tiles fill a second round of the chip, that is up to 128
