@@ -247,17 +247,15 @@ __global__ __launch_bounds__(64) void attention_kernel(const AttnArgs a) {
 // Key tiles in LDS.  A direct load puts lane l's 16 bytes at (wave-uniform address) + 16 l, so the layout is made on the global
 // side: each lane fetches the 16-byte chunk that belongs at its place.
 //   K rows [keys][256 bytes]: position pc of key row kr holds chunk pc ^ k_swizzle(kr);
-//   V^T rows [128 channels][KEYS * 2 bytes]: position pc of channel row r holds chunk pc ^ v_swizzle<KEYS>(r).
+//   V^T rows [128 channels][128 bytes = 64 keys]: position pc of channel row r holds chunk pc ^ v_swizzle(r).
 // A 16-byte read is served for lanes {0-7, 16-23} together (then {8-15, 24-31}, ...): the eight rows and two neighbouring
 // chunks of such a pass cover all 64 banks in both.
 __device__ __forceinline__ int k_swizzle(int kr) { return 2 * ((kr & 3) + 4 * ((kr >> 3) & 1)); }
-template <int KEYS>
-__device__ __forceinline__ int v_swizzle(int r) { return KEYS == 64 ? 2 * ((r >> 1) & 3) : 2 * ((r >> 2) & 1); }
+__device__ __forceinline__ int v_swizzle(int r) { return 2 * ((r >> 1) & 3); }
 // byte offsets of lane (j, g)'s fragments: chunk c of key key_row(0, j) (sub-tile 1 lies four rows = 1024 bytes on), and chunk c
 // = eight keys of channel row j (sixteen channels are 16 rows on)
 __device__ __forceinline__ uint32_t k_fragment(int j, int c) { return key_row(0, j) * 256 + ((c ^ k_swizzle(key_row(0, j))) << 4); }
-template <int KEYS>
-__device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * (KEYS * 2) + ((c ^ v_swizzle<KEYS>(j)) << 4); }
+__device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * 128 + ((c ^ v_swizzle(j)) << 4); }
 
 // ------------------------------------------------------------------------------------------------
 // Grouped variant: one work-group of NW = G * WQ wavefronts per (16 * QB * WQ consecutive queries, KV head, sequence).  A
@@ -329,7 +327,7 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
   const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vt_cache + ((int64_t)b * a.kv_heads + kvh) * (int64_t)HD * a.max_len);
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
   const int64_t vstep = (int64_t)a.max_len * 16;   // bytes of eight channel rows
-  const int vchunk = (lane & 7) ^ v_swizzle<64>(lane >> 3);
+  const int vchunk = (lane & 7) ^ v_swizzle(lane >> 3);
   const uint32_t vrow = (uint32_t)(lane >> 3) * (uint32_t)a.max_len * 2u;
   auto load_unit = [&](int unit, int slot) __attribute__((always_inline)) {
     const int k0 = min(unit * UNIT, a.max_len - 32);   // max_len is a multiple of 32
@@ -397,7 +395,7 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
   }
 #pragma unroll
   for (int hf = 0; hf < 2; hf++) {
-    vp[hf] = (lds_byte*)lds + UNIT * HD * 2 + v_fragment<64>(j, hf * 4 + g);
+    vp[hf] = (lds_byte*)lds + UNIT * HD * 2 + v_fragment(j, hf * 4 + g);
     asm volatile("" : "+v"(vp[hf]));
   }
   // tile hf of the two in a slot.  All fragments of an operand are asked for before the first MFMA that takes one (the
@@ -535,32 +533,35 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
 //     before the softmax of tile t, so the MFMA chain of one tile runs beside the exponentials of the other.
 //   * waves 4-7 do nothing but bring tiles in, with direct global->LDS loads (no staging registers, no LDS writes by a
 //     wave): a decode step is one dependent chain of key tiles per sequence, and every load a computing wave issues is a
-//     piece of that chain.  Loader i issues two of the eight 1 KiB load instructions of every K tile and V^T tile.
-// A direct load puts lane l's 16 bytes at (wave-uniform address) + 16 l, so the LDS layout is made on the global side:
-// each lane fetches the chunk that belongs at its fixed place.
-// The rows lie as k_swizzle and v_swizzle<32> say.
-// K tiles and V^T tiles have rings of NS slots each.  Iteration t reads K tile t + 1 and V^T tile t; the loaders request
-// K tile t + NS (slot t % NS, read during iteration t - 1) and V^T tile t + NS - 1 (slot (t - 1) % NS, likewise), wait
-// until what they requested NS - 2 iterations ago has landed (K tile t + 2, V^T tile t + 1: what iteration t + 1 reads),
-// and all eight waves meet at the barrier.  Tiles behind the last one are clamped to the last tile of the cache and
-// never used, so the number of loads in flight is static; nothing is in flight when a wave ends.
+//     piece of that chain.  Loader i issues two of the eight 1 KiB load instructions of every K tile and four of the sixteen
+//     of a pair of V^T tiles: whole 128-byte lines of the value cache, whose rows lie a cache length apart.
+// The rows lie in LDS as k_swizzle and v_swizzle say.
+// K tiles have a ring of NS slots, pairs of V^T tiles one of NP.  Iteration t reads K tile t + 1 and V^T tile t; the loaders request
+// K tile t + NS (slot t % NS, read during iteration t - 1) and in every second iteration the pair of V^T tiles t + 2 NP - 2,
+// t + 2 NP - 1 (the slot that iteration t - 1 finished), wait until what iteration t + 1 reads has landed (K tile t + 2, the
+// pair of V^T tile t + 1; the counts follow from the order of the requests), and all eight waves meet at the barrier.
+// Requests behind the last tile ask for the last one again (which comes from the L2: the tiles behind a context are up to 80 KB
+// that nobody needs, a fifth of the traffic at 700 keys) and are never used, so the number of loads in flight is static;
+// nothing is in flight when a wave ends.
 // A row's arithmetic -- the lanes that own it, the MFMA chains over channels and key slots, the order of the softmax
 // updates and of the chunks -- is that of the kernels above: the same bits.
 // SPLIT: gridDim.z work-groups per (KV head, sequence); work-group z takes the chunks z, z + gridDim.z, ... as one stream of
 // tiles and leaves each chunk's state in the workspace for attention_merge_kernel.  One work-group per (KV head,
-// sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8000 keys 102 us, with
-// the chunks spread over the chip 57 us, the merge included (the keys and values take 42 at the rate of a one-pass read).
+// sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8000 keys 102 us before their
+// chunks were spread over the chip (now 52, the merge included; the keys and values take 42 at the rate of a one-pass read).
 // ------------------------------------------------------------------------------------------------
-template <int G, bool FUSED, bool SPLIT>
+template <int G, bool FUSED, bool SPLIT, int NS, int NP>
 __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a, const QkvArgs f, const SplitArgs sp) {
-  constexpr int NS = 4;               // ring slots per operand (2 x 4 x 8 KiB of LDS)
+  // NS slots of K (tiles), NP of V^T (pairs of tiles)
+  constexpr int UNROLL = NS > 2 * NP ? NS : 2 * NP;
+  static_assert(NS == 4 && (NP == 2 || NP == 4) && CHUNK_TILES % UNROLL == 0, "the waits below count these");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_dyn[];
   uint8_t (*lds_k)[8192] = reinterpret_cast<uint8_t (*)[8192]>(lds_dyn);
-  uint8_t (*lds_v)[8192] = reinterpret_cast<uint8_t (*)[8192]>(lds_dyn + NS * 8192);
+  uint8_t (*lds_v)[16384] = reinterpret_cast<uint8_t (*)[16384]>(lds_dyn + NS * 8192);
   constexpr int QMAX = 16 / G;
   constexpr int CT = 2;
   constexpr int NL = 4;               // loader waves
-  constexpr int PI = 8 / NL;          // load instructions per tile, operand and loader wave
+  constexpr int PI = 8 / NL;          // load instructions per loader wave and K tile; a pair of V^T tiles takes twice as many
   const int b = blockIdx.y;
   const int kvh = blockIdx.x;
   const int z = SPLIT ? blockIdx.z : 0, nz = SPLIT ? gridDim.z : 1;
@@ -585,38 +586,43 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.k_cache + ((int64_t)b * a.kv_heads + kvh) * a.max_len * HD);
   const uint8_t* vbase = reinterpret_cast<const uint8_t*>(a.vt_cache + ((int64_t)b * a.kv_heads + kvh) * (int64_t)HD * a.max_len);
   if (wv >= 4) {
-    // ---------------- loader waves: loader li issues instructions li*PI .. li*PI+PI-1 of every K tile and V^T tile
+    // ---------------- loader waves: loader li issues instructions li*PI .. li*PI+PI-1 of every K tile, 2*li*PI .. of a V^T pair
     const int li = wv - 4;
     // K: instruction q covers key rows 4q .. 4q+3 (1 KiB): lane -> row 4q + (lane >> 4), chunk position lane & 15
-    // V^T: instruction q covers channel rows 16q .. 16q+15: lane -> row 16q + (lane >> 2), chunk position lane & 3
-    uint32_t kvoff[PI], vvoff[PI];
+    // V^T: instruction q covers channel rows 8q .. 8q+7, 128 bytes each: lane -> row 8q + (lane >> 3), chunk position lane & 7
+    // (a pair that reaches behind the cache: the second tile's lanes fetch what those of the first do, and nobody sees it)
+    uint32_t kvoff[PI], vrow[2 * PI];
 #pragma unroll
     for (int i = 0; i < PI; i++) {
-      const int q = li * PI + i;
-      const int kr = 4 * q + (lane >> 4), pc = lane & 15;
-      const int r = 16 * q + (lane >> 2), vc = (lane & 3) ^ v_swizzle<32>(r);
+      const int kr = 4 * (li * PI + i) + (lane >> 4), pc = lane & 15;
       kvoff[i] = (uint32_t)(kr * 256 + ((pc ^ k_swizzle(kr)) << 4));
-      vvoff[i] = (uint32_t)r * (uint32_t)a.max_len * 2u + vc * 16;
     }
+#pragma unroll
+    for (int i = 0; i < 2 * PI; i++) vrow[i] = (uint32_t)(8 * (2 * li * PI + i) + (lane >> 3)) * (uint32_t)a.max_len * 2u;
+    const int vchunk = (lane & 7) ^ v_swizzle(lane >> 3);   // (eight rows on, the swizzle is the same)
     const uint32_t lk = (uint32_t)(uintptr_t)&lds_k[0][0] + li * PI * 1024;
-    const uint32_t lv = (uint32_t)(uintptr_t)&lds_v[0][0] + li * PI * 1024;
+    const uint32_t lv = (uint32_t)(uintptr_t)&lds_v[0][0] + 2 * li * PI * 1024;
     auto load_k = [&](int tile, int slot) __attribute__((always_inline)) {
       const uint8_t* src = kbase + (int64_t)min(tile * 32, a.max_len - 32) * (HD * 2);
 #pragma unroll
       for (int i = 0; i < PI; i++) dma16(lk + slot * 8192 + i * 1024, kvoff[i], src);
     };
-    auto load_v = [&](int tile, int slot) __attribute__((always_inline)) {
-      const uint8_t* src = vbase + (int64_t)min(tile * 32, a.max_len - 32) * 2;
+    auto load_v = [&](int tile, int slot) __attribute__((always_inline)) {   // the pair that begins with tile `tile`
+      const int k0 = min(tile * 32, a.max_len - 32);
+      const uint8_t* src = vbase + (int64_t)k0 * 2;
+      const uint32_t at = (uint32_t)((k0 + 64 <= a.max_len ? vchunk : vchunk & 3) << 4);
 #pragma unroll
-      for (int i = 0; i < PI; i++) dma16(lv + slot * 8192 + i * 1024, vvoff[i], src);
+      for (int i = 0; i < 2 * PI; i++) dma16(lv + slot * 16384 + i * 1024, vrow[i] + at, src);
     };
     auto first_tiles = [&]() __attribute__((always_inline)) {
       load_k(tile_of(0), 0);
 #pragma unroll
       for (int i = 0; i < NS - 1; i++) {
         load_k(tile_of(i + 1), i + 1);
-        load_v(tile_of(i), i);
+        if (i % 2 == 0 && i / 2 < NP - 1) load_v(tile_of(i), i / 2);
       }
+#pragma unroll
+      for (int i = NS / 2; i < NP - 1; i++) load_v(tile_of(2 * i), i);
     };
     // on their way before the lengths are known, except where there may be no such chunk: in a cache that is mostly empty
     // most of these work-groups have nothing to do (8 sequences of 300 keys in a cache of 8192: 12.1 -> 9.0 us; the wait
@@ -641,7 +647,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       // below still count the tile loads alone
       // (SPLIT: the work-group that has the position's chunk)
       if (li < 2 && (!SPLIT || ((ctx - 1) / (32 * CHUNK_TILES)) % nz == z)) {
-        uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + 2 * NS * 8192);
+        uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + NS * 8192 + NP * 16384);
         const int pos = ctx - 1;
         const uint16_t* src = f.qkv + (int64_t)b * f.ld + (int64_t)(a.q_heads + (li == 0 ? 0 : a.kv_heads) + kvh) * HD;
         const uint16_t r1 = src[lane], r2 = src[lane + 64];
@@ -664,18 +670,20 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       }
       __syncthreads();  // the heads are in LDS
     }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PI * (NS - 1)) : "memory");  // K tile 0
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 5 : 9)) : "memory");  // K tile 0
     __syncthreads();
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PI * (NS - 2)) : "memory");  // K tile 1, V^T tile 0
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 2 : 6)) : "memory");  // K tile 1, V^T pair 0
     __syncthreads();
-    for (int t0 = 0; t0 < ntiles; t0 += NS) {
+    for (int t0 = 0; t0 < ntiles; t0 += UNROLL) {
 #pragma unroll
-      for (int d = 0; d < NS; d++) {
+      for (int d = 0; d < UNROLL; d++) {
         const int tile = t0 + d;
         if (tile >= ntiles) break;
-        load_k(tile_of(tile + NS), d);                       // slot t % NS, read during iteration t - 1
-        load_v(tile_of(tile + NS - 1), (d + NS - 1) % NS);   // slot (t - 1) % NS, likewise
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PI * (NS - 2)) : "memory");  // K tile t + 2, V^T tile t + 1
+        load_k(tile_of(min(tile + NS, ntiles - 1)), d % NS);                                        // slot of tile t, read during iteration t - 1
+        if (d % 2 == 0) load_v(tile_of(min(tile + 2 * NP - 2, (ntiles - 1) & ~1)), (d / 2 + NP - 1) % NP);   // slot of the pair that iteration t - 1 finished
+        // K tile t + 2, and the V^T pair of tile t + 1
+        if (d % 2 == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 4 : 6)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 1 : 4)) : "memory");
         __syncthreads();
       }
     }
@@ -700,7 +708,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   // value by two of the loader waves (per-head RMSNorm and rotary embedding as the stand-alone kernel does them); all are
   // left in LDS for the four computing waves and, the key and the value, filed in the caches for the steps to come.  This step takes them from LDS: the tile
   // that a loader brings in for their position holds whatever the cache held there, and is patched below.
-  uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + 2 * NS * 8192);  // [G + 2][128]: q heads, k, v
+  uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + NS * 8192 + NP * 16384);  // [G + 2][128]: q heads, k, v
   const int pos = ctx - 1;
   if (FUSED) {
     const uint16_t* row = f.qkv + (int64_t)b * f.ld;
@@ -728,13 +736,15 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   auto patch_v = [&](int slot) __attribute__((always_inline)) {
     if (lane < 16 * CT) {
       const int ch = 16 * CT * wv + lane;
-      *reinterpret_cast<uint16_t*>(&lds_v[slot][ch * 64 + (((pr >> 3) ^ v_swizzle<32>(ch)) << 4) + (pr & 7) * 2]) = hs[(G + 1) * HD + ch];
+      *reinterpret_cast<uint16_t*>(&lds_v[slot][ch * 128 + (((4 * (lt & 1) + (pr >> 3)) ^ v_swizzle(ch)) << 4) + (pr & 7) * 2]) = hs[(G + 1) * HD + ch];
     }
   };
   uint32_t kofs[4];
 #pragma unroll
   for (int c = 0; c < 4; c++) kofs[c] = k_fragment(j, c * 4 + g);
-  const uint32_t vofs = CT * wv * 1024 + v_fragment<32>(j, g);
+  uint32_t vofs[2];   // of the two tiles of a pair
+#pragma unroll
+  for (int hf = 0; hf < 2; hf++) vofs[hf] = CT * wv * 2048 + v_fragment(j, hf * 4 + g);
   auto scores = [&](int slot, f32x4 (&s)[2]) __attribute__((always_inline)) {
     const uint8_t* tb = &lds_k[slot][0];
 #pragma unroll
@@ -761,16 +771,16 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   __syncthreads();
   for (int c0 = 0; c0 < ntiles; c0 += CHUNK_TILES) {
     const int ce = min(c0 + CHUNK_TILES, ntiles);
-    for (int t0 = c0; t0 < ce; t0 += NS) {
+    for (int t0 = c0; t0 < ce; t0 += UNROLL) {
 #pragma unroll
-      for (int d = 0; d < NS; d++) {
+      for (int d = 0; d < UNROLL; d++) {
         if (t0 + d >= ce) break;
         const int tile = tile_of(t0 + d);
-        if (FUSED && tile == lt) patch_v(d);
+        if (FUSED && tile == lt) patch_v(d / 2 % NP);
         if (FUSED && tile_of(t0 + d + 1) == lt) patch_k((d + 1) % NS);
         bf16x8 vf[CT];
 #pragma unroll
-        for (int i = 0; i < CT; i++) vf[i] = *reinterpret_cast<const bf16x8*>(&lds_v[d][vofs + i * 1024]);
+        for (int i = 0; i < CT; i++) vf[i] = *reinterpret_cast<const bf16x8*>(&lds_v[d / 2 % NP][vofs[d % 2] + i * 2048]);
         f32x4 s_next[2];
         scores((d + 1) % NS, s_next);
         if (tile >= nfull) mask_scores(s_cur, tile * 32, g, qpos);
@@ -921,23 +931,33 @@ static void merge_launch(const AttnArgs& a, const SplitArgs& sp, int batch, hipS
   hipLaunchKernelGGL(attention_merge_kernel<FUSED>, grid, dim3(256), 0, stream, a, sp);
 }
 
+template <int G, bool FUSED, bool SPLIT, int NS, int NP>
+static int decode_run(const AttnArgs& a, const QkvArgs& f, const SplitArgs& sp, int batch, int nz, hipStream_t stream) {
+  const int lds = NS * 8192 + NP * 16384 + (FUSED ? (G + 2) * HD * 2 : 0);
+  static std::atomic<uint64_t> done{0};
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, SPLIT, NS, NP>), lds, done);
+  if (e != hipSuccess) return hip_code(e);
+  hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, SPLIT, NS, NP>), dim3((unsigned)a.kv_heads, (unsigned)batch, (unsigned)nz), dim3(512), lds, stream, a, f, sp);
+  return hip_code(hipGetLastError());
+}
+
+// Two slots of V^T pairs where two work-groups share a CU, four (96 KiB of LDS) where each has one of its own and its chain of
+// tiles is what a call takes.  Measured on MI355X, us, before (V^T tiles of 32 keys, half a line each, tiles behind the context
+// fetched) / now: two slots: 8 sequences of up to 8200 keys 66.5 / 58.5, 8 of 4200 30.5 / 27.7, 64 of 900 42.9 / 39.6, 48 of 1000
+// 40.3 / 34.2, 100 of 300 28.6 / 24.8, 128 of 1000 86.8 / 79.3 (12 of 8200, five work-groups to seventeen chunks, 92.6 / 93.9); four:
+// 8 of 900 13.9 / 12.6, 16 of 2300 35.5 / 30.7, 32 of 900 23.4 / 22.3, 32 of 4000 83.0 / 81.2 -- with two slots 13.1, 37.2, 24.6
+// and 89.5 there, and with four 44.4 for 64 of 900 and 68 for 8 of 8200 (both while tiles behind the context were still fetched).
+// Eight K slots beside the four cost 1 - 3 % again.
 template <int G, bool FUSED>
 static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max_q_len, void* ws, size_t ws_bytes, hipStream_t stream) {
-  const int lds = 2 * 4 * 8192 + (FUSED ? (G + 2) * HD * 2 : 0);
+  const int64_t pairs = (int64_t)batch * a.kv_heads;
   const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, a.q_heads, a.kv_heads, a.max_len) : 0;
-  if (need == 0 || ws_bytes < need) {
-    static std::atomic<uint64_t> done{0};
-    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, false>), lds, done);
-    if (e != hipSuccess) return hip_code(e);
-    hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, false>), dim3((unsigned)a.kv_heads, (unsigned)batch), dim3(512), lds, stream, a, f, SplitArgs{});
-    return hip_code(hipGetLastError());
-  }
+  if (need == 0 || ws_bytes < need)
+    return pairs <= 256 ? decode_run<G, FUSED, false, 4, 4>(a, f, SplitArgs{}, batch, 1, stream) : decode_run<G, FUSED, false, 4, 2>(a, f, SplitArgs{}, batch, 1, stream);
   const SplitArgs sp = split_args(ws, batch, max_q_len, a.q_heads, a.kv_heads, a.max_len);
-  static std::atomic<uint64_t> done{0};
-  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, true>), lds, done);
-  if (e != hipSuccess) return hip_code(e);
-  const int nz = decode_split((int64_t)batch * a.kv_heads, a.max_len);
-  hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, true>), dim3((unsigned)a.kv_heads, (unsigned)batch, (unsigned)nz), dim3(512), lds, stream, a, f, sp);
+  const int nz = decode_split(pairs, a.max_len);
+  const int rc = pairs * nz <= 256 ? decode_run<G, FUSED, true, 4, 4>(a, f, sp, batch, nz, stream) : decode_run<G, FUSED, true, 4, 2>(a, f, sp, batch, nz, stream);
+  if (rc != TBIK_OK) return rc;
   merge_launch<FUSED>(a, sp, batch, stream);
   return hip_code(hipGetLastError());
 }
