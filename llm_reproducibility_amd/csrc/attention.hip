@@ -261,7 +261,8 @@ __device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * 128 + 
 // Grouped variant: one work-group of NW = G * WQ wavefronts per (16 * QB * WQ consecutive queries, KV head, sequence).  A
 // wavefront holds one of the G query heads that share the KV head and QB blocks of 16 queries; the keys are brought in 64 at
 // a time (K and V^T, 32 KiB) by direct loads into an LDS ring of NS slots, once for the whole work-group, and every fragment
-// read from there serves the wavefront's QB blocks.  A row's arithmetic -- the lanes that own it, the MFMA chain, the order of
+// read from there serves the wavefront's QB blocks.  NLD > 0: that many more wavefronts do all the loading (their scalar
+// address arithmetic and the loads are a third of a tile's instructions) and none of the computing.  A row's arithmetic -- the lanes that own it, the MFMA chain, the order of
 // the softmax updates -- is exactly that of attention_kernel above, so the kernels produce the same bits.
 // SPLIT_CHUNKS: a work-group takes one chunk of the keys (blockIdx.z) and leaves its state in the workspace for
 // attention_merge_kernel: a few new tokens against a long cache are a handful of work-groups otherwise.
@@ -270,16 +271,20 @@ __device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * 128 + 
 // and 16 exponentials (47 %), no bank conflict, the LDS read port busy a quarter of the time.  One fragment read per 16
 // queries made it the LDS and the L2 (a 64-byte half of a V^T line per load and tile: 8.4 TB/s) instead; in work-groups of
 // 64 queries, which halve the key traffic once more, it takes the same time (532), and so does forming a tile's scores ahead.
-// Launches that leave CUs short of work-groups are a chain of 0.53 us per tile, a third of it the slot's barrier and waits.
+// Launches that leave CUs short of work-groups are a chain of tiles, 0.53 us each and 0.39 with loaders beside them.
+// (A wavefront's vector instructions do not run behind its own MFMAs: alone on a SIMD, one MFMA and three FMAs in turn take 32
+// cycles, the sum; two wavefronts of that hide a sixth of it.  Scores a tile ahead, and two blocks' exponentials between each
+// other's MFMAs, were therefore level.)
 // ------------------------------------------------------------------------------------------------
 // chunks: the cache has a single one / a work-group walks them all / a work-group takes one
 enum { ONE_CHUNK, ALL_CHUNKS, SPLIT_CHUNKS };
 constexpr int UNIT = 64, UNIT_BYTES = 4 * UNIT * HD;  // keys of a ring slot; 16 KiB of K, 16 KiB of V^T
-template <int G, int WQ, int QB, int NS, int CHUNKS>
-__global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
+template <int G, int WQ, int QB, int NS, int CHUNKS, int NLD>
+__global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1) void attention_group_kernel(const AttnArgs a, const SplitArgs sp) {
   constexpr bool SPLIT = CHUNKS == SPLIT_CHUNKS;
   constexpr int NW = G * WQ, ROWS = 16 * QB * WQ;
-  constexpr int PI = 16 / NW;                           // load instructions per slot, operand and wavefront
+  constexpr int NL = NLD ? NLD : NW;                    // wavefronts that load
+  constexpr int PI = 16 / NL;                           // load instructions per slot, operand and such a wavefront
   constexpr int CHUNK_UNITS = CHUNK_TILES * 32 / UNIT;
   static_assert((NW == 4 || NW == 8) && CHUNK_UNITS % NS == 0 && NS >= 2, "work-group shape");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -295,32 +300,16 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
   if (qb * ROWS >= qlen) return;  // uniform over the work-group
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = kvh * G + wave % G;
-  const int j = lane & 15;
-  const int g = lane >> 4;
   const int ctx = a.ctx_len[b];
-  const int row0 = qb * ROWS + wave / G * (16 * QB);   // this wavefront's first query
-  // the tiles of 32 keys that the work-group's queries see, and this wavefront's; SPLIT: up to the end of chunk blockIdx.z
+  // the tiles of 32 keys that the work-group's queries see; SPLIT: up to the end of chunk blockIdx.z
   const int tile0 = SPLIT ? (int)blockIdx.z * CHUNK_TILES : 0;
   const int all_tiles = (ctx - qlen + min(qb * ROWS + ROWS - 1, qlen - 1)) / 32 + 1;
   const int ntiles = SPLIT ? min(all_tiles, tile0 + CHUNK_TILES) : all_tiles;
   if (SPLIT && tile0 >= ntiles) return;  // uniform over the work-group
-  const int wave_tiles = min(ntiles, (ctx - qlen + min(row0 + 16 * QB - 1, qlen - 1)) / 32 + 1);
   const int unit0 = tile0 / 2, nunits = (ntiles + 1) / 2;
 
-  int qpos[QB];
-  bf16x8 qf[QB][4];
-#pragma unroll
-  for (int q = 0; q < QB; q++) {
-    const int qrow = min(row0 + 16 * q + j, qlen - 1);
-    qpos[q] = ctx - qlen + qrow;
-    const uint16_t* qp = a.q + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
-#pragma unroll
-    for (int c = 0; c < 4; c++) qf[q][c] = *reinterpret_cast<const bf16x8*>(qp + c * 32 + g * 8);
-  }
-
   // ---- staging: load instruction n of the sixteen of a slot covers key rows 4n .. 4n+3 / channel rows 8n .. 8n+7 (whole
-  // 128-byte lines of the V^T cache); this wavefront issues the instructions wave, wave + NW, ...
+  // 128-byte lines of the V^T cache); the wavefronts that load (all of them, or the NLD loaders) deal them out in turn
   // A cache whose length is an odd number of tiles ends in the middle of the last slot: K instructions behind its end fetch
   // the last rows again, and V^T lanes of the second half what those of the first half do (rows that nobody sees).
   const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.k_cache + ((int64_t)b * a.kv_heads + kvh) * a.max_len * HD);
@@ -334,13 +323,51 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
     const uint32_t voff = vrow + ((k0 + UNIT <= a.max_len ? vchunk : vchunk & 3) << 4);
 #pragma unroll
     for (int i = 0; i < PI; i++) {
-      const int n = wave + i * NW;
+      const int n = (NLD ? wave - NW : wave) + i * NL;
       const int kr = 4 * n + (lane >> 4);
       const uint32_t koff = (uint32_t)((lane >> 4) * 256 + (((lane & 15) ^ k_swizzle(kr)) << 4));
       dma16(lds0 + slot * UNIT_BYTES + n * 1024, koff, kbase + (int64_t)min(k0 + 4 * n, a.max_len - 4) * (HD * 2));
       dma16(lds0 + slot * UNIT_BYTES + UNIT * HD * 2 + n * 1024, voff, vbase + (int64_t)k0 * 2 + n * vstep);
     }
   };
+
+  // a slot has landed (this wavefront's share; up to NS - 2 slots stay in flight)
+  auto landed = [&](int unit) __attribute__((always_inline)) { wait_slices<2 * PI, NS - 2>(min(NS - 2, nunits - 1 - unit)); };
+  if (!NLD || wave >= NW) {
+#pragma unroll
+    for (int i = 0; i < NS - 1; i++)
+      if (unit0 + i < nunits) load_unit(unit0 + i, i);
+  }
+  if (NLD && wave >= NW) {   // a loader: the barriers of the loop below, and nothing else of it
+    for (int u0 = unit0; u0 < nunits; u0 += NS) {
+#pragma unroll
+      for (int d = 0; d < NS; d++) {
+        const int unit = u0 + d;
+        if (unit >= nunits) break;
+        landed(unit);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (unit + NS - 1 < nunits) load_unit(unit + NS - 1, (d + NS - 1) % NS);
+      }
+    }
+    return;
+  }
+
+  const int h = kvh * G + wave % G;
+  const int j = lane & 15;
+  const int g = lane >> 4;
+  const int row0 = qb * ROWS + wave / G * (16 * QB);   // this wavefront's first query
+  const int wave_tiles = min(ntiles, (ctx - qlen + min(row0 + 16 * QB - 1, qlen - 1)) / 32 + 1);
+  int qpos[QB];
+  bf16x8 qf[QB][4];
+#pragma unroll
+  for (int q = 0; q < QB; q++) {
+    const int qrow = min(row0 + 16 * q + j, qlen - 1);
+    qpos[q] = ctx - qlen + qrow;
+    const uint16_t* qp = a.q + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
+#pragma unroll
+    for (int c = 0; c < 4; c++) qf[q][c] = *reinterpret_cast<const bf16x8*>(qp + c * 32 + g * 8);
+  }
 
   f32x4 o[QB][8], ot[QB][8];   // this chunk's accumulators, and the merged chunks so far
   float m[QB], l[QB], mt[QB], lt[QB];
@@ -432,8 +459,8 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
 #pragma unroll
     for (int t = 0; t < 8; t++) o[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pf, o[q][t], 0, 0, 0);
   };
-  // eight MFMAs of one block beside the exponentials of another: an MFMA holds the matrix pipe for 16 cycles and takes one
-  // of its wave's issue slots, so three or four vector instructions fit behind each
+  // eight MFMAs of one block between the exponentials of another, so that neither kind comes in one long run (level within the
+  // box's noise with the order the compiler gives)
   auto interleave = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -467,9 +494,6 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
     accumulate(vf, QB - 1, pf[QB - 1]);
   };
 
-#pragma unroll
-  for (int i = 0; i < NS - 1; i++)
-    if (unit0 + i < nunits) load_unit(unit0 + i, i);
   // The queries are in their registers from here on.  (The compiler does not see the direct loads: left to the first use, its
   // wait for the queries would stand in the loop and drain every load in flight.)
 #pragma unroll
@@ -485,11 +509,11 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
         if (unit >= ce) break;
         // the slot has landed for every wave, and every wave is done with what it read from the slot before, which the
         // loads behind the barrier refill; up to NS - 2 slots stay in flight
-        wait_slices<2 * PI, NS - 2>(min(NS - 2, nunits - 1 - unit));
+        if (!NLD) landed(unit);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (unit + NS - 1 < nunits) load_unit(unit + NS - 1, (d + NS - 1) % NS);
+        if (!NLD && unit + NS - 1 < nunits) load_unit(unit + NS - 1, (d + NS - 1) % NS);
         if (2 * unit < wave_tiles) do_tile(2 * unit, d, 0);
         if (2 * unit + 1 < wave_tiles) do_tile(2 * unit + 1, d, 1);
       }
@@ -548,7 +572,7 @@ __global__ __launch_bounds__(64 * G * WQ, QB == 2 || G * WQ == 8 ? 2 : 1) void a
 // SPLIT: gridDim.z work-groups per (KV head, sequence); work-group z takes the chunks z, z + gridDim.z, ... as one stream of
 // tiles and leaves each chunk's state in the workspace for attention_merge_kernel.  One work-group per (KV head,
 // sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8000 keys 102 us before their
-// chunks were spread over the chip (now 52, the merge included; the keys and values take 42 at the rate of a one-pass read).
+// chunks were spread over the chip (now 54, the merge included; the keys and values take 42 at the rate of a one-pass read).
 // ------------------------------------------------------------------------------------------------
 template <int G, bool FUSED, bool SPLIT, int NS, int NP>
 __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a, const QkvArgs f, const SplitArgs sp) {
@@ -962,54 +986,63 @@ static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max
   return hip_code(hipGetLastError());
 }
 
-template <int G, int WQ, int QB, int NS, int CHUNKS>
+template <int G, int WQ, int QB, int NS, int CHUNKS, int NLD>
 static int group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_q_len, hipStream_t stream) {
   constexpr int ROWS = 16 * QB * WQ, LDS = NS * UNIT_BYTES;
   const int64_t blocks = ((int64_t)max_q_len + ROWS - 1) / ROWS;
   const dim3 grid((unsigned)(blocks * a.kv_heads), (unsigned)batch, CHUNKS == SPLIT_CHUNKS ? (unsigned)sp.nchunks : 1u);
   static std::atomic<uint64_t> done{0};
-  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_group_kernel<G, WQ, QB, NS, CHUNKS>), LDS, done);
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_group_kernel<G, WQ, QB, NS, CHUNKS, NLD>), LDS, done);
   if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((attention_group_kernel<G, WQ, QB, NS, CHUNKS>), grid, dim3(64 * G * WQ), LDS, stream, a, sp);
+  hipLaunchKernelGGL((attention_group_kernel<G, WQ, QB, NS, CHUNKS, NLD>), grid, dim3(64 * (G * WQ + NLD)), LDS, stream, a, sp);
   return hip_code(hipGetLastError());
 }
 
 // The form of the grouped kernel, same bits in all.  Lengths are the device's, so what is known is the number of
 // work-groups, the queries of the longest sequence and the cache length.
-//   one block of 16 queries per wavefront, two slots: two to four work-groups share a CU and fill each other's waits;
-//   the same with four slots (one work-group per CU, 96 KiB of keys on their way): a few new tokens of several sequences, whose
-//     work-groups stream keys that no other one has brought into the L2;
-//   two blocks per wavefront, two slots: half the fragment reads and half the key traffic per query, for launches that fill
-//     the chip in twice as large pieces.  That takes more work-groups where the longest sequence is as long as the cache: with
-//     nothing cached before it, its work-groups are of all lengths, and few large ones leave the chip with a tail.
-// Measured on MI355X, us, the three forms in this order (parentheses: the kernel with register staging and 16 queries per
-// fragment read that these replace):
-//   4 heads per KV head: 8192 tokens 629 / 961 / 503 (599), prompts of 4096, 3136 and 2176 321 / 488 / 256 (323), 1900 tokens at
-//     9000 keys 297 / 456 / 256 (299), 4 x 500 at 3000 116 / 170 / 100 (118), 32 x 64 at 4000 195 / 245 / 164 (182), 2 prompts of
-//     1020 29.6 / 43 / 37 (41), 526 at 3526 59 / 93 / 73 (75), 2 x 196 at 4251 62 / 66 / 88 (76), 8 x 60 at 8000
-//     130 / 118 / 161 (146), 24 x 16 at 4000 94 / 76 / 99 (80), 300 tokens 8.2 / 8.5 / 11.0 (8.8);
-//   8 heads: 4096 tokens 159 / 168 / 138 (175), 16 prompts of 400 43 / 57 / 52 (48), 32 x 64 at 4000 170 / 168 / 141 (191);
-//   2 heads: 8 x 400 at 4000 147 / 225 / 124 (184), 16 x 20 at 8000 154 / 125 / 165 (133);   1 head: 4096 tokens 91 / 136 / 95 (133).
+//   loaders: one block of 16 queries per wavefront and four more wavefronts that load, for launches of about one work-group per CU, which
+//     are a chain of tiles (and up to several rounds where the cache is one chunk: without the merged chunks in registers two such
+//     work-groups share a CU).  Two slots, and four (96 KiB of keys on their way) where keys were cached before: they come
+//     from the memory, and the work-groups that share them ask at the same time.
+//   plain: one block per wavefront, which loads for itself: two or three work-groups share a CU and fill each other's waits.
+//   two blocks: per wavefront, half the fragment reads and half the key traffic per query, for launches that fill the chip in
+//     twice as large pieces.  That takes more work-groups where the longest sequence is as long as the cache: with nothing
+//     cached before it, its work-groups are of all lengths, and few large ones leave the chip with a tail.
+// Work-groups of eight heads have eight wavefronts: no loaders beside them, and two share a CU in a cache of one chunk.
+// Measured on MI355X, us, loaders with two / with four slots, plain, two blocks (parentheses: the kernel with register staging and
+// 16 queries per fragment read that these replace):
+//   4 heads per KV head: 8192 tokens 724 / 769, 629, 503 (599), prompts of 4096, 3136 and 2176 358 / 396, 321, 256 (323), 1900 tokens
+//     at 9000 keys 346 / 365, 297, 256 (299), 4 x 500 at 3000 130 / 137, 116, 100 (118), 32 x 64 at 4000 288 / 217, 195, 152 (182),
+//     2 prompts of 1020 31 / 37, 29.3, 37 (41), 526 at 3526 71 / 75, 58, 73 (75), 1040 tokens 19.3 / 22.8, 21.4, 27.7 (26.9),
+//     2 x 196 at 4251 50 / 51, 61, 88 (76), 4 x 128 at 8000 93 / 95, 113, 160 (138), 8 x 60 at 8000 118 / 97, 130, 161 (146),
+//     24 x 16 at 4000 94 / 73, 94, 99 (80), one chunk: 16 x 400 45 / 66, 52, 47 (50), 32 x 512 144, -, 127;
+//   8 heads, plain and two blocks: 4096 tokens 159, 138 (175), 16 prompts of 400 43, 52 (48), 32 x 64 at 4000 170, 138 (191);
+//   2 heads: 8 x 400 at 4000 172 / 179, 147, 124 (184), 16 x 20 at 8000 151 / 102, 154, 165 (133), 300 at 2000 25.7 / 26.3, 30.0, 43 (34);
+//   1 head: 4096 tokens 104 / 107, 91, 95 (133), 1040 tokens 15.1 / 16.0, 18.4, 24.5 (21.1);
+//   the same with caches that hold nothing of it, 512 MB written in between: 2 x 196 at 4251 82 / 58, 88, 95 (84), 4 x 128 at 8000
+//     139 / 103, 155, 168 (149), 300 at 2000 of 2 heads 42 / 30, 44, 49 (37), 526 at 3526 93 / 81, 73, 78 (83), 16 x 400 69 / 81, 71, 60 (66).
+//   (A load per wavefront that touches the lines of the unit behind the next costs a warm L2 5 - 25 % and was not kept.)
 template <int G>
 static int group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
-  constexpr int WQ = G >= 4 ? 1 : 4 / G;   // at least four wavefronts per work-group
+  constexpr int WQ = G >= 4 ? 1 : 4 / G;   // at least four computing wavefronts per work-group
+  constexpr int NLD = G == 8 ? 0 : 4;
   const int64_t wgs = ((int64_t)max_q_len + 16 * WQ - 1) / (16 * WQ) * a.kv_heads * batch;
-  const bool one_chunk = chunks_of(a.max_len) == 1;
   const bool prompts = (int64_t)max_q_len * 4 > (int64_t)a.max_len * 3;
-  // (work-groups of eight wavefronts: two of them share a CU with one block each and one chunk only)
-  const int64_t few = G == 8 ? (one_chunk ? INT64_MAX : prompts ? 768 : 448) : prompts ? 1152 : 640;
-  const bool two_blocks = max_q_len > 16 && wgs > few;
 #define TBIK_ATTN_GROUP(...) return group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
-  if (split) TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS);
-  if (one_chunk) {
+  if (split) TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS, NLD);
+  if (chunks_of(a.max_len) == 1) {
     if constexpr (G != 8) {
-      if (two_blocks) TBIK_ATTN_GROUP(WQ, 2, 2, ONE_CHUNK);
+      if (max_q_len > 16 && wgs > 2500) TBIK_ATTN_GROUP(WQ, 2, 2, ONE_CHUNK, 0);
     }
-    TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK);
+    TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK, NLD);
   }
-  if (two_blocks) TBIK_ATTN_GROUP(WQ, 2, 2, ALL_CHUNKS);
-  if (wgs <= 256 && max_q_len <= 64) TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS);
-  TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS);
+  const int64_t few = G == 8 ? (prompts ? 768 : 448) : prompts ? 1152 : 640;
+  if (max_q_len > 16 && wgs > few) TBIK_ATTN_GROUP(WQ, 2, 2, ALL_CHUNKS, 0);
+  if (wgs <= 256 && (G == 8 ? max_q_len <= 64 : !prompts)) TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS, NLD);
+  if constexpr (NLD > 0) {
+    if (prompts && wgs <= 540) TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, NLD);
+  }
+  TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, 0);
 #undef TBIK_ATTN_GROUP
 }
 

@@ -1,5 +1,5 @@
-"""The forms of the grouped attention kernel (one or two blocks of queries per wavefront, two or four slots of 64 keys, a chunk
-per work-group) at caches that end in the middle of a slot: the bits of the one-wave kernel, and the float64 oracle's values."""
+"""The forms of the grouped attention kernel (one or two blocks of queries per wavefront, loaders beside them or not, two or
+four slots of 64 keys, a chunk per work-group) at caches that end in the middle of a slot: the bits of the one-wave kernel, and the float64 oracle's values."""
 import math
 
 import pytest
@@ -21,10 +21,11 @@ def _at_end_of_nan(t):
 
 # query heads, KV heads, sequences, longest number of new tokens, cache length
 @pytest.mark.parametrize("hq,hkv,B,new,L", [
-    (32, 8, 28, 33, 96), (32, 8, 28, 33, 1120), (16, 8, 41, 33, 96), (16, 8, 41, 33, 1120), (8, 8, 41, 70, 96), (8, 8, 41, 70, 1120),
+    (32, 8, 171, 33, 96), (32, 8, 28, 33, 1120), (16, 8, 260, 33, 96), (16, 8, 41, 33, 1120), (8, 8, 260, 70, 96), (8, 8, 41, 70, 1120),
     (64, 8, 20, 33, 1120),                                                            # two blocks of queries per wavefront
-    (64, 8, 20, 33, 96), (32, 8, 3, 100, 1120), (16, 8, 2, 40, 160), (4, 4, 2, 20, 32),   # one
-    (32, 8, 5, 50, 1120), (16, 8, 10, 50, 1120), (4, 4, 33, 64, 1120),                # one, four slots
+    (64, 8, 20, 33, 96), (32, 8, 36, 17, 1120), (16, 8, 4, 600, 1120),                # one
+    (32, 8, 28, 33, 96), (16, 8, 2, 40, 160), (4, 4, 2, 20, 32), (32, 8, 1, 1000, 1120),   # one, loaders
+    (32, 8, 3, 100, 1120), (32, 8, 5, 50, 1120), (16, 8, 10, 50, 1120), (4, 4, 33, 64, 1120), (64, 8, 5, 50, 1120),   # one, four slots
     (32, 8, 1, 40, 1120), (3, 3, 2, 20, 1568), (64, 8, 1, 17, 1120),                  # a chunk per work-group
 ])
 def test_forms_at_odd_cache_lengths(dev, hq, hkv, B, new, L):
