@@ -459,8 +459,8 @@ __global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1
 #pragma unroll
     for (int t = 0; t < 8; t++) o[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pf, o[q][t], 0, 0, 0);
   };
-  // eight MFMAs of one block between the exponentials of another, so that neither kind comes in one long run (level within the
-  // box's noise with the order the compiler gives)
+  // eight MFMAs of one block between the exponentials of another, so that neither kind comes in one long run (level, within
+  // 2 %, with the order the compiler gives)
   auto interleave = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -527,7 +527,8 @@ __global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1
 #pragma unroll
   for (int q = 0; q < QB; q++) {
     const int qrow = row0 + 16 * q + j;
-    if (qrow >= qlen) continue;
+    // (SPLIT: lengths are device data, and the workspace has rows for the caller's max_q_len, rounded up to 16)
+    if (qrow >= qlen || (SPLIT && qrow >= sp.q_rows)) continue;
     if (SPLIT && qpos[q] >= 32 * CHUNK_TILES) {   // (a row that sees one chunk only is complete here)
       const int64_t at = ((int64_t)(b * sp.q_rows + qrow) * a.q_heads + h) * sp.nchunks + blockIdx.z;
 #pragma unroll

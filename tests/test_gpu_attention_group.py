@@ -47,3 +47,19 @@ def test_forms_at_odd_cache_lengths(dev, hq, hkv, B, new, L):
         k, v = kc[b, :, : ctxs[b]].transpose(0, 1).cpu(), vt[b, :, :, : ctxs[b]].permute(2, 0, 1).cpu()
         mine = slice(starts[b], starts[b] + qlens[b])
         assert not O.outside_tolerance(got[mine].cpu(), O.causal_attention(q[mine].cpu(), k, v, SCALE).to(torch.bfloat16)).any()
+
+
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (4, 2), (8, 2)])
+def test_more_rows_than_the_caller_said(dev, monkeypatch, hq, hkv):
+    """q_len is device data: rows beyond the workspace's (max_q_len rounded up to 16) stay out of the states of the next sequence."""
+    print("case rows beyond", hq, hkv, flush=True)
+    gen = torch.Generator(device=dev).manual_seed(hq)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)  # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    L, new = 1600, 20
+    q, kc, vt = rnd(80, hq, D), rnd(2, hkv, L, D), rnd(2, hkv, D, L)
+    args = (i32([0, 60]), i32([60, 20]), i32([1590, 1500]), new, SCALE)
+    got = ops.bi_attention_bf16(q, kc, vt, *args)
+    monkeypatch.setattr(ops, "_attention_workspace", lambda *a: (None, 0))
+    want = ops.bi_attention_bf16(q, kc, vt, *args)
+    assert torch.equal(got[:32], want[:32]) and torch.equal(got[60:], want[60:])
