@@ -565,7 +565,7 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
 // transposing copy before: [8,6400]x[6400,5120] 67 -> 35, [212,6400]x[6400,5120] 82 -> 50, [128,25600]x[25600,5120] 206 -> 90.
 static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
   int T, flb, level_k;
-  if ((N & 7) || M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return 0.0;
+  if ((leaf_k != 256 && leaf_k != 128) || (N & 7) || M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return 0.0;
   const int lb = level_k - 1;
   const double slow = leaf_k == 128 ? 1.3 : 1.0;
   double best = 0.0;

@@ -110,6 +110,18 @@ def test_workspace_query_and_plan_come_from_one_decision():
     assert L.tbik_gemm_plan_info(8, 8, 256, 256, 0, 0, None) == _lib.TBIK_ERR_INVALID
 
 
+@pytest.mark.parametrize("leaf", [64, 192, 512])
+def test_a_row_major_operand_pays_only_with_leaves_a_kernel_takes(leaf):
+    """The tree kernels are built for leaves of 256 and 128 and every other product is refused: no kernel "takes the problem",
+    whatever the shape."""
+    L = _lib.lib()
+    for M in (1, 64, 300, 2048):
+        for N, K in ((4096, leaf), (2048, 6 * leaf), (5120, 24 * leaf)):
+            assert L.tbik_gemm_rowmajor_b_pays(M, N, K, leaf) == 0
+            assert L.tbik_gemm_bf16(16, K, 16, N, 1, 16, N, M, N, K, leaf, None, None, 0, None) == _lib.TBIK_ERR_UNSUPPORTED   # refused before any pointer is followed
+    assert L.tbik_gemm_rowmajor_b_pays(64, 4096, 6144, 256) == 1 and L.tbik_gemm_rowmajor_b_pays(64, 5120, 6400, 128) == 1
+
+
 @pytest.mark.parametrize("M,N,K,leaf", [(29, 151936, 8192, 256), (63, 262144, 8192, 256), (47, 200000, 25600, 128), (63, 40000, 12288, 256)])
 def test_decode_batches_fit_the_static_scratch(M, N, K, leaf):
     """However wide the matrix, a batch of fewer than 64 rows (64 may run on 128-row tiles) is not cut into more partial results than the array of
