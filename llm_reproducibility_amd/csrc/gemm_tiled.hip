@@ -1027,8 +1027,8 @@ static int gemm_dispatch_impl(bool tree, bool f16, const void* A, int64_t lda, c
     }
     return rc;
   }
-  if (tp.path == PATH_SINGLE && tp.single.kmajor && tp.bytes > ws_bytes) {
-    // less scratch than these tiles ask for (a fixed array, say): the 64-row tiles need less or none
+  if (tp.path == PATH_SINGLE && tp.single.kmajor && tp.bytes > 0 && (!ws || ws_bytes < tp.bytes || !aligned16(ws))) {
+    // less scratch than these tiles ask for (a fixed array, say), or none that can be used: the 64-row tiles need less or none
     if (!make_plan(M, N, K, leaf_k, f16, &tp.single, true)) return TBIK_ERR_INVALID;
     tp.bytes = tp.single.partial_bytes;
   }

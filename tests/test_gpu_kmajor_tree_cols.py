@@ -40,6 +40,23 @@ def test_row_major_tiles(leaf, M, K, N, f16):
             assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("leaf,M,K,N", [(128, 1000, 12800, 5120), (256, 2048, 6144, 2048)])
+def test_scratch_that_cannot_be_used(leaf, M, K, N):
+    """Enough scratch at an odd address, or none with its size: the 64-row tiles, which need none for these shapes."""
+    print("case unusable scratch", leaf, M, K, N, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A, B = torch.randn(M, K, device="cuda", generator=g).bfloat16(), (torch.randn(K, N, device="cuda", generator=g) * 0.05).bfloat16()
+    L, out, want = _lib.lib(), torch.empty(M, N, device="cuda", dtype=torch.bfloat16), ops.gemm_tree(A, B, None, leaf)
+    nbytes = L.tbik_gemm_workspace_bytes_rowmajor_b(M, N, K, leaf, 0)
+    assert nbytes > 0
+    ws = torch.empty(nbytes + 16, device="cuda", dtype=torch.uint8)
+    for ptr in (ws.data_ptr() + 8, None):
+        out.zero_()
+        assert L.tbik_gemm_bf16(A.data_ptr(), K, B.data_ptr(), N, 1, out.data_ptr(), N, M, N, K, leaf, None, ptr, nbytes,
+                                torch.cuda.current_stream().cuda_stream) == _lib.TBIK_OK
+        assert torch.equal(out, want)
+
+
 def test_leaves_of_128_against_the_oracle():
     x, w = O.integer_bf16((70, 3200), -9, 9, 0), O.integer_bf16((200, 3200), -7, 7, 1)
     B = w.t().contiguous()
