@@ -100,7 +100,7 @@ int tbik_gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k);
  *   out5[0] path: 0 one launch with K cut over the waves of a work-group (a few rows), 1 128x128 tiles (short K shards),
  *                 2 two column regions with a K split each, 3 one grid of any other kind with one K split
  *   out5[1] K split (of the first region for path 2, 0 if that region runs on 128x128 tiles; waves per strip for path 0)
- *   out5[2] columns of the first region (path 2), else 0
+ *   out5[2] columns of the first region (path 2) or of the tiles that read a row-major operand K-major (path 3: 128 or 64), else 0
  *   out5[3] K split of the second region (path 2), else 0
  *   out5[4] path 2: 1 when both regions go out as one launch; path 3: waves per work-group of the ring kernel that serves
  *           up to 64 rows (32 columns each), 0 where another kernel does; else 0

@@ -552,31 +552,41 @@ static bool make_plan(int M, int N, int K, int leaf_k, bool f16, Plan* pl, bool 
 }
 
 // A row-major B with columns in whole chunks of eight: in place on the tiles of gemm_tree_quad.hip, which take it K-major
-// (kmajor.h), 128 rows by 128 or 64 columns.  K is cut until at most two groups of leaves are left to a shard (the tree that
-// kernel holds), once or not at all beyond that.  The cheaper of all these, in us (returned; 0 where the kernel does not apply):
-//   128 columns, one work-group per CU: 3, and 0.3 + 12.3 ns per k of a shard (14.2 with leaves of 128) for every round of 256;
-//   64 columns, two per CU: 4.2, and per k of a shard 6.3 ns while the CUs are mostly idle, 2.6 + 11.5 ns per 512 work-groups
-//     beyond (a third more with leaves of 128): direct loads at some 15 TB/s from the L2s;
-//   and for a cut 3 us (7 behind tiles of 64 columns) and the combine's traffic.
-// Measured on MI355X over M = 16 .. 4096 and 26 shapes of K and N in both types (1.5 % from the best of the four on average),
-// against the 128-column tiles alone 7 % ahead on average with leaves of 256: [1024,1536]x[1536,2048] 19.0 -> 14.3 us,
-// [1024,1024]x[1024,5120] 28 -> 21.7, [16,1024]x[1024,4096] 15.9 -> 10.4; level at several rounds of a cut K, where
-// the 128-column tiles stay.  Leaves of 128 had the 64-row tiles of the tiled kernel or a
-// transposing copy before: [8,6400]x[6400,5120] 67 -> 35, [212,6400]x[6400,5120] 82 -> 50, [128,25600]x[25600,5120] 206 -> 90.
+// (kmajor.h), 128 rows by 128 (one work-group per CU) or 64 columns (two).  K is cut until at most two groups of leaves are left
+// to a shard (the tree that kernel holds), once or not at all beyond that.  The cheapest of all these by an estimate, us: a launch, the
+// rounds of 256 work-groups (a work-group's time per k of its shard, alone in its round and, of 64 columns, beside another) or
+// the weights from the memory, whichever takes longer, and for a cut the combine.  Fitted to 4648 timings on MI355X, M = 1 .. 4096,
+// K = 128 .. 25600, N = 64 .. 8192, both types, every tile and cut of 1336 shapes (9 % rms; 64 columns with leaves of 256 stand 4 %
+// high, since few rows of large weights scatter more on them); the choice is 0.9 % (leaves of 256) and 1.0 % (128) from the best of them on
+// average, p95 6 and 8 %.  (Before, with constants from the 128-column tiles, 5 and 11 %, and one in ten shapes slower than the 64-row
+// tiles or the copy that leaves of 128 had had: [3025,1536]x[1536,768] 34.1 -> 25.7 us, [1538,2048]x[2048,616] 26.9 -> 19.1,
+// [55,8192]x[8192,2560] 28.8 -> 19.8, [94,2560]x[2560,6144] with leaves of 256 20.6 -> 15.4.)
+struct KmajorCost {
+  double launch, round, per_k, per_k_full, more;   // more: per k and round beyond the first (64 columns)
+  double bytes_us;                                 // of the weights
+  double cut, cut_bytes_us;
+};
+static double kmajor_us(int cols, int leaf_k, int64_t wgs, double k, int split, double weight_bytes, double out_bytes) {
+  static const KmajorCost cost[2][2] = {
+      {{3.74, 0.0, 0.0055, 0.0023, 0.0060, 3.94e6, 2.3, 2.4e6}, {2.6, 2.4, 0.0069, 0.0034, 0.0, 3.8e6, 2.3, 3.3e6}},    // leaves of 256: 64, 128 columns
+      {{3.5, 0.0, 0.0069, 0.0027, 0.0062, 3.7e6, 2.0, 2.1e6}, {2.3, 2.8, 0.0104, 0.0030, 0.0, 3.9e6, 2.4, 3.5e6}}};   // leaves of 128
+  const KmajorCost& c = cost[leaf_k == 128][cols == 128];
+  const double rounds = (double)((wgs + 255) / 256), fill = std::min(1.0, (double)wgs / 256.0);
+  const double alone = c.round + k * (c.per_k + c.per_k_full * fill);
+  const double tiles = cols == 128 ? rounds * alone : rounds == 1.0 ? alone : rounds * k * c.more;
+  return c.launch + std::max(tiles, weight_bytes / c.bytes_us) + (split > 1 ? c.cut + (split + 1) * out_bytes / c.cut_bytes_us : 0.0);
+}
+// returns the estimate of the plan, 0 where the kernel does not apply
 static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
   int T, flb, level_k;
   if ((leaf_k != 256 && leaf_k != 128) || (N & 7) || M <= 0 || N <= 0 || tbik_tree_params(K, leaf_k, &T, &flb, &level_k) != TBIK_OK) return 0.0;
   const int lb = level_k - 1;
-  const double slow = leaf_k == 128 ? 1.3 : 1.0;
   double best = 0.0;
   for (int cols = 128; cols >= 64; cols -= 64) {
     const int64_t tiles = (((int64_t)N + cols - 1) / cols) * (((int64_t)M + 127) / 128);
     for (int ls = lb > 1 ? lb - 1 : 0; ls <= lb && ls <= 5; ls++) {
       const int sp = 1 << ls;
-      const double k = K / sp;
-      double t = cols == 128 ? 3.0 + (double)((tiles * sp + 255) / 256) * (0.3 + (leaf_k == 128 ? 0.0142 : 0.0123) * k)
-                             : 4.2 + k * slow * std::max(leaf_k == 128 ? 0.0070 : 0.0063, 0.0026 + 0.0115 * (double)(tiles * sp) / 512.0);
-      if (sp > 1) t += (cols == 128 ? 3.0 : 7.0) + (double)(sp + 1) * M * N * 2.0 / 5.0e6;
+      const double t = kmajor_us(cols, leaf_k, tiles * sp, (double)K / sp, sp, 2.0 * K * N, 2.0 * M * N);
       if (best > 0.0 && t >= best) continue;
       best = t;
       *pl = Plan{};
@@ -592,16 +602,15 @@ static double kmajor_plan(int M, int N, int K, int leaf_k, Plan* pl) {
 }
 
 // Whether a row-major B is better read by those tiles than through a transposing copy (23 us for 4096 x 4096, 45 us for 12288 x
-// 4096) and the kernels for [N,K] weights: the estimate above against the copy's two passes at 4.1 TB/s and the product at 1.1
-// PFLOP/s (700 rows: 4096 x 4096 51 us against 57, 8192 x 5120 128 against 107, 12288 x 4096 133 against 137; 0.4 % from the
-// better of the two on average over 99 shapes on tiles of 128 columns, 15 % at worst; the estimate for those stands 10 % high).
-// Tiles of 64 columns count in full: 1024 rows of 12288 x 4096 take 187 us on them and 153 through the copy.  With leaves of
-// 128 the product behind the copy takes 20 us more (500 rows of 3200 x 5120 66 us through the copy, 44 in place).
+// 4096) and the kernels for [N,K] weights: the estimate above against the copy's two passes at 4.1 TB/s, two more launches and the
+// product at 1.0 PFLOP/s (with leaves of 128 1.1 and 11 us on top).  On the shapes of the estimate the choice is 0.8 % (leaves of 256)
+// and 1.6 % (128) from the best of all tiles and the copy on average, p95 6 and 12 %; up to 128 rows the tiles always come out ahead, and did.
 bool gemm_rowmajor_b_pays(int M, int N, int K, int leaf_k) {
   Plan pl;
-  const double mkn = (double)M * K * N;
+  const double kn = (double)K * N;
   const double in_place = kmajor_plan(M, N, K, leaf_k, &pl);
-  return in_place > 0.0 && (pl.kmajor == 128 ? 0.9 : 1.0) * in_place < (leaf_k == 128 ? 29.0 : 9.0) + (double)K * N * 4.0 / 4.1e6 + std::max(mkn / 0.55e9, 3.0 + (double)K * N * 2.0 / 5.0e6);
+  const double product = std::max(M * kn / (leaf_k == 128 ? 0.55e9 : 0.5e9), 3.0 + kn * 2.0 / 5.0e6);
+  return in_place > 0.0 && in_place < (leaf_k == 128 ? 27.0 : 16.0) + kn * 4.0 / 4.1e6 + product;
 }
 
 // Short shards, leaves of 256: where K cannot be cut into long enough pieces, tiles of 128x256 leave half of the chip idle
@@ -789,7 +798,7 @@ bool gemm_sharded_pays(int M, int N, int K, int leaf_k, int shards, bool f16) {
 
 // What tree_plan() chose for a shape, for callers and tests that want to know (no effect on any result):
 // out[0] path (TreePath), out[1] K split (of the first region for path 2; waves per strip for path 0), out[2] columns of
-// the first region (path 2, else 0), out[3] K split of the second region (path 2, else 0), out[4] for path 2: 1 when the
+// the first region (path 2) or of the tiles that read a row-major operand K-major (path 3), else 0, out[3] K split of the second region (path 2, else 0), out[4] for path 2: 1 when the
 // two regions go out as one launch; for path 3: waves of the ring kernel for decode batches, 0 on the other kernels.
 int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, int out[5]) {
   TreePlan tp;
@@ -798,7 +807,7 @@ int gemm_plan_info(int M, int N, int K, int leaf_k, bool f16, bool rowmajor_b, i
   out[0] = (int)tp.path;
   out[1] = tp.path == PATH_STRIP ? tp.strip_waves : tp.path == PATH_NARROW ? tp.narrow.split
            : tp.path == PATH_REGIONS ? (tp.regions.narrow_a ? 0 : tp.regions.a.split) : tp.single.split;
-  out[2] = tp.path == PATH_REGIONS ? tp.regions.na : 0;
+  out[2] = tp.path == PATH_REGIONS ? tp.regions.na : tp.path == PATH_SINGLE ? tp.single.kmajor : 0;
   out[3] = tp.path == PATH_REGIONS ? (tp.regions.narrow_b ? 0 : tp.regions.b.split) : 0;
   out[4] = tp.path == PATH_REGIONS ? (tp.regions.pair ? 1 : 0) : tp.path == PATH_SINGLE ? tp.single.few_waves : 0;
   return TBIK_OK;

@@ -177,9 +177,9 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
     return out if len(shape) == 2 else out.reshape(shape)
 
 
-# Where a row-major [K,N] operand that the K-major kernels do not take (`_bi_gemm_kmajor`, `_tree_operand`: odd columns, a K
-# that is no multiple of 64) or not at a gain is repacked into the native [N,K] layout instead of being consumed in place.  In place
-# it runs on the 64-row tiled kernels; a repack is one pass of the transposing copy kernel (23 us for 4096 x 4096 in 16 bits,
+# Where a row-major [K,N] operand that the K-major kernels do not take (`_bi_gemm_kmajor`: odd columns, a K that is no multiple of
+# 64, or no gain; `_tree_operand`: columns that are no multiple of eight, 256 leaves and more) is repacked into the native [N,K]
+# layout instead of being consumed in place.  In place it runs on the 64-row tiled kernels; a repack is one pass of the transposing copy kernel (23 us for 4096 x 4096 in 16 bits,
 # 45 us for 12288 x 4096) and then whatever kernel is best.  Same bits either way.  Measured on MI355X, us in place against repacked:
 #   tree matmul: in place cuts K and holds out until its 64-row tiles fill a second round of the chip, that is up to 128
 #     rows (12288 x 4096: 68 against 73; at 192 rows 99 against 79, at 1024 448 against 164), later for small matrices
@@ -190,11 +190,10 @@ def _unflat(out: torch.Tensor, shape) -> torch.Tensor:
 #     64), wide ones not while they are one round (12288 x 16384: 220 against 273 at 64 rows, 248 against 318 at 256; 4096 x
 #     24576: 93 against 123 at 128 rows, 158 against 138 at 160).  K, the rounds and, for a K that is no multiple of 64, the type (fp16
 #     has the large tiles of bf16 for whole slices only) move the line, so both times are estimated.
-#   Both estimates are of whole column tiles (N a multiple of 128, of 64 up to 16 rows).  Of the operands that come here, 1 .. 3072
-#     rows, K = 512 .. 25600, N = 512 .. 48000 in both types: on whole tiles the choice is 0.5 % from the better of the two on average
-#     and 12 % at worst for the mm (62 points), 3 % and 32 % for the tree (33).  A last tile that is not whole costs the 64-row
-#     tiles two to four times the time, which the estimates do not know: where such an operand stays in place (118 of 655 points
-#     of the mm, 119 of 171 of the tree) a repack would nearly always be ahead, 1.8 times on average.
+#   Both estimates are of whole column tiles (N a multiple of 128, of 64 up to 16 rows): for the mm, 1 .. 3072 rows, K = 512 .. 25600, N =
+#     512 .. 48000 in both types, the choice is 0.5 % from the better of the two on average there and 12 % at worst (62 points).  A
+#     last tile that is not whole, which every tree operand has that comes here, costs the 64-row tiles two to four times the time, which the
+#     estimates do not know: where such an operand stays in place a repack would nearly always be ahead, 1.8 times on average.
 _TREE_IN_PLACE_MACS = 416 * 2048 * 1536
 
 
@@ -230,10 +229,15 @@ def _weight_operand(B: torch.Tensor, rows: int = 0, tree: bool = True):
 
 
 def _tree_operand(B: torch.Tensor, rows: int, leaf_k: int):
-    """`_weight_operand` of a tree matmul: a row-major operand also stays where the library reads it K-major at a gain."""
+    """`_weight_operand` of a tree matmul: a row-major operand that the library can read K-major (whole chunks of eight columns,
+    and a tree that those tiles hold: fewer than 256 leaves always are) stays in place where it says that this pays, and is
+    repacked where it does not."""
     (K, N), (s0, s1) = B.shape, B.stride()
-    if s1 == 1 and _aligned16(B) and s0 >= N and s0 % 8 == 0 and _lib.lib().tbik_gemm_rowmajor_b_pays(rows, N, K, leaf_k):
-        return B, s0, 1
+    if s1 == 1 and N % 8 == 0 and _aligned16(B) and s0 >= N and s0 % 8 == 0 and K < 256 * leaf_k:
+        if _lib.lib().tbik_gemm_rowmajor_b_pays(rows, N, K, leaf_k):
+            return B, s0, 1
+        w, ldw = _rows16(B.t())
+        return w, 1, ldw
     return _weight_operand(B, rows, True)
 
 

@@ -122,6 +122,19 @@ def test_a_row_major_operand_pays_only_with_leaves_a_kernel_takes(leaf):
     assert L.tbik_gemm_rowmajor_b_pays(64, 4096, 6144, 256) == 1 and L.tbik_gemm_rowmajor_b_pays(64, 5120, 6400, 128) == 1
 
 
+@pytest.mark.parametrize("M,N,K,leaf,cols,split", [
+    (3025, 768, 1536, 128, 64, 2),      # 25.7 us; on tiles of 128 columns 33.2, behind a transposing copy 25.7
+    (1538, 616, 2048, 128, 64, 4),      # 19.1; 26.4, 21.2
+    (55, 2560, 8192, 128, 64, 16),      # 19.8; 24.9, 32.9
+    (94, 6144, 2560, 256, 64, 2),       # 15.4; 19.3, 37.2
+    (1024, 2048, 1536, 256, 64, 1),     # 14.3; 19.0
+])
+def test_row_major_operands_run_on_the_tiles_measured_fastest(M, N, K, leaf, cols, split):
+    out = (ctypes.c_int * 5)()
+    assert _lib.lib().tbik_gemm_plan_info(M, N, K, leaf, 0, 1, out) == _lib.TBIK_OK
+    assert list(out) == [3, split, cols, 0, 0] and _lib.lib().tbik_gemm_rowmajor_b_pays(M, N, K, leaf) == 1
+
+
 @pytest.mark.parametrize("M,N,K,leaf", [(29, 151936, 8192, 256), (63, 262144, 8192, 256), (47, 200000, 25600, 128), (63, 40000, 12288, 256)])
 def test_decode_batches_fit_the_static_scratch(M, N, K, leaf):
     """However wide the matrix, a batch of fewer than 64 rows (64 may run on 128-row tiles) is not cut into more partial results than the array of
