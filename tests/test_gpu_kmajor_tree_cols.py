@@ -1,5 +1,7 @@
 """Tree matmuls on a row-major right operand, read in place on tiles of 64 and 128 columns, leaves of 256 and of 128: the bits of
 the same product on the K-contiguous copy."""
+import ctypes
+
 import pytest
 import torch
 
@@ -8,10 +10,27 @@ from oracle import tbik_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# shards of one and two groups of leaves, groups of one and of several, uncut and cut, ends in rows, columns and tiles of 64
+# groups of one leaf and of several, uncut and cut, ends in rows, columns and tiles of 64
 CASES = [(256, 1024, 1536, 2048), (256, 16, 1024, 4096), (256, 130, 768, 200), (256, 1000, 1024, 5112), (256, 300, 6144, 1032), (256, 1, 256, 72),
          (128, 1, 128, 8), (128, 8, 6400, 5120), (128, 212, 6400, 520), (128, 129, 3200, 136), (128, 50, 25600, 264), (128, 257, 1152, 72),
          (128, 1000, 6400, 1288), (128, 33, 896, 64), (128, 2100, 256, 4096)]
+
+
+# shards of one and of two groups of leaves (two: the carry and the binary level of the kernel), a group of two leaves and of
+# more, on both widths with both leaves: leaf, M, K, N, columns of a tile, cut, groups in a shard
+PLANNED = [(128, 129, 768, 2056, 64, 1, 2), (128, 100, 512, 72, 64, 1, 2), (128, 1, 6144, 5112, 64, 8, 2), (128, 33, 2048, 8184, 128, 4, 2),
+           (128, 1, 3072, 8184, 128, 4, 2), (128, 33, 5120, 8184, 128, 4, 2), (128, 1, 2560, 8184, 128, 4, 1), (128, 33, 1536, 8184, 128, 4, 1),
+           (256, 129, 1536, 4104, 64, 1, 2), (256, 257, 1024, 1032, 64, 1, 2), (256, 1, 8192, 5112, 64, 8, 2), (256, 33, 4096, 5112, 128, 4, 2),
+           (256, 129, 1024, 8200, 128, 1, 2), (256, 1, 6144, 5112, 128, 4, 2), (256, 1, 3072, 4104, 128, 4, 1)]
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("leaf,M,K,N,cols,split,groups", PLANNED)
+def test_each_form_of_the_tiles(leaf, M, K, N, cols, split, groups, f16):
+    info = (ctypes.c_int * 5)()
+    assert _lib.lib().tbik_gemm_plan_info(M, N, K, leaf, int(f16), 1, info) == _lib.TBIK_OK
+    assert (info[2], info[1]) == (cols, split) and _lib.tree_params(K // split, leaf)[2] == groups
+    test_row_major_tiles(leaf, M, K, N, f16)
 
 
 @pytest.mark.parametrize("f16", [False, True])
