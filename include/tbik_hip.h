@@ -298,6 +298,17 @@ int bi_attention_ws_bf16(const void* q, const void* k_cache, const void* vt_cach
                          const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
                          int batch, int max_q_len, int q_heads, int kv_heads, int head_dim, int max_len,
                          float scale, void* workspace_or_null, size_t workspace_bytes, tbik_stream_t stream);
+/*
+ * How such a call would run, for callers and tests that want to see it (host only, launches nothing, no effect on any result; the
+ * one-launch decode step runs as a call with max_q_len = 1):
+ *   out6[0] kernel: 0 one wavefront per 16 queries and head (caches of no whole number of 32 keys, more than 8 or an odd number of
+ *           query heads per KV head), 1 the query heads of a KV head in one work-group, 2 decode (max_q_len times those heads <= 16)
+ *   out6[1] work-groups that share the chunks of a row (1: none do)
+ *   out6[2] kernel 1: ring slots of 64 keys; kernel 2: ring slots of pairs of 32 keys of the value cache
+ *   out6[3] queries per work-group   out6[4] kernel 1: blocks of 16 queries per wavefront
+ *   out6[5] wavefronts that load beside the computing ones
+ */
+int bi_attention_plan_info(int batch, int max_q_len, int q_heads, int kv_heads, int max_len, size_t workspace_bytes, int* out6);
 
 /*
  * fp16 counterparts of tbik_gemm_bf16 / tbik_gemm_workspace_bytes / tbik_tree_combine_bf16 / bi_gemm_bf16: same

@@ -28,7 +28,7 @@ EXPORTS = (
     "tbik_gemm_bf16_static", "bi_log_softmax", "tbik_gemm_workspace_bytes_rowmajor_b", "tbik_gemm_rowmajor_b_pays", "tbik_gemm_plan_info",
     "bi_rmsnorm_gemm_bf16", "tbik_gemm_silu_mul_bf16", "bi_argmax_advance_bf16",
     "tbik_gemm_rmsnorm_bf16", "tbik_tree_combine_rmsnorm_bf16", "bi_attention_decode_qkv_bf16", "bi_gemm_silu_mul_bf16",
-    "tbik_gemm_sharded", "tbik_gemm_sharded_workspace_bytes", "tbik_gemm_sharded_pays", "bi_transpose", "bi_gemm_kmajor_bf16", "bi_gemm_kmajor_f16", "bi_attention_workspace_bytes", "bi_attention_ws_bf16", "bi_attention_decode_qkv_ws_bf16",
+    "tbik_gemm_sharded", "tbik_gemm_sharded_workspace_bytes", "tbik_gemm_sharded_pays", "bi_transpose", "bi_gemm_kmajor_bf16", "bi_gemm_kmajor_f16", "bi_attention_workspace_bytes", "bi_attention_plan_info", "bi_attention_ws_bf16", "bi_attention_decode_qkv_ws_bf16",
 )
 
 _lib = None
@@ -143,6 +143,8 @@ def lib() -> ctypes.CDLL:
     L.tbik_gemm_silu_mul_bf16.restype = i32
     L.bi_attention_bf16.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, f32, vp]
     L.bi_attention_bf16.restype = i32
+    L.bi_attention_plan_info.argtypes = [i32, i32, i32, i32, i32, sz, pi32]
+    L.bi_attention_plan_info.restype = i32
     L.bi_attention_workspace_bytes.argtypes = [i32, i32, i32, i32, i32]
     L.bi_attention_workspace_bytes.restype = sz
     L.bi_attention_ws_bf16.argtypes = L.bi_attention_bf16.argtypes[:-1] + [vp, sz, vp]

@@ -559,30 +559,35 @@ __global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1
 //   * waves 4-7 do nothing but bring tiles in, with direct global->LDS loads (no staging registers, no LDS writes by a
 //     wave): a decode step is one dependent chain of key tiles per sequence, and every load a computing wave issues is a
 //     piece of that chain.  Loader i issues two of the eight 1 KiB load instructions of every K tile and four of the sixteen
-//     of a pair of V^T tiles: whole 128-byte lines of the value cache, whose rows lie a cache length apart.
+//     of a pair of V^T tiles, 128 bytes of a channel row: whole lines of the value cache where the cache length is a
+//     multiple of 64 (of an odd number of tiles, every second row begins in the middle of a line and its pieces touch two).
 // The rows lie in LDS as k_swizzle and v_swizzle say.
 // K tiles have a ring of NS slots, pairs of V^T tiles one of NP.  Iteration t reads K tile t + 1 and V^T tile t; the loaders request
 // K tile t + NS (slot t % NS, read during iteration t - 1) and in every second iteration the pair of V^T tiles t + 2 NP - 2,
 // t + 2 NP - 1 (the slot that iteration t - 1 finished), wait until what iteration t + 1 reads has landed (K tile t + 2, the
-// pair of V^T tile t + 1; the counts follow from the order of the requests), and all eight waves meet at the barrier.
-// Requests behind the last tile ask for the last one again (which comes from the L2: the tiles behind a context are up to 80 KB
-// that nobody needs, a fifth of the traffic at 700 keys) and are never used, so the number of loads in flight is static;
-// nothing is in flight when a wave ends.
+// pair of V^T tile t + 1; the counts follow from the order of the requests, and with the K ring's depth that order keeps a fourth
+// slot of pairs from being any further ahead than a third), and all eight waves meet at the barrier.
+// Only the first two K tiles and the first pair, 32 KB, are asked for without a look at the context (with two slots of pairs two more K
+// tiles: 64 sequences of 300 keys 18.2 -> 17.8 us).  Requests behind its last tile ask for that one again (which
+// comes from the L2; the tiles behind a context are up to 80 KB that nobody needs, a fifth of the
+// traffic at 700 keys) and are never used, so the number of loads in flight is static; nothing is in flight when a wave ends.
 // A row's arithmetic -- the lanes that own it, the MFMA chains over channels and key slots, the order of the softmax
 // updates and of the chunks -- is that of the kernels above: the same bits.
 // SPLIT: gridDim.z work-groups per (KV head, sequence); work-group z takes the chunks z, z + gridDim.z, ... as one stream of
 // tiles and leaves each chunk's state in the workspace for attention_merge_kernel.  One work-group per (KV head,
 // sequence) is a chain of 0.35 us per tile on as many CUs as there are such pairs: 8 sequences of 8000 keys 102 us before their
-// chunks were spread over the chip (now 54, the merge included; the keys and values take 42 at the rate of a one-pass read).
+// chunks were spread over the chip (now 54, the merge included, in a cache of a multiple of 64 keys; the keys and values take 42
+// at the rate of a one-pass read).
 // ------------------------------------------------------------------------------------------------
-template <int G, bool FUSED, bool SPLIT, int NS, int NP>
+template <int G, bool FUSED, bool SPLIT, int NP>
 __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a, const QkvArgs f, const SplitArgs sp) {
-  // NS slots of K (tiles), NP of V^T (pairs of tiles)
-  constexpr int UNROLL = NS > 2 * NP ? NS : 2 * NP;
-  static_assert(NS == 4 && (NP == 2 || NP == 4) && CHUNK_TILES % UNROLL == 0, "the waits below count these");
+  constexpr int NS = 4;   // slots of K (tiles); NP of V^T (pairs of tiles)
+  static_assert((NP == 2 || NP == 3) && CHUNK_TILES % NS == 0, "the waits below count these");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_dyn[];
   uint8_t (*lds_k)[8192] = reinterpret_cast<uint8_t (*)[8192]>(lds_dyn);
   uint8_t (*lds_v)[16384] = reinterpret_cast<uint8_t (*)[16384]>(lds_dyn + NS * 8192);
+  // FUSED: [G + 2][128] q heads, new key, new value, in the slot that the first iteration's loads refill
+  uint16_t* hs = reinterpret_cast<uint16_t*>(lds_v[NP - 1]);
   constexpr int QMAX = 16 / G;
   constexpr int CT = 2;
   constexpr int NL = 4;               // loader waves
@@ -641,18 +646,17 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
     };
     auto first_tiles = [&]() __attribute__((always_inline)) {
       load_k(tile_of(0), 0);
-#pragma unroll
-      for (int i = 0; i < NS - 1; i++) {
-        load_k(tile_of(i + 1), i + 1);
-        if (i % 2 == 0 && i / 2 < NP - 1) load_v(tile_of(i), i / 2);
-      }
-#pragma unroll
-      for (int i = NS / 2; i < NP - 1; i++) load_v(tile_of(2 * i), i);
+      load_k(tile_of(1), 1);
+      load_v(tile_of(0), 0);
     };
     // on their way before the lengths are known, except where there may be no such chunk: in a cache that is mostly empty
     // most of these work-groups have nothing to do (8 sequences of 300 keys in a cache of 8192: 12.1 -> 9.0 us; the wait
     // costs full caches at most 1 us of 57)
     if (z == 0) first_tiles();
+    if (NP == 2 && z == 0) {
+      load_k(tile_of(2), 2);
+      load_k(tile_of(3), 3);
+    }
     const int ctx = a.ctx_len[b];
     const int qlen = FUSED ? (ctx > 0 ? 1 : 0) : a.q_len[b];
     if (qlen <= 0) {
@@ -666,13 +670,18 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       return;
     }
     if (z != 0) first_tiles();
+    const int last = max(ntiles - 1, 0);
+    if (NP == 3 || z != 0) {
+      load_k(tile_of(min(2, last)), 2);
+      load_k(tile_of(min(3, last)), 3);
+    }
+    if (NP == 3) load_v(tile_of(min(2, last & ~1)), 1);
     if (FUSED) {
       // loaders 0 and 1 form the new key and file the new value while the first tiles are on their way (the computing
       // waves form the query heads meanwhile); everything they have in flight is drained before the barrier, so the waits
       // below still count the tile loads alone
       // (SPLIT: the work-group that has the position's chunk)
       if (li < 2 && (!SPLIT || ((ctx - 1) / (32 * CHUNK_TILES)) % nz == z)) {
-        uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + NS * 8192 + NP * 16384);
         const int pos = ctx - 1;
         const uint16_t* src = f.qkv + (int64_t)b * f.ld + (int64_t)(a.q_heads + (li == 0 ? 0 : a.kv_heads) + kvh) * HD;
         const uint16_t r1 = src[lane], r2 = src[lane + 64];
@@ -695,17 +704,21 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
       }
       __syncthreads();  // the heads are in LDS
     }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 5 : 9)) : "memory");  // K tile 0
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 5 : 7)) : "memory");  // K tile 0
     __syncthreads();
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 2 : 6)) : "memory");  // K tile 1, V^T pair 0
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 2 : 4)) : "memory");  // K tile 1, V^T pair 0
     __syncthreads();
-    for (int t0 = 0; t0 < ntiles; t0 += UNROLL) {
+    int vslot = NP - 1;   // of the pair that is asked for next
+    for (int t0 = 0; t0 < ntiles; t0 += NS) {
 #pragma unroll
-      for (int d = 0; d < UNROLL; d++) {
+      for (int d = 0; d < NS; d++) {
         const int tile = t0 + d;
         if (tile >= ntiles) break;
-        load_k(tile_of(min(tile + NS, ntiles - 1)), d % NS);                                        // slot of tile t, read during iteration t - 1
-        if (d % 2 == 0) load_v(tile_of(min(tile + 2 * NP - 2, (ntiles - 1) & ~1)), (d / 2 + NP - 1) % NP);   // slot of the pair that iteration t - 1 finished
+        load_k(tile_of(min(tile + NS, last)), d);   // slot of tile t, read during iteration t - 1
+        if (d % 2 == 0) {
+          load_v(tile_of(min(tile + 2 * NP - 2, last & ~1)), NP == 2 ? 1 - d / 2 : vslot);   // slot of the pair that iteration t - 1 finished
+          vslot = vslot == NP - 1 ? 0 : vslot + 1;
+        }
         // K tile t + 2, and the V^T pair of tile t + 1
         if (d % 2 == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 4 : 6)) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PI * (NP == 2 ? 1 : 4)) : "memory");
@@ -733,8 +746,9 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   // value by two of the loader waves (per-head RMSNorm and rotary embedding as the stand-alone kernel does them); all are
   // left in LDS for the four computing waves and, the key and the value, filed in the caches for the steps to come.  This step takes them from LDS: the tile
   // that a loader brings in for their position holds whatever the cache held there, and is patched below.
-  uint16_t* hs = reinterpret_cast<uint16_t*>(lds_dyn + NS * 8192 + NP * 16384);  // [G + 2][128]: q heads, k, v
   const int pos = ctx - 1;
+  u32x4 new_k = {0, 0, 0, 0};   // lanes 0-15: the new key's chunk `lane`
+  uint16_t new_v = 0;           // lanes 0-31: the new value's channel 32 wv + lane
   if (FUSED) {
     const uint16_t* row = f.qkv + (int64_t)b * f.ld;
     for (int u = wv; u < G; u += 4) {  // wave-uniform: the query heads (loaders 0 and 1 take the key and the value)
@@ -746,6 +760,8 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; c++) qf[c] = *reinterpret_cast<const bf16x8*>(hs + (j % G) * HD + c * 32 + g * 8);
+    new_k = *reinterpret_cast<const u32x4*>(hs + G * HD + j * 8);
+    new_v = hs[(G + 1) * HD + 16 * CT * wv + (lane & 31)];
   } else {
     const uint16_t* qp = a.q + ((int64_t)(a.q_start[b] + qrow) * a.q_heads + h) * HD;
 #pragma unroll
@@ -756,12 +772,12 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   const int lt = pos >> 5, pr = pos & 31;
   auto patch_k = [&](int slot) __attribute__((always_inline)) {
     if (lane < 16)
-      *reinterpret_cast<u32x4*>(&lds_k[slot][pr * 256 + ((lane ^ k_swizzle(pr)) << 4)]) = *reinterpret_cast<const u32x4*>(hs + G * HD + lane * 8);
+      *reinterpret_cast<u32x4*>(&lds_k[slot][pr * 256 + ((lane ^ k_swizzle(pr)) << 4)]) = new_k;
   };
   auto patch_v = [&](int slot) __attribute__((always_inline)) {
     if (lane < 16 * CT) {
       const int ch = 16 * CT * wv + lane;
-      *reinterpret_cast<uint16_t*>(&lds_v[slot][ch * 128 + (((4 * (lt & 1) + (pr >> 3)) ^ v_swizzle(ch)) << 4) + (pr & 7) * 2]) = hs[(G + 1) * HD + ch];
+      *reinterpret_cast<uint16_t*>(&lds_v[slot][ch * 128 + (((4 * (lt & 1) + (pr >> 3)) ^ v_swizzle(ch)) << 4) + (pr & 7) * 2]) = new_v;
     }
   };
   uint32_t kofs[4];
@@ -794,18 +810,19 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
   f32x4 s_cur[2];
   scores(0, s_cur);
   __syncthreads();
+  int vslot = 0;   // of this iteration's pair
   for (int c0 = 0; c0 < ntiles; c0 += CHUNK_TILES) {
     const int ce = min(c0 + CHUNK_TILES, ntiles);
-    for (int t0 = c0; t0 < ce; t0 += UNROLL) {
+    for (int t0 = c0; t0 < ce; t0 += NS) {
 #pragma unroll
-      for (int d = 0; d < UNROLL; d++) {
+      for (int d = 0; d < NS; d++) {
         if (t0 + d >= ce) break;
-        const int tile = tile_of(t0 + d);
-        if (FUSED && tile == lt) patch_v(d / 2 % NP);
+        const int tile = tile_of(t0 + d), vs = NP == 2 ? d / 2 : vslot;
+        if (FUSED && tile == lt) patch_v(vs);
         if (FUSED && tile_of(t0 + d + 1) == lt) patch_k((d + 1) % NS);
         bf16x8 vf[CT];
 #pragma unroll
-        for (int i = 0; i < CT; i++) vf[i] = *reinterpret_cast<const bf16x8*>(&lds_v[d / 2 % NP][vofs[d % 2] + i * 2048]);
+        for (int i = 0; i < CT; i++) vf[i] = *reinterpret_cast<const bf16x8*>(&lds_v[vs][vofs[d % 2] + i * 2048]);
         f32x4 s_next[2];
         scores((d + 1) % NS, s_next);
         if (tile >= nfull) mask_scores(s_cur, tile * 32, g, qpos);
@@ -818,6 +835,7 @@ __global__ __launch_bounds__(512) void attention_decode_kernel(const AttnArgs a,
         __syncthreads();
         s_cur[0] = s_next[0];
         s_cur[1] = s_next[1];
+        if (d % 2 == 1) vslot = vslot == NP - 1 ? 0 : vslot + 1;
       }
     }
     // the chunk is complete
@@ -956,32 +974,37 @@ static void merge_launch(const AttnArgs& a, const SplitArgs& sp, int batch, hipS
   hipLaunchKernelGGL(attention_merge_kernel<FUSED>, grid, dim3(256), 0, stream, a, sp);
 }
 
-template <int G, bool FUSED, bool SPLIT, int NS, int NP>
+template <int G, bool FUSED, bool SPLIT, int NP>
 static int decode_run(const AttnArgs& a, const QkvArgs& f, const SplitArgs& sp, int batch, int nz, hipStream_t stream) {
-  const int lds = NS * 8192 + NP * 16384 + (FUSED ? (G + 2) * HD * 2 : 0);
+  constexpr int LDS = 4 * 8192 + NP * 16384;
   static std::atomic<uint64_t> done{0};
-  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, SPLIT, NS, NP>), lds, done);
+  const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(attention_decode_kernel<G, FUSED, SPLIT, NP>), LDS, done);
   if (e != hipSuccess) return hip_code(e);
-  hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, SPLIT, NS, NP>), dim3((unsigned)a.kv_heads, (unsigned)batch, (unsigned)nz), dim3(512), lds, stream, a, f, sp);
+  hipLaunchKernelGGL((attention_decode_kernel<G, FUSED, SPLIT, NP>), dim3((unsigned)a.kv_heads, (unsigned)batch, (unsigned)nz), dim3(512), LDS, stream, a, f, sp);
   return hip_code(hipGetLastError());
 }
 
-// Two slots of V^T pairs where two work-groups share a CU, four (96 KiB of LDS) where each has one of its own and its chain of
-// tiles is what a call takes.  Measured on MI355X, us, before (V^T tiles of 32 keys, half a line each, tiles behind the context
-// fetched) / now: two slots: 8 sequences of up to 8200 keys 66.5 / 58.5, 8 of 4200 30.5 / 27.7, 64 of 900 42.9 / 39.6, 48 of 1000
-// 40.3 / 34.2, 100 of 300 28.6 / 24.8, 128 of 1000 86.8 / 79.3 (12 of 8200, five work-groups to seventeen chunks, 92.6 / 93.9); four:
-// 8 of 900 13.9 / 12.6, 16 of 2300 35.5 / 30.7, 32 of 900 23.4 / 22.3, 32 of 4000 83.0 / 81.2 -- with two slots 13.1, 37.2, 24.6
-// and 89.5 there, and with four 44.4 for 64 of 900 and 68 for 8 of 8200 (both while tiles behind the context were still fetched).
-// Eight K slots beside the four cost 1 - 3 % again.
+// Slots of V^T pairs: three (80 KiB of LDS with the K ring, two work-groups per CU), or two where all work-groups of a launch are
+// resident at once and share the CUs: a deeper ring draws less from the memory there.  Measured on MI355X over 400 shapes (us,
+// queries of one token, 4 heads over 8 unless stated; in parentheses with V^T tiles of 32 keys, half a line each, and tiles behind the context
+// fetched; "same": contexts of one length, the others ragged), two slots / three:
+//   up to 256 work-groups: 32 of 900 24.6 / 23.5 (24.8), 8 of 900 13.1 / 12.8 (14.5), 32 of 176 - / 7.5 (8.2), 30 of 106 7.4 / 6.5 (7.4);
+//   257 .. 512: 8 of 8200 in a cache of 8224 59.5 / 65.6 (66.8), 48 of 1000 34.7 / 36.0 (41.0), 33 of 2707 78.3 / 82.6 (94.1),
+//     40 of 3579 105.6 / 110.3 (122.4), 64 of 900 same 44.2 / 45.5 (44.5), 5 of 6870 34.0 / 33.3 (37.5), 12 of 8200 in 8224 92.0 / 93.5
+//     (94.2), same 105.0 / 101.5 (100.5: the one shape found behind what it was);
+//   more: 81 of 1397 87.2 / 79.3 (89.6), 128 of 1000 same 95.0 / 93.8 (91.4), 33 of 3723 of one head over 16 185.9 / 169.6 (177.8), 189 of
+//     7508 same over 4 547.8 / 490.1 (490.4), 69 of 5195 of 8 heads same 312.7 / 285.5 (301.6), 112 of 151 of 8 heads 19.7 / 19.8 (26.7).
+// Four slots are level with three up to 256 work-groups (the order of the requests again) and leave a CU room for one.
+static bool two_pairs(int64_t wgs) { return wgs > 256 && wgs <= 512; }
 template <int G, bool FUSED>
 static int decode_launch(const AttnArgs& a, const QkvArgs& f, int batch, int max_q_len, void* ws, size_t ws_bytes, hipStream_t stream) {
   const int64_t pairs = (int64_t)batch * a.kv_heads;
   const size_t need = ws ? attention_workspace_bytes(batch, max_q_len, a.q_heads, a.kv_heads, a.max_len) : 0;
   if (need == 0 || ws_bytes < need)
-    return pairs <= 256 ? decode_run<G, FUSED, false, 4, 4>(a, f, SplitArgs{}, batch, 1, stream) : decode_run<G, FUSED, false, 4, 2>(a, f, SplitArgs{}, batch, 1, stream);
+    return two_pairs(pairs) ? decode_run<G, FUSED, false, 2>(a, f, SplitArgs{}, batch, 1, stream) : decode_run<G, FUSED, false, 3>(a, f, SplitArgs{}, batch, 1, stream);
   const SplitArgs sp = split_args(ws, batch, max_q_len, a.q_heads, a.kv_heads, a.max_len);
   const int nz = decode_split(pairs, a.max_len);
-  const int rc = pairs * nz <= 256 ? decode_run<G, FUSED, true, 4, 4>(a, f, sp, batch, nz, stream) : decode_run<G, FUSED, true, 4, 2>(a, f, sp, batch, nz, stream);
+  const int rc = two_pairs(pairs * nz) ? decode_run<G, FUSED, true, 2>(a, f, sp, batch, nz, stream) : decode_run<G, FUSED, true, 3>(a, f, sp, batch, nz, stream);
   if (rc != TBIK_OK) return rc;
   merge_launch<FUSED>(a, sp, batch, stream);
   return hip_code(hipGetLastError());
@@ -1023,28 +1046,73 @@ static int group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_
 //   the same with caches that hold nothing of it, 512 MB written in between: 2 x 196 at 4251 82 / 58, 88, 95 (84), 4 x 128 at 8000
 //     139 / 103, 155, 168 (149), 300 at 2000 of 2 heads 42 / 30, 44, 49 (37), 526 at 3526 93 / 81, 73, 78 (83), 16 x 400 69 / 81, 71, 60 (66).
 //   (A load per wavefront that touches the lines of the unit behind the next costs a warm L2 5 - 25 % and was not kept.)
-template <int G>
-static int group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
-  constexpr int WQ = G >= 4 ? 1 : 4 / G;   // at least four computing wavefronts per work-group
-  constexpr int NLD = G == 8 ? 0 : 4;
-  const int64_t wgs = ((int64_t)max_q_len + 16 * WQ - 1) / (16 * WQ) * a.kv_heads * batch;
-  const bool prompts = (int64_t)max_q_len * 4 > (int64_t)a.max_len * 3;
-#define TBIK_ATTN_GROUP(...) return group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
-  if (split) TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS, NLD);
-  if (chunks_of(a.max_len) == 1) {
-    if constexpr (G != 8) {
-      if (max_q_len > 16 && wgs > 2500) TBIK_ATTN_GROUP(WQ, 2, 2, ONE_CHUNK, 0);
-    }
-    TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK, NLD);
+struct GroupForm {
+  int wq, qb, ns, chunks, nld;   // the template arguments of group_run behind G
+  bool operator==(const GroupForm& o) const { return wq == o.wq && qb == o.qb && ns == o.ns && chunks == o.chunks && nld == o.nld; }
+};
+static GroupForm group_form(int G, bool split, int batch, int max_q_len, int kv_heads, int max_len) {
+  const int WQ = G >= 4 ? 1 : 4 / G;   // at least four computing wavefronts per work-group
+  const int NLD = G == 8 ? 0 : 4;
+  const int64_t wgs = ((int64_t)max_q_len + 16 * WQ - 1) / (16 * WQ) * kv_heads * batch;
+  const bool prompts = (int64_t)max_q_len * 4 > (int64_t)max_len * 3;
+  if (split) return {WQ, 1, 2, SPLIT_CHUNKS, NLD};
+  if (chunks_of(max_len) == 1) {
+    if (G != 8 && max_q_len > 16 && wgs > 2500) return {WQ, 2, 2, ONE_CHUNK, 0};
+    return {WQ, 1, 2, ONE_CHUNK, NLD};
   }
   const int64_t few = G == 8 ? (prompts ? 768 : 448) : prompts ? 1152 : 640;
-  if (max_q_len > 16 && wgs > few) TBIK_ATTN_GROUP(WQ, 2, 2, ALL_CHUNKS, 0);
-  if (wgs <= 256 && (G == 8 ? max_q_len <= 64 : !prompts)) TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS, NLD);
-  if constexpr (NLD > 0) {
-    if (prompts && wgs <= 540) TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, NLD);
-  }
+  if (max_q_len > 16 && wgs > few) return {WQ, 2, 2, ALL_CHUNKS, 0};
+  if (wgs <= 256 && (G == 8 ? max_q_len <= 64 : !prompts)) return {WQ, 1, 4, ALL_CHUNKS, NLD};
+  return {WQ, 1, 2, ALL_CHUNKS, prompts && wgs <= 540 ? NLD : 0};
+}
+template <int G>
+static int group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
+  constexpr int WQ = G >= 4 ? 1 : 4 / G;
+  constexpr int NLD = G == 8 ? 0 : 4;
+  const GroupForm f = group_form(G, split, batch, max_q_len, a.kv_heads, a.max_len);
+#define TBIK_ATTN_GROUP(...) if (f == GroupForm{__VA_ARGS__}) return group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
+  TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS, NLD);
+  TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK, NLD);
+  TBIK_ATTN_GROUP(WQ, 2, 2, ALL_CHUNKS, 0);
+  TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS, NLD);
   TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, 0);
+  if constexpr (G != 8) {
+    TBIK_ATTN_GROUP(WQ, 2, 2, ONE_CHUNK, 0);
+    TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, NLD);
+  }
 #undef TBIK_ATTN_GROUP
+  return TBIK_ERR_UNSUPPORTED;   // (a form that is not built)
+}
+
+// How a call would run (no effect on any result): out[0] kernel, 0 attention_kernel, 1 grouped, 2 decode; out[1] work-groups that
+// share the chunks of a row; out[2] ring slots of 64 keys (1) or of V^T pairs (2); out[3] queries per work-group; out[4] blocks of 16
+// queries per wavefront (1); out[5] wavefronts that load beside the computing ones (1, 2).
+int attention_plan_info(int batch, int max_q_len, int q_heads, int kv_heads, int max_len, size_t ws_bytes, int out[6]) {
+  if (!out || batch <= 0 || max_q_len <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || max_len < 32 || (max_len & 3)) return TBIK_ERR_INVALID;
+  const int G = q_heads / kv_heads;
+  const size_t need = attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len);
+  const bool split = need != 0 && ws_bytes >= need;
+  for (int i = 0; i < 6; i++) out[i] = 0;
+  out[1] = 1;
+  if (!grouped_cache(G, kv_heads, max_len)) {
+    out[3] = 16;
+  } else if ((int64_t)max_q_len * G <= 16) {
+    const int64_t pairs = (int64_t)batch * kv_heads;
+    out[0] = 2;
+    out[1] = split ? decode_split(pairs, max_len) : 1;
+    out[2] = two_pairs(pairs * out[1]) ? 2 : 3;
+    out[3] = 16 / G;
+    out[5] = 4;
+  } else {
+    const GroupForm f = group_form(G, split, batch, max_q_len, kv_heads, max_len);
+    out[0] = 1;
+    out[1] = f.chunks == SPLIT_CHUNKS ? chunks_of(max_len) : 1;
+    out[2] = f.ns;
+    out[3] = 16 * f.wq * f.qb;
+    out[4] = f.qb;
+    out[5] = f.nld;
+  }
+  return TBIK_OK;
 }
 
 int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache, void* out, const int* q_start,

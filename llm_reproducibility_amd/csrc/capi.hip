@@ -26,6 +26,7 @@ int attention_dispatch(const void* q, const void* k_cache, const void* vt_cache,
                        const int* q_len, const int* ctx_len, int batch, int max_q_len, int q_heads, int kv_heads,
                        int head_dim, int max_len, float scale, void* ws, size_t ws_bytes, hipStream_t stream);
 size_t attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len);
+int attention_plan_info(int batch, int max_q_len, int q_heads, int kv_heads, int max_len, size_t ws_bytes, int out[6]);
 int argmax_dispatch(const void* x, int64_t ld, void* out, int64_t rows, int cols, void* history, int64_t history_ld,
                     void* count, void* positions, void* ctx_len, hipStream_t stream);
 int mean_dispatch(const void* x, void* out, int64_t outer, int64_t n, int64_t inner, int dtype_code, hipStream_t stream);
@@ -235,6 +236,10 @@ int bi_attention_bf16(const void* q, const void* k_cache, const void* vt_cache, 
 
 size_t bi_attention_workspace_bytes(int batch, int max_q_len, int q_heads, int kv_heads, int max_len) {
   return tbik::attention_workspace_bytes(batch, max_q_len, q_heads, kv_heads, max_len);
+}
+
+int bi_attention_plan_info(int batch, int max_q_len, int q_heads, int kv_heads, int max_len, size_t workspace_bytes, int* out6) {
+  return tbik::attention_plan_info(batch, max_q_len, q_heads, kv_heads, max_len, workspace_bytes, out6);
 }
 
 int bi_attention_ws_bf16(const void* q, const void* k_cache, const void* vt_cache, void* out, const int32_t* q_start,
