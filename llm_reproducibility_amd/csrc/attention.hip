@@ -262,8 +262,9 @@ __device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * 128 + 
 // wavefront holds one of the G query heads that share the KV head and QB blocks of 16 queries; the keys are brought in 64 at
 // a time (K and V^T, 32 KiB) by direct loads into an LDS ring of NS slots, once for the whole work-group, and every fragment
 // read from there serves the wavefront's QB blocks.  NLD > 0: that many more wavefronts do all the loading (their scalar
-// address arithmetic and the loads are a third of a tile's instructions) and none of the computing.  A row's arithmetic -- the lanes that own it, the MFMA chain, the order of
-// the softmax updates -- is exactly that of attention_kernel above, so the kernels produce the same bits.
+// address arithmetic and the loads are a third of a tile's instructions) and none of the computing.  A row's arithmetic -- the
+// lanes that own it, the MFMA chain, the order of the softmax updates -- is exactly that of attention_kernel above, so the kernels
+// produce the same bits.
 // SPLIT_CHUNKS: a work-group takes one chunk of the keys (blockIdx.z) and leaves its state in the workspace for
 // attention_merge_kernel: a few new tokens against a long cache are a handful of work-groups otherwise.
 // What bounds it: vector issue and matrix pipes together.  8192 tokens of 32 heads on two blocks (503 us, 1.09 PFLOP/s; 599 before):
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1
   constexpr int NL = NLD ? NLD : NW;                    // wavefronts that load
   constexpr int PI = 16 / NL;                           // load instructions per slot, operand and such a wavefront
   constexpr int CHUNK_UNITS = CHUNK_TILES * 32 / UNIT;
-  static_assert((NW == 4 || NW == 8) && CHUNK_UNITS % NS == 0 && NS >= 2, "work-group shape");
+  static_assert((NW == 4 || NW == 8 || NLD == 4) && CHUNK_UNITS % NS == 0 && NS >= 2, "work-group shape");
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int b = blockIdx.y;
   // Work-groups are dealt to the eight XCDs round robin, each with an L2 of its own: with the KV head as the fastest
@@ -308,8 +309,9 @@ __global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1
   if (SPLIT && tile0 >= ntiles) return;  // uniform over the work-group
   const int unit0 = tile0 / 2, nunits = (ntiles + 1) / 2;
 
-  // ---- staging: load instruction n of the sixteen of a slot covers key rows 4n .. 4n+3 / channel rows 8n .. 8n+7 (whole
-  // 128-byte lines of the V^T cache); the wavefronts that load (all of them, or the NLD loaders) deal them out in turn
+  // ---- staging: load instruction n of the sixteen of a slot covers key rows 4n .. 4n+3 / channel rows 8n .. 8n+7, 128 bytes of
+  // each (whole lines of the V^T cache where its length is a multiple of 64); the wavefronts that load (all of them, or the NLD
+  // loaders) deal them out in turn
   // A cache whose length is an odd number of tiles ends in the middle of the last slot: K instructions behind its end fetch
   // the last rows again, and V^T lanes of the second half what those of the first half do (rows that nobody sees).
   const uint8_t* kbase = reinterpret_cast<const uint8_t*>(a.k_cache + ((int64_t)b * a.kv_heads + kvh) * a.max_len * HD);
@@ -1023,28 +1025,42 @@ static int group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_
 }
 
 // The form of the grouped kernel, same bits in all.  Lengths are the device's, so what is known is the number of
-// work-groups, the queries of the longest sequence and the cache length.
+// work-groups, the queries of the longest sequence and the cache length -- its capacity, not the keys in it.
 //   loaders: one block of 16 queries per wavefront and four more wavefronts that load, for launches of about one work-group per CU, which
 //     are a chain of tiles (and up to several rounds where the cache is one chunk: without the merged chunks in registers two such
 //     work-groups share a CU).  Two slots, and four (96 KiB of keys on their way) where keys were cached before: they come
-//     from the memory, and the work-groups that share them ask at the same time.
+//     from the memory, and the work-groups that share them ask at the same time.  Work-groups of one or two heads hold 64 or 32
+//     queries, and 16 in a cache of one chunk while those are few: five or six wavefronts instead of eight.
 //   plain: one block per wavefront, which loads for itself: two or three work-groups share a CU and fill each other's waits.
 //   two blocks: per wavefront, half the fragment reads and half the key traffic per query, for launches that fill the chip in
 //     twice as large pieces.  That takes more work-groups where the longest sequence is as long as the cache: with nothing
 //     cached before it, its work-groups are of all lengths, and few large ones leave the chip with a tail.
-// Work-groups of eight heads have eight wavefronts: no loaders beside them, and two share a CU in a cache of one chunk.
+//   Eight heads: plain only in one chunk (beside it another work-group fits a CU) and where work-groups take a chunk each (12 of 4 tokens
+//     at 4511 keys 55 us, 64 with loaders); else loaders, and two blocks later than the others: a work-group of eight computing wavefronts
+//     has twice the queries in flight already, and short or ragged sequences leave the second block empty.
 // Measured on MI355X, us, loaders with two / with four slots, plain, two blocks (parentheses: the kernel with register staging and
-// 16 queries per fragment read that these replace):
+// 16 queries per fragment read that these replace); the caches are as long as the longest context unless stated:
 //   4 heads per KV head: 8192 tokens 724 / 769, 629, 503 (599), prompts of 4096, 3136 and 2176 358 / 396, 321, 256 (323), 1900 tokens
 //     at 9000 keys 346 / 365, 297, 256 (299), 4 x 500 at 3000 130 / 137, 116, 100 (118), 32 x 64 at 4000 288 / 217, 195, 152 (182),
 //     2 prompts of 1020 31 / 37, 29.3, 37 (41), 526 at 3526 71 / 75, 58, 73 (75), 1040 tokens 19.3 / 22.8, 21.4, 27.7 (26.9),
 //     2 x 196 at 4251 50 / 51, 61, 88 (76), 4 x 128 at 8000 93 / 95, 113, 160 (138), 8 x 60 at 8000 118 / 97, 130, 161 (146),
 //     24 x 16 at 4000 94 / 73, 94, 99 (80), one chunk: 16 x 400 45 / 66, 52, 47 (50), 32 x 512 144, -, 127;
-//   8 heads, plain and two blocks: 4096 tokens 159, 138 (175), 16 prompts of 400 43, 52 (48), 32 x 64 at 4000 170, 138 (191);
-//   2 heads: 8 x 400 at 4000 172 / 179, 147, 124 (184), 16 x 20 at 8000 151 / 102, 154, 165 (133), 300 at 2000 25.7 / 26.3, 30.0, 43 (34);
-//   1 head: 4096 tokens 104 / 107, 91, 95 (133), 1040 tokens 15.1 / 16.0, 18.4, 24.5 (21.1);
-//   the same with caches that hold nothing of it, 512 MB written in between: 2 x 196 at 4251 82 / 58, 88, 95 (84), 4 x 128 at 8000
+//   the same in longer caches, where the rule takes them for cached keys: 2 prompts of 1020 in 8192 33.7 / 39.1, 31.8, 39.0 (42.7: two
+//     blocks), 2000 tokens in 8192 56 / 61, 49.7, 50.7 (58.9: two blocks), 1040 tokens in 8192 -, 22.9 (28.2: plain), 16 x 400 in 4096
+//     58 / 71, 56, 50.6 (53.4: two blocks);
+//   8 heads: 4096 tokens 154 / 161, 165, 142 (185), 16 prompts of 400 in one chunk 49 / 54, 46, 55 (49), 32 x 64 at 4000 169 / 167, 176, 154
+//     (208), 2 prompts of 1000 in 4096 28.4 / 28.9, 30.3, 38.6 (34.8), 36 x 37 at 3808 301 / 294, 309, 359 (311), 3 x 33 at 4649 46 / 45, 45,
+//     57 (56), 38 x 10 at 6645 137 / 122, 139, 193 (159), 12 x 290 in 1216 51 / 53, 52, 55 (49), 4 x 4 5.5 / 5.6, 5.8, 6.3 (5.5);
+//   2 heads: 8 x 400 at 4000 172 / 179, 147, 124 (184), 16 x 20 at 8000 151 / 102, 154, 165 (133), 300 at 2000 25.7 / 26.3, 30.0, 43 (34),
+//     with 16 queries per work-group against 32: 4 x 38 4.9, 5.4 (5.1), 35 x 37 over 4 6.1, 7.7 (6.2), 61 x 19 over 4 7.1, 5.3 (7.6);
+//   1 head: 4096 tokens 104 / 107, 91, 95 (133), 1040 tokens 15.1 / 16.0, 18.4, 24.5 (21.1), 16 queries per work-group against 64: 2 x 52
+//     4.8, 5.4 (5.0);
+//   with caches that hold nothing of it, 512 MB written in between: 2 x 196 at 4251 82 / 58, 88, 95 (84), 4 x 128 at 8000
 //     139 / 103, 155, 168 (149), 300 at 2000 of 2 heads 42 / 30, 44, 49 (37), 526 at 3526 93 / 81, 73, 78 (83), 16 x 400 69 / 81, 71, 60 (66).
+//   Over 919 random shapes (1 .. 64 sequences, 1 .. 8 heads over 1 .. 16, up to 4096 new tokens at up to 12,000 keys, caches of up to four times
+//   that) the choice is 10 % ahead of the replaced kernel on average, and more than 5 % behind it (26 % at most) in one of thirty: batches of
+//   prompts of up to a few hundred tokens in caches of several chunks, where the registers of the merged chunks and slots of 64 keys keep
+//   a third work-group from the CU.
 //   (A load per wavefront that touches the lines of the unit behind the next costs a warm L2 5 - 25 % and was not kept.)
 struct GroupForm {
   int wq, qb, ns, chunks, nld;   // the template arguments of group_run behind G
@@ -1052,33 +1068,38 @@ struct GroupForm {
 };
 static GroupForm group_form(int G, bool split, int batch, int max_q_len, int kv_heads, int max_len) {
   const int WQ = G >= 4 ? 1 : 4 / G;   // at least four computing wavefronts per work-group
-  const int NLD = G == 8 ? 0 : 4;
+  const int64_t blocks = ((int64_t)max_q_len + 15) / 16 * kv_heads * batch;
   const int64_t wgs = ((int64_t)max_q_len + 16 * WQ - 1) / (16 * WQ) * kv_heads * batch;
   const bool prompts = (int64_t)max_q_len * 4 > (int64_t)max_len * 3;
-  if (split) return {WQ, 1, 2, SPLIT_CHUNKS, NLD};
+  if (split) return {WQ, 1, 2, SPLIT_CHUNKS, G == 8 ? 0 : 4};
   if (chunks_of(max_len) == 1) {
-    if (G != 8 && max_q_len > 16 && wgs > 2500) return {WQ, 2, 2, ONE_CHUNK, 0};
-    return {WQ, 1, 2, ONE_CHUNK, NLD};
+    if (blocks <= 256 || (wgs > 256 && blocks <= 512 && G < 4)) return {1, 1, 2, ONE_CHUNK, 4};
+    if (G == 8) return {1, 1, 2, ONE_CHUNK, 0};
+    if (max_q_len > 16 && wgs > 2500) return {WQ, 2, 2, ONE_CHUNK, 0};
+    return {WQ, 1, 2, ONE_CHUNK, 4};
   }
-  const int64_t few = G == 8 ? (prompts ? 768 : 448) : prompts ? 1152 : 640;
-  if (max_q_len > 16 && wgs > few) return {WQ, 2, 2, ALL_CHUNKS, 0};
-  if (wgs <= 256 && (G == 8 ? max_q_len <= 64 : !prompts)) return {WQ, 1, 4, ALL_CHUNKS, NLD};
-  return {WQ, 1, 2, ALL_CHUNKS, prompts && wgs <= 540 ? NLD : 0};
+  const bool two_blocks = G != 8 ? wgs > (prompts ? 1152 : 640)
+                                 : wgs > 4500 || (max_q_len > 1200 && wgs > 1500) || (wgs > 850 && wgs > (int64_t)500 * batch);
+  if (max_q_len > 16 && two_blocks) return {WQ, 2, 2, ALL_CHUNKS, 0};
+  if (wgs <= 256 && (G == 8 ? max_q_len <= 64 && max_len >= 2048 : !prompts)) return {WQ, 1, 4, ALL_CHUNKS, 4};
+  return {WQ, 1, 2, ALL_CHUNKS, G == 8 || (prompts && wgs <= 540) ? 4 : 0};
 }
 template <int G>
 static int group_launch(const AttnArgs& a, const SplitArgs& sp, bool split, int batch, int max_q_len, hipStream_t stream) {
   constexpr int WQ = G >= 4 ? 1 : 4 / G;
-  constexpr int NLD = G == 8 ? 0 : 4;
   const GroupForm f = group_form(G, split, batch, max_q_len, a.kv_heads, a.max_len);
 #define TBIK_ATTN_GROUP(...) if (f == GroupForm{__VA_ARGS__}) return group_run<G, __VA_ARGS__>(a, sp, batch, max_q_len, stream)
-  TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS, NLD);
-  TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK, NLD);
+  TBIK_ATTN_GROUP(WQ, 1, 2, SPLIT_CHUNKS, G == 8 ? 0 : 4);
+  TBIK_ATTN_GROUP(1, 1, 2, ONE_CHUNK, 4);
+  TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, 4);
+  TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS, 4);
   TBIK_ATTN_GROUP(WQ, 2, 2, ALL_CHUNKS, 0);
-  TBIK_ATTN_GROUP(WQ, 1, 4, ALL_CHUNKS, NLD);
-  TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, 0);
-  if constexpr (G != 8) {
+  if constexpr (G == 8) {
+    TBIK_ATTN_GROUP(1, 1, 2, ONE_CHUNK, 0);
+  } else {
+    if constexpr (WQ > 1) TBIK_ATTN_GROUP(WQ, 1, 2, ONE_CHUNK, 4);
     TBIK_ATTN_GROUP(WQ, 2, 2, ONE_CHUNK, 0);
-    TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, NLD);
+    TBIK_ATTN_GROUP(WQ, 1, 2, ALL_CHUNKS, 0);
   }
 #undef TBIK_ATTN_GROUP
   return TBIK_ERR_UNSUPPORTED;   // (a form that is not built)
