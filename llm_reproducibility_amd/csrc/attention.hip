@@ -273,9 +273,10 @@ __device__ __forceinline__ uint32_t v_fragment(int j, int c) { return j * 128 + 
 // queries made it the LDS and the L2 (a 64-byte half of a V^T line per load and tile: 8.4 TB/s) instead; in work-groups of
 // 64 queries, which halve the key traffic once more, it takes the same time (532), and so does forming a tile's scores ahead.
 // Launches that leave CUs short of work-groups are a chain of tiles, 0.53 us each and 0.39 with loaders beside them.
-// (A wavefront's vector instructions do not run behind its own MFMAs: alone on a SIMD, one MFMA and three FMAs in turn take 32
-// cycles, the sum; two wavefronts of that hide a sixth of it.  Scores a tile ahead, and two blocks' exponentials between each
-// other's MFMAs, were therefore level.)
+// (Two vector instructions per MFMA issue behind it, each further one costs its 1.8 ns: on one CU 7.15 / 7.67 / 9.31 / 11.31 ns per MFMA
+// with 0 / 2 / 3 / 4 FMAs on two wavefronts per SIMD, 7.86 / 9.21 / 10.84 / 12.69 on one; on all 256 the clock pays for them, 8.10 /
+// 10.15 / 11.92 / 14.26.  A tile has three and half an exponential, so work moves the time only where it goes away: scores a tile
+// ahead, and two blocks' exponentials between each other's MFMAs, were level.)
 // ------------------------------------------------------------------------------------------------
 // chunks: the cache has a single one / a work-group walks them all / a work-group takes one
 enum { ONE_CHUNK, ALL_CHUNKS, SPLIT_CHUNKS };
@@ -461,8 +462,9 @@ __global__ __launch_bounds__(64 * (G * WQ + NLD), QB == 2 || G * WQ == 8 ? 2 : 1
 #pragma unroll
     for (int t = 0; t < 8; t++) o[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pf, o[q][t], 0, 0, 0);
   };
-  // eight MFMAs of one block between the exponentials of another, so that neither kind comes in one long run (level, within
-  // 2 %, with the order the compiler gives)
+  // eight MFMAs between the exponentials, so that neither kind comes in one long run: 1 - 3 % where a CU has one work-group (2 prompts of
+  // 1020 tokens 31.3 -> 30.8 us, 1040 tokens of one head 16.6 -> 16.1, 526 at 3526 60.8 -> 59.9) or few rounds (prompts of 4096, 3136
+  // and 2176 276 -> 271), level on the launches that fill the chip many times over
   auto interleave = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 8; i++) {
