@@ -68,8 +68,8 @@ int tbik_tree_params(int K, int leaf_k, int* T, int* flb, int* level_k);
  *   C: element (m,n) at C[m*ldc + n]
  *   workspace: at least tbik_gemm_workspace_bytes(M,N,K,leaf_k) bytes, 16-byte aligned (may be NULL when 0); fewer return
  *      TBIK_ERR_WORKSPACE before anything is launched.  A row-major B alone has a second way: with fewer bytes than its
- *      size above the 128x128 tiles give way to the 64-row tiles, which need less or none (and take longer), and only what
- *      does not suffice for those either is refused.
+ *      size above, or at an address that is not 16-byte aligned, the tiles of 128 rows give way to the 64-row tiles, which need less
+ *      or none (and take longer), and only what does not suffice for those either is refused.
  * Replaces: matmul_tp_persistent + matmul_kernel_tp_persistent,
  *           src/tbik/tree_based_matmul.py:190-277 and :50-187.
  */

@@ -1060,7 +1060,7 @@ static int group_run(const AttnArgs& a, const SplitArgs& sp, int batch, int max_
 //   with caches that hold nothing of it, 512 MB written in between: 2 x 196 at 4251 82 / 58, 88, 95 (84), 4 x 128 at 8000
 //     139 / 103, 155, 168 (149), 300 at 2000 of 2 heads 42 / 30, 44, 49 (37), 526 at 3526 93 / 81, 73, 78 (83), 16 x 400 69 / 81, 71, 60 (66).
 //   Over 919 random shapes (1 .. 64 sequences, 1 .. 8 heads over 1 .. 16, up to 4096 new tokens at up to 12,000 keys, caches of up to four times
-//   that) the choice is 10 % ahead of the replaced kernel on average, and more than 5 % behind it (26 % at most) in one of thirty: batches of
+//   that) the choice is 10 % ahead of the replaced kernel on average, and more than 5 % behind it (26 % at most) in one of 25: batches of
 //   prompts of up to a few hundred tokens in caches of several chunks, where the registers of the merged chunks and slots of 64 keys keep
 //   a third work-group from the CU.
 //   (A load per wavefront that touches the lines of the unit behind the next costs a warm L2 5 - 25 % and was not kept.)
